@@ -1,8 +1,9 @@
 // forage.hip -- collective-foraging agent step (Agent.update for every agent
 // in id order) in float64, plus the Agent.projection_field probe.
 //
-// One workgroup per replica; the replica's agents live in LDS and are
-// updated in place in id order (Group.update, abm/simulation/sims.py:861).
+// One workgroup per replica; the replica's agents live in LDS.  Without
+// visual exclusion all agents are updated at once (forage_update_kernel); with
+// it one after another, in id order (Group.update, abm/simulation/sims.py:861).
 // Per focal agent k:
 //   1. lanes over the other agents: cue class (agent.py:396-419) and the
 //      projection record of each obstacle (agent.py:501-556): closed angle with
@@ -300,10 +301,6 @@ __device__ inline int cue_class(const FGSmem& S, const FGRep& P, int j, int f, d
     return c;
 }
 
-// Whether the raster needs obstacle j's record: the cues, and with visual
-// exclusion every obstacle in range (agent.py:415-419).
-__device__ inline bool needs_record(int c, bool excl) { return c == kSocial || (excl && c != kNone); }
-
 // Per-replica float32 constants of the guarded record.
 struct FastRec {
     float inv_step;   // bins of linspace(-pi, pi, R) per radian
@@ -395,12 +392,12 @@ __device__ inline Rec record_of(const FGSmem& S, int j, int c, int N, const Foca
     return record_at(S.x[j], S.y[j], c, c * N + j, f, R, step, fov0, fov1, FR, need_dist);
 }
 
-// Classes of the agents j != skip for focal agent f into S.cls; those whose
-// records the raster needs are appended to lst (in any order: records are
+// Classes of the agents j != skip for focal agent f into S.cls; those in
+// range (agent.py:415-419) are appended to lst (in any order: records are
 // kept per agent and ranked by (distance, list position)).  Thread t0 of
 // `stride` threads, both multiples of 64 apart per wave.
-__device__ void classify(const FGSmem& S, const FGRep& P, int N, int f, int skip1, int skip2, bool excl,
-                         int* cls, int* lst, int* lst_n, int t0, int stride) {
+__device__ void classify(const FGSmem& S, const FGRep& P, int N, int f, int skip1, int skip2, int* cls,
+                         int* lst, int* lst_n, int t0, int stride) {
     const double cfx = S.x[f] + S.rad[f], cfy = S.y[f] + S.rad[f];
     const int pid_f = S.pid[f];
     const int lane = t0 & 63;
@@ -408,12 +405,9 @@ __device__ void classify(const FGSmem& S, const FGRep& P, int N, int f, int skip
         const int j = base + lane;
         bool need = false;
         if (j < N && j != skip1 && j != skip2) {
-            // without exclusion only a listed obstacle's class is read, and
-            // only an exploiting agent (overriding mode exploit) is listed
-            int c = kNone;
-            if (excl || S.over[j] == ABM_MODE_EXPLOIT) c = cue_class(S, P, j, f, cfx, cfy, pid_f);
+            const int c = cue_class(S, P, j, f, cfx, cfy, pid_f);
             cls[j] = c;
-            need = needs_record(c, excl);
+            need = c != kNone;
         }
         const uint64_t m = __ballot(need);
         if (m) {
@@ -426,11 +420,10 @@ __device__ void classify(const FGSmem& S, const FGRep& P, int N, int f, int skip
 }
 
 // make_focal with one sincos for the heading (the same values as cos, sin).
-__device__ inline Focal focal_of(const FGSmem& S, int k) {
+__device__ inline Focal focal_at(double px, double py, double th, double radius) {
 #pragma clang fp contract(off)
-    const double px = S.x[k], py = S.y[k], radius = S.rad[k];
     double sn, cs;
-    sincos(S.th[k], &sn, &cs);
+    sincos(th, &sn, &cs);
     Focal f;
     f.px = px; f.py = py; f.radius = radius;
     f.cx = px + radius;
@@ -443,6 +436,7 @@ __device__ inline Focal focal_of(const FGSmem& S, int k) {
     f.u1y = v1y / n1;
     return f;
 }
+__device__ inline Focal focal_of(const FGSmem& S, int k) { return focal_at(S.x[k], S.y[k], S.th[k], S.rad[k]); }
 
 // The heading agent f takes after a random-walk turn drawn from uniform
 // d + c (c = 0, 1) or after no turn (c = 2), with its sin and cos, into
@@ -507,45 +501,43 @@ __device__ inline uint32_t word_range_mask(int w, int a, int b) {
 // Visual exclusion (agent.py:421-445) over the listed records, then their
 // raster (agent.py:569-590) into the bit-packed raw field S.V (uint32
 // words, bit r = V[r]).  Every thread; ends synchronised.
-__device__ void raster_list(const FGSmem& S, int R, bool excl, const int* lst, int n0, int extra) {
+__device__ void raster_list(const FGSmem& S, int R, const int* lst, int n0, int extra) {
     const int tid = threadIdx.x, nthr = blockDim.x;
     // the listed records, and one more (extra >= 0) kept outside the list
     const int n = n0 + (extra >= 0 ? 1 : 0);
     auto item = [&](int q) { return q < n0 ? lst[q] : extra; };
-    if (excl) {
-        // rank = position in the stable ascending sort by distance
-        for (int q = tid; q < n; q += nthr) {
-            const int j = item(q);
-            const Rec rf = S.rec[j];
-            if (!rf.valid) continue;
-            int rank = 0;
-            for (int p = 0; p < n; ++p) {
-                const Rec ri = S.rec[item(p)];
-                if (ri.valid && (ri.dist < rf.dist || (ri.dist == rf.dist && ri.order < rf.order))) ++rank;
-            }
-            S.sorted[rank] = j;
+    // rank = position in the stable ascending sort by distance
+    for (int q = tid; q < n; q += nthr) {
+        const int j = item(q);
+        const Rec rf = S.rec[j];
+        if (!rf.valid) continue;
+        int rank = 0;
+        for (int p = 0; p < n; ++p) {
+            const Rec ri = S.rec[item(p)];
+            if (ri.valid && (ri.dist < rf.dist || (ri.dist == rf.dist && ri.order < rf.order))) ++rank;
         }
-        __syncthreads();
-        for (int q = tid; q < n; q += nthr) {
-            const int j = item(q);
-            Rec rf = S.rec[j];
-            if (!rf.valid) continue;
-            // walk the nearer records in rank order; rank 0 keeps its interval
-            for (int p = 0; p < n; ++p) {
-                const int i = S.sorted[p];
-                if (i == j) break;
-                const Rec ri = S.rec[i];
-                if (ri.dist < rf.dist) {
-                    if (rf.sx <= ri.start && ri.start <= rf.ex) rf.ex = ri.start;
-                    if (rf.sx <= ri.end && ri.end <= rf.ex) rf.sx = ri.end;
-                    if (ri.start <= rf.sx && ri.end >= rf.ex) { rf.sx = 0; rf.ex = 0; }
-                }
-            }
-            S.rec[j].sx = rf.sx;
-            S.rec[j].ex = rf.ex;
-        }
-        __syncthreads();
+        S.sorted[rank] = j;
     }
+    __syncthreads();
+    for (int q = tid; q < n; q += nthr) {
+        const int j = item(q);
+        Rec rf = S.rec[j];
+        if (!rf.valid) continue;
+        // walk the nearer records in rank order; rank 0 keeps its interval
+        for (int p = 0; p < n; ++p) {
+            const int i = S.sorted[p];
+            if (i == j) break;
+            const Rec ri = S.rec[i];
+            if (ri.dist < rf.dist) {
+                if (rf.sx <= ri.start && ri.start <= rf.ex) rf.ex = ri.start;
+                if (rf.sx <= ri.end && ri.end <= rf.ex) rf.sx = ri.end;
+                if (ri.start <= rf.sx && ri.end >= rf.ex) { rf.sx = 0; rf.ex = 0; }
+            }
+        }
+        S.rec[j].sx = rf.sx;
+        S.rec[j].ex = rf.ex;
+    }
+    __syncthreads();
     uint32_t* Vb = reinterpret_cast<uint32_t*>(S.V);
     for (int q = tid; q < n; q += nthr) {
         const Rec rc = S.rec[item(q)];
@@ -597,65 +589,6 @@ __device__ inline uint32_t interval_word(int w, int s, int e, int R) {
     }
     py_slice(s, e, R, &lo, &hi);
     return bits | word_slice_mask(w, lo, hi);
-}
-
-// Raster without visual exclusion, by one wave: raw-field word w of the
-// live social records lst[0..n).  Lane l loads records l, l + 64, ...; each
-// live interval reaches every lane by readlane, so there is no atomic.
-__device__ inline uint32_t list_word(const FGSmem& S, int R, const int* lst, int n, int w) {
-    const int lane = threadIdx.x & 63;
-    uint32_t bits = 0u;
-    for (int base = 0; base < n; base += 64) {
-        const int q = base + lane;
-        int sx = 0, ex = 0;
-        bool live = false;
-        if (q < n) {
-            const Rec& rc = S.rec[lst[q]];
-            live = rc.valid && rc.social;
-            sx = rc.sx;
-            ex = rc.ex;
-        }
-        uint64_t m = __ballot(live);
-        while (m) {
-            const int l = __builtin_ctzll(m);
-            m &= m - 1;
-            bits |= interval_word(w, __builtin_amdgcn_readlane(sx, l), __builtin_amdgcn_readlane(ex, l), R);
-        }
-    }
-    return bits;
-}
-
-// Counts of the field without visual exclusion, by wave 0: the words the
-// listed records made (S.V), with the interval [s, e] of the record kept
-// outside the list ORed in when live (wave-uniform): the rays set on the
-// kept raw range [ta, tb] and those in its left half [la, tb], to every lane.
-// m_tot / m_left: the lane's word masks of the two ranges when W <= 64.
-__device__ void count_wave(const FGSmem& S, int R, int W, bool live, int s, int e, int ta, int tb, int la,
-                           uint32_t m_tot, uint32_t m_left, int* n_set, int* n_left) {
-    const int lane = threadIdx.x & 63;
-    const uint32_t* Vb = reinterpret_cast<const uint32_t*>(S.V);
-    int tot = 0, left = 0;
-    if (W <= 64) {   // one word per lane
-        uint32_t bits = lane < W ? Vb[lane] : 0u;
-        if (live) bits |= interval_word(lane, s, e, R);
-        tot = __popc(bits & m_tot);
-        left = __popc(bits & m_left);
-    } else {
-        for (int w = lane; w < W; w += 64) {
-            uint32_t bits = Vb[w];
-            if (live) bits |= interval_word(w, s, e, R);
-            tot += __popc(bits & word_range_mask(w, ta, tb));
-            left += __popc(bits & word_range_mask(w, la, tb));
-        }
-    }
-    if (R < 65536) {   // one sum of both counts, each below 2^16
-        const int both = wave_sum(tot << 16 | left);
-        *n_set = both >> 16;
-        *n_left = both & 0xffff;
-    } else {
-        *n_set = wave_sum(tot);
-        *n_left = wave_sum(left);
-    }
 }
 
 // The returned field of agent k: counts for mean() and the left/right
@@ -763,10 +696,10 @@ __device__ inline double words_to_double(uint32_t w0, uint32_t w1) {
 // 32-bit outputs (words, two per draw, starting after the words the resource
 // loop consumed: u_used[b] on entry).  With status, only replicas marked
 // kWorldReady are updated, and they are marked ABM_WORLD_DONE.  FIELDS false:
-// a step that writes no fields (bits_out is ignored); EXCL false: no replica
-// of the launch has visual exclusion.  Either takes the other paths' tests
-// out of the agent loop.
-template <bool FIELDS, bool EXCL>
+// a step that writes no fields (bits_out is ignored).  The replicas of this
+// kernel have visual exclusion: every agent in range, as it stands in its
+// turn, occludes, so the agents are updated one after another.
+template <bool FIELDS>
 __global__ void __launch_bounds__(512)
 forage_step_kernel(const FGRep* __restrict__ reps, abm_forage_state st,
                    const double* __restrict__ uniforms, const uint32_t* __restrict__ words,
@@ -847,32 +780,21 @@ forage_step_kernel(const FGRep* __restrict__ reps, abm_forage_state st,
         }
     }
     int draws = 0;   // meaningful in thread 0
-    int xlive = 0, xs = 0, xe = 0;   // thread 0: agent k's social interval for agent k+1
     const int nl = R / 2;
-    const bool excl = EXCL && P.visual_exclusion != 0;
     const FastRec FR = fast_rec_const(R, P.step, P.fov0, P.fov1);
-    // without exclusion and field output, wave 0 rasters and counts alone
-    const bool wave_raster = !excl && !bits_out;
-    const int ta = R - 1 - P.keep_hi, tb = R - 1 - P.keep_lo, la = max(R - nl, ta);
-    // wave 0's lane masks of the kept range and its left half (one word per lane)
-    const int wl0 = tid & 63;
-    const uint32_t m_tot = wl0 < P.words ? word_range_mask(wl0, ta, tb) : 0u;
-    const uint32_t m_left = wl0 < P.words ? word_range_mask(wl0, la, tb) : 0u;
     int* const lst[2] = {S.lst, S.lst + maxN};
     int* const clsb[2] = {S.cls, S.cls2};
     int* const lst_n = S.cnt + 4;
     // Pipeline over the agents in id order.  Agent m's field depends on the
     // agents moved before it only through their records.  So while thread 0
     // moves agent k and then adds agent k's class (and record) for agent
-    // k+1, wave 1 builds agent k+1's records of every other obstacle
-    // (without exclusion, also their raster), and the other waves classify
-    // agent k+2's obstacles but k and k+1; one of them then builds agent
-    // k+1's speculative headings and the next agent k+2's focal geometry
-    // (agents move only in their own turn, so it is the start-of-step
-    // pose).  After one barrier come exclusion, raster and
-    // counts of agent k+1 (without exclusion: agent k's interval ORed in and
-    // the counts, by wave 0 alone), during which wave 2 adds agent k's class
-    // for agent k+2.
+    // k+1, wave 1 builds agent k+1's records of every other obstacle, and
+    // the other waves classify agent k+2's obstacles but k and k+1; one of
+    // them then builds agent k+1's speculative headings and the next agent
+    // k+2's focal geometry (agents move only in their own turn, so it is the
+    // start-of-step pose).  After one barrier come exclusion, raster and
+    // counts of agent k+1, during which wave 2 adds agent k's class for
+    // agent k+2.
     // Classes, lists, focal geometry and counts alternate between two
     // buffers by parity of the focal agent.
     const int rbase = 64, cbase = 128, cstride = nthr - 128;   // blockDim 256 or 512
@@ -891,26 +813,24 @@ forage_step_kernel(const FGRep* __restrict__ reps, abm_forage_state st,
     if (tid == 0) S.spec[24] = 0.0;    // uniforms drawn before agent 0
     if (tid == 0) S.focal[0] = focal_of(S, 0);
     if (tid == cbase && N > 1) S.focal[1] = focal_of(S, 1);
-    classify(S, P, N, 0, -1, -1, excl, clsb[0], lst[0], &lst_n[0], tid, nthr);
-    if (N > 1) classify(S, P, N, 1, 0, -1, excl, clsb[1], lst[1], &lst_n[1], tid, nthr);
+    classify(S, P, N, 0, -1, -1, clsb[0], lst[0], &lst_n[0], tid, nthr);
+    if (N > 1) classify(S, P, N, 1, 0, -1, clsb[1], lst[1], &lst_n[1], tid, nthr);
     __syncthreads();
     for (int q = tid; q < lst_n[0]; q += nthr) {
         const int j = lst[0][q];
-        S.rec[j] = record_of(S, j, clsb[0][j], N, S.focal[0], R, P.step, P.fov0, P.fov1, FR, excl);
+        S.rec[j] = record_of(S, j, clsb[0][j], N, S.focal[0], R, P.step, P.fov0, P.fov1, FR, true);
     }
     __syncthreads();
-    raster_list(S, R, excl, lst[0], lst_n[0], -1);
+    raster_list(S, R, lst[0], lst_n[0], -1);
     if (tid == 0) lst_n[0] = 0;   // rebuilt for agent 2
     count_field(S, P, R, S.cnt, bits_out, 0);
     __syncthreads();
 
-    // wave 0 carries the chain of moves: first issue on its SIMD.  It holds
-    // the focal agent's counts in registers (from LDS after count_field).
+    // wave 0 carries the chain of moves: first issue on its SIMD
     if (tid < 64) __builtin_amdgcn_s_setprio(3);
-    int n_set = S.cnt[0], n_left = S.cnt[1];
     for (int k = 0; k < N; ++k) {
         const int f1 = k + 1, par = f1 & 1, f2 = k + 2, par2 = par ^ 1;
-        if (!wave_raster && k > 0) { n_set = S.cnt[2 * (k & 1)]; n_left = S.cnt[2 * (k & 1) + 1]; }
+        const int n_set = S.cnt[2 * (k & 1)], n_left = S.cnt[2 * (k & 1) + 1];
         // ---- decision and motion (agent.py:168-283)
         if (tid == 0) {
             // every LDS operand first, in one batch: the replica's constants
@@ -994,71 +914,26 @@ forage_step_kernel(const FGRep* __restrict__ reps, abm_forage_state st,
         }
         // ---- thread 0, after the move: agent k's class and record for agent k+1
         if (tid == 0 && f1 < N) {
-            int extra = -1;
-            xlive = 0;
-            // without exclusion only an exploiting agent k (overriding mode
-            // exploit) can be a cue for agent k+1: skip the distance otherwise
-            int c = kNone;
-            if (excl || S.over[k] == ABM_MODE_EXPLOIT) {
-                const double cfx = S.x[f1] + S.rad[f1], cfy = S.y[f1] + S.rad[f1];
-                c = cue_class(S, P, k, f1, cfx, cfy, S.pid[f1]);
-            }
-            if (needs_record(c, excl)) {
-                const Rec rk = record_of(S, k, c, N, S.focal[par], R, P.step, P.fov0, P.fov1, FR, excl);
-                S.rec[k] = rk;
-                extra = k;
-                xlive = rk.valid && rk.social;
-                xs = rk.sx;
-                xe = rk.ex;
-            }
-            S.cnt[6] = extra;
+            const double cfx = S.x[f1] + S.rad[f1], cfy = S.y[f1] + S.rad[f1];
+            const int c = cue_class(S, P, k, f1, cfx, cfy, S.pid[f1]);
+            if (c != kNone) S.rec[k] = record_of(S, k, c, N, S.focal[par], R, P.step, P.fov0, P.fov1, FR, true);
+            S.cnt[6] = c != kNone ? k : -1;
             S.cnt[2 * par] = 0; S.cnt[2 * par + 1] = 0;   // agent k+1's counts (last read by k-1)
         }
         // ---- wave 1: agent k+1's records but agent k's
         if (f1 < N && tid >= rbase && tid < cbase) {
             uint32_t* Vb = reinterpret_cast<uint32_t*>(S.V);
-            if (!wave_raster)
-                for (int w = tid - rbase; w < P.words; w += 64) Vb[w] = 0u;
+            for (int w = tid - rbase; w < P.words; w += 64) Vb[w] = 0u;
             const Focal f = S.focal[par];
-            const int n = lst_n[par], wl = tid - rbase;
-            if (wave_raster && n <= 64 && P.words <= 64) {
-                // one record and one field word per lane: the live intervals
-                // go from registers to every lane by readlane (the records
-                // are not needed after the raster)
-                int sx = 0, ex = 0;
-                bool live = false;
-                if (wl < n) {
-                    const int j = lst[par][wl];
-                    const Rec rc = record_of(S, j, clsb[par][j], N, f, R, P.step, P.fov0, P.fov1, FR, excl);
-                    live = rc.valid && rc.social;
-                    sx = rc.sx;
-                    ex = rc.ex;
-                }
-                uint64_t m = __ballot(live);
-                uint32_t bits = 0u;
-                while (m) {
-                    const int l = __builtin_ctzll(m);
-                    m &= m - 1;
-                    bits |= interval_word(wl, __builtin_amdgcn_readlane(sx, l), __builtin_amdgcn_readlane(ex, l), R);
-                }
-                if (wl < P.words) Vb[wl] = bits;
-            } else {
-                for (int q = wl; q < n; q += 64) {
-                    const int j = lst[par][q];
-                    S.rec[j] = record_of(S, j, clsb[par][j], N, f, R, P.step, P.fov0, P.fov1, FR, excl);
-                }
-            }
-            if (wave_raster && !(n <= 64 && P.words <= 64)) {   // the listed records' raster; agent k's comes in phase 2
-                fg_wave_sync();
-                for (int w = wl; w - wl < P.words; w += 64) {
-                    const uint32_t bits = list_word(S, R, lst[par], lst_n[par], w);
-                    if (w < P.words) Vb[w] = bits;
-                }
+            const int n = lst_n[par];
+            for (int q = tid - rbase; q < n; q += 64) {
+                const int j = lst[par][q];
+                S.rec[j] = record_of(S, j, clsb[par][j], N, f, R, P.step, P.fov0, P.fov1, FR, true);
             }
         }
         // ---- waves 2 to 7: agent k+2's classes but agent k's and k+1's
         if (f2 < N && tid >= cbase)
-            classify(S, P, N, f2, k, f1, excl, clsb[par2], lst[par2], &lst_n[par2], tid - cbase, cstride);
+            classify(S, P, N, f2, k, f1, clsb[par2], lst[par2], &lst_n[par2], tid - cbase, cstride);
         // ---- one classifying wave, then: agent k+1's speculative headings,
         // from the uniforms drawn before agent k
         if (f1 < N && tid >= spec_tid && tid < spec_tid + 3)
@@ -1071,29 +946,18 @@ forage_step_kernel(const FGRep* __restrict__ reps, abm_forage_state st,
         if (f1 >= N) break;
         // ---- exclusion, raster and counts of agent k+1; meanwhile wave 2
         // adds agent k's class for agent k+2
-        if (wave_raster) {   // agent k's interval from thread 0's registers
-            if (tid < 64)
-                count_wave(S, R, P.words, __builtin_amdgcn_readlane(xlive, 0) != 0, __builtin_amdgcn_readlane(xs, 0),
-                           __builtin_amdgcn_readlane(xe, 0), ta, tb, la, m_tot, m_left, &n_set, &n_left);
-        } else {
-            raster_list(S, R, excl, lst[par], lst_n[par], S.cnt[6]);
-        }
+        raster_list(S, R, lst[par], lst_n[par], S.cnt[6]);
         if (tid == 0) lst_n[par] = 0;   // rebuilt for agent k+3
         if (tid == cbase && f2 < N) {   // agent k's class for agent k+2; its record comes with the others
-            // without exclusion only a listed obstacle's class is read, and
-            // only an exploiting agent k can be listed: skip the distance otherwise
-            int c2 = kNone;
-            if (excl || S.over[k] == ABM_MODE_EXPLOIT) {
-                const double gx = S.x[f2] + S.rad[f2], gy = S.y[f2] + S.rad[f2];
-                c2 = cue_class(S, P, k, f2, gx, gy, S.pid[f2]);
-            }
+            const double gx = S.x[f2] + S.rad[f2], gy = S.y[f2] + S.rad[f2];
+            const int c2 = cue_class(S, P, k, f2, gx, gy, S.pid[f2]);
             clsb[par2][k] = c2;
-            if (needs_record(c2, excl)) {
+            if (c2 != kNone) {
                 lst[par2][lst_n[par2]] = k;
                 lst_n[par2] += 1;
             }
         }
-        if (!wave_raster) count_field(S, P, R, S.cnt + 2 * par, bits_out, f1);
+        count_field(S, P, R, S.cnt + 2 * par, bits_out, f1);
         __syncthreads();
     }
     for (int i = tid; i < N; i += nthr) {
@@ -1124,6 +988,376 @@ forage_step_kernel(const FGRep* __restrict__ reps, abm_forage_state st,
         }
         if (tid == 0) mt[rb].pos = pos;
     }
+}
+
+// ------------------------------------------------ update without visual exclusion
+// Agent.update in id order (sims.py:861) without visual exclusion needs no
+// id-order chain.  Agent k reads the agents before it (already moved) and
+// after it (not yet) only as social cues, and what makes agent j a cue -- its
+// overriding mode exploit, its patch id and its position -- does not depend on
+// j's own field: the update leaves j exploiting exactly when u' > T_w with
+// env_status 1 (agent.py:215-283: the exploit branches; u' comes from I_priv,
+// u and the old w, agent.py:168-199), its patch id is never changed, and an
+// exploiting agent keeps its heading and slows by a fixed ratio.  So every
+// agent's moved cue is known before any field is, and all fields of a replica
+// are built at once: agent k's from the cues j < k as moved and j > k as they
+// started.  Only the walks' draw indices follow the id order (a scan of
+// flags).  A collide override (kept by the update) is never a cue.
+
+// u and I_priv after the update (agent.py:168-199), and whether the update
+// leaves the agent exploiting.
+struct Drive {
+    double u, ipriv;
+    bool exploit;
+};
+__device__ inline Drive drive_of(const FGRep& P, double w, double u, double nov, double cr, double crb,
+                                 int over, int env) {
+#pragma clang fp contract(off)
+    Drive q;
+    const double collected = cr - crb;
+    q.ipriv = P.F_N * nov + P.F_R * collected;
+    const double w_p = w > P.T_w ? w : 0.0;
+    const double du = P.Eps_u * q.ipriv - P.g_u * (u - P.B_u) - w_p * P.S_wu;
+    u = u + du;
+    if (u > P.u_max) u = P.u_max;
+    if (u < -P.u_max) u = -P.u_max;
+    q.u = u;
+    q.exploit = over != ABM_MODE_COLLIDE && u > P.T_w && env == 1;   // tr_u compares with T_w
+    return q;
+}
+
+// The decision of an agent (agent.py:168-283): its new w, modes, speed and
+// heading increments; kind 0 draws a walk turn.
+struct Choice {
+    double w, dth, dvel;
+    int over, mode, kind;
+};
+__device__ inline Choice choose(const FGRep& P, int R, int n_set, int n_left, double w, double u0, double u1,
+                                double vel0, int over, int mode, int env) {
+#pragma clang fp contract(off)
+    Choice c;
+    const int nl = R / 2;
+    const double count = (double)n_set, cleft = (double)n_left;
+    const double u_p = u0 > P.T_u ? u0 : 0.0;
+    const double mean = count / (double)R;
+    const double dw = P.Eps_w * mean - P.g_w * (w - P.B_w) - u_p * P.S_uw;
+    w = w + dw;
+    if (w > P.w_max) w = P.w_max;
+    if (w < -P.w_max) w = -P.w_max;
+    c.w = w; c.dth = 0.0; c.dvel = 0.0; c.over = over; c.mode = mode; c.kind = 1;
+    if (over == ABM_MODE_COLLIDE) return c;   // get_mode() == "collide" only via the override
+    const bool tw = w > P.T_w, tu = u1 > P.T_w;   // tr_u compares with T_w
+    if (tu && env == 1) {
+        c.over = ABM_MODE_EXPLOIT; c.mode = ABM_MODE_EXPLOIT;
+        c.dvel = -vel0 * P.exp_stop_ratio;
+    } else if (tw) {   // relocation towards the fuller half of the field
+        const double lm = cleft / (double)nl;
+        const double rm = (count - cleft) / (double)(R - nl);
+        c.dvel = P.exp_vel_max - vel0;
+        c.dth = (lm - rm) * P.reloc_theta_max;
+        c.over = -1; c.mode = ABM_MODE_RELOCATE;
+    } else {
+        c.dvel = P.exp_vel_max;
+        c.over = -1; c.mode = ABM_MODE_EXPLORE; c.kind = 0;
+    }
+    return c;
+}
+
+// The move (agent.py:200-283, 595-620): heading turned by dth, speed by
+// dvel, limited in explore mode only, one Euler step, the walls.
+__device__ inline Pose fg_move(const FGRep& P, Pose p, double dth, double dvel, int over, double w, double rad) {
+#pragma clang fp contract(off)
+    p.theta = prove_orientation(p.theta + dth);
+    double sn, cs;
+    sincos(p.theta, &sn, &cs);
+    p.v = p.v + dvel;
+    if (get_mode(over, w, P.T_w) == ABM_MODE_EXPLORE && fabs(p.v) > 1.0) p.v = P.exp_vel_max;
+    p.x = p.x + p.v * cs;
+    p.y = p.y - p.v * sn;
+    return reflect_walls(p, rad, P.pad, P.width, P.height);
+}
+
+// supcalc.distance <= vision_range of two centres: decided on the squared
+// distance outside a band far wider than its rounding, else by the norm.
+struct RangeTest {
+    double vr, lo, hi;
+};
+__device__ inline RangeTest range_test(double vr) {
+    RangeTest t;
+    t.vr = vr;
+    t.lo = vr > 0.0 ? vr * vr * (1.0 - 1e-9) : -1.0;
+    t.hi = vr > 0.0 ? vr * vr * (1.0 + 1e-9) : HUGE_VAL;
+    return t;
+}
+__device__ inline bool in_range(const RangeTest& t, double dx, double dy) {
+#pragma clang fp contract(off)
+    const double d2 = dx * dx + dy * dy;
+    if (d2 <= t.lo) return true;
+    if (d2 >= t.hi) return false;
+    return norm2(dx, dy) <= t.vr;
+}
+
+// Raw bits V[lo .. lo + 31] of a field of W words (zero outside it).
+__device__ inline uint32_t raw_window(const uint32_t* V, int W, int lo) {
+    const int w = lo >> 5, sh = lo & 31;
+    const uint32_t a = w >= 0 && w < W ? V[w] : 0u;
+    if (sh == 0) return a;
+    const uint32_t b = w + 1 >= 0 && w + 1 < W ? V[w + 1] : 0u;
+    return (a >> sh) | (b << (32 - sh));
+}
+
+// Counts of a wave's raw field on the kept rays and on their left half, to
+// every lane, and (dst not null) the returned field: soc_v_field[q] =
+// V[R - 1 - q] on the kept rays (agent.py:593-595), a word of it being a raw
+// window reversed.
+__device__ inline void wave_counts(const uint32_t* V, int R, int W, int keep_lo, int keep_hi, uint32_t* dst,
+                                   int* n_set, int* n_left) {
+    const int lane = threadIdx.x & 63;
+    const int nl = R / 2, ta = R - 1 - keep_hi, tb = R - 1 - keep_lo, la = max(R - nl, ta);
+    int tot = 0, left = 0;
+    for (int w = lane; w < W; w += 64) {
+        const uint32_t bits = V[w];
+        tot += __popc(bits & word_range_mask(w, ta, tb));
+        left += __popc(bits & word_range_mask(w, la, tb));
+        if (dst) dst[w] = __brev(raw_window(V, W, R - 32 - 32 * w)) & word_range_mask(w, keep_lo, keep_hi);
+    }
+    if (R < 32768) {   // one sum of both counts
+        const int both = wave_sum(tot << 16 | left);
+        *n_set = both >> 16;
+        *n_left = both & 0xffff;
+    } else {
+        *n_set = wave_sum(tot);
+        *n_left = wave_sum(left);
+    }
+}
+
+// LDS of the update kernel: the replica's agents at the step's start, their
+// moved poses where they are cues, and one raw field per wave.
+struct UpdSmem {
+    double *x, *y, *th, *v, *w, *u0, *u1, *ip, *cr, *u1x, *u1y, *xm, *ym;
+    int *rad, *pid, *over, *mode, *env, *flag, *cue, *nset, *nleft, *idx;
+    uint32_t *words, *key, *field;
+    int *wtot, *ctl;
+};
+constexpr int kUpdDoubles = 13, kUpdInts = 10, kUpdWaves = 16;
+
+__device__ inline UpdSmem upd_carve(void* base, int maxN) {
+    UpdSmem s;
+    char* p = reinterpret_cast<char*>(base);
+    double** d[] = {&s.x, &s.y, &s.th, &s.v, &s.w, &s.u0, &s.u1, &s.ip, &s.cr, &s.u1x, &s.u1y, &s.xm, &s.ym};
+    for (double** a : d) { *a = reinterpret_cast<double*>(p); p += sizeof(double) * maxN; }
+    s.words = reinterpret_cast<uint32_t*>(p); p += sizeof(uint32_t) * 2 * maxN;
+    int** i[] = {&s.rad, &s.pid, &s.over, &s.mode, &s.env, &s.flag, &s.cue, &s.nset, &s.nleft, &s.idx};
+    for (int** a : i) { *a = reinterpret_cast<int*>(p); p += sizeof(int) * maxN; }
+    s.key = reinterpret_cast<uint32_t*>(p); p += sizeof(uint32_t) * kMtN;
+    s.wtot = reinterpret_cast<int*>(p); p += sizeof(int) * 2 * kUpdWaves;
+    s.ctl = reinterpret_cast<int*>(p); p += sizeof(int) * 4;
+    s.field = reinterpret_cast<uint32_t*>(p);
+    return s;
+}
+
+size_t upd_lds_bytes(int maxN, int maxR, int waves) {
+    return (size_t)maxN * (8 * kUpdDoubles + 8 + 4 * kUpdInts) + 4 * (kMtN + 2 * kUpdWaves + 4) +
+           sizeof(uint32_t) * (size_t)waves * ((maxR + 31) / 32) + 16;
+}
+
+// What an agent is as a cue (UpdSmem.flag): where it started, and once moved.
+constexpr int kCueStart = 1, kCueMoved = 2;
+
+// One workgroup per replica, largest first.  Threads over agents: the drive,
+// the focal geometry and the moved pose of every cue; one wave per agent: its
+// cues' records (64 at a time, one per lane) ORed into the wave's raw field
+// (each interval is a few words: LDS atomics) and the counts; threads over
+// agents: the choice, the draw indices (a scan), the walk's words, the move.
+// Bound by the waves' records and their raster (64 cues at a time) for large
+// replicas, by the phases' latency for small ones.  Against the id-order chain
+// (one agent at a time, its cues' intervals spread over the lanes one by one):
+// 1000 replicas of 8 to 512 agents, a tenth of them cues, 3.95 ms -> 0.102 ms;
+// one replica of 10 agents 26.6 us -> 9.1 us.
+template <bool FIELDS>
+__global__ void __launch_bounds__(1024)
+forage_update_kernel(const FGRep* __restrict__ reps, abm_forage_state st,
+                     const double* __restrict__ uniforms, const uint32_t* __restrict__ words,
+                     const int64_t* __restrict__ u_off, const int32_t* __restrict__ u_cnt,
+                     int32_t* __restrict__ u_used, int32_t* __restrict__ status,
+                     uint32_t* __restrict__ bits_out, const int32_t* __restrict__ order,
+                     abm_mt19937_state* __restrict__ mt, int maxN) {
+#pragma clang fp contract(off)
+    extern __shared__ __align__(16) double smem[];
+    const int rb = order[blockIdx.x];
+    if (status && status[rb] != kWorldReady) return;   // uniform over the block
+    const int tid = threadIdx.x, nthr = blockDim.x;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), nw = nthr >> 6;
+    __shared__ FGRep sP;
+    if (tid < (int)(sizeof(FGRep) / 8))
+        reinterpret_cast<uint64_t*>(&sP)[tid] = reinterpret_cast<const uint64_t*>(reps + rb)[tid];
+    const UpdSmem S = upd_carve(smem, maxN);
+    if (tid == 0) S.ctl[0] = 0;
+    int mt_pos0 = 0;
+    if (mt) {
+        for (int i = tid; i < kMtN; i += nthr) S.key[i] = mt[rb].key[i];
+        mt_pos0 = mt[rb].pos;
+    }
+    const int ucount = mt ? 0 : u_cnt[rb];
+    const int used0 = (words || mt) ? u_used[rb] : 0;
+    __syncthreads();
+    const FGRep& P = sP;
+    const int N = P.n_agents, R = P.n_rays, W = P.words, a0 = P.agent_offset, tau = P.tau;
+    // ---- the agents, their drives and the cues
+    for (int base = tid - lane; base < N; base += nthr) {
+        const int i = base + lane;
+        int flag = 0;
+        if (i < N) {
+            const int g = a0 + i;
+            const double x = st.x[g], y = st.y[g], th = st.theta[g], v = st.v[g], w = st.w[g], u = st.u[g];
+            const double cr = st.collected_r[g], crb = st.collected_r_before[g];
+            const int rad = st.radius[g], over = st.overriding_mode[g], mode = st.mode[g];
+            const int env = st.env_status[g], pid = st.exploited_patch_id[g];
+            double m = st.novelty[(int64_t)g * tau];
+            for (int q = 1; q < tau; ++q) m = fmax(m, st.novelty[(int64_t)g * tau + q]);
+            const Drive d = drive_of(P, w, u, m, cr, crb, over, env);
+            S.x[i] = x; S.y[i] = y; S.th[i] = th; S.v[i] = v; S.w[i] = w; S.u0[i] = u; S.u1[i] = d.u;
+            S.ip[i] = d.ipriv; S.cr[i] = cr; S.rad[i] = rad; S.pid[i] = pid; S.over[i] = over;
+            S.mode[i] = mode; S.env[i] = env;
+            const Focal f = focal_at(x, y, th, (double)rad);
+            S.u1x[i] = f.u1x; S.u1y[i] = f.u1y;
+            if (pid != -1) {
+                if (over == ABM_MODE_EXPLOIT) flag |= kCueStart;
+                if (d.exploit) {
+                    flag |= kCueMoved;
+                    const Pose p = fg_move(P, Pose{x, y, th, v}, 0.0, -v * P.exp_stop_ratio, ABM_MODE_EXPLOIT,
+                                           w, (double)rad);
+                    S.xm[i] = p.x; S.ym[i] = p.y;
+                }
+            }
+            S.flag[i] = flag;
+        }
+        const uint64_t m = __ballot(flag != 0);
+        if (m) {
+            int at = 0;
+            if (lane == 0) at = atomicAdd(&S.ctl[0], (int)__popcll(m));
+            at = __builtin_amdgcn_readfirstlane(at);
+            if (flag) S.cue[at + (int)__popcll(m & ((1ull << lane) - 1ull))] = i;
+        }
+    }
+    __syncthreads();
+    // ---- the fields
+    const int n_cue = S.ctl[0];
+    {
+        const FastRec FR = fast_rec_const(R, P.step, P.fov0, P.fov1);
+        const RangeTest rt = range_test(P.vision_range);
+        const int keep_lo = P.keep_lo, keep_hi = P.keep_hi, patchwise = P.patchwise;
+        const double step = P.step, fov0 = P.fov0, fov1 = P.fov1;
+        uint32_t* V = S.field + wave * W;
+        for (int k = wave; k < N; k += nw) {
+            int n_set = 0, n_left = 0;
+            if (n_cue > 0) {
+                for (int w = lane; w < W; w += 64) V[w] = 0u;
+                fg_wave_sync();
+                Focal f;
+                f.radius = (double)S.rad[k];
+                f.px = S.x[k]; f.py = S.y[k];
+                f.cx = f.px + f.radius;
+                f.cy = f.py + f.radius;
+                f.u1x = S.u1x[k]; f.u1y = S.u1y[k];
+                const int pid_k = S.pid[k];
+                for (int q = lane; q < n_cue; q += 64) {
+                    const int j = S.cue[q];
+                    const int pid = S.pid[j];
+                    const bool moved = j < k;
+                    // agent.py:396-413: an exploiting agent in range with a
+                    // patch other than the focal's own (patchwise exclusion)
+                    if (j == k || !(S.flag[j] & (moved ? kCueMoved : kCueStart)) || (patchwise && pid == pid_k))
+                        continue;
+                    const double ox = moved ? S.xm[j] : S.x[j], oy = moved ? S.ym[j] : S.y[j];
+                    const double rj = (double)S.rad[j];
+                    if (!in_range(rt, (ox + rj) - f.cx, (oy + rj) - f.cy)) continue;
+                    const Rec rc = record_at(ox, oy, kSocial, j, f, R, step, fov0, fov1, FR, false);
+                    if (rc.valid) paint_bits(V, rc, R);
+                }
+                fg_wave_sync();
+                wave_counts(V, R, W, keep_lo, keep_hi, FIELDS ? bits_out + P.field_offset + (int64_t)k * W : nullptr,
+                            &n_set, &n_left);
+                fg_wave_sync();
+            } else if (FIELDS) {
+                uint32_t* dst = bits_out + P.field_offset + (int64_t)k * W;
+                for (int w = lane; w < W; w += 64) dst[w] = 0u;
+            }
+            if (lane == 0) { S.nset[k] = n_set; S.nleft[k] = n_left; }
+        }
+    }
+    __syncthreads();
+    // ---- the walks' draw indices, in id order
+    int draws = 0;
+    for (int c0 = 0, par = 0; c0 < N; c0 += nthr, par ^= 1) {
+        const int k = c0 + tid;
+        int kind = 1;
+        if (k < N)
+            kind = choose(P, R, S.nset[k], S.nleft[k], S.w[k], S.u0[k], S.u1[k], S.v[k], S.over[k], S.mode[k],
+                          S.env[k]).kind;
+        const uint64_t m = __ballot(kind == 0);
+        if (lane == 0) S.wtot[kUpdWaves * par + wave] = (int)__popcll(m);
+        __syncthreads();   // a half of wtot is rewritten two chunks later, after this chunk's barrier
+        int d = draws + (int)__popcll(m & ((1ull << lane) - 1ull));
+        for (int w = 0; w < nw; ++w) {
+            const int t = S.wtot[kUpdWaves * par + w];
+            if (w < wave) d += t;
+            draws += t;
+        }
+        if (k < N) S.idx[k] = d;
+    }
+    // ---- the walks' words from the replica's device generator: exactly the
+    // 2 * draws it consumes, so the key left is numpy's (which twists lazily,
+    // when a word is drawn at position 624)
+    if (mt) {
+        int made = 0, p = mt_pos0, twists = 0;
+        while (made < 2 * draws) {
+            if (p >= kMtN) {
+                mt_twist_block(S.key);
+                ++twists;
+                p = 0;
+            }
+            const int take = min(kMtN - p, 2 * draws - made);
+            for (int j = tid; j < take; j += nthr) S.words[made + j] = mt_temper(S.key[p + j]);
+            made += take;
+            p += take;
+        }
+        __syncthreads();
+        if (twists > 0)
+            for (int i = tid; i < kMtN; i += nthr) mt[rb].key[i] = S.key[i];
+        if (tid == 0) mt[rb].pos = p;
+    }
+    // ---- the moves (each thread its own agents of the scan)
+    for (int k = tid; k < N; k += nthr) {
+        const int g = a0 + k;
+        const double vel0 = S.v[k];
+        const Choice c = choose(P, R, S.nset[k], S.nleft[k], S.w[k], S.u0[k], S.u1[k], vel0, S.over[k], S.mode[k],
+                                S.env[k]);
+        double dth = c.dth;
+        if (c.kind == 0) {
+            // agent k's draw: doubles, or pairs of words after those the
+            // resource loop used; NaN past the end of the buffer
+            const int d = S.idx[k];
+            double uu = NAN;
+            if (mt) {
+                uu = words_to_double(S.words[2 * d], S.words[2 * d + 1]);
+            } else if (words) {
+                const uint32_t* wb = words + u_off[rb];
+                const int at = used0 + 2 * d;
+                if (at + 2 <= ucount) uu = words_to_double(wb[at], wb[at + 1]);
+            } else if (d < ucount) {
+                uu = uniforms[u_off[rb] + d];
+            }
+            dth = P.exp_theta_min + (P.exp_theta_max - P.exp_theta_min) * uu;
+        }
+        const Pose p = fg_move(P, Pose{S.x[k], S.y[k], S.th[k], vel0}, dth, c.dvel, c.over, c.w, (double)S.rad[k]);
+        st.x[g] = p.x; st.y[g] = p.y; st.theta[g] = p.theta; st.v[g] = p.v;
+        st.w[g] = c.w; st.u[g] = S.u1[k]; st.collected_r_before[g] = S.cr[k];
+        st.mode[g] = c.mode; st.overriding_mode[g] = c.over;
+        st.I_priv[g] = S.ip[k];
+    }
+    if (tid == 0 && u_used) u_used[rb] = used0 + (words || mt ? 2 : 1) * draws;
+    if (tid == 0 && status) status[rb] = ABM_WORLD_DONE;
 }
 
 // ------------------------------------------------ replicas beyond one workgroup
@@ -2374,34 +2608,54 @@ SweepMem sweep_carve(void* base, int M) {
     return m;
 }
 
-// Which replicas the step kernel updates and which are swept: sweeps for
-// those beyond one workgroup's LDS, or (ABM_FORAGE_PATH_SWEEP) for every
-// replica without visual exclusion.  The step kernel's blocks take their
-// replicas largest first (the id-order chain grows with the agents; rays add
-// to each agent's step).
+// Which kernel updates which replica: the update kernel those without visual
+// exclusion that fit one workgroup's LDS, the step kernel those with it, and
+// sweeps those beyond one workgroup's LDS, or (ABM_FORAGE_PATH_SWEEP) every
+// replica without visual exclusion.  A kernel's blocks take their replicas
+// largest first (the cost grows with the agents; rays add to each agent's).
 int plan_paths(abm_forage_batch* bt, int path) {
     const int n = bt->n_replicas;
-    std::vector<int32_t> small, big;
+    std::vector<int32_t> plain, occl, big;
     for (int b = 0; b < n; ++b) {
         const bool sweepable = !bt->exclusion[b] && bt->rep_r[b] <= 32 * kSweepMaxWords;
         if (bt->too_big[b] || (path == ABM_FORAGE_PATH_SWEEP && sweepable)) big.push_back(b);
-        else small.push_back(b);
+        else (bt->exclusion[b] ? occl : plain).push_back(b);
     }
     auto cost = [&](int b) { return (double)bt->rep_n[b] * (64.0 + bt->rep_r[b] / 32.0); };
-    std::stable_sort(small.begin(), small.end(), [&](int a, int c) { return cost(a) > cost(c); });
-    bt->order_host = small;
+    auto larger = [&](int a, int c) { return cost(a) > cost(c); };
+    std::stable_sort(plain.begin(), plain.end(), larger);
+    std::stable_sort(occl.begin(), occl.end(), larger);
+    bt->order_host = plain;
+    bt->order_host.insert(bt->order_host.end(), occl.begin(), occl.end());
     bt->order_host.insert(bt->order_host.end(), big.begin(), big.end());
-    bt->n_small = (int32_t)small.size();
-    bt->small_max_agents = 0;
-    bt->small_max_rays = 0;
-    for (int b : small) {
-        bt->small_max_agents = std::max(bt->small_max_agents, bt->rep_n[b]);
-        bt->small_max_rays = std::max(bt->small_max_rays, bt->rep_r[b]);
-    }
+    auto extent = [&](const std::vector<int32_t>& v, int32_t& count, int32_t& agents, int32_t& rays) {
+        count = (int32_t)v.size();
+        agents = rays = 0;
+        for (int b : v) {
+            agents = std::max(agents, bt->rep_n[b]);
+            rays = std::max(rays, bt->rep_r[b]);
+        }
+    };
+    extent(plain, bt->n_plain, bt->plain_max_agents, bt->plain_max_rays);
+    extent(occl, bt->n_occl, bt->occl_max_agents, bt->occl_max_rays);
     bt->sweep = big;
     bt->path = path;
     return check_hip(hipMemcpy(bt->order_dev, bt->order_host.data(), sizeof(int32_t) * n,
                                hipMemcpyHostToDevice), "upload forage order");
+}
+
+// Waves of the update kernel's workgroups: sixteen, so that a large replica's
+// agents share a CU's four SIMDs (1000 replicas of 8 to 512 agents: 0.140 ms a
+// step with sixteen, 0.161 with eight, 0.237 with four; 300 of 300 agents:
+// 0.126, 0.126, 0.179); four where more workgroups than two per CU queue and no
+// replica has work for more (1000 replicas of 10 agents: 0.048 ms with four,
+// 0.070 with sixteen; of 50: 0.068, 0.090; of 128: 0.121, 0.137).  Fewer too
+// where the waves' fields would not fit in LDS.
+int upd_waves(const abm_forage_batch* b) {
+    int waves = b->n_plain > 2 * b->cus && b->plain_max_agents <= 128 ? 4 : 16;
+    while (waves > 4 && upd_lds_bytes(b->plain_max_agents, b->plain_max_rays, waves) > (size_t)163840 - sizeof(FGRep))
+        waves /= 2;
+    return waves;
 }
 
 int check_state(const abm_forage_state* st, const char* who) {
@@ -2464,26 +2718,39 @@ int launch_forage_step(abm_forage_batch* b, const abm_forage_state* st, const do
                        const uint32_t* words, const int64_t* offset, const int32_t* count,
                        int32_t* used, int32_t* status, uint32_t* field_bits, void* stream,
                        abm_mt19937_state* mt = nullptr) {
-    // the step kernel overlaps one agent's move (wave 0) with the next
-    // agent's records (wave 1) and the classes of the one after (the other
-    // waves): eight waves when some replica has more agents than two waves
-    // classify in one pass, else four (two workgroups then share a CU)
-    if (b->n_small > 0) {
-        const int nthr = b->small_max_agents > 128 ? 512 : 256;
-        const size_t lds = fg_lds_bytes(b->small_max_agents, b->small_max_rays);
-        const bool ex = std::any_of(b->exclusion.begin(), b->exclusion.end(), [](uint8_t e) { return e != 0; });
-        auto kern = field_bits ? (ex ? forage_step_kernel<true, true> : forage_step_kernel<true, false>)
-                               : (ex ? forage_step_kernel<false, true> : forage_step_kernel<false, false>);
+    if (b->n_plain > 0) {
+        const int waves = upd_waves(b);
+        const size_t lds = upd_lds_bytes(b->plain_max_agents, b->plain_max_rays, waves);
+        auto kern = field_bits ? forage_update_kernel<true> : forage_update_kernel<false>;
         if (lds > 65536) {
             if (int rc = check_hip(hipFuncSetAttribute((const void*)kern,
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
                                    "hipFuncSetAttribute"))
                 return rc;
         }
-        hipLaunchKernelGGL(kern, dim3(b->n_small), dim3(nthr), lds, (hipStream_t)stream,
+        hipLaunchKernelGGL(kern, dim3(b->n_plain), dim3(64 * waves), lds, (hipStream_t)stream,
                            (const FGRep*)b->reps_dev, *st, uniforms, words, offset, count, used, status,
-                           field_bits, (const int32_t*)b->order_dev, mt, b->small_max_agents,
-                           b->small_max_rays);
+                           field_bits, (const int32_t*)b->order_dev, mt, b->plain_max_agents);
+        if (int rc = check_hip(hipGetLastError(), "forage_update_kernel launch")) return rc;
+    }
+    // the step kernel overlaps one agent's move (wave 0) with the next
+    // agent's records (wave 1) and the classes of the one after (the other
+    // waves): eight waves when some replica has more agents than two waves
+    // classify in one pass, else four (two workgroups then share a CU)
+    if (b->n_occl > 0) {
+        const int nthr = b->occl_max_agents > 128 ? 512 : 256;
+        const size_t lds = fg_lds_bytes(b->occl_max_agents, b->occl_max_rays);
+        auto kern = field_bits ? forage_step_kernel<true> : forage_step_kernel<false>;
+        if (lds > 65536) {
+            if (int rc = check_hip(hipFuncSetAttribute((const void*)kern,
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
+                                   "hipFuncSetAttribute"))
+                return rc;
+        }
+        hipLaunchKernelGGL(kern, dim3(b->n_occl), dim3(nthr), lds, (hipStream_t)stream,
+                           (const FGRep*)b->reps_dev, *st, uniforms, words, offset, count, used, status,
+                           field_bits, (const int32_t*)b->order_dev + b->n_plain, mt, b->occl_max_agents,
+                           b->occl_max_rays);
         if (int rc = check_hip(hipGetLastError(), "forage_step_kernel launch")) return rc;
     }
     for (int rb : b->sweep)
@@ -2549,6 +2816,8 @@ int abm_forage_batch_create(const abm_forage_replica* reps, int32_t n, abm_forag
     bt->n_replicas = n; bt->n_agents_total = (int32_t)agents; bt->field_words = words;
     bt->max_agents = max_n; bt->max_rays = max_r;
     int rc = check_hip(hipGetDevice(&bt->device), "hipGetDevice");
+    if (!rc) rc = check_hip(hipDeviceGetAttribute(&bt->cus, hipDeviceAttributeMultiprocessorCount, bt->device),
+                            "hipDeviceGetAttribute");
     int dev_max = 0;
     if (!rc) rc = check_hip(hipDeviceGetAttribute(&dev_max, hipDeviceAttributeMaxSharedMemoryPerBlock,
                                                   bt->device), "hipDeviceGetAttribute");

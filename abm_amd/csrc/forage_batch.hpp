@@ -15,17 +15,19 @@ struct abm_forage_batch {
     int32_t max_agents = 0;
     int32_t max_rays = 0;
     int device = 0;
+    int cus = 0;                       // compute units of the device
     void* reps_dev = nullptr;
     void* order_dev = nullptr;        // replicas by descending cost: the blocks' update order
     int32_t* agent_offset_host = nullptr;
     int64_t* field_offset_host = nullptr;
-    // Replicas the step kernel updates (the first n_small of order_dev) and
-    // the ones it cannot hold in one workgroup's LDS, updated by sweeps.
-    int32_t n_small = 0;
-    int32_t small_max_agents = 0, small_max_rays = 0;
+    // Replicas the update kernel takes (the first n_plain of order_dev), those
+    // with visual exclusion, which the step kernel takes (the next n_occl),
+    // and the ones beyond one workgroup's LDS, updated by sweeps.
+    int32_t n_plain = 0, n_occl = 0;
+    int32_t plain_max_agents = 0, plain_max_rays = 0, occl_max_agents = 0, occl_max_rays = 0;
     int32_t path = 0;                  // ABM_FORAGE_PATH_*
     std::vector<int32_t> rep_n, rep_r; // agents and rays of every replica
-    std::vector<int32_t> order_host;   // every replica, step-kernel ones first by cost
+    std::vector<int32_t> order_host;   // every replica: update kernel's, step kernel's, swept
     std::vector<uint8_t> too_big;      // [b]: beyond one workgroup's LDS
     std::vector<uint8_t> exclusion;    // [b]: visual exclusion
     std::vector<int32_t> sweep;        // replicas updated by sweeps
