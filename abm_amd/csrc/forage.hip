@@ -546,11 +546,6 @@ __device__ void raster_list(const FGSmem& S, int R, const int* lst, int n0, int 
     __syncthreads();
 }
 
-// Bits [lo, hi) of a field that fall in word w.
-__device__ inline uint32_t word_slice_mask(int w, int lo, int hi) {
-    return hi > lo ? word_range_mask(w, lo, hi - 1) : 0u;
-}
-
 // Sum over the 64 lanes of wave 0 with DPP moves (no LDS round trips):
 // prefix sums inside each row of 16 lanes (row_shr 1, 2, 4, 8), then row
 // 15's and row 31's lane carried into the rows above (row_bcast 15, 31), so
@@ -569,26 +564,6 @@ __device__ inline void fg_wave_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
-// Raw-field word w of one social interval [s, e] of a record: the pieces
-// paint_bits ORs (agent.py:577-590).
-__device__ inline uint32_t interval_word(int w, int s, int e, int R) {
-    if (s >= 0 && e < R) return word_slice_mask(w, s, e > s ? e : s);   // one piece: py_slice(s, e)
-    uint32_t bits = 0u;
-    int lo, hi;
-    if (s < 0) {
-        py_slice(R + s, R, R, &lo, &hi);
-        bits |= word_slice_mask(w, lo, hi);
-        s = 0;
-    }
-    if (e >= R) {
-        py_slice(0, e - R, R, &lo, &hi);
-        bits |= word_slice_mask(w, lo, hi);
-        e = R - 1;
-    }
-    py_slice(s, e, R, &lo, &hi);
-    return bits | word_slice_mask(w, lo, hi);
 }
 
 // The returned field of agent k: counts for mean() and the left/right
@@ -1360,402 +1335,255 @@ forage_update_kernel(const FGRep* __restrict__ reps, abm_forage_state st,
     if (tid == 0 && status) status[rb] = ABM_WORLD_DONE;
 }
 
-// ------------------------------------------------ replicas beyond one workgroup
-// Agent.update in id order (sims.py:861) for a replica whose agents do not fit
-// one workgroup's LDS, without visual exclusion.  Agent k's update reads the
-// agents j < k after their own update and j > k before it, and only through
-// what makes j a social cue for k: j's overriding mode (exploit), its patch
-// id (never changed by the update) and its position.  Sweeps recompute every
-// agent from the latest tentative states X^m (j < k) and the step's start
-// (j >= k) at once:
-//   X^{m+1}_k = F_k(X^m_0, .., X^m_{k-1}, start_k, .., start_{N-1}),
-// the walk's draw index being the number of draws in X^{m+1}_j, j < k.
-// Agent k is final after k + 1 sweeps, and the only fixed point X = F(X) is
-// the reference's sequential result, so the sweeps stop at the first
-// X^{m+1} == X^m (every value bitwise), which is that result; in practice a
-// few sweeps, as only exploiting agents carry dependencies.
-struct SweepX {
-    double *x, *y, *th, *v, *w, *u, *ip, *dth, *dvel;
-    int32_t *over, *mode, *kind;   // kind: 0 = draws a walk turn, 1 = fixed increments, -1 = unset
+// ------------------------------------------------ replicas over the whole GPU
+// The same update for replicas beyond one workgroup's LDS, and for large ones:
+// three launches over the agents of all of them, 64 (a chunk) to a wave in the
+// first and last, one to a wave in the middle, with the cues in global memory.
+// No host round trip, so a caller may capture the step.  Its predecessor swept
+// all agents until a fixed point (three sweeps a step, checked on the host):
+// one replica of 8192 agents with 100 to 700 cues took 0.41 ms in the sweeps,
+// 0.04 ms now.
+struct WideRep {
+    int32_t rb, chunk0;   // the replica, its first chunk
+    int64_t keys;         // its twisted keys in WideMem.keys, in words
 };
+struct WideCue {
+    double x, y, xm, ym;         // at the step's start, and moved
+    int32_t rad, j, pid, flag;   // flag: kCueStart, kCueMoved
+};
+// Agent k of a replica is entry 64 * chunk0 + k of every array.
+struct WideMem {
+    const WideRep* rep;          // the replicas
+    const int32_t* of;           // [chunk]: which of them
+    WideCue* cue;                // from the replica's first entry on
+    double *u1, *ip, *u1x, *u1y;
+    int32_t *nset, *nleft;
+    uint32_t *uni;               // the next 2N words of a device generator
+    uint32_t* keys;              // its key after each twist
+    uint8_t* walk;               // 1: the agent draws a walk turn
+    int32_t* ctl;                // [replica][kWdWords]
+};
+constexpr int kWdCues = 0, kWdSkip = 1, kWdUsed0 = 2, kWdUpdates = 3, kWdWords = 4;
 
-// Sweep control words.
-constexpr int kSwConverged = 0, kSwSkip = 1, kSwCand = 2, kSwIters = 3, kSwDraws = 4,
-              kSwUsed0 = 5, kSwPos0 = 6, kSwBad = 7, kSwTwists = 8, kSwWords = 9;
-
-constexpr int kSweepMaxWords = 256;   // R <= 8192: four field words per lane
-
-// Exploiting agents with a patch (at the step's start or in X), the only
-// candidates for a social cue.
-__device__ inline void sweep_candidates(const abm_forage_state& st, int a0, int N, const int32_t* xover,
-                                        int32_t* cand, int32_t* ctrl) {
-    if (threadIdx.x == 0) ctrl[kSwCand] = 0;
-    __syncthreads();
-    const int lane = threadIdx.x & 63;
-    for (int base = threadIdx.x - lane; base < N; base += blockDim.x) {
-        const int j = base + lane;
-        bool c = false;
-        if (j < N) {
-            const int g = a0 + j;
-            c = st.exploited_patch_id[g] != -1 &&
-                (st.overriding_mode[g] == ABM_MODE_EXPLOIT || (xover && xover[j] == ABM_MODE_EXPLOIT));
-        }
-        const uint64_t m = __ballot(c);
-        if (m) {
-            int at = 0;
-            if (lane == 0) at = atomicAdd(&ctrl[kSwCand], (int)__popcll(m));
-            at = __builtin_amdgcn_readfirstlane(at);
-            if (c) cand[at + (int)__popcll(m & ((1ull << lane) - 1ull))] = j;
-        }
-    }
-    __syncthreads();
-}
-
-// One block of 1024 threads: status, the step's uniforms, X^0 = the start
-// state, the first candidates.
-__global__ void __launch_bounds__(1024)
-sweep_prep_kernel(const FGRep* __restrict__ reps, int rb, abm_forage_state st,
-                  const double* __restrict__ uniforms, const uint32_t* __restrict__ words,
-                  const int64_t* __restrict__ u_off, const int32_t* __restrict__ u_cnt,
-                  const int32_t* __restrict__ u_used, const int32_t* __restrict__ status,
-                  const abm_mt19937_state* __restrict__ mt, SweepX X0, double* __restrict__ uni,
-                  uint32_t* __restrict__ keys, int32_t* __restrict__ cand, int32_t* __restrict__ ctrl) {
-    __shared__ uint32_t key[kMtN];
-    const FGRep& P = reps[rb];
-    const int N = P.n_agents, a0 = P.agent_offset, tid = threadIdx.x, nthr = blockDim.x;
-    const bool skip = status && status[rb] != kWorldReady;
-    if (tid == 0) {
-        ctrl[kSwConverged] = 0; ctrl[kSwSkip] = skip ? 1 : 0; ctrl[kSwIters] = 0;
-        ctrl[kSwDraws] = 0; ctrl[kSwBad] = 0; ctrl[kSwTwists] = 0;
-        ctrl[kSwUsed0] = (words || mt) ? u_used[rb] : 0;
-        ctrl[kSwPos0] = mt ? mt[rb].pos : 0;
-    }
-    if (skip) return;   // uniform over the block
-    for (int i = tid; i < N; i += nthr) {
-        const int g = a0 + i;
-        X0.x[i] = st.x[g]; X0.y[i] = st.y[g]; X0.th[i] = st.theta[g]; X0.v[i] = st.v[g];
-        X0.w[i] = st.w[g]; X0.u[i] = st.u[g]; X0.ip[i] = st.I_priv[g];
-        X0.dth[i] = 0.0; X0.dvel[i] = 0.0;
-        X0.over[i] = st.overriding_mode[g]; X0.mode[i] = st.mode[g]; X0.kind[i] = -1;
-    }
-    // agent i's walk draws the i-th uniform at most: doubles, pairs of words
-    // after those the resource loop used, or the device generator's next 2N
-    // words; NaN past the end of a buffer
-    if (mt) {
-        for (int i = tid; i < kMtN; i += nthr) key[i] = mt[rb].key[i];
-        __syncthreads();
-        uint32_t* wb = reinterpret_cast<uint32_t*>(uni);
-        int made = 0, p = mt[rb].pos, twists = 0;
-        while (made < 2 * N) {
-            if (p >= kMtN) {
-                // each twisted key is kept, so the commit takes the state
-                // after the words drawn without twisting again
-                mt_twist_block(key);
-                for (int i = tid; i < kMtN; i += nthr) keys[(int64_t)twists * kMtN + i] = key[i];
-                ++twists;
-                p = 0;
-            }
-            const int take = min(kMtN - p, 2 * N - made);
-            for (int j = tid; j < take; j += nthr) wb[made + j] = mt_temper(key[p + j]);
-            made += take;
-            p += take;
-            __syncthreads();
-        }
-        for (int i = tid; i < N; i += nthr) {   // each thread rewrites its own 8 bytes
-            const uint32_t w0 = wb[2 * i], w1 = wb[2 * i + 1];
-            uni[i] = words_to_double(w0, w1);
-        }
-        if (tid == 0) ctrl[kSwTwists] = twists;
-    } else {
-        const int ucount = u_cnt[rb];
-        const int used0 = words ? u_used[rb] : 0;
-        for (int i = tid; i < N; i += nthr) {
-            double uu = NAN;
-            if (words) {
-                const int at = used0 + 2 * i;
-                if (at + 2 <= ucount) uu = words_to_double(words[u_off[rb] + at], words[u_off[rb] + at + 1]);
-            } else if (i < ucount) {
-                uu = uniforms[u_off[rb] + i];
-            }
-            uni[i] = uu;
-        }
-    }
-    __syncthreads();
-    sweep_candidates(st, a0, N, nullptr, cand, ctrl);
-}
-
-// One wave per focal agent k: its social field from the view (X^m for j < k,
-// the start for j > k), the counts, and the decision (agent.py:168-265)
-// into X^{m+1}; the field bits when asked for.
+// One thread per agent: the drive, the focal geometry, the cues.
 __global__ void __launch_bounds__(256)
-sweep_field_kernel(const FGRep* __restrict__ reps, int rb, abm_forage_state st, SweepX Xc, SweepX Xn,
-                   const int32_t* __restrict__ cand, const int32_t* __restrict__ ctrl,
-                   uint32_t* __restrict__ bits_out) {
+wide_drive_kernel(const FGRep* __restrict__ reps, int n_chunks, abm_forage_state st,
+                  const int32_t* __restrict__ status, const int32_t* __restrict__ u_used, int words_or_mt,
+                  WideMem M) {
 #pragma clang fp contract(off)
-    __shared__ uint32_t raw[4][kSweepMaxWords];
-    if (ctrl[kSwConverged] | ctrl[kSwSkip]) return;
+    const int lane = threadIdx.x & 63;
+    const int chunk = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+    if (chunk >= n_chunks) return;
+    const int q = M.of[chunk], rb = M.rep[q].rb, chunk0 = M.rep[q].chunk0;
+    int32_t* const ctl = M.ctl + kWdWords * q;
+    const bool skip = status && status[rb] != kWorldReady;
+    if (chunk == chunk0 && lane == 0) {
+        ctl[kWdSkip] = skip;
+        ctl[kWdUsed0] = words_or_mt ? u_used[rb] : 0;
+    }
+    if (skip) return;
     const FGRep& P = reps[rb];
-    const int N = P.n_agents, R = P.n_rays, W = P.words, a0 = P.agent_offset;
-    const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    const int k = blockIdx.x * 4 + wv;
-    if (k >= N) return;   // uniform over the wave
-    const int gk = a0 + k;
-    const double rk = (double)st.radius[gk];
-    const double pxk = st.x[gk], pyk = st.y[gk];
-    const int pid_k = st.exploited_patch_id[gk];
-    Focal f;
-    {
-        double sn, cs;
-        sincos(st.theta[gk], &sn, &cs);
-        f.px = pxk; f.py = pyk; f.radius = rk;
-        f.cx = pxk + rk;
-        f.cy = pyk + rk;
-        const double ex = pxk + (1.0 + cs) * rk;
-        const double ey = pyk + (1.0 - sn) * rk;
-        const double v1x = ex - f.cx, v1y = ey - f.cy;
-        const double n1 = norm2(v1x, v1y);
-        f.u1x = v1x / n1;
-        f.u1y = v1y / n1;
-    }
-    const FastRec FR = fast_rec_const(R, P.step, P.fov0, P.fov1);
-    const int ncand = ctrl[kSwCand];
-    uint32_t bits[4] = {0u, 0u, 0u, 0u};
-    for (int base = 0; base < ncand; base += 64) {
-        const int q = base + lane;
-        bool live = false;
-        int sx = 0, ex = 0;
-        if (q < ncand) {
-            const int j = cand[q];
-            const int g = a0 + j;
-            const bool moved = j < k;
-            const int over = moved ? Xc.over[j] : st.overriding_mode[g];
-            const int pid = st.exploited_patch_id[g];
-            // agent.py:396-413: a cue is an exploiting agent in range with a
-            // patch other than the focal's own (patchwise exclusion)
-            if (j != k && over == ABM_MODE_EXPLOIT && pid != -1 && !(P.patchwise && pid == pid_k)) {
-                const double ox = moved ? Xc.x[j] : st.x[g];
-                const double oy = moved ? Xc.y[j] : st.y[g];
-                const double rj = (double)st.radius[g];
-                if (norm2((ox + rj) - f.cx, (oy + rj) - f.cy) <= P.vision_range) {
-                    const Rec rc = record_at(ox, oy, kSocial, j, f, R, P.step, P.fov0, P.fov1, FR, false);
-                    live = rc.valid != 0;
-                    sx = rc.sx;
-                    ex = rc.ex;
-                }
+    const int i = (chunk - chunk0) * 64 + lane, e = chunk * 64 + lane;
+    int flag = 0;
+    WideCue c;
+    if (i < P.n_agents) {
+        const int g = P.agent_offset + i, tau = P.tau;
+        const double th = st.theta[g], v = st.v[g], w = st.w[g];
+        c.x = st.x[g]; c.y = st.y[g]; c.rad = st.radius[g]; c.pid = st.exploited_patch_id[g]; c.j = i;
+        const int over = st.overriding_mode[g];
+        double m = st.novelty[(int64_t)g * tau];
+        for (int q = 1; q < tau; ++q) m = fmax(m, st.novelty[(int64_t)g * tau + q]);
+        const Drive d = drive_of(P, w, st.u[g], m, st.collected_r[g], st.collected_r_before[g], over,
+                                 st.env_status[g]);
+        const Focal f = focal_at(c.x, c.y, th, (double)c.rad);
+        M.u1[e] = d.u; M.ip[e] = d.ipriv; M.u1x[e] = f.u1x; M.u1y[e] = f.u1y;
+        c.xm = c.x; c.ym = c.y;
+        if (c.pid != -1) {
+            if (over == ABM_MODE_EXPLOIT) flag |= kCueStart;
+            if (d.exploit) {
+                flag |= kCueMoved;
+                const Pose p = fg_move(P, Pose{c.x, c.y, th, v}, 0.0, -v * P.exp_stop_ratio, ABM_MODE_EXPLOIT, w,
+                                       (double)c.rad);
+                c.xm = p.x; c.ym = p.y;
             }
         }
-        uint64_t m = __ballot(live);
-        while (m) {
-            const int l = __builtin_ctzll(m);
-            m &= m - 1;
-            const int s = __builtin_amdgcn_readlane(sx, l), e = __builtin_amdgcn_readlane(ex, l);
-#pragma unroll
-            for (int qw = 0; qw < 4; ++qw) {
-                const int w = lane + 64 * qw;
-                if (w < W) bits[qw] |= interval_word(w, s, e, R);
-            }
-        }
+        c.flag = flag;
     }
-    // counts of the returned field: the kept raw range [ta, tb] and its left half
-    const int nl = R / 2;
-    const int ta = R - 1 - P.keep_hi, tb = R - 1 - P.keep_lo, la = max(R - nl, ta);
-    int tot = 0, left = 0;
-#pragma unroll
-    for (int qw = 0; qw < 4; ++qw) {
-        const int w = lane + 64 * qw;
-        if (w < W) {
-            tot += __popc(bits[qw] & word_range_mask(w, ta, tb));
-            left += __popc(bits[qw] & word_range_mask(w, la, tb));
-        }
+    const uint64_t m = __ballot(flag != 0);
+    if (m) {
+        int at = 0;
+        if (lane == 0) at = atomicAdd(&ctl[kWdCues], (int)__popcll(m));
+        at = __builtin_amdgcn_readfirstlane(at) + 64 * chunk0;
+        if (flag) M.cue[at + (int)__popcll(m & ((1ull << lane) - 1ull))] = c;
     }
-    const int n_set = wave_sum(tot), n_left = wave_sum(left);
-    if (bits_out) {
-        // soc_v_field[q] = V[R-1-q] on the kept rays
-#pragma unroll
-        for (int qw = 0; qw < 4; ++qw) {
-            const int w = lane + 64 * qw;
-            if (w < W) raw[wv][w] = bits[qw];
-        }
-        fg_wave_sync();
-        uint32_t* dst = bits_out + P.field_offset + (int64_t)k * W;
-        for (int wd = lane; wd < W; wd += 64) {
-            uint32_t mm = 0u;
-            for (int b = 0; b < 32; ++b) {
-                const int q = wd * 32 + b, r = R - 1 - q;
-                if (q >= P.keep_lo && q <= P.keep_hi && ((raw[wv][r >> 5] >> (r & 31)) & 1u)) mm |= 1u << b;
-            }
-            dst[wd] = mm;
-        }
-    }
-    if (lane != 0) return;
-    // ---- the decision of agent k (agent.py:168-265), as in the step kernel
-    double w = st.w[gk], u = st.u[gk];
-    const double vel0 = st.v[gk], cr = st.collected_r[gk], crb = st.collected_r_before[gk];
-    double nov = st.novelty[(int64_t)gk * P.tau];
-    for (int q = 1; q < P.tau; ++q) nov = fmax(nov, st.novelty[(int64_t)gk * P.tau + q]);
-    int over = st.overriding_mode[gk], mode = st.mode[gk];
-    const int env = st.env_status[gk];
-    const double count = (double)n_set, cleft = (double)n_left;
-    const double collected = cr - crb;
-    const double ipriv = P.F_N * nov + P.F_R * collected;
-    const double w_p = w > P.T_w ? w : 0.0;
-    const double u_p = u > P.T_u ? u : 0.0;
-    const double mean = count / (double)R;
-    const double dw = P.Eps_w * mean - P.g_w * (w - P.B_w) - u_p * P.S_uw;
-    const double du = P.Eps_u * ipriv - P.g_u * (u - P.B_u) - w_p * P.S_wu;
-    w = w + dw;
-    u = u + du;
-    if (w > P.w_max) w = P.w_max;
-    if (w < -P.w_max) w = -P.w_max;
-    if (u > P.u_max) u = P.u_max;
-    if (u < -P.u_max) u = -P.u_max;
-    double dvel = 0.0, dth = 0.0;
-    int kind = 1;
-    const bool tw = w > P.T_w, tu = u > P.T_w;   // tr_u compares with T_w
-    auto walk = [&]() {
-        kind = 0;
-        dvel = P.exp_vel_max;
-        over = -1; mode = ABM_MODE_EXPLORE;
-    };
-    auto reloc = [&]() {
-        const double lm = cleft / (double)nl;
-        const double rm = (count - cleft) / (double)(R - nl);
-        dvel = P.exp_vel_max - vel0;
-        dth = (lm - rm) * P.reloc_theta_max;
-        over = -1; mode = ABM_MODE_RELOCATE;
-    };
-    auto exploit = [&]() {
-        over = ABM_MODE_EXPLOIT; mode = ABM_MODE_EXPLOIT;
-        dvel = -vel0 * P.exp_stop_ratio;
-        dth = 0.0;
-    };
-    if (over != ABM_MODE_COLLIDE) {
-        if (!tw && !tu) walk();
-        else if (tw && tu) { if (env == 1) exploit(); else reloc(); }
-        else if (tw && !tu) reloc();
-        else { if (env == 1) exploit(); else walk(); }
-    }
-    Xn.w[k] = w; Xn.u[k] = u; Xn.ip[k] = ipriv;
-    Xn.over[k] = over; Xn.mode[k] = mode; Xn.kind[k] = kind;
-    Xn.dth[k] = dth; Xn.dvel[k] = dvel;
 }
 
-// One block of 1024 threads: the draw indices (a scan of the walk flags in
-// id order), the moves of X^{m+1}, the comparison with X^m and the next
-// candidates.  The agents go in chunks of one per thread, so every load is
-// coalesced; a chunk's draw indices come from wave ballots and the waves'
-// totals in LDS.
-__global__ void __launch_bounds__(1024)
-sweep_motion_kernel(const FGRep* __restrict__ reps, int rb, abm_forage_state st, SweepX Xc, SweepX Xn,
-                    const double* __restrict__ uni, int32_t* __restrict__ cand, int32_t* __restrict__ ctrl) {
+// One wave per agent, sixteen blocks per chunk: its field from the cues, the
+// counts and whether it walks.  With device generators the first n_reps blocks
+// make each replica's next 2N words meanwhile.
+template <bool FIELDS>
+__global__ void __launch_bounds__(256)
+wide_field_kernel(const FGRep* __restrict__ reps, int n_reps, abm_forage_state st, WideMem M,
+                  const abm_mt19937_state* __restrict__ mt, uint32_t* __restrict__ bits_out) {
 #pragma clang fp contract(off)
-    __shared__ int wtot[2][16];
-    __shared__ int changed;
-    if (ctrl[kSwConverged] | ctrl[kSwSkip]) return;   // uniform over the block
-    const FGRep& P = reps[rb];
-    const int N = P.n_agents, a0 = P.agent_offset, tid = threadIdx.x, nthr = blockDim.x;
-    const int lane = tid & 63, wave = tid >> 6, nw = nthr >> 6;
-    if (tid == 0) changed = 0;
-    auto bits_ne = [](double a, double b) { return __double_as_longlong(a) != __double_as_longlong(b); };
-    bool diff = false;
-    int d_base = 0;   // draws before the chunk (uniform over the block)
-    for (int c0 = 0, par = 0; c0 < N; c0 += nthr, par ^= 1) {
-        const int k = c0 + tid;
-        const bool in = k < N;
-        const int kind = in ? Xn.kind[k] : 1;
-        const uint64_t m = __ballot(kind == 0);
-        if (lane == 0) wtot[par][wave] = (int)__popcll(m);
-        __syncthreads();   // wtot[par] is rewritten two chunks later, after this chunk's barrier
-        int d = d_base + (int)__popcll(m & ((1ull << lane) - 1ull)), tot = 0;
-        for (int w = 0; w < nw; ++w) {
-            const int t = wtot[par][w];
-            if (w < wave) d += t;
-            tot += t;
+    extern __shared__ uint32_t lds_u[];
+    const int tid = threadIdx.x;
+    int block = blockIdx.x;
+    if (mt) {
+        if (block < n_reps) {
+            if (M.ctl[kWdWords * block + kWdSkip]) return;   // uniform over the block
+            const int rb = M.rep[block].rb, N = reps[rb].n_agents;
+            uint32_t* const keys = M.keys + M.rep[block].keys;
+            uint32_t* const uni = M.uni + 128 * (int64_t)M.rep[block].chunk0;
+            for (int i = tid; i < kMtN; i += 256) lds_u[i] = mt[rb].key[i];
+            __syncthreads();
+            int made = 0, p = mt[rb].pos, twists = 0;
+            while (made < 2 * N) {
+                if (p >= kMtN) {
+                    mt_twist_block(lds_u);
+                    for (int i = tid; i < kMtN; i += 256) keys[(int64_t)twists * kMtN + i] = lds_u[i];
+                    ++twists;
+                    p = 0;
+                }
+                const int take = min(kMtN - p, 2 * N - made);
+                for (int j = tid; j < take; j += 256) uni[made + j] = mt_temper(lds_u[p + j]);
+                made += take;
+                p += take;
+                __syncthreads();
+            }
+            return;
         }
-        d_base += tot;
-        if (!in) continue;
+        block -= n_reps;
+    }
+    const int chunk = block >> 4, q = M.of[chunk], chunk0 = M.rep[q].chunk0;
+    const int32_t* const ctl = M.ctl + kWdWords * q;
+    if (ctl[kWdSkip]) return;
+    const FGRep& P = reps[M.rep[q].rb];
+    const int N = P.n_agents, R = P.n_rays, W = P.words, a0 = P.agent_offset;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int k = (chunk - chunk0) * 64 + (block & 15) * 4 + wave, e = chunk0 * 64 + k;
+    if (k >= N) return;   // uniform over the wave; no block barrier below
+    const int gk = a0 + k;
+    uint32_t* V = lds_u + wave * W;
+    for (int w = lane; w < W; w += 64) V[w] = 0u;
+    Focal f;
+    f.radius = (double)st.radius[gk];
+    f.px = st.x[gk]; f.py = st.y[gk];
+    f.cx = f.px + f.radius;
+    f.cy = f.py + f.radius;
+    f.u1x = M.u1x[e]; f.u1y = M.u1y[e];
+    const int pid_k = st.exploited_patch_id[gk], patchwise = P.patchwise;
+    const FastRec FR = fast_rec_const(R, P.step, P.fov0, P.fov1);
+    const RangeTest rt = range_test(P.vision_range);
+    const double step = P.step, fov0 = P.fov0, fov1 = P.fov1;
+    const int n_cue = ctl[kWdCues];
+    const WideCue* const cues = M.cue + 64 * (int64_t)chunk0;
+    fg_wave_sync();
+    for (int i = lane; i < n_cue; i += 64) {
+        const WideCue c = cues[i];
+        const bool moved = c.j < k;
+        // agent.py:396-413, as the update kernel
+        if (c.j == k || !(c.flag & (moved ? kCueMoved : kCueStart)) || (patchwise && c.pid == pid_k)) continue;
+        const double ox = moved ? c.xm : c.x, oy = moved ? c.ym : c.y, rj = (double)c.rad;
+        if (!in_range(rt, (ox + rj) - f.cx, (oy + rj) - f.cy)) continue;
+        const Rec rc = record_at(ox, oy, kSocial, c.j, f, R, step, fov0, fov1, FR, false);
+        if (rc.valid) paint_bits(V, rc, R);
+    }
+    fg_wave_sync();
+    int n_set, n_left;
+    wave_counts(V, R, W, P.keep_lo, P.keep_hi, FIELDS ? bits_out + P.field_offset + (int64_t)k * W : nullptr,
+                &n_set, &n_left);
+    if (lane == 0) {
+        M.nset[e] = n_set; M.nleft[e] = n_left;
+        M.walk[e] = choose(P, R, n_set, n_left, st.w[gk], st.u[gk], M.u1[e], st.v[gk], st.overriding_mode[gk],
+                           st.mode[gk], st.env_status[gk]).kind == 0;
+    }
+}
+
+// One thread per agent: the walk's draw index (the flags of every agent
+// before it), the choice and the move, written to the state.  A replica's
+// first chunk also leaves the words used, the status and the device generator
+// advanced by them.
+__global__ void __launch_bounds__(256)
+wide_move_kernel(const FGRep* __restrict__ reps, int n_chunks, abm_forage_state st,
+                 const double* __restrict__ uniforms, const uint32_t* __restrict__ words,
+                 const int64_t* __restrict__ u_off, const int32_t* __restrict__ u_cnt,
+                 int32_t* __restrict__ u_used, int32_t* __restrict__ status,
+                 abm_mt19937_state* __restrict__ mt, WideMem M) {
+#pragma clang fp contract(off)
+    const int lane = threadIdx.x & 63;
+    const int chunk = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+    if (chunk >= n_chunks) return;
+    const int q = M.of[chunk], rb = M.rep[q].rb, chunk0 = M.rep[q].chunk0;
+    int32_t* const ctl = M.ctl + kWdWords * q;
+    if (ctl[kWdSkip]) return;
+    const FGRep& P = reps[rb];
+    const int N = P.n_agents, R = P.n_rays, a0 = P.agent_offset;
+    const bool first = chunk == chunk0;
+    // walks before this chunk (the first: in all), sixteen flags at a time
+    const uint8_t* const walk = M.walk + 64 * (int64_t)chunk0;
+    const int upto = first ? N : (chunk - chunk0) * 64;
+    int n = 0;
+    for (int i = lane * 16; i < upto; i += 1024) {
+        const uint4 f = *reinterpret_cast<const uint4*>(walk + i);
+        const uint32_t four[4] = {f.x, f.y, f.z, f.w};
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const int left = upto - i - 4 * t;   // flags of this word that count
+            n += __popc(left >= 4 ? four[t] : (left <= 0 ? 0u : four[t] & ((1u << (8 * left)) - 1u)));
+        }
+    }
+    const int total = wave_sum(n);
+    const int k = (chunk - chunk0) * 64 + lane, e = chunk * 64 + lane;
+    const bool walks = k < N && M.walk[e] != 0;
+    const uint64_t m = __ballot(walks);
+    const int d = (first ? 0 : total) + (int)__popcll(m & ((1ull << lane) - 1ull));
+    const int used0 = ctl[kWdUsed0];
+    if (k < N) {
         const int g = a0 + k;
-        double dth = Xn.dth[k];
-        if (kind == 0) {
-            const double uu = d < N ? uni[d] : NAN;
+        const double vel0 = st.v[g];
+        const Choice c = choose(P, R, M.nset[e], M.nleft[e], st.w[g], st.u[g], M.u1[e], vel0,
+                                st.overriding_mode[g], st.mode[g], st.env_status[g]);
+        double dth = c.dth;
+        if (walks) {
+            double uu = NAN;   // past the end of the buffer
+            if (mt) {
+                const uint32_t* uni = M.uni + 128 * (int64_t)chunk0;
+                uu = words_to_double(uni[2 * d], uni[2 * d + 1]);
+            } else if (words) {
+                const uint32_t* wb = words + u_off[rb];
+                const int at = used0 + 2 * d;
+                if (at + 2 <= u_cnt[rb]) uu = words_to_double(wb[at], wb[at + 1]);
+            } else if (d < u_cnt[rb]) {
+                uu = uniforms[u_off[rb] + d];
+            }
             dth = P.exp_theta_min + (P.exp_theta_max - P.exp_theta_min) * uu;
         }
-        Pose p{st.x[g], st.y[g], st.theta[g], st.v[g]};
-        p.theta = prove_orientation(p.theta + dth);
-        double sn, cs;
-        sincos(p.theta, &sn, &cs);
-        p.v = p.v + Xn.dvel[k];
-        // prove_velocity (agent.py:612-620): only in explore mode
-        if (get_mode(Xn.over[k], Xn.w[k], P.T_w) == ABM_MODE_EXPLORE && fabs(p.v) > 1.0) p.v = P.exp_vel_max;
-        p.x = p.x + p.v * cs;
-        p.y = p.y - p.v * sn;
-        p = reflect_walls(p, (double)st.radius[g], P.pad, P.width, P.height);
-        Xn.x[k] = p.x; Xn.y[k] = p.y; Xn.th[k] = p.theta; Xn.v[k] = p.v;
-        diff = diff || bits_ne(p.x, Xc.x[k]) || bits_ne(p.y, Xc.y[k]) || bits_ne(p.theta, Xc.th[k]) ||
-               bits_ne(p.v, Xc.v[k]) || bits_ne(Xn.w[k], Xc.w[k]) || bits_ne(Xn.u[k], Xc.u[k]) ||
-               bits_ne(Xn.ip[k], Xc.ip[k]) || Xn.over[k] != Xc.over[k] || Xn.mode[k] != Xc.mode[k] ||
-               kind != Xc.kind[k];
-    }
-    if (diff) changed = 1;   // benign race: every writer stores 1
-    __syncthreads();
-    if (tid == 0) {
-        ctrl[kSwDraws] = d_base;
-        ctrl[kSwIters] += 1;
-    }
-    if (!changed) {
-        if (tid == 0) ctrl[kSwConverged] = 1;
-        return;   // uniform over the block
-    }
-    sweep_candidates(st, a0, N, Xn.over, cand, ctrl);
-}
-
-// Writes the converged sweep into the state (one block of 1024 threads):
-// poses, decision state, collected_r_before, the words used and status, and
-// the device generator advanced by the words drawn (the key the prep
-// twisted to).
-__global__ void __launch_bounds__(1024)
-sweep_commit_kernel(const FGRep* __restrict__ reps, int rb, abm_forage_state st, SweepX X,
-                    int32_t* __restrict__ u_used, int32_t* __restrict__ status, int words_or_mt,
-                    abm_mt19937_state* __restrict__ mt, const uint32_t* __restrict__ keys,
-                    int32_t* __restrict__ ctrl) {
-    __shared__ uint32_t key[kMtN];
-    if (ctrl[kSwSkip]) return;
-    if (!ctrl[kSwConverged]) {
-        if (threadIdx.x == 0) ctrl[kSwBad] = 1;
-        return;
-    }
-    const FGRep& P = reps[rb];
-    const int N = P.n_agents, a0 = P.agent_offset, tid = threadIdx.x, nthr = blockDim.x;
-    for (int i = tid; i < N; i += nthr) {
-        const int g = a0 + i;
-        st.x[g] = X.x[i]; st.y[g] = X.y[i]; st.theta[g] = X.th[i]; st.v[g] = X.v[i];
-        st.w[g] = X.w[i]; st.u[g] = X.u[i]; st.I_priv[g] = X.ip[i];
+        const Pose p = fg_move(P, Pose{st.x[g], st.y[g], st.theta[g], vel0}, dth, c.dvel, c.over, c.w,
+                               (double)st.radius[g]);
+        st.x[g] = p.x; st.y[g] = p.y; st.theta[g] = p.theta; st.v[g] = p.v;
+        st.w[g] = c.w; st.u[g] = M.u1[e]; st.I_priv[g] = M.ip[e];
         st.collected_r_before[g] = st.collected_r[g];
-        st.mode[g] = X.mode[i]; st.overriding_mode[g] = X.over[i];
+        st.mode[g] = c.mode; st.overriding_mode[g] = c.over;
     }
-    const int draws = ctrl[kSwDraws];
-    if (tid == 0 && u_used) u_used[rb] = ctrl[kSwUsed0] + (words_or_mt ? 2 : 1) * draws;
-    if (tid == 0 && status) status[rb] = ABM_WORLD_DONE;
+    if (!first) return;
     if (mt) {
-        // numpy's state after the 2 * draws words: the key twisted v times at
-        // position pos0 + c - 624 v (as the step kernel)
-        const int c = 2 * draws;
-        int v = 0, pos = ctrl[kSwPos0] + c;
+        // numpy's state after the 2 * total words: the key twisted v times at
+        // position pos0 + c - 624 v (it twists lazily, when a word is drawn)
+        int v = 0, pos = mt[rb].pos + 2 * total;
         if (pos > kMtN) {
             v = (pos - 1) / kMtN;
             pos -= kMtN * v;
+            const uint32_t* const key = M.keys + M.rep[q].keys + (int64_t)(v - 1) * kMtN;
+            for (int i = lane; i < kMtN; i += 64) mt[rb].key[i] = key[i];
         }
-        // the prep kept every key it twisted, and c <= 2N words never need
-        // more; twisting here again is only the fallback
-        if (v > ctrl[kSwTwists]) {   // uniform over the block
-            for (int i = tid; i < kMtN; i += nthr) key[i] = mt[rb].key[i];
-            __syncthreads();
-            for (int t = 0; t < v; ++t) mt_twist_block(key);
-            for (int i = tid; i < kMtN; i += nthr) mt[rb].key[i] = key[i];
-        } else if (v > 0) {
-            for (int i = tid; i < kMtN; i += nthr) mt[rb].key[i] = keys[(int64_t)(v - 1) * kMtN + i];
-        }
-        if (tid == 0) mt[rb].pos = pos;
+        if (lane == 0) mt[rb].pos = pos;
+    }
+    if (lane == 0) {
+        ctl[kWdCues] = 0;   // for the next step's drive kernel
+        ctl[kWdUpdates] += 1;
+        if (u_used) u_used[rb] = used0 + (words || mt ? 2 : 1) * total;
+        if (status) status[rb] = ABM_WORLD_DONE;
     }
 }
 
@@ -2568,57 +2396,107 @@ using namespace abm;
 namespace {
 
 constexpr int kForageMaxAgents = 65536;
+constexpr int kWideMaxRays = 8192;   // of the update over the whole GPU
+constexpr int kWideMinAgents = 64, kWideMaxPerCu = 96;   // where it is the better one (plan_paths)
 
-// Device bytes of the sweep buffers for replicas of up to M agents: two
-// tentative states (nine double and three int arrays each), the uniforms,
-// the candidates and the control words.
-// generator keys the prep may twist to while making 2M words
-int sweep_key_slots(int M) { return (2 * M + kMtN) / kMtN + 1; }
+// Generator keys a step may twist to while making 2M words.
+int wide_key_slots(int M) { return (2 * M + kMtN) / kMtN + 1; }
 
-size_t sweep_bytes(int M) {
-    return 2 * (size_t)M * (9 * sizeof(double) + 3 * sizeof(int32_t)) + (size_t)M * sizeof(double) +
-           (size_t)M * sizeof(int32_t) + sizeof(uint32_t) * kMtN * (size_t)sweep_key_slots(M) +
-           kSwWords * sizeof(int32_t) + 256;
+// Device memory of the update over the whole GPU for so many replicas, chunks
+// and twisted key words; with base null only its size is found.
+size_t wide_carve(void* base, size_t reps, size_t chunks, size_t key_words, WideMem* m) {
+    const size_t n = 64 * chunks;
+    size_t at = 0;
+    auto take = [&](size_t bytes) {
+        char* p = reinterpret_cast<char*>(base) + at;
+        at += (bytes + 255) & ~(size_t)255;
+        return p;
+    };
+    m->rep = reinterpret_cast<WideRep*>(take(sizeof(WideRep) * reps));
+    m->of = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * chunks));
+    m->cue = reinterpret_cast<WideCue*>(take(sizeof(WideCue) * n));
+    for (double** d : {&m->u1, &m->ip, &m->u1x, &m->u1y}) *d = reinterpret_cast<double*>(take(sizeof(double) * n));
+    for (int32_t** i : {&m->nset, &m->nleft}) *i = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * n));
+    m->uni = reinterpret_cast<uint32_t*>(take(sizeof(uint32_t) * 2 * n));
+    m->keys = reinterpret_cast<uint32_t*>(take(sizeof(uint32_t) * key_words));
+    m->walk = reinterpret_cast<uint8_t*>(take(n));
+    m->ctl = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * kWdWords * reps));
+    return at;
 }
 
-struct SweepMem {
-    SweepX X[2];
-    double* uni;
-    int32_t* cand;
-    uint32_t* keys;
-    int32_t* ctrl;
-};
+// Updates the wide replicas' move kernels have made since the plan.
+int wide_updates(const abm_forage_batch* bt, int64_t* total) {
+    *total = 0;
+    if (!bt->wide_mem) return ABM_OK;
+    WideMem m;
+    const size_t n = bt->wide.size();
+    wide_carve(bt->wide_mem, n, (size_t)bt->wide_chunks, (size_t)bt->wide_keys, &m);
+    std::vector<int32_t> ctl(kWdWords * n);
+    if (int rc = check_hip(hipDeviceSynchronize(), "hipDeviceSynchronize")) return rc;
+    if (int rc = check_hip(hipMemcpy(ctl.data(), m.ctl, sizeof(int32_t) * ctl.size(), hipMemcpyDeviceToHost),
+                           "read wide control"))
+        return rc;
+    for (size_t i = 0; i < n; ++i) *total += ctl[kWdWords * i + kWdUpdates];
+    return ABM_OK;
+}
 
-SweepMem sweep_carve(void* base, int M) {
-    SweepMem m;
-    char* p = reinterpret_cast<char*>(base);
-    for (int q = 0; q < 2; ++q) {
-        double** d[] = {&m.X[q].x, &m.X[q].y, &m.X[q].th, &m.X[q].v, &m.X[q].w, &m.X[q].u, &m.X[q].ip,
-                        &m.X[q].dth, &m.X[q].dvel};
-        for (double** a : d) { *a = reinterpret_cast<double*>(p); p += sizeof(double) * (size_t)M; }
+// The wide replicas' chunks and scratch, laid out once per plan.
+int plan_wide(abm_forage_batch* bt) {
+    if (bt->wide_mem) (void)hipFree(bt->wide_mem);
+    bt->wide_mem = nullptr;
+    bt->wide_chunks = 0;
+    bt->wide_keys = 0;
+    bt->wide_max_rays = 0;
+    if (bt->wide.empty()) return ABM_OK;
+    std::vector<WideRep> rep;
+    std::vector<int32_t> of;
+    for (int b : bt->wide) {
+        rep.push_back(WideRep{b, (int32_t)of.size(), bt->wide_keys});
+        of.insert(of.end(), (bt->rep_n[b] + 63) / 64, (int32_t)rep.size() - 1);
+        bt->wide_keys += (int64_t)kMtN * wide_key_slots(bt->rep_n[b]);
+        bt->wide_max_rays = std::max(bt->wide_max_rays, bt->rep_r[b]);
     }
-    m.uni = reinterpret_cast<double*>(p); p += sizeof(double) * (size_t)M;
-    for (int q = 0; q < 2; ++q) {
-        int32_t** i[] = {&m.X[q].over, &m.X[q].mode, &m.X[q].kind};
-        for (int32_t** a : i) { *a = reinterpret_cast<int32_t*>(p); p += sizeof(int32_t) * (size_t)M; }
-    }
-    m.cand = reinterpret_cast<int32_t*>(p); p += sizeof(int32_t) * (size_t)M;
-    m.keys = reinterpret_cast<uint32_t*>(p); p += sizeof(uint32_t) * kMtN * (size_t)sweep_key_slots(M);
-    m.ctrl = reinterpret_cast<int32_t*>(p);
-    return m;
+    bt->wide_chunks = (int32_t)of.size();
+    WideMem m;
+    const size_t bytes = wide_carve(nullptr, rep.size(), of.size(), (size_t)bt->wide_keys, &m);
+    int rc = check_hip(hipMalloc(&bt->wide_mem, bytes), "hipMalloc(wide update)");
+    if (rc) return rc;
+    wide_carve(bt->wide_mem, rep.size(), of.size(), (size_t)bt->wide_keys, &m);
+    rc = check_hip(hipMemcpy(const_cast<WideRep*>(m.rep), rep.data(), sizeof(WideRep) * rep.size(),
+                             hipMemcpyHostToDevice), "upload wide replicas");
+    if (!rc) rc = check_hip(hipMemcpy(const_cast<int32_t*>(m.of), of.data(), sizeof(int32_t) * of.size(),
+                                      hipMemcpyHostToDevice), "upload wide chunks");
+    if (!rc) rc = check_hip(hipMemset(m.ctl, 0, sizeof(int32_t) * kWdWords * rep.size()), "clear wide control");
+    if (!rc) rc = check_hip(hipDeviceSynchronize(), "plan wide update");
+    return rc;
 }
 
 // Which kernel updates which replica: the update kernel those without visual
 // exclusion that fit one workgroup's LDS, the step kernel those with it, and
-// sweeps those beyond one workgroup's LDS, or (ABM_FORAGE_PATH_SWEEP) every
-// replica without visual exclusion.  A kernel's blocks take their replicas
+// the wide launches those beyond one workgroup's LDS, or every replica without
+// visual exclusion: on request (ABM_FORAGE_PATH_SWEEP), or when the batch's
+// agents are too few to fill the GPU a workgroup per replica and some replica
+// has work for more than one CU (ms a step, wide against a workgroup each: one
+// replica of 512 agents 0.039 and 0.090, of 128 0.029 and 0.037, of 60 0.026
+// both, of 10 0.025 and 0.020; 30 of 512 0.067 and 0.132, 50 of 300 0.066 and
+// 0.093, 100 of 8 to 512 0.064 and 0.113; 300 of 100 0.085 and 0.074, 1000 of 8
+// to 512 0.226 and 0.148).  A kernel's blocks take their replicas
 // largest first (the cost grows with the agents; rays add to each agent's).
 int plan_paths(abm_forage_batch* bt, int path) {
     const int n = bt->n_replicas;
     std::vector<int32_t> plain, occl, big;
+    int64_t agents = 0;
+    int largest = 0;
+    for (int b = 0; b < n; ++b)
+        if (!bt->exclusion[b] && bt->rep_r[b] <= kWideMaxRays) {
+            agents += bt->rep_n[b];
+            largest = std::max(largest, bt->rep_n[b]);
+        }
+    const bool spread = path == ABM_FORAGE_PATH_SWEEP ||
+                        (largest >= kWideMinAgents && agents <= (int64_t)kWideMaxPerCu * bt->cus);
     for (int b = 0; b < n; ++b) {
-        const bool sweepable = !bt->exclusion[b] && bt->rep_r[b] <= 32 * kSweepMaxWords;
-        if (bt->too_big[b] || (path == ABM_FORAGE_PATH_SWEEP && sweepable)) big.push_back(b);
+        const bool wideable = !bt->exclusion[b] && bt->rep_r[b] <= kWideMaxRays;
+        if (bt->too_big[b] || (spread && wideable)) big.push_back(b);
         else (bt->exclusion[b] ? occl : plain).push_back(b);
     }
     auto cost = [&](int b) { return (double)bt->rep_n[b] * (64.0 + bt->rep_r[b] / 32.0); };
@@ -2638,8 +2516,13 @@ int plan_paths(abm_forage_batch* bt, int path) {
     };
     extent(plain, bt->n_plain, bt->plain_max_agents, bt->plain_max_rays);
     extent(occl, bt->n_occl, bt->occl_max_agents, bt->occl_max_rays);
-    bt->sweep = big;
+    // updates counted so far, and no launch left on the scratch that goes
+    int64_t made = 0;
+    if (int rc = wide_updates(bt, &made)) return rc;
+    bt->wide_steps += made;
+    bt->wide = big;
     bt->path = path;
+    if (int rc = plan_wide(bt)) return rc;
     return check_hip(hipMemcpy(bt->order_dev, bt->order_host.data(), sizeof(int32_t) * n,
                                hipMemcpyHostToDevice), "upload forage order");
 }
@@ -2667,50 +2550,26 @@ int check_state(const abm_forage_state* st, const char* who) {
     return ABM_OK;
 }
 
-// Agent.update of replica rb by sweeps (see sweep_field_kernel): the
-// start, then sweeps in rounds of a few (a sweep after convergence returns
-// at once) until the control words report a fixed point, then the commit.
-// Reads the control words after each round, so the call synchronises the
-// stream.
-int sweep_replica(abm_forage_batch* b, int rb, const abm_forage_state* st, const double* uniforms,
-                  const uint32_t* words, const int64_t* offset, const int32_t* count, int32_t* used,
-                  int32_t* status, uint32_t* field_bits, hipStream_t s, abm_mt19937_state* mt) {
-    const int N = b->rep_n[rb];
-    if (N > b->sweep_max_agents || !b->sweep_mem || !b->sweep_ctrl_host)
-        return set_error(ABM_ERR_UNSUPPORTED, "forage replica %d: no sweep buffers for %d agents", rb, N);
-    const SweepMem m = sweep_carve(b->sweep_mem, b->sweep_max_agents);
+// Agent.update of the wide replicas (see wide_drive_kernel).
+int launch_wide(abm_forage_batch* b, const abm_forage_state* st, const double* uniforms,
+                const uint32_t* words, const int64_t* offset, const int32_t* count, int32_t* used,
+                int32_t* status, uint32_t* field_bits, hipStream_t s, abm_mt19937_state* mt) {
+    WideMem m;
+    const int n = (int)b->wide.size(), chunks = b->wide_chunks, W = (b->wide_max_rays + 31) / 32;
+    wide_carve(b->wide_mem, n, chunks, (size_t)b->wide_keys, &m);
     const FGRep* reps = (const FGRep*)b->reps_dev;
-    hipLaunchKernelGGL(sweep_prep_kernel, dim3(1), dim3(1024), 0, s, reps, rb, *st, uniforms, words, offset,
-                       count, used, status, mt, m.X[0], m.uni, m.keys, m.cand, m.ctrl);
-    if (int rc = check_hip(hipGetLastError(), "sweep_prep_kernel launch")) return rc;
-    int par = 0, sweeps = 0, round = 3;
-    for (;;) {
-        for (int i = 0; i < round; ++i) {
-            hipLaunchKernelGGL(sweep_field_kernel, dim3((N + 3) / 4), dim3(256), 0, s, reps, rb, *st,
-                               m.X[par], m.X[par ^ 1], m.cand, m.ctrl, field_bits);
-            hipLaunchKernelGGL(sweep_motion_kernel, dim3(1), dim3(1024), 0, s, reps, rb, *st, m.X[par],
-                               m.X[par ^ 1], m.uni, m.cand, m.ctrl);
-            par ^= 1;
-        }
-        if (int rc = check_hip(hipGetLastError(), "sweep kernels launch")) return rc;
-        sweeps += round;
-        if (int rc = check_hip(hipMemcpyAsync(b->sweep_ctrl_host, m.ctrl, sizeof(int32_t) * kSwWords,
-                                              hipMemcpyDeviceToHost, s), "read sweep control"))
-            return rc;
-        if (int rc = check_hip(hipStreamSynchronize(s), "hipStreamSynchronize(sweeps)")) return rc;
-        if (b->sweep_ctrl_host[kSwSkip]) break;
-        if (b->sweep_ctrl_host[kSwConverged]) {
-            b->sweep_steps += 1;
-            b->sweeps_done += b->sweep_ctrl_host[kSwIters];
-            break;
-        }
-        if (sweeps > N + 2)   // agent k is final after k + 1 sweeps: cannot happen
-            return set_error(ABM_ERR_HIP, "forage replica %d: no fixed point after %d sweeps", rb, sweeps);
-        round = 2;
-    }
-    hipLaunchKernelGGL(sweep_commit_kernel, dim3(1), dim3(1024), 0, s, reps, rb, *st, m.X[par], used, status,
-                       (words || mt) ? 1 : 0, mt, m.keys, m.ctrl);
-    return check_hip(hipGetLastError(), "sweep_commit_kernel launch");
+    const int blocks = (chunks + 3) / 4;
+    hipLaunchKernelGGL(wide_drive_kernel, dim3(blocks), dim3(256), 0, s, reps, chunks, *st, status, used,
+                       (words || mt) ? 1 : 0, m);
+    if (int rc = check_hip(hipGetLastError(), "wide_drive_kernel launch")) return rc;
+    const size_t lds = sizeof(uint32_t) * (size_t)std::max(kMtN, 4 * W);
+    hipLaunchKernelGGL(field_bits ? wide_field_kernel<true> : wide_field_kernel<false>,
+                       dim3(16 * chunks + (mt ? n : 0)), dim3(256), lds, s, reps, n, *st, m, mt, field_bits);
+    if (int rc = check_hip(hipGetLastError(), "wide_field_kernel launch")) return rc;
+    hipLaunchKernelGGL(wide_move_kernel, dim3(blocks), dim3(256), 0, s, reps, chunks, *st, uniforms, words, offset,
+                       count, used, status, mt, m);
+    if (int rc = check_hip(hipGetLastError(), "wide_move_kernel launch")) return rc;
+    return ABM_OK;
 }
 
 // Agent.update for every replica (all, or those a status array marks ready).
@@ -2753,10 +2612,8 @@ int launch_forage_step(abm_forage_batch* b, const abm_forage_state* st, const do
                            b->occl_max_rays);
         if (int rc = check_hip(hipGetLastError(), "forage_step_kernel launch")) return rc;
     }
-    for (int rb : b->sweep)
-        if (int rc = sweep_replica(b, rb, st, uniforms, words, offset, count, used, status, field_bits,
-                                   (hipStream_t)stream, mt))
-            return rc;
+    if (!b->wide.empty())
+        return launch_wide(b, st, uniforms, words, offset, count, used, status, field_bits, (hipStream_t)stream, mt);
     return ABM_OK;
 }
 
@@ -2821,21 +2678,19 @@ int abm_forage_batch_create(const abm_forage_replica* reps, int32_t n, abm_forag
     int dev_max = 0;
     if (!rc) rc = check_hip(hipDeviceGetAttribute(&dev_max, hipDeviceAttributeMaxSharedMemoryPerBlock,
                                                   bt->device), "hipDeviceGetAttribute");
-    // a replica beyond one workgroup's LDS is updated by sweeps, which do
-    // not implement visual exclusion and hold at most 8192 rays
+    // a replica beyond one workgroup's LDS is updated over the whole GPU,
+    // without visual exclusion and with at most 8192 rays
     bt->too_big.assign(n, 0);
     bt->exclusion.assign(n, 0);
     for (int b = 0; !rc && b < n; ++b) {
         const size_t need = fg_lds_bytes(host[b].n_agents, host[b].n_rays) + sizeof(FGRep);
         bt->too_big[b] = need > (size_t)dev_max;
         bt->exclusion[b] = host[b].visual_exclusion != 0;
-        if (bt->too_big[b] && (host[b].visual_exclusion || host[b].n_rays > 32 * kSweepMaxWords))
+        if (bt->too_big[b] && (host[b].visual_exclusion || host[b].n_rays > kWideMaxRays))
             rc = set_error(ABM_ERR_UNSUPPORTED, "forage replica %d: %d agents x %d rays need %zu B of LDS "
-                           "(one workgroup has %d B); replicas that large are updated by sweeps, which "
-                           "support neither visual exclusion nor more than %d rays", b, host[b].n_agents,
-                           host[b].n_rays, need, dev_max, 32 * kSweepMaxWords);
-        if (!host[b].visual_exclusion && host[b].n_rays <= 32 * kSweepMaxWords)
-            bt->sweep_max_agents = std::max(bt->sweep_max_agents, host[b].n_agents);
+                           "(one workgroup has %d B); replicas that large are updated over the whole GPU, which "
+                           "supports neither visual exclusion nor more than %d rays", b, host[b].n_agents,
+                           host[b].n_rays, need, dev_max, kWideMaxRays);
     }
     bt->order_host.resize(n);
     bt->rep_n.resize(n);
@@ -2845,11 +2700,6 @@ int abm_forage_batch_create(const abm_forage_replica* reps, int32_t n, abm_forag
     if (!rc) rc = check_hip(hipMemcpy(bt->reps_dev, host.data(), sizeof(FGRep) * n, hipMemcpyHostToDevice),
                            "upload forage replicas");
     if (!rc) rc = check_hip(hipMalloc(&bt->order_dev, sizeof(int32_t) * n), "hipMalloc(forage order)");
-    if (!rc && bt->sweep_max_agents > 0)
-        rc = check_hip(hipMalloc(&bt->sweep_mem, sweep_bytes(bt->sweep_max_agents)), "hipMalloc(sweeps)");
-    if (!rc && bt->sweep_max_agents > 0)
-        rc = check_hip(hipHostMalloc((void**)&bt->sweep_ctrl_host, sizeof(int32_t) * kSwWords),
-                       "hipHostMalloc(sweep control)");
     if (!rc) rc = plan_paths(bt, ABM_FORAGE_PATH_AUTO);
     if (rc) { abm_forage_batch_destroy(bt); return rc; }
     bt->agent_offset_host = new int32_t[n + 1];
@@ -2868,8 +2718,7 @@ int abm_forage_batch_destroy(abm_forage_batch* b) {
     if (!b) return ABM_OK;
     if (b->reps_dev) (void)hipFree(b->reps_dev);
     if (b->order_dev) (void)hipFree(b->order_dev);
-    if (b->sweep_mem) (void)hipFree(b->sweep_mem);
-    if (b->sweep_ctrl_host) (void)hipHostFree(b->sweep_ctrl_host);
+    if (b->wide_mem) (void)hipFree(b->wide_mem);
     delete[] b->agent_offset_host;
     delete[] b->field_offset_host;
     delete b;
@@ -2893,8 +2742,9 @@ int abm_forage_batch_get_offsets(const abm_forage_batch* b, int32_t* agent_offse
 
 int abm_forage_sweep_counts(const abm_forage_batch* b, int64_t* updates, int64_t* sweeps) {
     if (!b || !updates || !sweeps) return set_error(ABM_ERR_INVALID, "abm_forage_sweep_counts: NULL argument");
-    *updates = b->sweep_steps;
-    *sweeps = b->sweeps_done;
+    int64_t made = 0;
+    if (int rc = wide_updates(b, &made)) return rc;
+    *updates = *sweeps = b->wide_steps + made;
     return ABM_OK;
 }
 

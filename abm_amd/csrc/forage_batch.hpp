@@ -22,19 +22,19 @@ struct abm_forage_batch {
     int64_t* field_offset_host = nullptr;
     // Replicas the update kernel takes (the first n_plain of order_dev), those
     // with visual exclusion, which the step kernel takes (the next n_occl),
-    // and the ones beyond one workgroup's LDS, updated by sweeps.
+    // and the ones beyond one workgroup's LDS, updated over the whole GPU.
     int32_t n_plain = 0, n_occl = 0;
     int32_t plain_max_agents = 0, plain_max_rays = 0, occl_max_agents = 0, occl_max_rays = 0;
     int32_t path = 0;                  // ABM_FORAGE_PATH_*
     std::vector<int32_t> rep_n, rep_r; // agents and rays of every replica
-    std::vector<int32_t> order_host;   // every replica: update kernel's, step kernel's, swept
+    std::vector<int32_t> order_host;   // every replica: update kernel's, step kernel's, wide
     std::vector<uint8_t> too_big;      // [b]: beyond one workgroup's LDS
     std::vector<uint8_t> exclusion;    // [b]: visual exclusion
-    std::vector<int32_t> sweep;        // replicas updated by sweeps
-    int32_t sweep_max_agents = 0;      // the sweep buffers' capacity
-    void* sweep_mem = nullptr;         // two tentative states, uniforms, candidates, control
-    int32_t* sweep_ctrl_host = nullptr;   // pinned copy of the control words
-    int64_t sweep_steps = 0, sweeps_done = 0;   // replica updates by sweeps, sweeps they took
+    std::vector<int32_t> wide;         // replicas updated over the whole GPU
+    int32_t wide_chunks = 0, wide_max_rays = 0;   // their 64-agent chunks, their largest field
+    int64_t wide_keys = 0;             // words of their generators' twisted keys
+    void* wide_mem = nullptr;          // their map, cues, drives, counts, words, control
+    int64_t wide_steps = 0;            // replica updates made that way under earlier plans
 };
 
 // The resource patches' per-replica constants and pending-placement scratch

@@ -166,16 +166,16 @@ class ForageSwarm:
         return slice(int(self.agent_offset[b]), int(self.agent_offset[b + 1]))
 
     def set_path(self, path: str = "auto"):
-        """How replicas are updated: "auto" (the step kernel for replicas that
-        fit one workgroup's LDS, sweeps for larger ones) or "sweep" (sweeps for
-        every replica without visual exclusion; the same results, used to
-        compare the two).  Sweeps read a few control words per round, so a
-        step with swept replicas synchronises the stream."""
+        """How replicas are updated: "auto" (one workgroup each for replicas
+        that fit its LDS, a sweep over the whole GPU for larger ones) or
+        "sweep" (that sweep for every replica without visual exclusion; the
+        same results, used to compare the two)."""
         code = {"auto": L.FORAGE_PATH_AUTO, "sweep": L.FORAGE_PATH_SWEEP}[path]
         L.check(self.lib.abm_forage_set_path(self.handle, code))
 
     def sweep_counts(self):
-        """(replica updates made by sweeps, sweeps they took) since creation."""
+        """(replica updates made by sweeps over the whole GPU, sweeps they took:
+        one each) since creation."""
         u, s = C.c_int64(), C.c_int64()
         L.check(self.lib.abm_forage_sweep_counts(self.handle, C.byref(u), C.byref(s)))
         return u.value, s.value

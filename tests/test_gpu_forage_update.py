@@ -66,3 +66,44 @@ def test_many_small_replicas_equal_few(gpu):
             assert np.array_equal(gm[k][-n:], gf[k]), (step, k)
         fm, ff = many.fields.cpu().numpy(), few.fields.cpu().numpy()
         assert np.array_equal(fm[-len(ff):], ff), step
+
+
+# a chunk of 64 agents less one, full and one more, several chunks, several
+# replicas in the three launches; host words and device generators
+@pytest.mark.parametrize("device_rng", [False, True])
+def test_update_over_the_whole_gpu_equals_a_workgroup_each(gpu, device_rng):
+    from abm_amd.forage import ResourceWorld, WorldConfig
+    worlds = []
+    for b, (n, R) in enumerate([(63, 100), (64, 64), (65, 1024), (1, 33), (200, 2081), (130, 512)]):
+        ags, kw = make_world(9000 + b, N=n, R=R, W=500, mixed=False)
+        worlds.append((ags, R, kw))
+    pair = []
+    for path in ("auto", "sweep"):
+        rngs = [np.random.RandomState(50 + b) for b in range(len(worlds))]
+        sw = _swarm(worlds, rngs)
+        if path == "auto":   # enough other replicas that the batch takes a workgroup each
+            extra = [make_world(9100 + b, N=80, R=96, W=400, mixed=False) for b in range(400)]
+            rngs += [np.random.RandomState(1000 + b) for b in range(400)]
+            sw = _swarm(worlds + [(a, 96, kw) for a, kw in extra], rngs)
+        else:
+            sw.set_path(path)
+        rw = ResourceWorld(sw, [WorldConfig(N_resc=4, min_resc_perpatch=3, max_resc_perpatch=9)] * len(rngs),
+                           device_rng=device_rng)
+        rw.create_resources()
+        pair.append((sw, rw, rngs))
+    (a, ra, ga), (s, rs, gs) = pair
+    n = len(s.get_state("x")["x"])
+    for step in range(40):
+        ra.step(fields=True)
+        rs.step(fields=True)
+        fa, fs = a.get_state(), s.get_state()
+        for k in ("x", "y", "theta", "v", "w", "u", "I_priv", "collected_r_before", "mode", "overriding_mode"):
+            assert np.array_equal(fa[k][:n], fs[k]), (step, k)
+        bits = s.fields.cpu().numpy()
+        assert np.array_equal(a.fields.cpu().numpy()[:len(bits)], bits), step
+    ra.sync_rng()
+    rs.sync_rng()
+    for b in range(len(worlds)):
+        assert ga[b].get_state()[2] == gs[b].get_state()[2], b
+        assert np.array_equal(ga[b].get_state()[1], gs[b].get_state()[1]), b
+    assert s.sweep_counts()[0] == 40 * len(worlds) and a.sweep_counts()[0] == 0
