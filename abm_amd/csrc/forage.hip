@@ -612,18 +612,34 @@ __device__ inline uint32_t mt_twist_word(uint32_t cur, uint32_t nxt, uint32_t fa
     return far ^ (y >> 1) ^ ((y & 1u) ? 0x9908b0dfu : 0u);
 }
 
-// key[i] for i = 0..623 in order, in place, by one thread.
-__device__ inline void mt_twist_serial(uint32_t* key) {
-    int i = 0;
-    for (; i < kMtN - kMtM; ++i) key[i] = mt_twist_word(key[i], key[i + 1], key[i + kMtM]);
-    for (; i < kMtN - 1; ++i) key[i] = mt_twist_word(key[i], key[i + 1], key[i + kMtM - kMtN]);
-    key[kMtN - 1] = mt_twist_word(key[kMtN - 1], key[0], key[kMtM - 1]);
+// key[i] for i = 0..623 in order, in place, by one wave: in the chunks [0, 227),
+// [227, 454), [454, 623) and {623} every element reads key[i + 1] not yet
+// rewritten and key[(i + 397) % 624] already final, so each chunk is read in
+// full, then written.
+__device__ inline void mt_twist_wave(uint32_t* key) {
+    const int lane = threadIdx.x & 63;
+    constexpr int lo[4] = {0, kMtN - kMtM, 2 * (kMtN - kMtM), kMtN - 1};
+    constexpr int hi[4] = {kMtN - kMtM, 2 * (kMtN - kMtM), kMtN - 1, kMtN};
+#pragma unroll
+    for (int c = 0; c < 4; ++c) {
+        uint32_t v[4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const int i = lo[c] + lane + 64 * t;
+            const int far = i + kMtM < kMtN ? i + kMtM : i + kMtM - kMtN;
+            v[t] = i < hi[c] ? mt_twist_word(key[i], key[i + 1 < kMtN ? i + 1 : 0], key[far]) : 0u;
+        }
+        fg_wave_sync();
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const int i = lo[c] + lane + 64 * t;
+            if (i < hi[c]) key[i] = v[t];
+        }
+        fg_wave_sync();
+    }
 }
 
-// The same by a block of at least 227 threads: in the chunks [0, 227),
-// [227, 454), [454, 623) and {623} every element reads key[i + 1] not yet
-// rewritten and key[(i + 397) % 624] already final, so each chunk is read
-// in full, then written.  Every thread of the block calls it.
+// The same by a block of at least 227 threads, all of which call it.
 __device__ inline void mt_twist_block(uint32_t* key) {
     const int tid = threadIdx.x;
     constexpr int lo[4] = {0, kMtN - kMtM, 2 * (kMtN - kMtM), kMtN - 1};
@@ -643,14 +659,15 @@ __device__ inline void mt_twist_block(uint32_t* key) {
     }
 }
 
-// Draws from a generator state held in LDS by one thread; never runs out.
+// Draws from a generator state held in LDS, by one wave (every lane the same
+// draw); never runs out.
 struct MtCursor {
     uint32_t* key;
     int pos, used;
     bool out;
     __device__ uint32_t next() {
         if (pos >= kMtN) {
-            mt_twist_serial(key);
+            mt_twist_wave(key);
             pos = 0;
         }
         ++used;
@@ -1589,7 +1606,6 @@ wide_move_kernel(const FGRep* __restrict__ reps, int n_chunks, abm_forage_state 
 
 // ------------------------------------------------ agent-resource interaction
 constexpr int kMaxPatches = 64;     // patches per replica (one 64-bit membership word)
-constexpr int kMaxWorldChunks = 1024;   // 64-agent words of a replica's membership (65536 agents)
 constexpr int kMaxRetries = 10000;  // add_new_resource_patch's max_retries (sims.py:335)
 
 // Pending patch placements of a replica, kept between a phase that ran out of
@@ -1598,7 +1614,7 @@ constexpr int kPendNone = 0, kPendKill = 1, kPendFill = 2;
 
 // Per-replica world constants on the device.
 struct WRep {
-    int32_t n_patches, patch_radius, pooling_time, regenerate, teleport, collide, ghost, pad_;
+    int32_t n_patches, patch_radius, pooling_time, regenerate, teleport, collide, ghost, n_agents;
     int64_t patch_offset;
     int64_t x_lo, x_hi, y_lo, y_hi, units_lo, units_hi;   // randint bounds [lo, hi)
     double consumption, q_lo, q_hi;
@@ -1695,83 +1711,69 @@ struct FreshPatch {
 // Place the replica's pending patches (regenerations of the patches killed
 // this step, in kill order, or create_resources' new patches) from the word
 // buffer, then compact the list: live patches in order, new ones appended.
-// One thread.  Commits nothing unless every placement fits in the buffer.
+// One wave, lane t holding patch t and new patch t (at most 64 of each): the
+// draws are the same on every lane, the overlap tests one patch per lane.
+// Commits nothing unless every placement fits in the buffer.
+static_assert(kMaxPatches == 64, "a lane per patch");
 template <typename Cursor>
-__device__ int place_patches(const WRep& W, abm_patch_state ps, int b, int kind, int n_pending,
-                             const int32_t* __restrict__ pend_id, int32_t* __restrict__ kill_rank,
-                             Cursor& cur, FreshPatch* fresh) {
+__device__ int place_patches(const WRep& W, const abm_patch_state& ps, int b, int kind, int n_pending,
+                             const int32_t* __restrict__ pend_id, int32_t* __restrict__ kill_rank, Cursor& cur) {
     const int64_t po = W.patch_offset;
-    const int count = ps.count[b];
+    const int lane = threadIdx.x & 63, count = ps.count[b];
     int n_new = 0;
     if (kind == kPendKill) n_new = W.regenerate ? n_pending : 0;
     else if (kind == kPendFill) n_new = W.n_patches - count;
-    const int64_t r = W.patch_radius;
+    const int64_t r = W.patch_radius, s = po + lane;
+    const bool held = lane < count;
+    double px = 0.0, py = 0.0, pr = 0.0, units = 0.0, left = 0.0, quality = 0.0;
+    int32_t id = 0, rank = -1, pend = 0;
+    if (held) {
+        px = ps.x[s]; py = ps.y[s]; pr = ps.radius[s]; units = ps.units[s]; left = ps.left[s];
+        quality = ps.quality[s]; id = ps.id[s]; rank = kill_rank[s];
+    }
+    if (kind == kPendKill && lane < n_new) pend = pend_id[s];   // force_id: the killed patch's id
+    const int64_t pcx = (int64_t)trunc(px + pr), pcy = (int64_t)trunc(py + pr), pri = (int64_t)pr;
+    int32_t top = held ? id : INT32_MIN;   // the largest id, for create_resources
+    for (int d = 1; d < 64; d <<= 1) top = max(top, __shfl_xor(top, d, 64));
+    if (count == 0) top = 0;
+    FreshPatch mine{0, 0, 0, 0.0, 0.0};
     for (int k = 0; k < n_new; ++k) {
-        int32_t id;
-        if (kind == kPendKill) {
-            id = pend_id[po + k];                 // force_id: the killed patch's id
-        } else {
-            bool any = false;                     // max(ids) + 1, or 1 for an empty list
-            int32_t mx = 0;
-            for (int t = 0; t < count; ++t) {
-                const int32_t v = ps.id[po + t];
-                if (!any || v > mx) mx = v;
-                any = true;
-            }
-            for (int f = 0; f < k; ++f) {
-                if (!any || fresh[f].id > mx) mx = fresh[f].id;
-                any = true;
-            }
-            id = (any ? mx : 0) + 1;
-        }
-        int retries = 0;
-        for (;;) {
+        for (int retries = 0;; ++retries) {
             if (retries > kMaxRetries) return ABM_WORLD_TIMEOUT;
             const int64_t x = np_randint(cur, W.x_lo, W.x_hi);
             const int64_t y = np_randint(cur, W.y_lo, W.y_hi);
-            const int64_t units = np_randint(cur, W.units_lo, W.units_hi);
+            const int64_t u = np_randint(cur, W.units_lo, W.units_hi);
             const double q = np_uniform(cur, W.q_lo, W.q_hi);
             if (cur.out) return ABM_WORLD_NEED_WORDS;
             const int64_t cx = x + r, cy = y + r;
-            bool ok = true;
             // the Group at the time: live patches, those killed later this
             // step, and the ones placed before this one
-            for (int t = 0; t < count && ok; ++t) {
-                const int64_t s = po + t;
-                if (kill_rank[s] >= 0 && kill_rank[s] <= k) continue;
-                const double pr = ps.radius[s];
-                const int64_t pcx = (int64_t)trunc(ps.x[s] + pr), pcy = (int64_t)trunc(ps.y[s] + pr);
-                if (patches_collide(pcx, pcy, (int64_t)pr, cx, cy, r)) ok = false;
+            bool hit = held && !(rank >= 0 && rank <= k) && patches_collide(pcx, pcy, pri, cx, cy, r);
+            hit = hit || (lane < k && patches_collide(mine.x + r, mine.y + r, r, cx, cy, r));
+            if (__ballot(hit)) continue;
+            if (lane == k) {
+                mine.id = kind == kPendKill ? pend : top + 1 + k;
+                mine.x = x; mine.y = y; mine.units = (double)u; mine.quality = q;
             }
-            for (int f = 0; f < k && ok; ++f)
-                if (patches_collide(fresh[f].x + r, fresh[f].y + r, r, cx, cy, r)) ok = false;
-            ++retries;
-            if (ok) {
-                fresh[k].id = id; fresh[k].x = x; fresh[k].y = y;
-                fresh[k].units = (double)units; fresh[k].quality = q;
-                break;
-            }
+            break;
         }
     }
     // commit: drop the killed patches, keep the order, append the new ones
-    int wpos = 0;
-    for (int t = 0; t < count; ++t) {
-        const int64_t s = po + t;
-        if (kill_rank[s] >= 0) { kill_rank[s] = -1; continue; }
-        if (wpos != t) {
-            const int64_t d = po + wpos;
-            ps.id[d] = ps.id[s]; ps.x[d] = ps.x[s]; ps.y[d] = ps.y[s]; ps.radius[d] = ps.radius[s];
-            ps.units[d] = ps.units[s]; ps.left[d] = ps.left[s]; ps.quality[d] = ps.quality[s];
-        }
-        ++wpos;
+    const bool stays = held && rank < 0;
+    const uint64_t m = __ballot(stays);
+    const int kept = (int)__popcll(m);
+    if (held && rank >= 0) kill_rank[s] = -1;
+    if (stays) {
+        const int64_t d = po + (int)__popcll(m & ((1ull << lane) - 1ull));
+        ps.id[d] = id; ps.x[d] = px; ps.y[d] = py; ps.radius[d] = pr; ps.units[d] = units; ps.left[d] = left;
+        ps.quality[d] = quality;
     }
-    for (int k = 0; k < n_new; ++k) {
-        const int64_t d = po + wpos + k;
-        ps.id[d] = fresh[k].id; ps.x[d] = (double)fresh[k].x; ps.y[d] = (double)fresh[k].y;
-        ps.radius[d] = (double)r; ps.units[d] = fresh[k].units; ps.left[d] = fresh[k].units;
-        ps.quality[d] = fresh[k].quality;
+    if (lane < n_new) {
+        const int64_t d = po + kept + lane;
+        ps.id[d] = mine.id; ps.x[d] = (double)mine.x; ps.y[d] = (double)mine.y; ps.radius[d] = (double)r;
+        ps.units[d] = mine.units; ps.left[d] = mine.units; ps.quality[d] = mine.quality;
     }
-    ps.count[b] = wpos + n_new;
+    if (lane == 0) ps.count[b] = kept + n_new;
     return ABM_WORLD_DONE;
 }
 
@@ -2003,12 +2005,287 @@ forage_collide_kernel(const FGRep* __restrict__ reps, const WRep* __restrict__ w
     if (tid == 0) status[b] = kWorldReady;
 }
 
-// One replica per block.  STEP: agent-resource interaction (sims.py:789-855)
-// then the placement of regenerated patches; FILL: create_resources; RESUME:
-// the placements a previous phase left pending.  Membership is computed for
-// every (patch, agent) pair in parallel from the poses at the start of the
-// step; the loop over patches and their agents runs per agent in parallel,
-// with only each patch's depletion chain in id order (one thread per patch).
+// Replicas above this many agents take the resource loop over the whole GPU
+// (one workgroup spent about 0.2 of its 0.26 ms on testing 8192 agents against
+// 64 patches on one CU).  At or below it a replica has one thread per agent of
+// a single workgroup.
+constexpr int kWorldBlockAgents = 1024;
+
+// An agent's part of the resource loop that depends on nobody else: the patch
+// its centre lies on (supcalc.distance(resc, agent) < resc.radius).  The norm
+// (a sqrt) is taken only where both centre differences are within the radius,
+// with a margin far above the rounding of the norm, so no pair inside is
+// skipped.  each(p, in) sees every patch in order.
+struct PatchLds {
+    double pr[kMaxPatches], cx[kMaxPatches], cy[kMaxPatches];   // radius, resc.center
+    double pq[kMaxPatches], pl[kMaxPatches];                    // quality, units left
+    int32_t pid[kMaxPatches];
+};
+template <class Each>
+__device__ inline void patch_tests(const PatchLds& L, int p0, int p1, bool live, double cx, double cy,
+                                   const Each& each) {
+#pragma unroll 4
+    for (int p = p0; p < p1; ++p) {
+        const double pr = L.pr[p], dx = cx - L.cx[p], dy = cy - L.cy[p];
+        const double lim = pr * 1.0000001;
+        bool in = false;
+        if (live && fabs(dx) <= lim && fabs(dy) <= lim) in = norm2(dx, dy) < pr;
+        each(p, in);
+    }
+}
+
+// bias_agent_towards_res_center (sims.py:544-552) for the patch's centre.
+__device__ inline double biased_heading(double th, double cx, double cy, double pcx, double pcy) {
+#pragma clang fp contract(off)
+    const double cl = py_mod_2pi(atan2(pcy - cy, pcx - cx) + th);
+    return th + (cl - kPi) * 0.02;
+}
+
+// Rescource.deplete (rescource.py:118-133) by n exploiting agents in turn:
+// every one up to the last served takes `units`, the last takes `last` (what
+// is left, when that is less); the one that empties the patch is the last
+// served and destroys it.
+struct Depletion {
+    double left, units, last;
+    int served;
+    bool destroyed;
+};
+__device__ inline Depletion deplete(double consumption, double quality, double left, int n) {
+#pragma clang fp contract(off)
+    Depletion d;
+    d.units = consumption > quality ? quality : consumption;
+    d.last = 0.0; d.served = 0; d.destroyed = false;
+    while (d.served < n && !d.destroyed) {
+        if (left >= d.units) { left = left - d.units; d.last = d.units; }
+        else { d.last = left; left = 0.0; }
+        d.destroyed = !(left > 0.0);
+        ++d.served;
+    }
+    d.left = left;
+    return d;
+}
+
+// What the agents need of a patch after its depletion.
+struct PatchAfter {
+    double units, last;
+    int32_t served, destroyer;   // destroyer: its agent, or n_agents
+};
+
+// Index of the n-th set bit (n from 0) of m.
+__device__ inline int nth_bit(uint64_t m, int n) {
+    for (; n > 0; --n) m &= m - 1;
+    return __builtin_ctzll(m);
+}
+
+// The depletions of np_ patches by their exploiting agents in id order,
+// word(p, c) being those of patch p in the 64-agent chunk c of C.  The waves of
+// the block (nw, at most 16) share the chunks out, a patch per lane; one lane
+// per patch then runs its subtractions.  base(p, c, n) takes the number of a
+// patch's exploiting agents before chunk c.  Every thread; ends synchronised.
+template <class Word, class Base>
+__device__ inline void deplete_patches(const Word& word, const Base& base, int np_, int C, int N, int nw,
+                                       double consumption, PatchLds& L, int (*seg)[kMaxPatches],
+                                       PatchAfter* after) {
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int per = (C + nw - 1) / nw, c0 = wave * per, c1 = min(C, c0 + per);
+    int cnt = 0;
+    if (lane < np_)
+        for (int c = c0; c < c1; ++c) cnt += (int)__popcll(word(lane, c));
+    seg[wave][lane] = cnt;
+    __syncthreads();
+    int before = 0, n = 0;
+    for (int w = 0; w < nw; ++w) {
+        const int t = seg[w][lane];
+        if (w < wave) before += t;
+        n += t;
+    }
+    if (lane < np_) {
+        int run = before;
+        for (int c = c0; c < c1; ++c) {
+            base(lane, c, run);
+            run += (int)__popcll(word(lane, c));
+        }
+        if (wave == 0) {
+            const Depletion d = deplete(consumption, L.pq[lane], L.pl[lane], n);
+            L.pl[lane] = d.left;
+            after[lane] = PatchAfter{d.units, d.last, d.served, d.destroyed ? -1 : N};
+        }
+    }
+    __syncthreads();
+    if (lane < np_ && after[lane].destroyer < N) {   // whose wave holds the last agent served
+        int r = after[lane].served - 1 - before;
+        if (r >= 0 && r < cnt)
+            for (int c = c0; c < c1; ++c) {
+                const uint64_t m = word(lane, c);
+                const int t = (int)__popcll(m);
+                if (r < t) {
+                    after[lane].destroyer = c * 64 + nth_bit(m, r);
+                    break;
+                }
+                r -= t;
+            }
+    }
+    __syncthreads();
+}
+
+// The agent's share of the walk over its patch (sims.py:803-845), everything
+// the walk does to agent j of patch p: its heading, what it takes (rank: its
+// place among the patch's exploiting agents), the notify of its own turn (a
+// pooled agent up to the destroyer hears of the patch, and teleports), the
+// destroyer's notify-all, and for agents after the destroyer the notify of
+// their own turn.
+__device__ inline void walk_agent(const abm_forage_state& st, int32_t* pool_success, const WRep& W, int tau, int g,
+                                  int j, double theta, bool exploits, int rank, bool pool, const PatchAfter& a,
+                                  int32_t pid, double pcx, double pcy) {
+#pragma clang fp contract(off)
+    st.theta[g] = theta;
+    if (exploits && rank < a.served) {
+        const double cr = st.collected_r[g];
+        st.collected_r_before[g] = cr;
+        st.collected_r[g] = cr + (rank == a.served - 1 ? a.last : a.units);
+    }
+    const int d = a.destroyer, N = W.n_agents;
+    if (j <= d && pool) {
+        notify(st, pool_success, tau, g, 1, pid);
+        if (W.teleport) {
+            const double ra = (double)st.radius[g];
+            st.x[g] = pcx - ra;
+            st.y[g] = pcy - ra;
+        }
+    }
+    if (d < N) notify(st, pool_success, tau, g, -1, -1);   // the destroyer's notify-all
+    if (j > d) notify(st, pool_success, tau, g, -1, -1);   // its own turn after it
+}
+
+// Scratch of the resource loop over the whole GPU.  Replica q of rep[] has
+// its 64-agent chunks from chunk0 on; agent j is entry 64 * chunk0 + j.
+struct WideWorldRep {
+    int32_t b, chunk0;
+};
+struct WideWorldBlock {
+    int32_t q, agent0;         // 64 agents of replica rep[q]
+};
+struct WideWorld {
+    const WideWorldRep* rep;
+    const WideWorldBlock* block;
+    uint64_t *member, *expl;   // [chunk][64 patches]: agents on the patch; those exploiting
+    int32_t* before;           // [chunk][64 patches]: exploiting agents of earlier chunks
+    double* theta;             // the biased headings
+    uint8_t *patch, *flag;     // the agent's patch (255: none), kExploits | kPools
+    PatchAfter* after;         // [replica][64]
+    PatchLds* geo;             // [replica]: the patches before any placement
+    int32_t* ctl;              // [replica][kWwWords]
+};
+constexpr int kExploits = 1, kPools = 2;
+constexpr int kWwGo = 0, kWwMulti = 1, kWwWords = 2;
+
+__device__ inline void stage_patches(PatchLds& L, const abm_patch_state& ps, int64_t po, int np_, int tid, int nthr) {
+    for (int p = tid; p < np_; p += nthr) {
+        const int64_t s = po + p;
+        const double pr = ps.radius[s];
+        L.pr[p] = pr; L.cx[p] = ps.x[s] + pr; L.cy[p] = ps.y[s] + pr;
+        L.pq[p] = ps.quality[s]; L.pl[p] = ps.left[s]; L.pid[p] = ps.id[s];
+    }
+}
+
+// The agents' own parts of the loop (a replica above kWorldBlockAgents), 64
+// agents per block: its four waves test a quarter of the patches each (128
+// blocks of one wave left 8192 agents waiting on their tests' LDS reads).
+// Membership words, headings, flags.
+__global__ void __launch_bounds__(256)
+wide_member_kernel(const FGRep* __restrict__ reps, const WRep* __restrict__ wreps, abm_forage_state st,
+                   const int32_t* __restrict__ pool_success, abm_patch_state ps, WideWorld ww) {
+#pragma clang fp contract(off)
+    __shared__ PatchLds L;
+    __shared__ uint64_t words[kMaxPatches];
+    __shared__ int s_on[64], s_times[64];
+    const WideWorldBlock B = ww.block[blockIdx.x];
+    const int b = ww.rep[B.q].b, chunk0 = ww.rep[B.q].chunk0;
+    const FGRep& P = reps[b];
+    const WRep& W = wreps[b];
+    const int N = P.n_agents, np_ = ps.count[b], tid = threadIdx.x, lane = tid & 63;
+    if (np_ < 0 || np_ > W.n_patches) return;   // reported by the world kernel
+    stage_patches(L, ps, W.patch_offset, np_, tid, blockDim.x);
+    if (tid < 64) { words[tid] = 0ull; s_on[tid] = kMaxPatches; s_times[tid] = 0; }
+    const int j = B.agent0 + lane, g = P.agent_offset + j;
+    const bool live = j < N;
+    double cx = 0.0, cy = 0.0;
+    if (live) {
+        const double ra = (double)st.radius[g];
+        cx = st.x[g] + ra;
+        cy = st.y[g] + ra;
+    }
+    __syncthreads();
+    const int wave = tid >> 6, per = (np_ + 3) / 4;
+    int on = kMaxPatches, times = 0;
+    patch_tests(L, wave * per, min(np_, wave * per + per), live, cx, cy, [&](int p, bool in) {
+        const uint64_t m = __ballot(in);
+        if (lane == 0) words[p] = m;
+        if (in) { on = min(on, p); ++times; }
+    });
+    if (times) { atomicMin(&s_on[lane], on); atomicAdd(&s_times[lane], times); }
+    __syncthreads();
+    if (wave != 0) return;
+    on = s_on[lane];
+    int flag = 0;
+    if (live) {
+        const int mode = get_mode(st.overriding_mode[g], st.w[g], P.T_w);
+        flag = (mode == ABM_MODE_EXPLOIT ? kExploits : 0) | (pooled(mode, pool_success[g], W.pooling_time) ? kPools : 0);
+    }
+    const uint64_t ex = __ballot((flag & kExploits) != 0);
+    const int64_t chunk = chunk0 + (B.agent0 >> 6), at = chunk * kMaxPatches + lane, e = chunk * 64 + lane;
+    ww.member[at] = words[lane];
+    ww.expl[at] = words[lane] & ex;
+    if (__ballot(s_times[lane] > 1) && lane == 0) atomicOr(&ww.ctl[kWwWords * B.q + kWwMulti], 1);
+    if (!live) return;
+    ww.patch[e] = on < kMaxPatches ? (uint8_t)on : 255;
+    ww.flag[e] = (uint8_t)flag;
+    if (on < kMaxPatches) ww.theta[e] = biased_heading(st.theta[g], cx, cy, L.cx[on], L.cy[on]);
+}
+
+// The walk's effects on each agent, after the world kernel's depletions.
+__global__ void __launch_bounds__(64)
+wide_notify_kernel(const FGRep* __restrict__ reps, const WRep* __restrict__ wreps, abm_forage_state st,
+                   int32_t* __restrict__ pool_success, WideWorld ww) {
+    const WideWorldBlock B = ww.block[blockIdx.x];
+    if (!ww.ctl[kWwWords * B.q + kWwGo]) return;
+    const int b = ww.rep[B.q].b;
+    const FGRep& P = reps[b];
+    const int j = B.agent0 + threadIdx.x;
+    if (j >= P.n_agents) return;
+    const int64_t e = 64 * (int64_t)ww.rep[B.q].chunk0 + j;
+    const int g = P.agent_offset + j, p = ww.patch[e], flag = ww.flag[e];
+    if (p == 255) {   // agents on no patch (sims.py:847-855)
+        if (flag) notify(st, pool_success, P.tau, g, -1, -1);
+        return;
+    }
+    const int64_t at = (e >> 6) * kMaxPatches + p;
+    const PatchLds& geo = ww.geo[B.q];
+    const int rank = ww.before[at] + (int)__popcll(ww.expl[at] & ((1ull << (j & 63)) - 1ull));
+    walk_agent(st, pool_success, wreps[b], P.tau, g, j, ww.theta[e], (flag & kExploits) != 0, rank,
+               (flag & kPools) != 0, ww.after[kMaxPatches * B.q + p], geo.pid[p], geo.cx[p], geo.cy[p]);
+}
+
+// STEP: agent-resource interaction (sims.py:789-855) then the placement of
+// regenerated patches; FILL: create_resources; RESUME: the placements a
+// previous phase left pending.  One replica per block, one thread per agent;
+// WIDE: the replicas above kWorldBlockAgents, whose agents' own parts come from
+// wide_member_kernel and go to wide_notify_kernel.
+// An agent's centre lies on at most one patch (patches never overlap), so of
+// the walk over the patches and their agents in id order only each patch's
+// depletion is sequential, a count of its exploiting agents and as many
+// subtractions; each agent then takes its share by its rank.  Patches a caller
+// loaded that overlap take the walk itself, in the reference's order, on one
+// lane.  Waves that neither hold an agent nor are among the first four end at
+// once (a barrier waits for those that live).  Bound by latency: the loads
+// (each agent's in one batch), the notify's round trip, the barriers, and in
+// steps that regenerate patches the placements' draws.  Against passes over the
+// agents one after another, a lane per patch walking its agents' records in
+// global memory and one thread twisting, drawing and compacting: 1000 replicas
+// of 8 to 512 agents with ten patches 46 -> 31 us, one replica of 10 agents
+// 10.2 -> 8.2, 8192 agents with 64 patches 261 -> 29 in three launches (7 us
+// membership, 16 here, 6 notify).
+template <bool WIDE>
 __global__ void __launch_bounds__(1024)
 forage_world_kernel(const FGRep* __restrict__ reps, const WRep* __restrict__ wreps, int phase,
                     abm_forage_state st, int32_t* __restrict__ pool_success, abm_patch_state ps,
@@ -2016,13 +2293,19 @@ forage_world_kernel(const FGRep* __restrict__ reps, const WRep* __restrict__ wre
                     int32_t* __restrict__ pend_id, const uint32_t* __restrict__ words,
                     const int64_t* __restrict__ w_off, const int32_t* __restrict__ w_cnt,
                     int32_t* __restrict__ w_used, int32_t* __restrict__ status,
-                    abm_mt19937_state* __restrict__ mt) {
+                    abm_mt19937_state* __restrict__ mt, WideWorld ww) {
 #pragma clang fp contract(off)
-    extern __shared__ __align__(16) uint64_t member[];   // [patch][64-agent chunk]
-    __shared__ FreshPatch fresh[kMaxPatches];
+    extern __shared__ __align__(16) uint64_t member_lds[];   // [patch][chunk], then the exploiting ones
     __shared__ uint32_t mkey[kMtN];
-    __shared__ int s_kind, s_pending, s_pos;
-    const int b = blockIdx.x, tid = threadIdx.x, nthr = blockDim.x;
+    __shared__ int s_kind, s_pending, s_pos, s_multi;
+    __shared__ PatchLds L;
+    __shared__ PatchAfter s_after[kMaxPatches];
+    __shared__ int s_seg[16][kMaxPatches];
+    const int b = WIDE ? ww.rep[blockIdx.x].b : blockIdx.x, tid = threadIdx.x;
+    const int nthr = WIDE ? 1024 : min((int)blockDim.x, max(256, (reps[b].n_agents + 63) & ~63));
+    if (tid >= nthr) return;   // uniform over the wave
+    const int64_t chunk0 = WIDE ? ww.rep[blockIdx.x].chunk0 : 0;
+    int32_t* const wctl = WIDE ? ww.ctl + kWwWords * blockIdx.x : nullptr;
     // the replica's parameters in LDS, read where used
     __shared__ FGRep sP;
     __shared__ WRep sW;
@@ -2031,19 +2314,26 @@ forage_world_kernel(const FGRep* __restrict__ reps, const WRep* __restrict__ wre
         reinterpret_cast<uint64_t*>(&sP)[tid] = reinterpret_cast<const uint64_t*>(reps + b)[tid];
     else if (tid >= 64 && tid < 64 + (int)(sizeof(WRep) / 8))
         reinterpret_cast<uint64_t*>(&sW)[tid - 64] = reinterpret_cast<const uint64_t*>(wreps + b)[tid - 64];
+    int kind = pend[2 * b], n_pending = pend[2 * b + 1];
+    const int n_live = ps.count[b], status0 = status[b];
+    if (tid == 0) {
+        // taken and cleared in one operation: a plain read of this uniform
+        // address is a scalar load, which the clearing store may overtake
+        s_multi = WIDE ? atomicExch(&wctl[kWwMulti], 0) : 0;
+        if (WIDE) wctl[kWwGo] = 0;
+    }
     __syncthreads();
     const FGRep& P = sP;
     const WRep& W = sW;
     const int N = P.n_agents, a0 = P.agent_offset, C = (N + 63) / 64;
     const int64_t po = W.patch_offset;
-    int kind = pend[2 * b], n_pending = pend[2 * b + 1];
-    const int n_live = ps.count[b];
+    if (!WIDE && phase == ABM_WORLD_STEP && N > kWorldBlockAgents) return;   // the WIDE launch's
     if (n_live < 0 || n_live > W.n_patches) {
         if (tid == 0) { w_used[b] = 0; status[b] = ABM_WORLD_BAD_COUNT; }
         return;
     }
     if (phase == ABM_WORLD_RESUME) {
-        if (status[b] != ABM_WORLD_NEED_WORDS || kind == kPendNone) {
+        if (status0 != ABM_WORLD_NEED_WORDS || kind == kPendNone) {
             if (tid == 0) w_used[b] = 0;
             return;
         }
@@ -2054,130 +2344,91 @@ forage_world_kernel(const FGRep* __restrict__ reps, const WRep* __restrict__ wre
     }
     if (phase == ABM_WORLD_STEP) {
         // a replica the collision kernel found crowded is left as it is
-        if (W.collide && status[b] == ABM_WORLD_CROWDED) {
+        if (W.collide && status0 == ABM_WORLD_CROWDED) {
             if (tid == 0) w_used[b] = 0;
             return;
         }
-        const int np_ = n_live;
-        // the live patches' geometry, quality and units staged in LDS
-        __shared__ double s_pr[kMaxPatches], s_px[kMaxPatches], s_py[kMaxPatches];
-        __shared__ double s_pq[kMaxPatches], s_pl[kMaxPatches];
-        __shared__ int32_t s_pid[kMaxPatches];
-        for (int p = tid; p < np_; p += nthr) {
-            const int64_t s = po + p;
-            s_pr[p] = ps.radius[s]; s_px[p] = ps.x[s]; s_py[p] = ps.y[s];
-            s_pq[p] = ps.quality[s]; s_pl[p] = ps.left[s]; s_pid[p] = ps.id[s];
+        const int np_ = n_live, lane = tid & 63, g = a0 + tid;
+        uint64_t* const member = member_lds;
+        uint64_t* const expl = member_lds + (size_t)np_ * C;
+        auto member_word = [&](int p, int c) {
+            return WIDE ? ww.member[(chunk0 + c) * kMaxPatches + p] : member[p * C + c];
+        };
+        // the live patches' geometry, quality and units staged in LDS, and
+        // (one thread per agent) the agent's own part
+        stage_patches(L, ps, po, np_, tid, nthr);
+        const bool live = !WIDE && tid < N;
+        double cx = 0.0, cy = 0.0, th = 0.0;
+        int flag = 0;
+        if (live) {
+            const double ra = (double)st.radius[g];
+            cx = st.x[g] + ra;
+            cy = st.y[g] + ra;
+            th = st.theta[g];
+            const int mode = get_mode(st.overriding_mode[g], st.w[g], P.T_w);
+            flag = (mode == ABM_MODE_EXPLOIT ? kExploits : 0) |
+                   (pooled(mode, pool_success[g], W.pooling_time) ? kPools : 0);
         }
         __syncthreads();
-        // ---- membership: supcalc.distance(resc, agent) < resc.radius.  A
-        // wave takes 64 agents, loads their centres once and tests them
-        // against every patch; the norm (a sqrt) only where both centre
-        // differences are within the radius (with a margin far above the
-        // rounding of the norm, so no pair inside is skipped)
-        for (int base = tid & ~63; base < C * 64; base += nthr) {
-            const int j = base + (tid & 63);
-            double cx = 0.0, cy = 0.0;
-            if (j < N) {
-                const int g = a0 + j;
-                const double ra = (double)st.radius[g];
-                cx = st.x[g] + ra;
-                cy = st.y[g] + ra;
-            }
-            for (int p = 0; p < np_; ++p) {
-                const double pr = s_pr[p];
-                const double dx = cx - (s_px[p] + pr), dy = cy - (s_py[p] + pr);
-                const double lim = pr * 1.0000001;
-                bool in = false;
-                if (j < N && fabs(dx) <= lim && fabs(dy) <= lim) in = norm2(dx, dy) < pr;
+        int on = -1;
+        if (!WIDE && (tid & ~63) < N) {
+            const uint64_t ex = __ballot((flag & kExploits) != 0);
+            int times = 0;
+            patch_tests(L, 0, np_, live, cx, cy, [&](int p, bool in) {
                 const uint64_t m = __ballot(in);
-                if ((tid & 63) == 0) member[p * C + (j >> 6)] = m;
-            }
+                if (lane == 0) { member[p * C + (tid >> 6)] = m; expl[p * C + (tid >> 6)] = m & ex; }
+                if (in) { if (on < 0) on = p; ++times; }
+            });
+            if (__ballot(times > 1) && lane == 0) s_multi = 1;   // every writer stores 1
         }
-        __syncthreads();
-        // ---- the patches' agent groups (sims.py:803-845).  The reference
-        // walks the patches in Group order and their agents in id order; an
-        // agent's centre lies in at most one patch (patches never overlap),
-        // so only the depletion chain of each patch is sequential (patches a
-        // caller loaded that overlap take the serial walk).  Phase A
-        // (every thread): per agent on a patch, the bias towards the patch
-        // centre and its mode and pooling flags, read before any notify of
-        // the walk (a notify never changes them; a later notify of the same
-        // agent only follows its own pooling test).  Phase B (one thread per
-        // patch): the exploiting agents deplete the patch in id order until
-        // its last unit; the agent that took it is the destroyer.  Phase C
-        // (every thread): each agent's notifies in the walk's order: a
-        // pooled agent up to the destroyer hears of the patch (and teleports),
-        // then every agent of a destroyed patch hears -1 from the
-        // destroyer's notify-all, and agents after the destroyer hear -1
-        // once more in their own turn.
-        __shared__ uint64_t s_on[kMaxWorldChunks], s_expl[kMaxWorldChunks], s_pool[kMaxWorldChunks];
-        __shared__ int32_t s_destroyer[kMaxPatches];
-        __shared__ int s_multi;
-        if (tid == 0) s_multi = 0;
-        __syncthreads();
-        for (int c = tid; c < C; c += nthr) {
-            uint64_t on = 0, dup = 0;
-            for (int p = 0; p < np_; ++p) {
-                dup |= on & member[p * C + c];
-                on |= member[p * C + c];
+        if (WIDE)
+            for (int p = tid; p < np_; p += nthr) {
+                PatchLds& geo = ww.geo[blockIdx.x];
+                geo.cx[p] = L.cx[p]; geo.cy[p] = L.cy[p]; geo.pid[p] = L.pid[p];
             }
-            s_on[c] = on;
-            if (dup) s_multi = 1;
-        }
-        for (int p = tid; p < np_; p += nthr) s_destroyer[p] = N;
         __syncthreads();
-        if (s_multi) {
+        const bool multi = s_multi != 0;
+        if (multi) {
             // patches loaded by the caller that overlap: the walk in the
             // reference's order, in one thread
             if (tid == 0) {
                 int n_kill = 0;
                 for (int p = 0; p < np_; ++p) {
                     const int64_t s = po + p;
-                    const double pr = s_pr[p];
-                    const double pcx = s_px[p] + pr, pcy = s_py[p] + pr;   // resc.center
-                    const int32_t pid = s_pid[p];
+                    const double pcx = L.cx[p], pcy = L.cy[p];   // resc.center
+                    const int32_t pid = L.pid[p];
                     bool destroy = false;
                     for (int c = 0; c < C; ++c) {
-                        uint64_t m = member[p * C + c];
+                        uint64_t m = member_word(p, c);
                         while (m) {
-                            const int g = a0 + c * 64 + __builtin_ctzll(m);
+                            const int gi = a0 + c * 64 + __builtin_ctzll(m);
                             m &= m - 1;
-                            const double ra = (double)st.radius[g];
-                            // bias_agent_towards_res_center (sims.py:544-552)
-                            const double x1 = st.x[g] + ra, y1 = st.y[g] + ra;
-                            const double th = st.theta[g];
-                            const double cl = py_mod_2pi(atan2(pcy - y1, pcx - x1) + th);
-                            st.theta[g] = th + (cl - kPi) * 0.02;
+                            const double ra = (double)st.radius[gi];
+                            st.theta[gi] = biased_heading(st.theta[gi], st.x[gi] + ra, st.y[gi] + ra, pcx, pcy);
                             if (destroy) {
-                                notify(st, pool_success, P.tau, g, -1, -1);
+                                notify(st, pool_success, P.tau, gi, -1, -1);
                                 continue;
                             }
-                            const int mode = get_mode(st.overriding_mode[g], st.w[g], P.T_w);
-                            if (pooled(mode, pool_success[g], W.pooling_time)) {
-                                notify(st, pool_success, P.tau, g, 1, pid);
+                            const int mode = get_mode(st.overriding_mode[gi], st.w[gi], P.T_w);
+                            if (pooled(mode, pool_success[gi], W.pooling_time)) {
+                                notify(st, pool_success, P.tau, gi, 1, pid);
                                 if (W.teleport) {
-                                    st.x[g] = (s_px[p] + pr) - ra;
-                                    st.y[g] = (s_py[p] + pr) - ra;
+                                    st.x[gi] = pcx - ra;
+                                    st.y[gi] = pcy - ra;
                                 }
                             }
                             if (mode == ABM_MODE_EXPLOIT) {
-                                // Rescource.deplete (rescource.py:118-133)
-                                double units = W.consumption;
-                                const double q = s_pq[p];
-                                if (units > q) units = q;
-                                double left = s_pl[p], dep;
-                                if (left >= units) { left = left - units; dep = units; }
-                                else { dep = left; left = 0.0; }
-                                s_pl[p] = left;
-                                ps.left[s] = left;
-                                destroy = !(left > 0.0);
-                                const double cr = st.collected_r[g];
-                                st.collected_r_before[g] = cr;
-                                st.collected_r[g] = cr + dep;
+                                const Depletion d = deplete(W.consumption, L.pq[p], L.pl[p], 1);
+                                L.pl[p] = d.left;
+                                ps.left[s] = d.left;
+                                destroy = d.destroyed;
+                                const double cr = st.collected_r[gi];
+                                st.collected_r_before[gi] = cr;
+                                st.collected_r[gi] = cr + d.last;
                                 if (destroy) {
                                     // every agent of the group hears of it
                                     for (int c2 = 0; c2 < C; ++c2) {
-                                        uint64_t m2 = member[p * C + c2];
+                                        uint64_t m2 = member_word(p, c2);
                                         while (m2) {
                                             const int g2 = a0 + c2 * 64 + __builtin_ctzll(m2);
                                             m2 &= m2 - 1;
@@ -2194,162 +2445,107 @@ forage_world_kernel(const FGRep* __restrict__ reps, const WRep* __restrict__ wre
                         ++n_kill;
                     }
                 }
+                // agents on no patch (sims.py:847-855)
+                for (int j = 0; j < N; ++j) {
+                    uint64_t any = 0ull;
+                    for (int p = 0; p < np_; ++p) any |= member_word(p, j >> 6);
+                    if ((any >> (j & 63)) & 1ull) continue;
+                    const int mode = get_mode(st.overriding_mode[a0 + j], st.w[a0 + j], P.T_w);
+                    if (pooled(mode, pool_success[a0 + j], W.pooling_time) || mode == ABM_MODE_EXPLOIT)
+                        notify(st, pool_success, P.tau, a0 + j, -1, -1);
+                }
                 kind = n_kill ? kPendKill : kPendNone;
                 n_pending = n_kill;
             }
         } else {
-            for (int base = tid & ~63; base < C * 64; base += nthr) {
-                const int j = base + (tid & 63);
-                bool ex = false, pl = false;
-                if (j < N && ((s_on[j >> 6] >> (j & 63)) & 1ull)) {
-                    int p = 0;
-                    while (!((member[p * C + (j >> 6)] >> (j & 63)) & 1ull)) ++p;
-                    const int g = a0 + j;
-                    const double pr = s_pr[p];
-                    const double pcx = s_px[p] + pr, pcy = s_py[p] + pr;   // resc.center
-                    const double ra = (double)st.radius[g];
-                    // bias_agent_towards_res_center (sims.py:544-552)
-                    const double x1 = st.x[g] + ra, y1 = st.y[g] + ra;
-                    const double th = st.theta[g];
-                    const double cl = py_mod_2pi(atan2(pcy - y1, pcx - x1) + th);
-                    st.theta[g] = th + (cl - kPi) * 0.02;
-                    const int mode = get_mode(st.overriding_mode[g], st.w[g], P.T_w);
-                    ex = mode == ABM_MODE_EXPLOIT;
-                    pl = pooled(mode, pool_success[g], W.pooling_time);
-                }
-                const uint64_t me = __ballot(ex), mp = __ballot(pl);
-                if ((tid & 63) == 0 && base < C * 64) { s_expl[base >> 6] = me; s_pool[base >> 6] = mp; }
-            }
-            __syncthreads();
+            deplete_patches([&](int p, int c) { return WIDE ? ww.expl[(chunk0 + c) * kMaxPatches + p] : expl[p * C + c]; },
+                            [&](int p, int c, int n) { if (WIDE) ww.before[(chunk0 + c) * kMaxPatches + p] = n; }, np_, C,
+                            N, nthr >> 6, W.consumption, L, s_seg, s_after);
             for (int p = tid; p < np_; p += nthr) {
-                // Rescource.deplete (rescource.py:118-133) by the exploiting
-                // agents of patch p in id order
-                const int64_t s = po + p;
-                double units = W.consumption;
-                const double q = s_pq[p];
-                if (units > q) units = q;
-                double left = s_pl[p];
-                bool destroy = false;
-                for (int c = 0; c < C && !destroy; ++c) {
-                    uint64_t m = member[p * C + c] & s_expl[c];
-                    while (m && !destroy) {
-                        const int j = c * 64 + __builtin_ctzll(m);
-                        m &= m - 1;
-                        const int g = a0 + j;
-                        double dep;
-                        if (left >= units) { left = left - units; dep = units; }
-                        else { dep = left; left = 0.0; }
-                        destroy = !(left > 0.0);
-                        const double cr = st.collected_r[g];
-                        st.collected_r_before[g] = cr;
-                        st.collected_r[g] = cr + dep;
-                        if (destroy) s_destroyer[p] = j;
-                    }
-                }
-                s_pl[p] = left;
-                ps.left[s] = left;
+                ps.left[po + p] = L.pl[p];
+                if (WIDE) ww.after[kMaxPatches * blockIdx.x + p] = s_after[p];
             }
-            __syncthreads();
-            for (int j = tid; j < N; j += nthr) {
-                if (!((s_on[j >> 6] >> (j & 63)) & 1ull)) continue;
-                int p = 0;
-                while (!((member[p * C + (j >> 6)] >> (j & 63)) & 1ull)) ++p;
-                const int g = a0 + j;
-                const int d = s_destroyer[p];
-                if (j <= d && ((s_pool[j >> 6] >> (j & 63)) & 1ull)) {
-                    notify(st, pool_success, P.tau, g, 1, s_pid[p]);
-                    if (W.teleport) {
-                        const double pr = s_pr[p], ra = (double)st.radius[g];
-                        st.x[g] = (s_px[p] + pr) - ra;
-                        st.y[g] = (s_py[p] + pr) - ra;
-                    }
+            if (WIDE && tid == 0) wctl[kWwGo] = 1;
+            if (live) {
+                if (on < 0) {
+                    if (flag) notify(st, pool_success, P.tau, g, -1, -1);   // agents on no patch (sims.py:847-855)
+                } else {
+                    int rank = (int)__popcll(expl[on * C + (tid >> 6)] & ((1ull << lane) - 1ull));
+                    for (int c = 0; c < tid >> 6; ++c) rank += (int)__popcll(expl[on * C + c]);
+                    walk_agent(st, pool_success, W, P.tau, g, tid, biased_heading(th, cx, cy, L.cx[on], L.cy[on]),
+                               (flag & kExploits) != 0, rank, (flag & kPools) != 0, s_after[on], L.pid[on], L.cx[on],
+                               L.cy[on]);
                 }
-                if (d < N) notify(st, pool_success, P.tau, g, -1, -1);   // the destroyer's notify-all
-                if (j > d) notify(st, pool_success, P.tau, g, -1, -1);   // its own turn after it
             }
-            if (tid == 0) {
-                int n_kill = 0;
-                for (int p = 0; p < np_; ++p) {
-                    if (s_destroyer[p] >= N) continue;
-                    kill_rank[po + p] = n_kill;
-                    pend_id[po + n_kill] = s_pid[p];
-                    ++n_kill;
+            if (tid < 64) {   // the destroyed patches, in Group order
+                const bool dead = tid < np_ && s_after[tid].destroyer < N;
+                const uint64_t m = __ballot(dead);
+                if (dead) {
+                    const int k = (int)__popcll(m & ((1ull << tid) - 1ull));
+                    kill_rank[po + tid] = k;
+                    pend_id[po + k] = L.pid[tid];
                 }
-                kind = n_kill ? kPendKill : kPendNone;
-                n_pending = n_kill;
+                kind = m ? kPendKill : kPendNone;
+                n_pending = (int)__popcll(m);
             }
-        }
-        // ---- agents on no patch (sims.py:847-855)
-        for (int j = tid; j < N; j += nthr) {
-            if ((s_on[j >> 6] >> (j & 63)) & 1ull) continue;
-            const int g = a0 + j;
-            const int mode = get_mode(st.overriding_mode[g], st.w[g], P.T_w);
-            if (pooled(mode, pool_success[g], W.pooling_time) || mode == ABM_MODE_EXPLOIT)
-                notify(st, pool_success, P.tau, g, -1, -1);
         }
     } else if (phase == ABM_WORLD_FILL) {
         kind = kPendFill;
         n_pending = 0;
     }
-    if (mt) {
-        // ---- placements from the replica's generator on the device: its
-        // state in LDS for thread 0's draws, written back after
-        if (tid == 0) { s_kind = kind; s_pending = n_pending; }
-        __syncthreads();
-        kind = s_kind;
-        n_pending = s_pending;
-        const bool update_follows = kind != kPendFill;
-        if (kind == kPendNone) {
-            if (tid == 0) {
-                pend[2 * b] = kPendNone; pend[2 * b + 1] = 0;
-                w_used[b] = 0;
-                status[b] = kWorldReady;
-            }
-            return;
-        }
-        for (int i = tid; i < kMtN; i += nthr) mkey[i] = mt[b].key[i];
-        if (tid == 0) s_pos = mt[b].pos;
-        __syncthreads();
+    // ---- placements, by the first wave: from the words the caller drew
+    // ahead, but for those of the random walk of the update that follows, or
+    // from the replica's generator on the device, its key in LDS meanwhile
+    if (tid == 0) { s_kind = kind; s_pending = n_pending; }
+    __syncthreads();
+    kind = s_kind;
+    n_pending = s_pending;
+    const bool update_follows = kind != kPendFill;
+    if (kind == kPendNone) {
         if (tid == 0) {
-            MtCursor cur{mkey, s_pos, 0, false};
-            const int rc = place_patches(W, ps, b, kind, n_pending, pend_id, kill_rank, cur, fresh);
-            w_used[b] = cur.used;
-            if (rc == ABM_WORLD_DONE) {
-                pend[2 * b] = kPendNone; pend[2 * b + 1] = 0;
-                status[b] = update_follows ? kWorldReady : ABM_WORLD_DONE;
-                s_pos = cur.pos;
-            } else {
-                // too many retries: the reference raises; nothing placed, the
-                // generator stays where it was
-                pend[2 * b] = kind; pend[2 * b + 1] = n_pending;
-                status[b] = rc;
-                s_pos = -1;
-            }
-        }
-        __syncthreads();
-        if (s_pos >= 0) {
-            for (int i = tid; i < kMtN; i += nthr) mt[b].key[i] = mkey[i];
-            if (tid == 0) mt[b].pos = s_pos;
+            pend[2 * b] = kPendNone; pend[2 * b + 1] = 0;
+            w_used[b] = 0;
+            status[b] = kWorldReady;
         }
         return;
     }
-    if (tid != 0) return;
-    // ---- placements: kept words for the random walk of the update that follows
-    const bool update_follows = kind != kPendFill;
-    const int reserve = update_follows ? 2 * N : 0;
-    const int limit = w_cnt ? max(0, w_cnt[b] - reserve) : 0;
-    WordCursor cur{words ? words + w_off[b] : nullptr, 0, words ? limit : 0, false};
-    int rc = ABM_WORLD_DONE;
-    if (kind != kPendNone) rc = place_patches(W, ps, b, kind, n_pending, pend_id, kill_rank, cur, fresh);
-    if (rc == ABM_WORLD_DONE) {
-        pend[2 * b] = kPendNone; pend[2 * b + 1] = 0;
-        w_used[b] = cur.used;
-        status[b] = update_follows ? kWorldReady : ABM_WORLD_DONE;
-    } else {
-        // nothing placed and nothing drawn; the kill ranks stay for the resume
-        pend[2 * b] = kind; pend[2 * b + 1] = n_pending;
-        w_used[b] = rc == ABM_WORLD_TIMEOUT ? cur.used : 0;
-        status[b] = rc;
+    if (mt) {
+        for (int i = tid; i < kMtN; i += nthr) mkey[i] = mt[b].key[i];
+        if (tid == 0) s_pos = mt[b].pos;
+        __syncthreads();
+    }
+    if (tid < 64) {
+        int rc, used;
+        if (mt) {
+            MtCursor cur{mkey, s_pos, 0, false};
+            rc = place_patches(W, ps, b, kind, n_pending, pend_id, kill_rank, cur);
+            used = cur.used;
+            // a timeout: the generator stays where it was
+            if (tid == 0) s_pos = rc == ABM_WORLD_DONE ? cur.pos : -1;
+        } else {
+            const int limit = w_cnt ? max(0, w_cnt[b] - (update_follows ? 2 * N : 0)) : 0;
+            WordCursor cur{words ? words + w_off[b] : nullptr, 0, words ? limit : 0, false};
+            rc = place_patches(W, ps, b, kind, n_pending, pend_id, kill_rank, cur);
+            used = rc == ABM_WORLD_NEED_WORDS ? 0 : cur.used;   // nothing placed, nothing drawn
+        }
+        if (tid == 0) {
+            w_used[b] = used;
+            if (rc == ABM_WORLD_DONE) {
+                pend[2 * b] = kPendNone; pend[2 * b + 1] = 0;
+                status[b] = update_follows ? kWorldReady : ABM_WORLD_DONE;
+            } else {
+                // out of words (the kill ranks stay for the resume), or too
+                // many retries: the reference raises
+                pend[2 * b] = kind; pend[2 * b + 1] = n_pending;
+                status[b] = rc;
+            }
+        }
+    }
+    if (!mt) return;
+    __syncthreads();
+    if (s_pos >= 0) {
+        for (int i = tid; i < kMtN; i += nthr) mt[b].key[i] = mkey[i];
+        if (tid == 0) mt[b].pos = s_pos;
     }
 }
 
@@ -2469,6 +2665,30 @@ int plan_wide(abm_forage_batch* bt) {
     if (!rc) rc = check_hip(hipMemset(m.ctl, 0, sizeof(int32_t) * kWdWords * rep.size()), "clear wide control");
     if (!rc) rc = check_hip(hipDeviceSynchronize(), "plan wide update");
     return rc;
+}
+
+// Device memory of the resource loop over the whole GPU; with base null only
+// its size is found.
+size_t wide_world_carve(void* base, const abm_forage_world* w, WideWorld* m) {
+    const size_t reps = (size_t)w->wide_reps, chunks = (size_t)w->wide_chunks, agents = 64 * chunks;
+    size_t at = 0;
+    auto take = [&](size_t bytes) {
+        char* p = reinterpret_cast<char*>(base) + at;
+        at += (bytes + 255) & ~(size_t)255;
+        return p;
+    };
+    m->rep = reinterpret_cast<WideWorldRep*>(take(sizeof(WideWorldRep) * reps));
+    m->block = reinterpret_cast<WideWorldBlock*>(take(sizeof(WideWorldBlock) * (size_t)w->wide_blocks));
+    m->member = reinterpret_cast<uint64_t*>(take(sizeof(uint64_t) * chunks * kMaxPatches));
+    m->expl = reinterpret_cast<uint64_t*>(take(sizeof(uint64_t) * chunks * kMaxPatches));
+    m->before = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * chunks * kMaxPatches));
+    m->theta = reinterpret_cast<double*>(take(sizeof(double) * agents));
+    m->patch = reinterpret_cast<uint8_t*>(take(agents));
+    m->flag = reinterpret_cast<uint8_t*>(take(agents));
+    m->after = reinterpret_cast<PatchAfter*>(take(sizeof(PatchAfter) * reps * kMaxPatches));
+    m->geo = reinterpret_cast<PatchLds*>(take(sizeof(PatchLds) * reps));
+    m->ctl = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * kWwWords * reps));
+    return at;
 }
 
 // Which kernel updates which replica: the update kernel those without visual
@@ -2797,6 +3017,7 @@ int abm_forage_world_create(abm_forage_batch* b, const abm_forage_world_params* 
                              "agents per replica (got %d)", i, kCollideMaxAgents, reps[i].n_agents);
         if (w.collide)
             collide_lds = std::max(collide_lds, collide_lds_bytes(reps[i].n_agents, reps[i].n_rays));
+        w.n_agents = reps[i].n_agents;
         w.patch_offset = total;
         // the bounds numpy sees: int() of the Python expressions (sims.py:349-356)
         const double r = (double)q.patch_radius, pad = reps[i].pad;
@@ -2824,6 +3045,29 @@ int abm_forage_world_create(abm_forage_batch* b, const abm_forage_world_params* 
     abm_forage_world* wd = new abm_forage_world();
     wd->batch = b; wd->n_replicas = n; wd->patch_total = total; wd->member_lds = lds;
     wd->collide_lds = collide_lds;
+    // the world kernel's workgroups: a thread per agent of the replicas that
+    // take one workgroup, membership words of every patch and of its
+    // exploiting agents; the larger replicas' blocks and chunks
+    std::vector<WideWorldRep> wide;
+    std::vector<WideWorldBlock> blocks;
+    int64_t chunks = 0;
+    int threads = 256;
+    for (int i = 0; i < n; ++i) {
+        const int N = reps[i].n_agents;
+        if (N > kWorldBlockAgents) {
+            for (int a = 0; a < N; a += 64) blocks.push_back(WideWorldBlock{(int32_t)wide.size(), a});
+            wide.push_back(WideWorldRep{i, (int32_t)chunks});
+            chunks += (N + 63) / 64;
+        } else {
+            while (threads < N) threads *= 2;
+            wd->world_lds = std::max(wd->world_lds, 2 * sizeof(uint64_t) * (size_t)host[i].n_patches *
+                                                        (size_t)((N + 63) / 64));
+        }
+    }
+    wd->threads = threads;
+    wd->wide_reps = (int32_t)wide.size();
+    wd->wide_blocks = (int32_t)blocks.size();
+    wd->wide_chunks = chunks;
     if (collide_lds > (size_t)163840) {
         delete wd;
         return set_error(ABM_ERR_UNSUPPORTED, "forage world: the collision kernel needs %zu B of LDS",
@@ -2838,6 +3082,21 @@ int abm_forage_world_create(abm_forage_batch* b, const abm_forage_world_params* 
                            "upload world replicas");
     if (!rc) rc = check_hip(hipMemset(wd->kill_rank, 0xff, sizeof(int32_t) * slots), "clear kill ranks");
     if (!rc) rc = check_hip(hipMemset(wd->pend, 0, sizeof(int32_t) * 2 * n), "clear pending");
+    if (!rc && wd->wide_reps > 0) {
+        WideWorld ww;
+        const size_t bytes = wide_world_carve(nullptr, wd, &ww);
+        rc = check_hip(hipMalloc(&wd->wide_mem, bytes), "hipMalloc(wide world)");
+        if (!rc) {
+            wide_world_carve(wd->wide_mem, wd, &ww);
+            rc = check_hip(hipMemset(ww.ctl, 0, sizeof(int32_t) * kWwWords * wide.size()), "clear wide world control");
+        }
+        if (!rc) rc = check_hip(hipMemcpy(const_cast<WideWorldRep*>(ww.rep), wide.data(),
+                                          sizeof(WideWorldRep) * wide.size(), hipMemcpyHostToDevice),
+                                "upload wide world replicas");
+        if (!rc) rc = check_hip(hipMemcpy(const_cast<WideWorldBlock*>(ww.block), blocks.data(),
+                                          sizeof(WideWorldBlock) * blocks.size(), hipMemcpyHostToDevice),
+                                "upload wide world blocks");
+    }
     if (!rc) rc = check_hip(hipDeviceSynchronize(), "world create");
     if (rc) { abm_forage_world_destroy(wd); return rc; }
     wd->patch_offset_host = new int64_t[n + 1];
@@ -2853,6 +3112,7 @@ int abm_forage_world_destroy(abm_forage_world* w) {
     if (w->kill_rank) (void)hipFree(w->kill_rank);
     if (w->pend) (void)hipFree(w->pend);
     if (w->pend_id) (void)hipFree(w->pend_id);
+    if (w->wide_mem) (void)hipFree(w->wide_mem);
     delete[] w->patch_offset_host;
     delete w;
     return ABM_OK;
@@ -2883,8 +3143,8 @@ int world_run(abm_forage_world* w, int32_t phase, const abm_forage_state* st, in
         return set_error(ABM_ERR_INVALID, "%s: every patch array is required", who);
     if (!ps->count) return set_error(ABM_ERR_INVALID, "%s: patch count array is required", who);
     abm_forage_batch* b = w->batch;
-    const size_t lds = w->member_lds;
-    if (lds > 65536) return set_error(ABM_ERR_UNSUPPORTED, "%s: %zu B of membership masks", who, lds);
+    if (w->member_lds > 65536)
+        return set_error(ABM_ERR_UNSUPPORTED, "%s: %zu B of membership masks", who, w->member_lds);
     if (phase == ABM_WORLD_STEP && w->collide_lds > 0) {
         // agent-agent collisions first (sims.py:736-787)
         if (w->collide_lds > 65536) {
@@ -2898,14 +3158,29 @@ int world_run(abm_forage_world* w, int32_t phase, const abm_forage_state* st, in
                            pool_success, w->pend, status);
         if (int rc = check_hip(hipGetLastError(), "forage_collide_kernel launch")) return rc;
     }
-    // a replica above 1024 agents takes a block of 1024 threads for the
-    // per-agent parts; smaller ones share a CU in blocks of 256
-    const int threads = b->max_agents > 1024 ? 1024 : 256;
-    hipLaunchKernelGGL(forage_world_kernel, dim3(b->n_replicas), dim3(threads), lds, (hipStream_t)stream,
-                       (const FGRep*)b->reps_dev, (const WRep*)w->wreps_dev, (int)phase, *st, pool_success,
-                       *ps, w->kill_rank, w->pend, w->pend_id, words, word_offset, word_count, words_used,
-                       status, mt);
-    if (int rc = check_hip(hipGetLastError(), "forage_world_kernel launch")) return rc;
+    const bool wide = phase == ABM_WORLD_STEP && w->wide_reps > 0;
+    const FGRep* reps = (const FGRep*)b->reps_dev;
+    const WRep* wreps = (const WRep*)w->wreps_dev;
+    WideWorld ww{};
+    if (!wide || w->wide_reps < b->n_replicas) {
+        hipLaunchKernelGGL(forage_world_kernel<false>, dim3(b->n_replicas), dim3(w->threads), w->world_lds,
+                           (hipStream_t)stream, reps, wreps, (int)phase, *st, pool_success, *ps, w->kill_rank,
+                           w->pend, w->pend_id, words, word_offset, word_count, words_used, status, mt, ww);
+        if (int rc = check_hip(hipGetLastError(), "forage_world_kernel launch")) return rc;
+    }
+    if (wide) {
+        wide_world_carve(w->wide_mem, w, &ww);
+        hipLaunchKernelGGL(wide_member_kernel, dim3(w->wide_blocks), dim3(256), 0, (hipStream_t)stream, reps, wreps,
+                           *st, pool_success, *ps, ww);
+        if (int rc = check_hip(hipGetLastError(), "wide_member_kernel launch")) return rc;
+        hipLaunchKernelGGL(forage_world_kernel<true>, dim3(w->wide_reps), dim3(1024), 0, (hipStream_t)stream, reps,
+                           wreps, (int)phase, *st, pool_success, *ps, w->kill_rank, w->pend, w->pend_id, words,
+                           word_offset, word_count, words_used, status, mt, ww);
+        if (int rc = check_hip(hipGetLastError(), "forage_world_kernel launch")) return rc;
+        hipLaunchKernelGGL(wide_notify_kernel, dim3(w->wide_blocks), dim3(64), 0, (hipStream_t)stream, reps, wreps,
+                           *st, pool_success, ww);
+        if (int rc = check_hip(hipGetLastError(), "wide_notify_kernel launch")) return rc;
+    }
     if (phase == ABM_WORLD_FILL) return ABM_OK;
     // the update draws its walk after the placements
     return launch_forage_step(b, st, nullptr, words, word_offset, word_count, words_used, status,

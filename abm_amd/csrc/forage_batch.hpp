@@ -43,7 +43,12 @@ struct abm_forage_world {
     abm_forage_batch* batch = nullptr;
     int32_t n_replicas = 0;
     int64_t patch_total = 0;
-    size_t member_lds = 0;           // bytes of the membership masks per block
+    size_t member_lds = 0;           // bytes of the largest replica's membership masks
+    size_t world_lds = 0;            // LDS of the world kernel's workgroups
+    int32_t threads = 0;             // their threads
+    int32_t wide_reps = 0, wide_blocks = 0;   // replicas whose loop runs over the whole GPU, their blocks
+    int64_t wide_chunks = 0;         // their 64-agent chunks
+    void* wide_mem = nullptr;        // their scratch (the control words zeroed once)
     size_t collide_lds = 0;          // LDS of the collision kernel (0: no replica collides)
     void* wreps_dev = nullptr;
     int32_t* kill_rank = nullptr;    // [patch_total], -1 = not killed
