@@ -1,6 +1,8 @@
-// vf_f64.hip -- plain float64 VSWRM step: the reference arithmetic on the GPU.
+// vf_f64.hip -- float64 VSWRM step.  Two kernels with the same results: the
+// guarded one (below), and the plain one, the reference arithmetic on the GPU,
+// for what the guarded one does not take.
 //
-// One workgroup per replica.  The replica's poses live in LDS for the whole
+// The plain kernel: one workgroup per replica.  The replica's poses live in LDS for the whole
 // step and are updated in place, agent by agent in id order, which is the
 // reference's Group.update semantics (vf_sims.py:302; agent k sees agents <k
 // at their new poses).  Per agent:
@@ -11,8 +13,11 @@
 //   3. one lane: VSWRM motion, Euler step and boundary (vf_agent.py:188-204,
 //      263-326; agent.py:347-395, 605-610).
 // Built with -ffp-contract=off.
+#include <algorithm>
+
 #include "vf_batch.hpp"
 #include "vf_exact.hpp"
+#include "vf_f32_common.hpp"
 
 namespace abm {
 
@@ -183,6 +188,308 @@ vf_step_f64_kernel(const VFRep* __restrict__ reps, const double* __restrict__ tc
     if (count && n_near) atomicAdd(&counters[3], n_near);
 }
 
+// ---------------------------------------------------------------------------
+// The same step with the pairs' integer decisions made in float32 where
+// float32 is certain of them and by the exact float64 replica elsewhere;
+// state, sums and motion stay float64.  A pair's decision is its bin and its
+// half-width; the centre difference (periodic image included) is the float64
+// one, rounded once, the heading the float64 sine and cosine, rounded once, so
+// the float32 angle is within 1e-6 rad of the exact one and the guard bands of
+// the fused kernels (4e-6 rad around a bin tie and the +-pi wrap, 4e-6 relative
+// + 1e-6 around an integer half-width) cover it and the reference's own error
+// (vf_f32_common.hpp).  About 1 pair in 1000 takes the replica.
+//
+// One workgroup of NW waves per replica, largest first.  Lanes over objects
+// decide and OR each interval into a bit-packed field in LDS; every lane owns
+// RPL rays whose table entries it keeps in registers for the whole step; the
+// sums meet by DPP.  Bound by VALU
+// issue (batches) or the id-order chain's latency (few replicas).  Against the
+// plain kernel (exact decisions, a byte per ray, tables from memory): 4096
+// replicas of 50 agents at R = 512 0.773 -> 0.169 ms a step (1332 -> 461 VALU
+// instructions per agent-step, an eighth of them the motion's sincos; 0.91 of
+// the VALU issue slots filled), 512 of 37 at R = 300 in a walled arena 0.265 ->
+// 0.088 ms.
+constexpr int kGuardMaxWaves = 8;
+
+struct GuardSmem {
+    double *x, *y, *th, *v, *a0, *b0, *v0, *ox, *oy, *red;
+    float2* u;       // heading vectors (agents move only in their own turn)
+    int* rad;
+    uint2* D;        // the focal agent's field and its edges, a word of each
+    uint32_t* F;     // the field as the pairs set it
+};
+
+constexpr int kGuardRays = 8;   // at most, per lane
+
+__host__ __device__ inline size_t guard_lds_bytes(int N, int R, int nw, bool sync_order) {
+    return (size_t)N * (sizeof(double) * (sync_order ? 9 : 7) + sizeof(float2) + sizeof(int)) +
+           sizeof(double) * 4 * nw + sizeof(uint2) * 2 * kGuardRays * nw + sizeof(uint32_t) * ((size_t)(R + 31) / 32) + 16;
+}
+
+__device__ inline GuardSmem guard_carve(void* base, int N, int nw, bool sync_order) {
+    GuardSmem s;
+    char* p = reinterpret_cast<char*>(base);
+    for (double** d : {&s.x, &s.y, &s.th, &s.v, &s.a0, &s.b0, &s.v0}) {
+        *d = reinterpret_cast<double*>(p);
+        p += sizeof(double) * N;
+    }
+    s.ox = s.x; s.oy = s.y;
+    if (sync_order) {
+        s.ox = reinterpret_cast<double*>(p); p += sizeof(double) * N;
+        s.oy = reinterpret_cast<double*>(p); p += sizeof(double) * N;
+    }
+    s.red = reinterpret_cast<double*>(p); p += sizeof(double) * 4 * nw;
+    s.u = reinterpret_cast<float2*>(p); p += sizeof(float2) * N;
+    s.D = reinterpret_cast<uint2*>(p); p += sizeof(uint2) * 2 * kGuardRays * nw;
+    s.rad = reinterpret_cast<int*>(p); p += sizeof(int) * N;
+    s.F = reinterpret_cast<uint32_t*>(p);
+    return s;
+}
+
+// The float64 decision of a pair inside a guard band, out of line.
+struct Interval {
+    int start, end, drawn;
+};
+__device__ __noinline__ Interval exact_interval(double px, double py, double theta, double radius, double ox,
+                                                double oy, double osize, const VFRep* rp) {
+    const Focal f = make_focal(px, py, theta, radius);
+    const PairVF p = pair_vf_exact(f, ox, oy, osize, rp->boundary == ABM_BOUNDARY_INFINITE ? 1 : 0, rp->width,
+                                   rp->height, rp->n_rays, rp->step, rp->fov_px0, rp->fov_px1);
+    return Interval{p.start, p.end, p.skipped ? 0 : p.drawn};
+}
+
+// sincos out of line: inlined, its constants are held over the agent loop and
+// spilled to scratch, nine loads per agent.
+__device__ __noinline__ double2 sincos_f64(double x) {
+    double s, c;
+    sincos(x, &s, &c);
+    return make_double2(s, c);
+}
+
+template <int CTRL>
+__device__ inline double dpp_f64(double v) {
+    return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true),
+                            __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true));
+}
+// Wave sum, to every lane: quads, half rows, rows (every lane its row's), then
+// rows carried up to lane 63.
+__device__ inline double wave_total_f64(double x) {
+    x += dpp_f64<0xB1>(x);
+    x += dpp_f64<0x4E>(x);
+    x += dpp_f64<0x141>(x);
+    x += dpp_f64<0x140>(x);
+    x += f32::dpp_f64_masked<0x142, 0xa>(x);
+    x += f32::dpp_f64_masked<0x143, 0xc>(x);
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), 63),
+                            __builtin_amdgcn_readlane(__double2loint(x), 63));
+}
+
+// OR the rays [a, b) into the field: one or two words nearly always.
+__device__ inline void or_rays(uint32_t* F, int a, int b) {
+    if (a >= b) return;
+    const int w0 = a >> 5, w1 = (b - 1) >> 5;
+    const uint32_t m0 = 0xffffffffu << (a & 31), m1 = 0xffffffffu >> (31 - ((b - 1) & 31));
+    atomicOr(&F[w0], w0 == w1 ? m0 & m1 : m0);
+    if (w0 < w1) {
+        atomicOr(&F[w1], m1);
+        for (int w = w0 + 1; w < w1; ++w) atomicOr(&F[w], 0xffffffffu);
+    }
+}
+
+template <int NW, int RPL>
+__global__ void __launch_bounds__(64 * NW) __attribute__((amdgpu_waves_per_eu(4)))
+vf_step_f64_guard_kernel(const VFRep* __restrict__ reps, const int32_t* __restrict__ order,
+                         const double* __restrict__ tcos, const double* __restrict__ tsin,
+                         const double* __restrict__ tdphi, abm_vf_state_f64 st,
+                         uint32_t* __restrict__ bits_out, double* __restrict__ diag, uint32_t flags, int maxN) {
+#pragma clang fp contract(off)
+    extern __shared__ double smem[];
+    constexpr int NT = 64 * NW;
+    const VFRep* rp = reps + order[blockIdx.x];
+    const int N = rp->n_agents, R = rp->n_rays, W = rp->words, a0 = rp->agent_offset;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const bool sync_order = (flags & ABM_ORDER_SYNCHRONOUS) != 0;
+    const bool want_diag = diag != nullptr && (flags & ABM_WANT_DIAG) != 0;
+    const GuardSmem S = guard_carve(smem, maxN, NW, sync_order);
+    // this lane's rays, tid + NT i, and their table entries (zero at or beyond
+    // R): cos, sin and the trapz weight d_{r-1} / 2 + d_r / 2 (numpy's trapz
+    // terms d_k (y_{k+1} + y_k) / 2 gathered by ray).  Rays spread over the circle
+    // cancel within a lane, so the lanes' sums stay small and the tree rounds as
+    // little as the plain kernel's (spans of consecutive rays: 1.5 times its error).
+    double tw[RPL], tc[RPL], ts[RPL];
+#pragma unroll
+    for (int i = 0; i < RPL; ++i) {
+        const int r = tid + NT * i, e = rp->table_offset + (r < R ? r : 0);
+        const double left = r > 0 && r < R ? tdphi[e - 1] : 0.0, right = r < R - 1 ? tdphi[e] : 0.0;
+        tw[i] = left / 2.0 + right / 2.0;
+        tc[i] = r < R ? tcos[e] : 0.0;
+        ts[i] = r < R ? tsin[e] : 0.0;
+    }
+    for (int w = tid; w < 2 * kGuardRays * NW; w += NT) S.D[w] = make_uint2(0u, 0u);   // beyond the field: no ray
+    for (int i = tid; i < N; i += NT) {
+        const int g = a0 + i;
+        const double th = st.theta[g];
+        S.x[i] = st.x[g]; S.y[i] = st.y[g]; S.th[i] = th; S.v[i] = st.v[g];
+        S.rad[i] = st.radius[g];
+        S.a0[i] = st.alp0 ? st.alp0[g] : rp->alp0;
+        S.b0[i] = st.bet0 ? st.bet0[g] : rp->bet0;
+        S.v0[i] = st.v0 ? st.v0[g] : rp->v0;
+        const double2 sc = sincos_f64(th);
+        S.u[i] = make_float2((float)sc.y, -(float)sc.x);   // unit(v1) = (cos th, -sin th)
+        if (sync_order) { S.ox[i] = S.x[i]; S.oy[i] = S.y[i]; }
+    }
+    const bool torus = rp->boundary == ABM_BOUNDARY_INFINITE;
+    const double Wd = rp->width, Hd = rp->height, hw = Wd / 2.0, hh = Hd / 2.0;
+    const float inv_step = (float)(1.0 / rp->step), hs = (float)((double)R / kTwoPi);
+    const float g_bins = (float)(f32::kAngleGuardF / rp->step + 1.5e-7 * R);
+    const int px0 = rp->fov_px0, px1 = rp->fov_px1;
+    __syncthreads();
+
+    for (int k = 0; k < N; ++k) {
+        // a SIMD's arbiter favours its oldest wave: each lowers its own
+        // priority as it advances, so that a batch's waves finish together
+        if (NW == 1) {
+            if (k == 0) __builtin_amdgcn_s_setprio(3);
+            else if (k == N / 2) __builtin_amdgcn_s_setprio(2);
+            else if (k == 3 * N / 4) __builtin_amdgcn_s_setprio(1);
+            else if (k == 15 * N / 16) __builtin_amdgcn_s_setprio(0);
+        }
+        for (int w = tid; w < W; w += NT) S.F[w] = 0u;
+        const double fx = S.x[k], fy = S.y[k], fr = (double)S.rad[k], cx = fx + fr, cy = fy + fr;
+        const float2 u = S.u[k];
+        __syncthreads();
+        // ---- pairs
+        for (int j = tid; j < N; j += NT) {
+            const double ojx = S.ox[j], ojy = S.oy[j], os = (double)S.rad[j];
+            if (j == k || (ojx == fx && ojy == fy)) continue;   // coincident (vf_supcalc.py:57)
+            // the centre difference exactly as pair_vf_exact forms it (a
+            // difference beyond half the arena is not zero, so its sign is
+            // that of the comparison there)
+            const double ocx = ojx + os, ocy = ojy + os;
+            double vx = ocx - cx, vy = ocy - cy;
+            if (torus) {
+                vx = (ocx - (fabs(vx) > hw ? copysign(Wd, vx) : 0.0)) - cx;
+                vy = (ocy - (fabs(vy) > hh ? copysign(Hd, vy) : 0.0)) - cy;
+            }
+            const float dx = (float)vx, dy = (float)vy;
+            const float d2 = fmaf(dy, dy, dx * dx);
+            const float a = f32::atan2_f32(fmaf(u.x, dy, -u.y * dx), fmaf(u.x, dx, u.y * dy));
+            const float z = (float)os * __builtin_amdgcn_rsqf(d2);
+            const float xb = (f32::kPiF - a) * inv_step;   // bin coordinate of the closed angle -a
+            const float tr = rintf(xb), dfr = xb - tr;
+            const float half = f32::atan_unit_f32(z) * hs;   // proj_size / 2
+            const float hfl = floorf(half), hfrac = half - hfl, hg = 4e-6f * fabsf(half) + 1e-6f;
+            const bool ok = (d2 > 1e-30f) & (fabsf(z) < 1.0f) & (fabsf(a) < f32::kPiF - f32::kAngleGuardF) &
+                            (hfrac >= hg) & (hfrac <= 1.0f - hg) & (fabsf(dfr) <= 0.5f - g_bins);
+            const int t = (int)tr, h = (int)hfl;
+            Interval p{t - h, t + h, 0};
+            p.drawn = ((px0 < p.start) & (p.start < px1)) | ((px0 < p.end) & (p.end < px1));
+            if (!ok) p = exact_interval(fx, fy, S.th[k], fr, ojx, ojy, os, rp);
+            if (p.drawn) {
+                // vf_pieces: the part inside, and the part that wraps (at
+                // most one end does; an end at or beyond R wraps one ray less)
+                or_rays(S.F, clamp_ray(p.start, R), p.end >= R ? R : clamp_ray(p.end, R));
+                if (p.start < 0 || p.end >= R)
+                    or_rays(S.F, p.end >= R ? 0 : clamp_ray(R + p.start, R), p.end >= R ? clamp_ray(p.end - (R - 1), R) : R);
+            }
+        }
+        __syncthreads();
+        // ---- sums: the field's edges by the dPhi alignment rule
+        // (vf_supcalc.py:266-274), then the table entries added where a bit is
+        // set (as fma(bit ? w : 0, t, acc), one rounding)
+        const bool case1 = (S.F[0] & 1u) == 1u && f32::field_bit(S.F, R - 1) == 0u;
+        for (int w = tid; w < W; w += NT) {
+            const uint32_t cur = S.F[w];
+            const int nb = w == W - 1 ? R - 32 * w : 32;   // the word's rays
+            const uint32_t other = case1 ? (cur << 1) | (w ? S.F[w - 1] >> 31 : 0u)
+                                         : (cur >> 1) | ((w == W - 1 ? S.F[0] & 1u : S.F[w + 1] & 1u) << (nb - 1));
+            S.D[w] = make_uint2(cur, (cur ^ other) & f32::low_mask(nb));
+        }
+        __syncthreads();
+        const uint2* const D = S.D + (tid >> 5);
+        const int sh = tid & 31;
+        double bc = 0.0, bs = 0.0, ec = 0.0, es = 0.0;
+#pragma unroll
+        for (int i = 0; i < RPL; ++i) {
+            const uint2 d = D[(NT / 32) * i];
+            const int vm = __builtin_amdgcn_sbfe((int)d.x, sh, 1), sm = __builtin_amdgcn_sbfe((int)d.y, sh, 1);
+            const double vb = __hiloint2double(vm & __double2hiint(tw[i]), vm & __double2loint(tw[i]));
+            const double sb = __hiloint2double(sm & 0x3ff00000, 0);
+            bc = __builtin_fma(vb, tc[i], bc);
+            bs = __builtin_fma(vb, ts[i], bs);
+            ec = __builtin_fma(sb, tc[i], ec);
+            es = __builtin_fma(sb, ts[i], es);
+        }
+        const double alp0 = S.a0[k], bet0 = S.b0[k], vel = S.v[k];
+        const double ae0 = alp0 * rp->alp1, be0 = bet0 * rp->bet1;
+        // blob terms: trapz(cos(PHI) * (-V)) = -sum(w cos V)
+        double Sv, Sp, ab = 0.0, ae = 0.0, bb = 0.0, be = 0.0;
+        if (!want_diag) {
+            Sv = wave_total_f64(__builtin_fma(ae0, ec, -(alp0 * bc)));
+            Sp = wave_total_f64(__builtin_fma(be0, es, -(bet0 * bs)));
+            if (NW > 1) {
+                if (lane == 0) { S.red[2 * (tid >> 6)] = Sv; S.red[2 * (tid >> 6) + 1] = Sp; }
+                __syncthreads();
+                Sv = Sp = 0.0;
+#pragma unroll
+                for (int w = 0; w < NW; ++w) { Sv += S.red[2 * w]; Sp += S.red[2 * w + 1]; }
+            }
+        } else {
+            double c[4] = {wave_total_f64(bc), wave_total_f64(bs), wave_total_f64(ec), wave_total_f64(es)};
+            if (NW > 1) {
+                if (lane == 0)
+                    for (int q = 0; q < 4; ++q) S.red[4 * (tid >> 6) + q] = c[q];
+                __syncthreads();
+                for (int q = 0; q < 4; ++q) {
+                    c[q] = 0.0;
+                    for (int w = 0; w < NW; ++w) c[q] += S.red[4 * w + q];
+                }
+            }
+            ab = alp0 * -c[0]; bb = bet0 * -c[1]; ae = ae0 * c[2]; be = be0 * c[3];
+            Sv = ab + ae;
+            Sp = bb + be;
+        }
+        if (bits_out) {
+            uint32_t* dst = bits_out + rp->field_offset + (int64_t)k * W;
+            for (int w = tid; w < W; w += NT) dst[w] = S.F[w];
+        }
+        // ---- motion, on every lane (one writes it)
+        double dv = 0.0, dpsi = 0.0;
+        if (rp->phi_ok) {
+            dv = __builtin_fma(rp->gam, S.v0[k] - vel, Sv);
+            dpsi = Sp;
+        } else {
+            ab = ae = bb = be = 0.0;
+        }
+        // vf_move with one sincos for both values
+        double turn = dpsi;
+        if (rp->limit_movement && fabs(turn) > rp->max_th) turn = turn < 0.0 ? -rp->max_th : rp->max_th;
+        Pose p{fx, fy, prove_orientation(S.th[k] + turn), vel + dv};
+        if (rp->limit_movement && fabs(p.v) > rp->max_vel) p.v = p.v < 0.0 ? -rp->max_vel : rp->max_vel;
+        const double2 sc = sincos_f64(p.theta);
+        p.x = fx + p.v * sc.y;
+        p.y = fy - p.v * sc.x;
+        p = torus ? teleport(p, fr, rp->pad, Wd, Hd) : reflect_walls(p, fr, rp->pad, Wd, Hd);
+        // every wave has read agent k's pose and the field
+        if (NW > 1) __syncthreads();
+        if (tid == 0) {
+            S.x[k] = p.x; S.y[k] = p.y; S.th[k] = p.theta; S.v[k] = p.v;
+            if (want_diag) {
+                double* d = diag + 6 * (int64_t)(a0 + k);
+                d[0] = dv; d[1] = dpsi; d[2] = ab; d[3] = ae; d[4] = bb; d[5] = be;
+            }
+        }
+    }
+    __syncthreads();
+    for (int i = tid; i < N; i += NT) {
+        const int g = a0 + i;
+        st.x[g] = S.x[i];
+        st.y[g] = S.y[i];
+        st.theta[g] = S.th[i];
+        st.v[g] = S.v[i];
+    }
+}
+
 }  // namespace
 
 size_t vf_f64_lds_bytes(int max_agents, int max_rays, int nthr, bool sync_order) {
@@ -190,9 +497,55 @@ size_t vf_f64_lds_bytes(int max_agents, int max_rays, int nthr, bool sync_order)
     return d * sizeof(double) + (size_t)max_rays + 16;
 }
 
+namespace {
+
+// Waves per replica of the guarded kernel, 0 where it does not apply: the
+// near-tie count (it needs every pair's float64 angle), R beyond 4096 (eight
+// waves of eight rays a lane) or replicas beyond its LDS.  As few waves as hold
+// the rays at eight a lane, or, while the batch leaves SIMDs with fewer than two
+// waves, up to four that bring the rays to four a lane or the objects to one
+// (us a step with 1, 2, 4, 8 waves: one replica of 100 agents at R = 1024 -, 251,
+// 235, 288; of 300 at 512 1279, 961, 842, 903; 256 replicas of 100 at 512 281,
+// 224, 236, 289; 512 of 150 at 300 496, 432, 381, 522; 1000 of 64 at 1000 -, 190,
+// 220, 450; 2048 of 50 at 512 139, 168, 304, 654).
+int guard_waves(const abm_vf_batch* b, uint32_t flags) {
+    if ((flags & ABM_COUNT_RECHECKS) != 0 || b->max_rays > 64 * 8 * kGuardMaxWaves) return 0;
+    int nw = 1;
+    while (64 * 8 * nw < b->max_rays) nw *= 2;
+    const int want = std::max((b->max_rays + 255) / 256, (b->max_agents + 63) / 64);
+    while (nw < want && nw < 4 && (int64_t)b->n_replicas * nw * 2 <= 8ll * b->n_cu) nw *= 2;
+    const size_t lds = guard_lds_bytes(b->max_agents, b->max_rays, nw, (flags & ABM_ORDER_SYNCHRONOUS) != 0);
+    return lds <= (size_t)b->dev_max_lds ? nw : 0;
+}
+
+int launch_guard(abm_vf_batch* b, const abm_vf_state_f64* st, uint32_t* bits, double* diag, uint32_t flags,
+                 hipStream_t s, int nw, int rpl) {
+    const size_t lds = guard_lds_bytes(b->max_agents, b->max_rays, nw, (flags & ABM_ORDER_SYNCHRONOUS) != 0);
+    auto kern = rpl == 4 ? (nw == 1 ? vf_step_f64_guard_kernel<1, 4>
+                            : nw == 2 ? vf_step_f64_guard_kernel<2, 4>
+                            : nw == 4 ? vf_step_f64_guard_kernel<4, 4> : vf_step_f64_guard_kernel<8, 4>)
+                         : (nw == 1 ? vf_step_f64_guard_kernel<1, 8>
+                            : nw == 2 ? vf_step_f64_guard_kernel<2, 8>
+                            : nw == 4 ? vf_step_f64_guard_kernel<4, 8> : vf_step_f64_guard_kernel<8, 8>);
+    if (lds > 65536)
+        if (int rc = check_hip(hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                                   (int)lds), "hipFuncSetAttribute"))
+            return rc;
+    hipLaunchKernelGGL(kern, dim3(b->n_replicas), dim3(64 * nw), lds, s, b->reps_dev, b->order_dev, b->tab_cos,
+                       b->tab_sin, b->tab_dphi, *st, bits, diag, flags, b->max_agents);
+    b->last_kernels = ABM_KERNEL_F64;
+    return check_hip(hipGetLastError(), "vf_step_f64_guard_kernel launch");
+}
+
+}  // namespace
+
 int launch_vf_step_f64(abm_vf_batch* b, const abm_vf_state_f64* st, uint32_t* bits,
                        double* diag, uint32_t flags, hipStream_t s) {
     const bool sync_order = (flags & ABM_ORDER_SYNCHRONOUS) != 0;
+    if (const int nw = guard_waves(b, flags)) {
+        const int per = (b->max_rays + 64 * nw - 1) / (64 * nw);
+        return launch_guard(b, st, bits, diag, flags, s, nw, per <= 4 ? 4 : 8);
+    }
     int nthr = 64;
     if (b->max_rays >= 1024 || b->max_agents > 128) nthr = 128;
     if (b->max_agents > 512) nthr = 256;
