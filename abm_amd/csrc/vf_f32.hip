@@ -1045,38 +1045,57 @@ int launch_big_any(abm_vf_batch* b, const abm_vf_state_f32* st, uint32_t* bits, 
 // from LDS, the loads of the sums waited on the other waves' LDS traffic.
 constexpr int kPushThreads = 64 * kPushWaves;
 
+// Rays added to a field in registers: up to two pieces [a, b) (wave-uniform).
+struct Pieces {
+    int a0, b0, a1, b1;
+};
+
+// Bits of the lane's rays [rs, rs + RPL) inside [a, b).
+template <int RPL>
+__device__ __forceinline__ uint32_t span_mask(int a, int b, int rs) {
+    const int lo = min(max(a - rs, 0), RPL), hi = min(max(b - rs, lo), RPL);
+    if (RPL < 32) return (1u << hi) - (1u << lo);
+    return low_mask(hi) & ~low_mask(lo);
+}
+
 // The one-wave sums of a field Fk, as the one-wave per-replica kernel takes
 // them: lane l sums its rays [l RPL, (l + 1) RPL) (table entries T) in float32,
 // the wave totals are float64.  Without diagnostics the two integrals are
 // totalled directly (Sv, Sp); with them the four parts (Bc, Bs, Ec, Es) and
 // the integrals from those.  Shared by the push kernel and the chain step's
-// segment kernel, which thereby give the same results bit for bit.
+// segment kernel, which thereby give the same results bit for bit.  A lane's
+// rays lie in one word (RPL divides 32), its neighbours' rays come from the
+// lanes beside it, so one LDS read starts the sums; `more` holds rays that are
+// not in Fk yet.
 template <int RPL>
 __device__ __forceinline__ void one_wave_sums(const uint32_t* Fk, const RayTab32* T, int lane, const RepConst& C,
-                                              bool want_diag, float alp0, float bet0, double& Sv, double& Sp,
-                                              double& Bc, double& Bs, double& Ec, double& Es) {
+                                              bool want_diag, float alp0, float bet0, const Pieces& more,
+                                              double& Sv, double& Sp, double& Bc, double& Bs, double& Ec,
+                                              double& Es) {
     const int rs = lane * RPL;
     const int rn = rs >= C.R ? 0 : (C.R - rs < RPL ? C.R - rs : RPL);
-    const bool case1 = (Fk[0] & 1u) == 1u && field_bit(Fk, C.R - 1) == 0u;
     float bc = 0.f, bs = 0.f, ec = 0.f, es = 0.f;
     {
-        const int w0 = rs >> 5;
-        const uint32_t lo = w0 < C.W ? Fk[w0] : 0u;
-        const uint32_t hi = (RPL > 1 && w0 + 1 < C.W) ? Fk[w0 + 1] : 0u;
-        const uint64_t v64 = (((uint64_t)hi << 32) | lo) >> (rs & 31);
         const uint32_t m = low_mask(rn);
-        const uint32_t cur = (uint32_t)v64 & m;
-        uint32_t spike = 0u;
-        if (rn > 0) {
-            if (case1) {
-                const uint32_t prev = field_bit(Fk, rs == 0 ? C.R - 1 : rs - 1);
-                spike = (cur ^ ((cur << 1) | prev)) & m;
-            } else {
-                const int nx = rs + rn;
-                const uint32_t next = field_bit(Fk, nx >= C.R ? 0 : nx);
-                spike = (cur ^ ((cur >> 1) | (next << (rn - 1)))) & m;
-            }
+        uint32_t cur = Fk[min(rs >> 5, C.W - 1)] >> (rs & 31);
+        if (more.b0 > more.a0) cur |= span_mask<RPL>(more.a0, more.b0, rs);
+        if (more.b1 > more.a1) cur |= span_mask<RPL>(more.a1, more.b1, rs);
+        cur &= m;
+        // edges by the dPhi alignment rule (vf_supcalc.py:266-274): against the
+        // ray before when ray 0 is set and ray R - 1 is not, else the ray after
+        const int end_lane = (C.R - 1) / RPL;
+        const uint32_t first = (uint32_t)__builtin_amdgcn_readfirstlane((int)cur) & 1u;
+        const uint32_t last = ((uint32_t)__builtin_amdgcn_readlane((int)cur, end_lane) >> ((C.R - 1) % RPL)) & 1u;
+        uint32_t other;
+        if (first == 1u && last == 0u) {   // wave_shr:1; lane 0's ray before is R - 1, not set
+            const uint32_t low = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)cur, 0x138, 0xf, 0xf, false);
+            other = (cur << 1) | (low >> (RPL - 1));
+        } else {                           // wave_shl:1; the last ray's next is ray 0
+            uint32_t up = (uint32_t)__builtin_amdgcn_update_dpp(0, (int)cur, 0x130, 0xf, 0xf, false) & 1u;
+            up = lane == end_lane ? first : up;
+            other = (cur >> 1) | (up << ((rn - 1) & 31));
         }
+        const uint32_t spike = (cur ^ other) & m;
         // acc + (bit ? t : 0) as fma(bit, t, acc): the same value (a 0 bit adds
         // a zero to an accumulator that is never -0), without a lane mask
 #pragma unroll
@@ -1251,16 +1270,23 @@ vf_step_f32_push_kernel(const VFRep* __restrict__ reps, const int32_t* __restric
     }
     __syncthreads();
     if (wave == 0) __builtin_amdgcn_s_setprio(3);   // the chain's wave issues first
+    float4 f1 = P0[0], d1 = dyn[0];   // wave 0: the next agent's
+    Pieces more{0, 0, 0, 0};          // wave 0: the pair (k, k - 1)'s rays, not in F
     for (int k = 0; k < C.N; ++k) {
         if (wave == 0) {
-            // ---- agent k's sums, as the one-wave per-replica kernel
+            // ---- agent k's sums, as the one-wave per-replica kernel; the next
+            // agent's start pose, heading and parameters (constant over the
+            // step) load meanwhile
             const uint32_t* Fk = F + (size_t)k * W1;
-            const float4 fp = P0[k];
-            const float4 dk = dyn[k];
+            const float4 fp = f1, dk = d1;
+            const int k1 = min(k + 1, C.N - 1);
+            f1 = P0[k1];
+            d1 = dyn[k1];
+            const float2 u1 = U[k1];
             const float fx = fp.x, fy = fp.y, fr = fp.z, fth = fp.w;
             const float alp0 = dk.y, bet0 = dk.z, v0 = dk.w;
             double Sv, Sp, Bc, Bs, Ec, Es;
-            one_wave_sums<RPL>(Fk, T, lane, C, want_diag, alp0, bet0, Sv, Sp, Bc, Bs, Ec, Es);
+            one_wave_sums<RPL>(Fk, T, lane, C, want_diag, alp0, bet0, more, Sv, Sp, Bc, Bs, Ec, Es);
             if (!PLAIN && bits_out) {
                 uint32_t* dst = bits_out + C.field_offset + (int64_t)k * C.W;
                 for (int w = lane; w < C.W; w += 64) dst[w] = Fk[w];
@@ -1285,13 +1311,24 @@ vf_step_f32_push_kernel(const VFRep* __restrict__ reps, const int32_t* __restric
                     dd[4] = C.phi_ok ? (float)((double)bet0 * -Bs) : 0.f;
                     dd[5] = C.phi_ok ? (float)((double)(bet0 * C.bet1) * Es) : 0.f;
                 }
-                if (k + 1 < C.N) {
-                    const float4 f1 = P0[k + 1];
+                if (!PLAIN && k + 1 < C.N) {
                     if (push_culled(f1, moved, C, cull_c))
                         push_culled_check(f1, moved, rp, count, verify, n_pairs, n_disagree);
                     else
-                        push_pair(F + (size_t)(k + 1) * W1, U[k + 1], f1, moved, rp, C, count, verify,
+                        push_pair(F + (size_t)(k + 1) * W1, u1, f1, moved, rp, C, count, verify,
                                   n_pairs, n_recheck, n_disagree);
+                }
+            }
+            if (PLAIN) {
+                // on every lane alike: its rays go into agent k + 1's sums
+                // from registers (a pair beyond the cut-off decides to none)
+                PairF32 pr;
+                more = Pieces{0, 0, 0, 0};
+                if (decide_pair(pr, u1, f1, moved, rp, C, false, false, n_pairs, n_recheck, n_disagree)) {
+                    Pieces q;
+                    vf_pieces(pr.start, pr.end, C.R, &q.a0, &q.b0, &q.a1, &q.b1);
+                    more.a0 = __builtin_amdgcn_readfirstlane(q.a0); more.b0 = __builtin_amdgcn_readfirstlane(q.b0);
+                    more.a1 = __builtin_amdgcn_readfirstlane(q.a1); more.b1 = __builtin_amdgcn_readfirstlane(q.b1);
                 }
             }
         } else {
@@ -1496,7 +1533,7 @@ vf_step_f32_segment_kernel(const VFRep* __restrict__ rp, const RayTab32* __restr
     auto sums = [&](int kk, int buf) {
         const float4 d = sdyn[kk];
         double Sv, Sp, Bc, Bs, Ec, Es;
-        one_wave_sums<RPL>(rows[kk], T, lane, C, want_diag, d.y, d.z, Sv, Sp, Bc, Bs, Ec, Es);
+        one_wave_sums<RPL>(rows[kk], T, lane, C, want_diag, d.y, d.z, Pieces{0, 0, 0, 0}, Sv, Sp, Bc, Bs, Ec, Es);
         if (lane == 0) {
             double* r = red[buf];
             r[0] = Sv; r[1] = Sp; r[2] = Bc; r[3] = Bs; r[4] = Ec; r[5] = Es;
