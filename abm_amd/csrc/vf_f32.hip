@@ -1029,20 +1029,29 @@ int launch_big_any(abm_vf_batch* b, const abm_vf_state_f32* st, uint32_t* bits, 
 // is the OR of its pairs with every other agent j, seen at j's new pose for
 // j < m and at its start pose for j > m, and m itself at its start pose.
 // Step k of the chain (one barrier each):
-//   * wave 0 sums agent k's field, moves agent k and decides the pair
-//     (k + 1, k) at k's new pose;
-//   * waves 1..7 decide the pairs (m, k - 1) for m > k with agent k - 1's
+//   * wave 0 moves agent k by the sums of its field and decides the pairs
+//     (k + 1, k) and (k + 2, k) at k's new pose;
+//   * wave 1 sums agent k + 1's field, complete but for the pair (k + 1, k),
+//     with the rays that pair would set if agent k kept its heading and speed;
+//     where the decided rays differ, wave 0 takes agent k + 1's sums again
+//     with the decided ones, so a wrong guess costs time and no result;
+//   * waves 2..7 decide the pairs (m, k - 1) for m > k + 1 with agent k - 1's
 //     new pose.
 // The start-pose pairs (m, j > m) are decided before the chain by every
 // wave.  Pairs beyond the visibility cut-off are dropped by a cheap float32
 // test (as in the 16-wave kernel) and the rest queued, so that the exact
 // decisions run on full waves.
-// So only one pair, agent k's sums and its move stay on the chain.  Wave 0
-// sums and moves exactly as the one-wave per-replica kernel does (same ray
-// spans, table order and reductions), and the decisions are exact, so the
-// two kernels give identical results bit for bit.  Wave 0 keeps its rays'
-// table entries in registers (up to 128), which two waves per SIMD allow;
-// from LDS, the loads of the sums waited on the other waves' LDS traffic.
+// So only agent k's move and one pair deep of decisions stay on the chain
+// (about 0.5 + 1.0 thousand cycles of latency; the sums are another 1.3, which
+// the guess takes off the chain).  The sums and moves are exactly those of the
+// one-wave per-replica kernel (same ray spans, table order and reductions),
+// and the decisions are exact, so the two kernels give identical results bit
+// for bit.  Waves 0 and 1 keep their rays' table entries in registers (up to
+// 128), which two waves per SIMD allow; from LDS, the loads of the sums waited
+// on the other waves' LDS traffic.  Measured, one replica of 100 agents at
+// R = 1024: 0.160 ms a step with the sums and their LDS round trips on the
+// chain, 0.141 with the pair handed over in registers, 0.123 with wave 1
+// summing ahead; 1000 replicas of 8 to 512 agents, 1.025, 0.989, 0.931.
 constexpr int kPushThreads = 64 * kPushWaves;
 
 // Rays added to a field in registers: up to two pieces [a, b) (wave-uniform).
@@ -1203,6 +1212,7 @@ vf_step_f32_push_kernel(const VFRep* __restrict__ reps, const int32_t* __restric
     float2* U = reinterpret_cast<float2*>(p); p += sizeof(float2) * (size_t)C.N;     // (cos, -sin) of start headings
     uint32_t* queue = reinterpret_cast<uint32_t*>(p); p += sizeof(uint32_t) * kPushQueue * kPushWaves;
     uint32_t* F = reinterpret_cast<uint32_t*>(p);                                     // [N][W + 1] fields
+    __shared__ double red[2][6];   // Sv, Sp, Bc, Bs, Ec, Es of agents k and k + 1
     const float cull_c = (float)rp->cull_c;
     uint32_t* wq = queue + wave * kPushQueue;   // this wave's ring of queued pairs
     const float a0d = (float)rp->alp0, b0d = (float)rp->bet0, v0d = (float)rp->v0;
@@ -1216,9 +1226,9 @@ vf_step_f32_push_kernel(const VFRep* __restrict__ reps, const int32_t* __restric
         sincos_f32(q.w, &sth, &cth);
         U[i] = make_float2(cth, -sth);
     }
-    // wave 0's lane l owns rays [l RPL, (l + 1) RPL) and their table entries
+    // in waves 0 and 1 lane l owns rays [l RPL, (l + 1) RPL) and their table entries
     RayTab32 T[RPL];
-    if (wave == 0) {
+    if (wave <= 1) {
 #pragma unroll
         for (int i = 0; i < RPL; ++i) {
             const int r = lane * RPL + i;
@@ -1268,30 +1278,70 @@ vf_step_f32_push_kernel(const VFRep* __restrict__ reps, const int32_t* __restric
                       n_disagree);
         }
     }
+    // ---- where agent i will be if it keeps its heading and speed, and the
+    // rays its pair (i + 1, i) then sets: a prediction, left in P1[i + 1] until
+    // agent i + 1's new pose goes there
+    for (int i = tid; i < C.N; i += kPushThreads) {
+        Pieces q{0, 0, 0, 0};
+        if (i > 0) {
+            const float4 b = P0[i - 1];
+            const float2 ub = U[i - 1];
+            const float vb = dyn[i - 1].x;
+            const float4 f = P0[i];
+            const PairF32 pr = fast_pair(U[i].x, U[i].y, f.x, f.y, f.z, b.x + vb * ub.x, b.y + vb * ub.y, b.z, C);
+            if (pr.drawn) vf_pieces(pr.start, pr.end, C.R, &q.a0, &q.b0, &q.a1, &q.b1);
+        }
+        P1[i] = make_float4(__int_as_float(q.a0), __int_as_float(q.b0), __int_as_float(q.a1), __int_as_float(q.b1));
+    }
     __syncthreads();
-    if (wave == 0) __builtin_amdgcn_s_setprio(3);   // the chain's wave issues first
-    float4 f1 = P0[0], d1 = dyn[0];   // wave 0: the next agent's
-    Pieces more{0, 0, 0, 0};          // wave 0: the pair (k, k - 1)'s rays, not in F
+    auto predicted = [&](int i) {
+        const float4 q = P1[i];
+        return Pieces{__float_as_int(q.x), __float_as_int(q.y), __float_as_int(q.z), __float_as_int(q.w)};
+    };
+    auto sums_into = [&](int i, const Pieces& more, double* r) {   // wave 1
+        const float4 d = dyn[i];
+        double Sv, Sp, Bc, Bs, Ec, Es;
+        one_wave_sums<RPL>(F + (size_t)i * W1, T, lane, C, want_diag, d.y, d.z, more, Sv, Sp, Bc, Bs, Ec, Es);
+        if (lane == 0) {
+            r[0] = Sv; r[1] = Sp;
+            if (want_diag) { r[2] = Bc; r[3] = Bs; r[4] = Ec; r[5] = Es; }
+        }
+    };
+    if (wave == 1) sums_into(0, Pieces{0, 0, 0, 0}, red[0]);   // agent 0's field is complete
+    __syncthreads();
+    if (wave == 0) __builtin_amdgcn_s_setprio(3);   // the chain's wave issues first,
+    if (wave == 1) __builtin_amdgcn_s_setprio(2);   // then the summing wave
+    const int last = C.N - 1;
+    float4 f0 = P0[0], f1 = P0[min(1, last)];   // wave 0: start poses of agents k, k + 1
+    float2 u1 = U[min(1, last)];
+    Pieces more{0, 0, 0, 0};   // wave 0: the rays of the pair (k, k - 1)
+    bool hit = true;           // wave 0: they are the ones wave 1 summed with
     for (int k = 0; k < C.N; ++k) {
         if (wave == 0) {
-            // ---- agent k's sums, as the one-wave per-replica kernel; the next
-            // agent's start pose, heading and parameters (constant over the
-            // step) load meanwhile
+            // ---- agent k's sums: wave 1's, or taken again where the
+            // prediction missed; what the next steps need loads meanwhile
             const uint32_t* Fk = F + (size_t)k * W1;
-            const float4 fp = f1, dk = d1;
-            const int k1 = min(k + 1, C.N - 1);
-            f1 = P0[k1];
-            d1 = dyn[k1];
-            const float2 u1 = U[k1];
-            const float fx = fp.x, fy = fp.y, fr = fp.z, fth = fp.w;
+            const double* r = red[k & 1];
+            double Sv = r[0], Sp = r[1], Bc = 0.0, Bs = 0.0, Ec = 0.0, Es = 0.0;
+            const float4 dk = dyn[k], f2 = P0[min(k + 2, last)];
+            const float2 u2 = U[min(k + 2, last)];
+            const Pieces guess = predicted(min(k + 1, last));
+            const float fx = f0.x, fy = f0.y, fr = f0.z, fth = f0.w;
             const float alp0 = dk.y, bet0 = dk.z, v0 = dk.w;
-            double Sv, Sp, Bc, Bs, Ec, Es;
-            one_wave_sums<RPL>(Fk, T, lane, C, want_diag, alp0, bet0, more, Sv, Sp, Bc, Bs, Ec, Es);
-            if (!PLAIN && bits_out) {
-                uint32_t* dst = bits_out + C.field_offset + (int64_t)k * C.W;
-                for (int w = lane; w < C.W; w += 64) dst[w] = Fk[w];
+            if (!PLAIN) {
+                if (want_diag) { Bc = r[2]; Bs = r[3]; Ec = r[4]; Es = r[5]; }
+                if (bits_out) {   // the one pair that is not in the row
+                    if (lane == 0) {
+                        or_range(F + (size_t)k * W1, more.a0, more.b0);
+                        or_range(F + (size_t)k * W1, more.a1, more.b1);
+                    }
+                    wave_lds_sync();
+                    uint32_t* dst = bits_out + C.field_offset + (int64_t)k * C.W;
+                    for (int w = lane; w < C.W; w += 64) dst[w] = Fk[w];
+                }
             }
-            // ---- agent k's move, then the pair (k + 1, k) at its new pose
+            if (!hit) one_wave_sums<RPL>(Fk, T, lane, C, want_diag, alp0, bet0, more, Sv, Sp, Bc, Bs, Ec, Es);
+            // ---- agent k's move
             float vel, o, dv, dpsi;
             steer(C, fth, dk.x, v0, (float)Sv, (float)Sp, &o, &vel, &dv, &dpsi);
             float so, co;
@@ -1299,6 +1349,33 @@ vf_step_f32_push_kernel(const VFRep* __restrict__ reps, const int32_t* __restric
             float nx, ny;
             euler_boundary(C, fx, fy, fr, vel, so, co, &o, &nx, &ny);
             const float4 moved = make_float4(nx, ny, fr, o);
+            // ---- the pairs (k + 1, k), on even lanes, and (k + 2, k), on odd
+            // ones, at its new pose; counted on lanes 0 and 1
+            const bool odd = (lane & 1) != 0;
+            const bool there = k + (odd ? 2 : 1) < C.N;
+            const bool once = lane < 2 && there;
+            const float4 f = odd ? f2 : f1;
+            const float2 u = odd ? u2 : u1;
+            PairF32 pr;
+            pr.drawn = false;
+            Pieces q{0, 0, 0, 0};
+            bool culled = false;
+            if (count && odd && there && push_culled(f, moved, C, cull_c)) {   // counted as every pushed pair
+                culled = true;
+                if (once) push_culled_check(f, moved, rp, count, verify, n_pairs, n_disagree);
+            }
+            if (there && !culled &&
+                decide_pair(pr, u, f, moved, rp, C, count && once, verify && once, n_pairs, n_recheck, n_disagree))
+                vf_pieces(pr.start, pr.end, C.R, &q.a0, &q.b0, &q.a1, &q.b1);
+            if (lane == 1) {
+                or_range(F + (size_t)(k + 2) * W1, q.a0, q.b0);
+                or_range(F + (size_t)(k + 2) * W1, q.a1, q.b1);
+            }
+            more.a0 = __builtin_amdgcn_readfirstlane(q.a0); more.b0 = __builtin_amdgcn_readfirstlane(q.b0);
+            more.a1 = __builtin_amdgcn_readfirstlane(q.a1); more.b1 = __builtin_amdgcn_readfirstlane(q.b1);
+            hit = more.a0 == __builtin_amdgcn_readfirstlane(guess.a0) && more.b0 == __builtin_amdgcn_readfirstlane(guess.b0) &&
+                  more.a1 == __builtin_amdgcn_readfirstlane(guess.a1) && more.b1 == __builtin_amdgcn_readfirstlane(guess.b1);
+            f0 = f1; f1 = f2; u1 = u2;
             if (lane == 0) {
                 const int gk = C.a0 + k;
                 P1[k] = moved;
@@ -1311,60 +1388,20 @@ vf_step_f32_push_kernel(const VFRep* __restrict__ reps, const int32_t* __restric
                     dd[4] = C.phi_ok ? (float)((double)bet0 * -Bs) : 0.f;
                     dd[5] = C.phi_ok ? (float)((double)(bet0 * C.bet1) * Es) : 0.f;
                 }
-                if (!PLAIN && k + 1 < C.N) {
-                    if (push_culled(f1, moved, C, cull_c))
-                        push_culled_check(f1, moved, rp, count, verify, n_pairs, n_disagree);
-                    else
-                        push_pair(F + (size_t)(k + 1) * W1, u1, f1, moved, rp, C, count, verify,
-                                  n_pairs, n_recheck, n_disagree);
-                }
             }
-            if (PLAIN) {
-                // on every lane alike: its rays go into agent k + 1's sums
-                // from registers (a pair beyond the cut-off decides to none)
-                PairF32 pr;
-                more = Pieces{0, 0, 0, 0};
-                if (decide_pair(pr, u1, f1, moved, rp, C, false, false, n_pairs, n_recheck, n_disagree)) {
-                    Pieces q;
-                    vf_pieces(pr.start, pr.end, C.R, &q.a0, &q.b0, &q.a1, &q.b1);
-                    more.a0 = __builtin_amdgcn_readfirstlane(q.a0); more.b0 = __builtin_amdgcn_readfirstlane(q.b0);
-                    more.a1 = __builtin_amdgcn_readfirstlane(q.a1); more.b1 = __builtin_amdgcn_readfirstlane(q.b1);
-                }
-            }
-        } else {
-            // ---- agent k - 1's new pose into the fields of agents k + 1 ..:
-            // each wave tests its focal agents against the cut-off 64 at a
-            // time and queues the rest in a ring of 128 in LDS, deciding 64
-            // at a time
-            if (k >= 1) {
-                const float4 o = P1[k - 1];
-                int head = 0, tail = 0;   // wave-uniform ring positions
-                for (int mb = k + 1 + (wave - 1) * 64; mb < C.N; mb += kPushThreads - 64) {
-                    const int m = mb + lane;
-                    bool keep = false;
-                    if (m < C.N) {
-                        const float4 f = P0[m];
-                        if (!(o.x == f.x && o.y == f.y)) {   // coincident pairs are skipped (vf_supcalc.py:57)
-                            keep = !push_culled(f, o, C, cull_c);
-                            if (!keep) push_culled_check(f, o, rp, count, verify, n_pairs, n_disagree);
-                        }
-                    }
-                    const uint64_t mk = __ballot(keep);
-                    if (keep) wq[(tail + (int)__popcll(mk & ((1ull << lane) - 1ull))) & (kPushQueue - 1)] = (uint32_t)m;
-                    tail += (int)__popcll(mk);
-                    wave_lds_sync();
-                    if (tail - head >= 64) {
-                        const int mm = (int)wq[(head + lane) & (kPushQueue - 1)];
-                        push_pair(F + (size_t)mm * W1, U[mm], P0[mm], o, rp, C, count, verify, n_pairs,
-                                  n_recheck, n_disagree);
-                        head += 64;
-                        wave_lds_sync();
-                    }
-                }
-                if (lane < tail - head) {
-                    const int mm = (int)wq[(head + lane) & (kPushQueue - 1)];
-                    push_pair(F + (size_t)mm * W1, U[mm], P0[mm], o, rp, C, count, verify, n_pairs, n_recheck,
-                              n_disagree);
+        } else if (wave == 1) {
+            // ---- agent k + 1's sums: its row lacks only the pair (k + 1, k),
+            // whose rays are the predicted ones
+            if (k + 1 < C.N) sums_into(k + 1, predicted(k + 1), red[(k + 1) & 1]);
+        } else if (k >= 1) {
+            // ---- agent k - 1's new pose into the fields of agents k + 2 ..
+            const float4 ob = P1[k - 1];
+            for (int m = k + 2 + (wave - 2) * 64 + lane; m < C.N; m += (kPushWaves - 2) * 64) {
+                const float4 f = P0[m];
+                if (push_culled(f, ob, C, cull_c)) {
+                    push_culled_check(f, ob, rp, count, verify, n_pairs, n_disagree);
+                } else {
+                    push_pair(F + (size_t)m * W1, U[m], f, ob, rp, C, count, verify, n_pairs, n_recheck, n_disagree);
                 }
             }
         }
