@@ -319,6 +319,19 @@ __device__ inline FastRec fast_rec_const(int R, double step, double fov0, double
     return q;
 }
 
+// The exact record (rare): visible, start, end.  Out of line, or its constants
+// (acos, atan) would be held in registers over every caller's loop.
+__device__ __attribute__((noinline)) int4 record_exact(double ox, double oy, double px, double py, double radius,
+                                                       double u1x, double u1y, int R, double step, double fov0,
+                                                       double fov1) {
+    Focal f;
+    f.px = px; f.py = py; f.radius = radius;
+    f.cx = px + radius; f.cy = py + radius;
+    f.u1x = u1x; f.u1y = u1y;
+    const PairFG p = pair_forage_exact(f, ox, oy, R, step, fov0, fov1);
+    return make_int4(!p.skipped && p.visible, p.start, p.end, 0);
+}
+
 // Record of obstacle j (class c) for focal geometry f.  The bin, the
 // interval and the FOV test come from a float32 decision when it is outside
 // every guard band, else from the exact float64 record (agent.py:501-556):
@@ -374,15 +387,14 @@ __device__ inline Rec record_at(double ox, double oy, int c, int order, const Fo
             return rc;
         }
     }
-    const PairFG p = pair_forage_exact(f, ox, oy, R, step, fov0, fov1);
-    if (!p.skipped && p.visible) {
+    const int4 p = record_exact(ox, oy, f.px, f.py, f.radius, f.u1x, f.u1y, R, step, fov0, fov1);
+    if (p.x) {
         rc.valid = 1;
         rc.social = c == kSocial;
         rc.order = order;
-        rc.start = rc.sx = p.start;
-        rc.end = rc.ex = p.end;
-        rc.dist = p.dist;
-        rc.vis = p.vis;
+        rc.start = rc.sx = p.y;
+        rc.end = rc.ex = p.z;
+        if (need_dist) rc.dist = norm2(v2x, v2y);
     }
     return rc;
 }
@@ -419,11 +431,16 @@ __device__ void classify(const FGSmem& S, const FGRep& P, int N, int f, int skip
     }
 }
 
-// make_focal with one sincos for the heading (the same values as cos, sin).
-__device__ inline Focal focal_at(double px, double py, double th, double radius) {
-#pragma clang fp contract(off)
+// sin and cos (out of line for the same reason).
+__device__ __attribute__((noinline)) double2 sin_cos(double th) {
     double sn, cs;
     sincos(th, &sn, &cs);
+    return make_double2(sn, cs);
+}
+
+// make_focal with one sincos for the heading (the same values as cos, sin).
+__device__ inline Focal focal_at(double px, double py, double sn, double cs, double radius) {
+#pragma clang fp contract(off)
     Focal f;
     f.px = px; f.py = py; f.radius = radius;
     f.cx = px + radius;
@@ -435,6 +452,11 @@ __device__ inline Focal focal_at(double px, double py, double th, double radius)
     f.u1x = v1x / n1;
     f.u1y = v1y / n1;
     return f;
+}
+__device__ inline Focal focal_at(double px, double py, double th, double radius) {
+    double sn, cs;
+    sincos(th, &sn, &cs);
+    return focal_at(px, py, sn, cs, radius);
 }
 __device__ inline Focal focal_of(const FGSmem& S, int k) { return focal_at(S.x[k], S.y[k], S.th[k], S.rad[k]); }
 
@@ -690,7 +712,8 @@ __device__ inline double words_to_double(uint32_t w0, uint32_t w1) {
 // kWorldReady are updated, and they are marked ABM_WORLD_DONE.  FIELDS false:
 // a step that writes no fields (bits_out is ignored).  The replicas of this
 // kernel have visual exclusion: every agent in range, as it stands in its
-// turn, occludes, so the agents are updated one after another.
+// turn, occludes, so the agents are updated one after another.  It takes those
+// with more agents than forage_occlude_kernel holds in registers.
 template <bool FIELDS>
 __global__ void __launch_bounds__(512)
 forage_step_kernel(const FGRep* __restrict__ reps, abm_forage_state st,
@@ -789,7 +812,7 @@ forage_step_kernel(const FGRep* __restrict__ reps, abm_forage_state st,
     // agent k+2.
     // Classes, lists, focal geometry and counts alternate between two
     // buffers by parity of the focal agent.
-    const int rbase = 64, cbase = 128, cstride = nthr - 128;   // blockDim 256 or 512
+    const int rbase = 64, cbase = 128, cstride = nthr - 128;   // blockDim 512
     if (tid == 0) {
         for (int q = 0; q < 8; ++q) S.cnt[q] = 0;
     }
@@ -799,8 +822,8 @@ forage_step_kernel(const FGRep* __restrict__ reps, abm_forage_state st,
     // speculative headings (slot 0, draw index 0)
     // two waves that classify once per focal agent also build the
     // speculative headings and the focal geometry: waves 4 and 5 of eight
-    // (waves 2 and 3 classify twice for 512 agents), waves 2 and 3 of four
-    const int spec_tid = nthr == 512 ? 256 : 128, focal_tid = spec_tid + 64;
+    // (waves 2 and 3 classify twice for 512 agents)
+    const int spec_tid = 256, focal_tid = spec_tid + 64;
     if (tid >= spec_tid && tid < spec_tid + 3) spec_heading(S, P, N, 0, 0, tid - spec_tid, S.spec);
     if (tid == 0) S.spec[24] = 0.0;    // uniforms drawn before agent 0
     if (tid == 0) S.focal[0] = focal_of(S, 0);
@@ -1350,6 +1373,627 @@ forage_update_kernel(const FGRep* __restrict__ reps, abm_forage_state st,
     }
     if (tid == 0 && u_used) u_used[rb] = used0 + (words || mt ? 2 : 1) * draws;
     if (tid == 0 && status) status[rb] = ABM_WORLD_DONE;
+}
+
+// ------------------------------------------------ update with visual exclusion
+// Agent.update in id order (sims.py:861) with visual exclusion: every agent in
+// range, as it stands in agent k's turn, may occlude the others, so agent k + 1's
+// field waits for agent k's move.  But only for the one record of agent k: the
+// rest of the field is known a turn earlier.  Wave 0 carries the chain alone
+// (decide and move agent k, its record in agent k + 1's view, what it occludes,
+// the counts of agent k + 1's field) and the other H = 7 waves prepare the fields,
+// each that of every 7th agent over the 7 turns before its own:
+//   turn 0      the focal geometry and the records of the agents that will
+//               not move before the focal agent does (a lane each)
+//   turns 1, 2  how many of them are nearer than each
+//   turns 3, 4  which nearer ones overlap each; the headings after a walk turn
+//   turn 5      the records of the agents moved meanwhile, one by one
+//   turn 6      the last but one's, the visible intervals, the field: to wave 0
+// One barrier a turn.  A record's visible interval is cut by the nearer records
+// in the order of their distance (agent.py:421-445); one that does not overlap it
+// cuts nothing, so the walk goes over the others alone (few: the agents along
+// one line of sight), and agent k's record changes only the intervals it overlaps.
+// Bound by the chain's latency (about 4.0 thousand cycles a turn of 5.7 with 40
+// agents: 1.9 decision and move, 1.0 record, 0.5 cuts, 0.5 counts), beyond 64
+// agents by the preparing waves (12 thousand a turn with 80).  Against one
+// kernel that ranked and cut all records between two agents' moves (still the one
+// beyond 256 agents, where K would not fit in registers), ms a step: 200 replicas
+// of 10 to 40 agents at R = 600 0.72 -> 0.134, 1000 of 10 to 64 1.68 -> 0.226,
+// 700 of 80 5.23 -> 0.87, 20 of 250 24.3 -> 4.0, one of 10 0.085 -> 0.040.
+// K <= 2 is held to 128 registers, so that two workgroups share a CU (700 of 80:
+// 1.15 with one; 50 of 80 then take 0.495 instead of 0.472).
+constexpr int kOcclMaxAgents = 256;   // K = 1, 2 or 4 records per lane
+
+// A focal agent's records, K per lane (record j in lane j & 63, slot j >> 6):
+// bins, distance, place in the reference's obstacle list, rank by distance
+// (equal ones by place) and the nearer records that overlap it, a bit each.
+// A record that a nearer one covers from end to end is hidden, whatever else
+// cuts it (its interval only shrinks): its set is not needed.
+template <int K>
+struct Seen {
+    int start[K], end[K], ord[K];   // ord: place, negative: no record
+    int rank[K];                    // place by (distance, ord)
+    int below[K];                   // nearer records
+    int hid[K];                     // negative: hidden
+    double dist[K];                 // no record: NaN, neither nearer nor as near as any
+    uint32_t over[K][2 * K];        // [slot of the record][32 of the nearer ones]
+};
+struct OcclRec {                    // a record as the other records meet it
+    double dist;
+    int ord, start, end;
+};
+
+// LDS of the kernel: the agents, and by parity of the focal agent the records
+// handed to wave 0.
+struct OcclSmem {
+    double *x, *y, *rad, *th, *v, *w, *u0, *u1, *ip, *uni;
+    double* spec;      // [kOcclSpec q ..]: prepared headings, by agent mod 4; [4 kOcclSpec + p]: uniforms drawn before
+    double* dist;      // the handed records, by rank: [64 K p ..]
+    uint64_t* over;    // [64 K K p + 64 K c ..]: nearer records of rank 64 c .. that overlap
+    int2 *span, *cut;  // [64 K p ..]: bins, and after exclusion
+    int* ord;          // [64 K p ..]: place, + kOrdHidden
+    int4* rec;         // [64 K h ..]: preparing wave h's records of its focal's first turn: below, start, end, ord
+    double* rdist;     // [64 K h ..]: their distances
+    int* rank;         // [64 K h ..]: their ranks when handed over
+    Focal* focal;      // [wave]
+    int *pid, *mode_over, *mode, *env, *kept;
+    uint32_t* key;
+    uint32_t* field;   // [4][W]: raw fields by focal agent mod 4
+};
+constexpr int kOcclDoubles = 10, kOcclInts = 4;
+constexpr int kOrdHidden = 1 << 30;
+constexpr int kOcclSpec = 16;   // four turns' headings and none's (each with sin, cos), the first's draw
+constexpr int kOcclWaves = 8, kOcclPrep = kOcclWaves - 1;
+
+__device__ inline OcclSmem occl_carve(void* base, int maxN, int K) {
+    OcclSmem s;
+    const int L = 128 * K;
+    char* p = reinterpret_cast<char*>(base);
+    s.focal = reinterpret_cast<Focal*>(p); p += 64 * kOcclWaves;
+    s.rec = reinterpret_cast<int4*>(p); p += sizeof(int4) * 64 * K * kOcclPrep;
+    s.rdist = reinterpret_cast<double*>(p); p += sizeof(double) * 64 * K * kOcclPrep;
+    double** d[] = {&s.x, &s.y, &s.rad, &s.th, &s.v, &s.w, &s.u0, &s.u1, &s.ip, &s.uni};
+    for (double** a : d) { *a = reinterpret_cast<double*>(p); p += sizeof(double) * maxN; }
+    s.spec = reinterpret_cast<double*>(p); p += sizeof(double) * (4 * kOcclSpec + 2);
+    s.dist = reinterpret_cast<double*>(p); p += sizeof(double) * L;
+    s.over = reinterpret_cast<uint64_t*>(p); p += sizeof(uint64_t) * L * K;
+    s.span = reinterpret_cast<int2*>(p); p += sizeof(int2) * L;
+    s.cut = reinterpret_cast<int2*>(p); p += sizeof(int2) * L;
+    s.ord = reinterpret_cast<int*>(p); p += sizeof(int) * L;
+    s.rank = reinterpret_cast<int*>(p); p += sizeof(int) * 64 * K * kOcclPrep;
+    int** i[] = {&s.pid, &s.mode_over, &s.mode, &s.env};
+    for (int** a : i) { *a = reinterpret_cast<int*>(p); p += sizeof(int) * maxN; }
+    s.kept = reinterpret_cast<int*>(p); p += sizeof(int) * 2;
+    s.key = reinterpret_cast<uint32_t*>(p); p += sizeof(uint32_t) * kMtN;
+    s.field = reinterpret_cast<uint32_t*>(p);
+    return s;
+}
+
+size_t occl_lds_bytes(int maxN, int maxR, int K) {
+    return 64 * (size_t)kOcclWaves + (size_t)maxN * (8 * kOcclDoubles + 4 * kOcclInts) + 8 * (4 * kOcclSpec + 2) +
+           (size_t)128 * K * (8 + 8 * K + 8 + 8 + 4) + (size_t)64 * K * kOcclPrep * (16 + 8 + 4) +
+           4 * (kMtN + 2) + 4 * sizeof(uint32_t) * (size_t)((maxR + 31) / 32);
+}
+
+__device__ inline int occl_class(const OcclSmem& S, int patchwise, const RangeTest& rt, int j, double cfx, double cfy,
+                                 int pid_f) {
+    if (!in_range(rt, (S.x[j] + S.rad[j]) - cfx, (S.y[j] + S.rad[j]) - cfy)) return kNone;
+    if (S.mode_over[j] != ABM_MODE_EXPLOIT) return kNonExpl;   // get_mode() == "exploit" only via the override
+    if (patchwise && S.pid[j] == pid_f) return kSamePatch;
+    return S.pid[j] != -1 ? kSocial : kNone;
+}
+
+// A record's visible interval after nearer ones (agent.py:421-445): those of
+// rank 64 c + (bit of m), nearest first.
+struct Interval {
+    int s, e;
+};
+__device__ inline bool cut_by(Interval& v, int2 i) {   // false: nothing is left to cut
+    if (v.s <= i.x && i.x <= v.e) v.e = i.x;
+    if (v.s <= i.y && i.y <= v.e) v.s = i.y;
+    const bool covered = i.x <= v.s && i.y >= v.e;
+    if (covered) v.s = v.e = 0;   // (no record moves an interval from there)
+    return !covered;
+}
+__device__ inline bool cut_by_all(Interval& v, uint64_t m, const int2* span) {
+    if (!m) return true;
+    int2 i = span[__builtin_ctzll(m)];
+    for (m &= m - 1; m; m &= m - 1) {
+        const int2 next = span[__builtin_ctzll(m)];
+        if (!cut_by(v, i)) return false;
+        i = next;
+    }
+    return cut_by(v, i);
+}
+
+__device__ inline void paint_cut(uint32_t* V, Interval cut, int R) {
+    Rec rc;
+    rc.sx = cut.s; rc.ex = cut.e;
+    paint_bits(V, rc, R);
+}
+
+template <int K, bool FIELDS>
+__global__ void __launch_bounds__(64 * kOcclWaves) __attribute__((amdgpu_waves_per_eu(K < 4 ? 4 : 2)))
+forage_occlude_kernel(const FGRep* __restrict__ reps, abm_forage_state st,
+                      const double* __restrict__ uniforms, const uint32_t* __restrict__ words,
+                      const int64_t* __restrict__ u_off, const int32_t* __restrict__ u_cnt,
+                      int32_t* __restrict__ u_used, int32_t* __restrict__ status,
+                      uint32_t* __restrict__ bits_out, const int32_t* __restrict__ order,
+                      abm_mt19937_state* __restrict__ mt, int maxN) {
+#pragma clang fp contract(off)
+    extern __shared__ __align__(16) double smem[];
+    const int rb = order[blockIdx.x];
+    if (status && status[rb] != kWorldReady) return;   // uniform over the block
+    const int tid = threadIdx.x, nthr = blockDim.x;
+    const int lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    constexpr int H = kOcclPrep;
+    __shared__ FGRep sP;
+    if (tid < (int)(sizeof(FGRep) / 8))
+        reinterpret_cast<uint64_t*>(&sP)[tid] = reinterpret_cast<const uint64_t*>(reps + rb)[tid];
+    __syncthreads();
+    const FGRep& P = sP;
+    const int N = P.n_agents, R = P.n_rays, W = P.words, a0 = P.agent_offset, tau = P.tau;
+    const OcclSmem S = occl_carve(smem, maxN, K);
+    for (int i = tid; i < N; i += nthr) {
+        const int g = a0 + i;
+        const double w = st.w[g], u = st.u[g], cr = st.collected_r[g], crb = st.collected_r_before[g];
+        const int over = st.overriding_mode[g], env = st.env_status[g];
+        double m = st.novelty[(int64_t)g * tau];
+        for (int q = 1; q < tau; ++q) m = fmax(m, st.novelty[(int64_t)g * tau + q]);
+        const Drive d = drive_of(P, w, u, m, cr, crb, over, env);
+        S.x[i] = st.x[g]; S.y[i] = st.y[g]; S.th[i] = st.theta[g]; S.v[i] = st.v[g];
+        S.w[i] = w; S.u0[i] = u; S.u1[i] = d.u; S.ip[i] = d.ipriv; S.rad[i] = (double)st.radius[g];
+        S.pid[i] = st.exploited_patch_id[g]; S.mode_over[i] = over; S.mode[i] = st.mode[g]; S.env[i] = env;
+        st.collected_r_before[g] = cr;
+    }
+    // the step's uniforms: agent i's draw is the i-th at the latest (at most
+    // one per agent); doubles, or pairs of words after those the resource
+    // loop used (u_used[b] on entry); NaN past the end of the buffer
+    const int ucount = mt ? 0 : u_cnt[rb];
+    const int used0 = (words || mt) ? u_used[rb] : 0;
+    int mt_pos0 = 0;
+    if (mt) {
+        for (int i = tid; i < kMtN; i += nthr) S.key[i] = mt[rb].key[i];
+        mt_pos0 = mt[rb].pos;
+        __syncthreads();
+        uint32_t* wb = reinterpret_cast<uint32_t*>(S.uni);
+        int made = 0, p = mt_pos0;
+        while (made < 2 * N) {
+            if (p >= kMtN) {
+                mt_twist_block(S.key);
+                p = 0;
+            }
+            const int take = min(kMtN - p, 2 * N - made);
+            for (int j = tid; j < take; j += nthr) wb[made + j] = mt_temper(S.key[p + j]);
+            made += take;
+            p += take;
+        }
+        __syncthreads();
+        for (int i = tid; i < N; i += nthr) {   // each thread rewrites its own 8 bytes
+            const uint32_t w0 = wb[2 * i], w1 = wb[2 * i + 1];
+            S.uni[i] = words_to_double(w0, w1);
+        }
+    } else {
+        for (int i = tid; i < N; i += nthr) {
+            double uu = NAN;
+            if (words) {
+                const uint32_t* wb = words + u_off[rb];
+                const int at = used0 + 2 * i;
+                if (at + 2 <= ucount) uu = words_to_double(wb[at], wb[at + 1]);
+            } else if (i < ucount) {
+                uu = uniforms[u_off[rb] + i];
+            }
+            S.uni[i] = uu;
+        }
+    }
+    if (tid < 2) S.spec[4 * kOcclSpec + tid] = 0.0;
+    const FastRec FR = fast_rec_const(R, P.step, P.fov0, P.fov1);
+    const RangeTest rt = range_test(P.vision_range);
+    const double step = P.step, fov0 = P.fov0, fov1 = P.fov1;
+    const int patchwise = P.patchwise;
+    constexpr int L = 64 * K;
+    __syncthreads();
+
+    const int h = wave - 1;   // the preparing wave's number (wave 0: none)
+    Seen<K> seen;
+    // ---- the pieces of a focal agent's preparation (a whole wave each)
+    auto record = [&](int j, int f, const Focal& fo) {
+        Rec rc;
+        rc.valid = 0;
+        const int c = occl_class(S, patchwise, rt, j, fo.cx, fo.cy, S.pid[f]);
+        if (c != kNone) rc = record_at(S.x[j], S.y[j], c, c * N + j, fo, R, step, fov0, fov1, FR, true);
+        return rc;
+    };
+    auto begin = [&](int f, int lo) {   // every record but those of agents lo .. f
+        const double2 sc = sin_cos(S.th[f]);
+        const Focal fo = focal_at(S.x[f], S.y[f], sc.x, sc.y, S.rad[f]);
+        if (lane == 0) S.focal[wave] = fo;
+#pragma unroll
+        for (int c = 0; c < K; ++c) {
+            const int j = 64 * c + lane;
+            seen.ord[c] = -1; seen.start[c] = seen.end[c] = seen.rank[c] = seen.below[c] = seen.hid[c] = 0;
+            seen.dist[c] = NAN;
+#pragma unroll
+            for (int b = 0; b < 2 * K; ++b) seen.over[c][b] = 0;
+            if (j < N && (j < lo || j > f)) {
+                const Rec rc = record(j, f, fo);
+                if (rc.valid) { seen.start[c] = rc.start; seen.end[c] = rc.end; seen.ord[c] = rc.order; seen.dist[c] = rc.dist; }
+            }
+            S.rdist[L * h + j] = seen.dist[c];
+        }
+        fg_wave_sync();
+    };
+    // whether a record (distance d, bins [s, e]) is nearer than this lane's
+    // record in slot c and overlaps it
+    auto cuts = [&](const OcclRec& r, int c) {
+        return (r.dist < seen.dist[c]) & (r.start <= seen.end[c]) & (r.end >= seen.start[c]);
+    };
+    auto hides = [&](const OcclRec& r, int c) {
+        return (r.dist < seen.dist[c]) & (r.start <= seen.start[c]) & (r.end >= seen.end[c]);
+    };
+    auto before = [&](const OcclRec& r, int c) {
+        return (r.dist < seen.dist[c]) | ((r.dist == seen.dist[c]) & (r.ord < seen.ord[c]));
+    };
+    // the first turn's records against each other, in two passes over j0 ..
+    // j1 - 1: how many are nearer than each, then which of them overlap or hide it.
+    // (Vector operations only: sign bits, and carries into the counts.)
+    int same[K];
+    auto count_nearer = [&](int j0, int j1) {
+        const double* q = S.rdist + L * h;
+        for (int j = j0; j < j1; j += 4) {
+            double d[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) d[i] = j + i < j1 ? q[min(j + i, L - 1)] : NAN;
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int c = 0; c < K; ++c) {
+                    seen.below[c] += d[i] < seen.dist[c] ? 1 : 0;
+                    same[c] += d[i] == seen.dist[c] ? 1 : 0;
+                }
+        }
+    };
+    auto end_count = [&]() {   // places, ties in the obstacle list's order (rare); the records for the second pass
+        bool tie = false;
+#pragma unroll
+        for (int c = 0; c < K; ++c) {
+            seen.rank[c] = seen.below[c];
+            tie |= same[c] > 1;
+            S.rec[L * h + 64 * c + lane] = make_int4(seen.ord[c] < 0 ? 1 << 30 : seen.below[c], seen.start[c],
+                                                     seen.end[c], seen.ord[c]);
+        }
+        fg_wave_sync();
+        if (__ballot(tie) != 0)
+            for (int j = 0; j < N; ++j) {
+                const double d = S.rdist[L * h + j];
+                const int o = S.rec[L * h + j].w;
+#pragma unroll
+                for (int c = 0; c < K; ++c) seen.rank[c] += (d == seen.dist[c]) & (o < seen.ord[c]) ? 1 : 0;
+            }
+    };
+    auto overlaps = [&](int j0, int j1) {
+        const int4* q = S.rec + L * h;
+#pragma unroll
+        for (int b = 0; b < 2 * K; ++b) {
+            const int e = min(j1, 32 * b + 32);
+            for (int j = max(j0, 32 * b); j < e; j += 4) {   // (records past e are met again: the same bits)
+                int4 r[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) r[i] = q[min(j + i, 32 * b + 31)];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const uint32_t bit = 1u << (min(j + i, 32 * b + 31) & 31);
+#pragma unroll
+                    for (int c = 0; c < K; ++c) {
+                        const int nearer = r[i].x - seen.below[c];
+                        seen.over[c][b] |= (uint32_t)((nearer & (r[i].y - seen.end[c] - 1) & (seen.start[c] - r[i].z - 1)) >> 31) & bit;
+                        seen.hid[c] |= nearer & (r[i].y - seen.start[c] - 1) & (seen.end[c] - r[i].z - 1);
+                    }
+                }
+            }
+        }
+    };
+    // a record more, of agent j: the ranks and sets it enters, and its own
+    auto enter = [&](int j, const OcclRec& r) {
+        const int cj = j >> 6, lj = j & 63;
+        const uint32_t bit = 1u << (j & 31);
+        int rank = 0, below = 0;
+        uint64_t on[K], hidden = 0;
+#pragma unroll
+        for (int c = 0; c < K; ++c) {
+            const bool after = before(r, c), nearer = seen.dist[c] < r.dist;
+            rank += (int)__popcll(__ballot((seen.ord[c] >= 0) & !after));
+            below += (int)__popcll(__ballot(nearer));
+            seen.rank[c] += after ? 1 : 0;
+            seen.below[c] += r.dist < seen.dist[c] ? 1 : 0;
+            const bool by = cuts(r, c);
+            seen.hid[c] |= hides(r, c) ? -1 : 0;
+#pragma unroll
+            for (int b = 0; b < 2 * K; ++b)
+                if (b == j >> 5) seen.over[c][b] |= by ? bit : 0u;
+            on[c] = __ballot(nearer & (seen.start[c] <= r.end) & (seen.end[c] >= r.start));
+            hidden |= __ballot(nearer & (seen.start[c] <= r.start) & (seen.end[c] >= r.end));
+        }
+#pragma unroll
+        for (int c = 0; c < K; ++c)
+            if (c == cj && lane == lj) {
+                seen.start[c] = r.start; seen.end[c] = r.end; seen.ord[c] = r.ord; seen.dist[c] = r.dist;
+                seen.rank[c] = rank; seen.below[c] = below; seen.hid[c] = hidden != 0 ? -1 : 0;
+#pragma unroll
+                for (int b = 0; b < K; ++b) {
+                    seen.over[c][2 * b] = (uint32_t)on[b];
+                    seen.over[c][2 * b + 1] = (uint32_t)(on[b] >> 32);
+                }
+            }
+    };
+    auto insert = [&](int f, int j0, int j1) {   // the records of agents j0 .. j1 - 1 (at most 64), which have moved
+        Rec rc;
+        rc.valid = 0;
+        const Focal fo = S.focal[wave];
+        if (j0 + lane < j1) rc = record(j0 + lane, f, fo);
+        const long long db = __double_as_longlong(rc.valid ? rc.dist : 0.0);
+        for (uint64_t t = __ballot(rc.valid != 0); t; t &= t - 1) {
+            const int l = __builtin_ctzll(t);
+            OcclRec r;
+            const uint32_t dl = (uint32_t)__builtin_amdgcn_readlane((int)db, l);
+            const uint32_t dh = (uint32_t)__builtin_amdgcn_readlane((int)(db >> 32), l);
+            r.dist = __longlong_as_double((long long)((uint64_t)dh << 32 | dl));
+            r.ord = __builtin_amdgcn_readlane(rc.order, l);
+            r.start = __builtin_amdgcn_readlane(rc.start, l);
+            r.end = __builtin_amdgcn_readlane(rc.end, l);
+            enter(j0 + l, r);
+        }
+    };
+    // the headings after a walk turn by uniform d .. d + 3, or none
+    // (agent.py:187-200, 595-603), d uniforms drawn before agent f - 3
+    auto headings = [&](int f, int d) {
+        if (lane < 5) {
+            double dth = 0.0;
+            if (lane < 4) dth = P.exp_theta_min + (P.exp_theta_max - P.exp_theta_min) * (d + lane < N ? S.uni[d + lane] : 0.0);
+            const double th = prove_orientation(S.th[f] + dth);
+            const double2 sc = sin_cos(th);
+            double* q = S.spec + kOcclSpec * (f & 3) + 3 * lane;
+            q[0] = th; q[1] = sc.x; q[2] = sc.y;
+            if (lane == 0) S.spec[kOcclSpec * (f & 3) + 15] = (double)d;
+        }
+    };
+    auto publish = [&](int f) {   // to wave 0, by rank, with the field of these records
+        const int p = f & 1;
+        double* dist = S.dist + L * p;
+        int2 *span = S.span + L * p, *cut = S.cut + L * p;
+        int* ord = S.ord + L * p;
+        int* rank = S.rank + L * h;
+        uint32_t* V = S.field + (f & 3) * W;
+        for (int w = lane; w < W; w += 64) V[w] = 0u;
+        int n = 0;
+#pragma unroll
+        for (int c = 0; c < K; ++c) n += (int)__popcll(__ballot(seen.ord[c] >= 0));
+#pragma unroll
+        for (int c = 0; c < K; ++c) {
+            const int j = 64 * c + lane;
+            if (j >= n) { dist[j] = NAN; ord[j] = -1; }
+            if (seen.ord[c] >= 0) {
+                const int r = seen.rank[c];
+                rank[j] = r;
+                dist[r] = seen.dist[c];
+                span[r] = make_int2(seen.start[c], seen.end[c]);
+                ord[r] = seen.ord[c] | (seen.hid[c] < 0 ? kOrdHidden : 0);
+            }
+        }
+        fg_wave_sync();
+#pragma unroll
+        for (int c = 0; c < K; ++c) {
+            // the cues lead the obstacle list; only they are painted
+            if ((unsigned)seen.ord[c] >= (unsigned)N || seen.hid[c] < 0) continue;
+            uint64_t m[K];
+#pragma unroll
+            for (int b = 0; b < K; ++b) m[b] = 0;
+#pragma unroll
+            for (int b = 0; b < 2 * K; ++b)
+                for (uint32_t t = seen.over[c][b]; t; t &= t - 1) {
+                    const int r = rank[32 * b + __builtin_ctz(t)];
+#pragma unroll
+                    for (int a = 0; a < K; ++a) m[a] |= r >> 6 == a ? 1ull << (r & 63) : 0ull;
+                }
+            Interval v{seen.start[c], seen.end[c]};
+            bool on = true;
+#pragma unroll
+            for (int b = 0; b < K; ++b)
+                if (on) on = cut_by_all(v, m[b], span + 64 * b);
+            paint_cut(V, v, R);
+            const int r = seen.rank[c];
+            cut[r] = make_int2(v.s, v.e);
+#pragma unroll
+            for (int b = 0; b < K; ++b) S.over[(size_t)L * (K * p + b) + r] = m[b];
+        }
+    };
+    auto output = [&](int f) {   // soc_v_field[q] = V[R - 1 - q] on the kept rays (agent.py:593-595)
+        const uint32_t* V = S.field + (f & 3) * W;
+        const int lo = P.keep_lo, hi = P.keep_hi;
+        uint32_t* dst = bits_out + P.field_offset + (int64_t)f * W;
+        for (int w = lane; w < W; w += 64) dst[w] = __brev(raw_window(V, W, R - 32 - 32 * w)) & word_range_mask(w, lo, hi);
+    };
+
+    // ---- before the first turn: agents 0 .. H - 1 begun, agent 0's field
+    if (wave > 0 && h < N) {
+        begin(h, 0);
+#pragma unroll
+        for (int c = 0; c < K; ++c) same[c] = 0;
+        count_nearer(0, N);
+        end_count();
+        overlaps(0, N);
+        if (h == 0) publish(0);
+        if (h < 3) headings(h, 0);
+    }
+    __syncthreads();
+    int draws = 0, n_set = 0, n_left = 0;   // wave 0
+    if (wave == 0) {
+        wave_counts(S.field, R, W, P.keep_lo, P.keep_hi, nullptr, &n_set, &n_left);
+        __builtin_amdgcn_s_setprio(3);   // the chain issues first
+    }
+    for (int k = 0; k < N; ++k) {
+        const int f1 = k + 1;
+        Rec rc;
+        rc.valid = 0;
+        if (wave == 0) {
+            // ---- agent k's decision and move (agent.py:168-283), on every lane
+            const int fn = min(f1, N - 1), pid_k = S.pid[k], pid_f = S.pid[fn];
+            const Focal fo = S.focal[1 + fn % H];
+            const double w0 = S.w[k], u0 = S.u0[k], u1 = S.u1[k], vel0 = S.v[k];
+            const double x0 = S.x[k], y0 = S.y[k], th0 = S.th[k], rad = S.rad[k];
+            const int env = S.env[k];
+            const double* spec = S.spec + kOcclSpec * (k & 3);
+            const int spec_d = (int)spec[15];
+            const Choice c = choose(P, R, n_set, n_left, w0, u0, u1, vel0, S.mode_over[k], S.mode[k], env);
+            Pose p{x0, y0, th0, vel0};
+            double sn, cs;
+            if (c.mode == ABM_MODE_RELOCATE && c.over == -1) {
+                p.theta = prove_orientation(p.theta + c.dth);
+                const double2 sc = sin_cos(p.theta);
+                sn = sc.x; cs = sc.y;
+            } else {   // prepared: prove_orientation(theta + turn) and its sin, cos
+                const double* q = spec + 3 * (c.kind == 0 ? draws - spec_d : 4);
+                p.theta = q[0]; sn = q[1]; cs = q[2];
+                draws += c.kind == 0 ? 1 : 0;
+            }
+            p.v = p.v + c.dvel;
+            // prove_velocity (agent.py:612-620): only in explore mode
+            if (get_mode(c.over, c.w, P.T_w) == ABM_MODE_EXPLORE && fabs(p.v) > 1.0) p.v = P.exp_vel_max;
+            p.x = p.x + p.v * cs;
+            p.y = p.y - p.v * sn;
+            p = reflect_walls(p, rad, P.pad, P.width, P.height);
+            if (lane == 0) {
+                S.x[k] = p.x; S.y[k] = p.y; S.th[k] = p.theta; S.v[k] = p.v;
+                S.w[k] = c.w; S.mode_over[k] = c.over; S.mode[k] = c.mode;
+                S.spec[4 * kOcclSpec + (f1 & 1)] = (double)draws;
+            }
+            // ---- its record in agent k + 1's view
+            if (f1 < N && in_range(rt, (p.x + rad) - fo.cx, (p.y + rad) - fo.cy)) {
+                const int cls = c.over != ABM_MODE_EXPLOIT ? kNonExpl
+                                : patchwise && pid_k == pid_f ? kSamePatch : pid_k != -1 ? kSocial : kNone;
+                if (cls != kNone) rc = record_at(p.x, p.y, cls, cls * N + k, fo, R, step, fov0, fov1, FR, true);
+            }
+        } else {
+            const int f = f1 + (((h - f1) % H) + H) % H, s = k + H - f;   // turns since f's first
+            if (FIELDS && k >= 1 && (k - 1) % H == h) output(k - 1);
+            if (f < N) {
+                if (s == 0) {
+                    begin(f, k);
+#pragma unroll
+                    for (int c = 0; c < K; ++c) same[c] = 0;
+                } else if (s <= 2) {
+                    if (f >= H) count_nearer(N * (s - 1) / 2, N * s / 2);
+                    if (f >= H && s == 2) end_count();
+                } else if (s <= H - 3) {
+                    if (f >= H) overlaps(N * (s - 3) / (H - 5), N * (s - 2) / (H - 5));
+                    if (s == H - 3) headings(f, (int)S.spec[4 * kOcclSpec + (k & 1)]);
+                } else if (s == H - 2) {
+                    insert(f, max(f - H, 0), k);
+                } else if (k >= 1) {
+                    insert(f, k - 1, k);
+                }
+                if (s == H - 1) publish(f);
+            }
+        }
+        __syncthreads();
+        if (f1 >= N) break;
+        if (wave == 0) {
+            // ---- agent k + 1's field: the prepared one, with agent k's record
+            const int p = f1 & 1;
+            double* dist = S.dist + L * p;
+            int2 *span = S.span + L * p, *cut = S.cut + L * p;
+            int* ord = S.ord + L * p;
+            uint32_t* V = S.field + (f1 & 3) * W;
+            if (rc.valid) {
+                const OcclRec r{rc.dist, rc.order, rc.start, rc.end};
+                bool walk[K], any = false;
+                uint64_t on[K], hidden = 0;
+                int at = 0;   // its rank
+#pragma unroll
+                for (int c = 0; c < K; ++c) {
+                    const int q = 64 * c + lane;
+                    seen.dist[c] = dist[q];
+                    const int o = ord[q];
+                    seen.ord[c] = o < 0 ? o : o & ~kOrdHidden;
+                    seen.hid[c] = o < 0 || (o & kOrdHidden) != 0 || seen.ord[c] >= N;   // hidden, no cue or no record
+                    const int2 b = span[q];
+                    seen.start[c] = b.x; seen.end[c] = b.y;
+                    at += (int)__popcll(__ballot((o >= 0) & !before(r, c)));
+                    walk[c] = !seen.hid[c] & cuts(r, c);   // a cue, cut by the record
+                    any |= walk[c];
+                    const bool nearer = seen.dist[c] < r.dist;
+                    on[c] = __ballot(nearer & (b.x <= r.end) & (b.y >= r.start));
+                    hidden |= __ballot(nearer & (b.x <= r.start) & (b.y >= r.end));
+                }
+                const bool repaint = __ballot(any) != 0;
+                if (repaint) {
+                    for (int w = lane; w < W; w += 64) V[w] = 0u;
+                    fg_wave_sync();
+#pragma unroll
+                    for (int c = 0; c < K; ++c) {
+                        const int q = 64 * c + lane;
+                        if (seen.hid[c]) continue;
+                        const int2 had = cut[q];
+                        Interval v{had.x, had.y};
+                        if (walk[c]) {
+                            v = Interval{seen.start[c], seen.end[c]};
+                            bool open = true;
+#pragma unroll
+                            for (int b = 0; b < K; ++b) {   // the nearer ones before it, itself, those after it
+                                const uint64_t m = S.over[(size_t)L * (K * p + b) + q];
+                                const int l = min(max(at - 64 * b, 0), 64);
+                                const uint64_t low = l == 64 ? ~0ull : (1ull << l) - 1ull;
+                                if (open) open = cut_by_all(v, m & low, span + 64 * b);
+                                if (open && at >= 64 * b && (at < 64 * b + 64 || b == K - 1)) open = cut_by(v, make_int2(r.start, r.end));
+                                if (open) open = cut_by_all(v, m & ~low, span + 64 * b);
+                            }
+                        }
+                        paint_cut(V, v, R);
+                    }
+                }
+                if (rc.social && hidden == 0) {
+                    Interval v{r.start, r.end};
+                    bool open = true;
+#pragma unroll
+                    for (int b = 0; b < K; ++b)
+                        if (open) open = cut_by_all(v, on[b], span + 64 * b);
+                    if (lane == 0) paint_cut(V, v, R);
+                }
+                fg_wave_sync();
+            }
+            wave_counts(V, R, W, P.keep_lo, P.keep_hi, nullptr, &n_set, &n_left);
+        }
+    }
+    if (FIELDS && wave > 0 && (N - 1) % H == h) output(N - 1);
+    for (int i = tid; i < N; i += nthr) {
+        const int g = a0 + i;
+        st.x[g] = S.x[i]; st.y[g] = S.y[i]; st.theta[g] = S.th[i]; st.v[g] = S.v[i];
+        st.w[g] = S.w[i]; st.u[g] = S.u1[i];
+        st.mode[g] = S.mode[i]; st.overriding_mode[g] = S.mode_over[i];
+        st.I_priv[g] = S.ip[i];
+    }
+    if (tid == 0) S.kept[0] = draws;
+    __syncthreads();
+    draws = S.kept[0];
+    if (tid == 0 && u_used) u_used[rb] = used0 + (words || mt ? 2 : 1) * draws;
+    if (tid == 0 && status) status[rb] = ABM_WORLD_DONE;
+    if (mt) {
+        // advance the generator by the 2 * draws words used: numpy's state
+        // after them is the key twisted v times at position pos0 + c - 624 v
+        const int c = 2 * draws;
+        int v = 0, pos = mt_pos0 + c;
+        if (pos > kMtN) {
+            v = (pos - 1) / kMtN;
+            pos -= kMtN * v;
+        }
+        if (v > 0) {
+            for (int i = tid; i < kMtN; i += nthr) S.key[i] = mt[rb].key[i];
+            __syncthreads();
+            for (int t = 0; t < v; ++t) mt_twist_block(S.key);
+            for (int i = tid; i < kMtN; i += nthr) mt[rb].key[i] = S.key[i];
+        }
+        if (tid == 0) mt[rb].pos = pos;
+    }
 }
 
 // ------------------------------------------------ replicas over the whole GPU
@@ -2704,7 +3348,7 @@ size_t wide_world_carve(void* base, const abm_forage_world* w, WideWorld* m) {
 // largest first (the cost grows with the agents; rays add to each agent's).
 int plan_paths(abm_forage_batch* bt, int path) {
     const int n = bt->n_replicas;
-    std::vector<int32_t> plain, occl, big;
+    std::vector<int32_t> plain, occl, crowd, big;
     int64_t agents = 0;
     int largest = 0;
     for (int b = 0; b < n; ++b)
@@ -2717,14 +3361,16 @@ int plan_paths(abm_forage_batch* bt, int path) {
     for (int b = 0; b < n; ++b) {
         const bool wideable = !bt->exclusion[b] && bt->rep_r[b] <= kWideMaxRays;
         if (bt->too_big[b] || (spread && wideable)) big.push_back(b);
-        else (bt->exclusion[b] ? occl : plain).push_back(b);
+        else (!bt->exclusion[b] ? plain : bt->rep_n[b] <= kOcclMaxAgents ? occl : crowd).push_back(b);
     }
     auto cost = [&](int b) { return (double)bt->rep_n[b] * (64.0 + bt->rep_r[b] / 32.0); };
     auto larger = [&](int a, int c) { return cost(a) > cost(c); };
     std::stable_sort(plain.begin(), plain.end(), larger);
     std::stable_sort(occl.begin(), occl.end(), larger);
+    std::stable_sort(crowd.begin(), crowd.end(), larger);
     bt->order_host = plain;
     bt->order_host.insert(bt->order_host.end(), occl.begin(), occl.end());
+    bt->order_host.insert(bt->order_host.end(), crowd.begin(), crowd.end());
     bt->order_host.insert(bt->order_host.end(), big.begin(), big.end());
     auto extent = [&](const std::vector<int32_t>& v, int32_t& count, int32_t& agents, int32_t& rays) {
         count = (int32_t)v.size();
@@ -2736,6 +3382,7 @@ int plan_paths(abm_forage_batch* bt, int path) {
     };
     extent(plain, bt->n_plain, bt->plain_max_agents, bt->plain_max_rays);
     extent(occl, bt->n_occl, bt->occl_max_agents, bt->occl_max_rays);
+    extent(crowd, bt->n_crowd, bt->crowd_max_agents, bt->crowd_max_rays);
     // updates counted so far, and no launch left on the scratch that goes
     int64_t made = 0;
     if (int rc = wide_updates(bt, &made)) return rc;
@@ -2812,13 +3459,26 @@ int launch_forage_step(abm_forage_batch* b, const abm_forage_state* st, const do
                            field_bits, (const int32_t*)b->order_dev, mt, b->plain_max_agents);
         if (int rc = check_hip(hipGetLastError(), "forage_update_kernel launch")) return rc;
     }
-    // the step kernel overlaps one agent's move (wave 0) with the next
-    // agent's records (wave 1) and the classes of the one after (the other
-    // waves): eight waves when some replica has more agents than two waves
-    // classify in one pass, else four (two workgroups then share a CU)
     if (b->n_occl > 0) {
-        const int nthr = b->occl_max_agents > 128 ? 512 : 256;
-        const size_t lds = fg_lds_bytes(b->occl_max_agents, b->occl_max_rays);
+        const int K = b->occl_max_agents <= 64 ? 1 : (b->occl_max_agents <= 128 ? 2 : 4);
+        const size_t lds = occl_lds_bytes(b->occl_max_agents, b->occl_max_rays, K);
+        auto kern = field_bits ? (K == 1 ? forage_occlude_kernel<1, true>
+                                         : (K == 2 ? forage_occlude_kernel<2, true> : forage_occlude_kernel<4, true>))
+                               : (K == 1 ? forage_occlude_kernel<1, false>
+                                         : (K == 2 ? forage_occlude_kernel<2, false> : forage_occlude_kernel<4, false>));
+        if (lds > 65536) {
+            if (int rc = check_hip(hipFuncSetAttribute((const void*)kern,
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
+                                   "hipFuncSetAttribute"))
+                return rc;
+        }
+        hipLaunchKernelGGL(kern, dim3(b->n_occl), dim3(64 * kOcclWaves), lds, (hipStream_t)stream,
+                           (const FGRep*)b->reps_dev, *st, uniforms, words, offset, count, used, status,
+                           field_bits, (const int32_t*)b->order_dev + b->n_plain, mt, b->occl_max_agents);
+        if (int rc = check_hip(hipGetLastError(), "forage_occlude_kernel launch")) return rc;
+    }
+    if (b->n_crowd > 0) {   // the replicas with visual exclusion beyond its registers
+        const size_t lds = fg_lds_bytes(b->crowd_max_agents, b->crowd_max_rays);
         auto kern = field_bits ? forage_step_kernel<true> : forage_step_kernel<false>;
         if (lds > 65536) {
             if (int rc = check_hip(hipFuncSetAttribute((const void*)kern,
@@ -2826,10 +3486,10 @@ int launch_forage_step(abm_forage_batch* b, const abm_forage_state* st, const do
                                    "hipFuncSetAttribute"))
                 return rc;
         }
-        hipLaunchKernelGGL(kern, dim3(b->n_occl), dim3(nthr), lds, (hipStream_t)stream,
+        hipLaunchKernelGGL(kern, dim3(b->n_crowd), dim3(512), lds, (hipStream_t)stream,
                            (const FGRep*)b->reps_dev, *st, uniforms, words, offset, count, used, status,
-                           field_bits, (const int32_t*)b->order_dev + b->n_plain, mt, b->occl_max_agents,
-                           b->occl_max_rays);
+                           field_bits, (const int32_t*)b->order_dev + b->n_plain + b->n_occl, mt,
+                           b->crowd_max_agents, b->crowd_max_rays);
         if (int rc = check_hip(hipGetLastError(), "forage_step_kernel launch")) return rc;
     }
     if (!b->wide.empty())

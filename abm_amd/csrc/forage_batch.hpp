@@ -21,13 +21,15 @@ struct abm_forage_batch {
     int32_t* agent_offset_host = nullptr;
     int64_t* field_offset_host = nullptr;
     // Replicas the update kernel takes (the first n_plain of order_dev), those
-    // with visual exclusion, which the step kernel takes (the next n_occl),
-    // and the ones beyond one workgroup's LDS, updated over the whole GPU.
-    int32_t n_plain = 0, n_occl = 0;
+    // with visual exclusion, which the occlude kernel takes (the next n_occl) or
+    // the step kernel (the next n_crowd), and the ones beyond one workgroup's
+    // LDS, updated over the whole GPU.
+    int32_t n_plain = 0, n_occl = 0, n_crowd = 0;
     int32_t plain_max_agents = 0, plain_max_rays = 0, occl_max_agents = 0, occl_max_rays = 0;
+    int32_t crowd_max_agents = 0, crowd_max_rays = 0;
     int32_t path = 0;                  // ABM_FORAGE_PATH_*
     std::vector<int32_t> rep_n, rep_r; // agents and rays of every replica
-    std::vector<int32_t> order_host;   // every replica: update kernel's, step kernel's, wide
+    std::vector<int32_t> order_host;   // every replica: update kernel's, occlude kernel's, step kernel's, wide
     std::vector<uint8_t> too_big;      // [b]: beyond one workgroup's LDS
     std::vector<uint8_t> exclusion;    // [b]: visual exclusion
     std::vector<int32_t> wide;         // replicas updated over the whole GPU
