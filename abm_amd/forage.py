@@ -82,6 +82,7 @@ class ForageConfig:
 
 _F64 = ("x", "y", "theta", "v", "w", "u", "I_priv", "collected_r", "collected_r_before")
 _I32 = ("mode", "overriding_mode", "env_status", "exploited_patch_id", "radius")
+_STATE = tuple(name for name, _ in L.ForageState._fields_)
 
 
 class ForageSwarm:
@@ -181,12 +182,15 @@ class ForageSwarm:
         return u.value, s.value
 
     # ---------------------------------------------------------------- step
+    def _state(self):
+        t = self.t
+        return L.ForageState(*[t[k].data_ptr() for k in _STATE])
+
     def _state_addrs(self):
         """Addresses of the replicas' MT19937 states (numpy's mt19937_state,
         the layout of abm_mt19937_state)."""
         gens = self.rngs if self.rngs is not None else [np.random.mtrand._rand]
-        if self.rngs is None or self._addr is None or any(
-                g is not c for g, c in zip(gens, self._addr_of)):
+        if self.rngs is None or self._addr is None or gens != self._addr_of:   # (by identity)
             self._addr_of = list(gens)
             self._addr = np.array([g._bit_generator.ctypes.state_address for g in gens],
                                   dtype=np.uint64)
@@ -232,8 +236,7 @@ class ForageSwarm:
                 # the pinned staging buffer is free again: the previous step
                 # ended with a synchronising read of u_used on this stream
                 self.u_dev.copy_(self._draw_ahead(), non_blocking=True)
-                st = L.ForageState(**{k: self.t[k].data_ptr() for k in
-                                      _F64 + ("novelty",) + _I32})
+                st = self._state()
                 fb = L.ptr(self.fields) if fields else None
                 L.check(self.lib.abm_forage_step_f64(self.handle, C.byref(st), L.ptr(self.u_dev),
                                                      L.ptr(self.u_off), L.ptr(self.u_cnt),
@@ -290,6 +293,7 @@ class WorldConfig:
 
 
 _PATCH_F64 = ("x", "y", "radius", "units", "left", "quality")
+_PATCH_STATE = tuple(name for name, _ in L.PatchState._fields_)
 _MT_WORDS = 625                       # abm_mt19937_state: 624 key words and the position
 _MT_BYTES = 4 * _MT_WORDS
 TIMEOUT_MESSAGE = "Reached timeout while trying to create resources without overlap!"
@@ -345,10 +349,10 @@ class ResourceWorld:
         self.p["count"] = torch.zeros(nb, dtype=torch.int32, device=dev)
         self.pool_success = torch.zeros(int(swarm.info.n_agents_total), dtype=torch.int32, device=dev)
         self._ret = torch.zeros((2, nb), dtype=torch.int32, device=dev)   # used, status
-        self._woff = torch.zeros(nb, dtype=torch.int64, device=dev)
-        self._wcnt = torch.zeros(nb, dtype=torch.int32, device=dev)
-        self._words_host = torch.zeros(0, dtype=torch.int32).pin_memory()
-        self._words = torch.zeros(1, dtype=torch.int32, device=dev)
+        # staging of the words and their ranges, sent in one copy (int32 words):
+        # offsets (int64) | counts | the replicas' words
+        self._stage_host = torch.zeros(0, dtype=torch.int32).pin_memory()
+        self._stage = torch.zeros(0, dtype=torch.int32, device=dev)
         self.regen_words = int(regen_words)
         self.resumes = 0      # phases resumed for want of words
         self._n = np.diff(swarm.agent_offset).astype(np.int64)
@@ -427,42 +431,51 @@ class ResourceWorld:
         """One loop body for every replica: interaction, regeneration, update."""
         self._run(L.WORLD_STEP, fields, stream)
 
+    def _patch_state(self):
+        p = self.p
+        return L.PatchState(*[p[k].data_ptr() for k in _PATCH_STATE])
+
     def _run(self, phase, fields, stream):
         if self.device_rng:
             return self._run_dev(phase, fields, stream)
         sw = self.swarm
         nb = len(sw.configs)
         reserve = np.zeros(nb, dtype=np.int64) if phase == L.WORLD_FILL else 2 * self._n
+        cnt = reserve + self.regen_words
         active = np.ones(nb, dtype=bool)
         budget, ph = self.regen_words, phase
-        st = L.ForageState(**{k: sw.t[k].data_ptr() for k in _F64 + ("novelty",) + _I32})
-        ps = L.PatchState(**{k: self.p[k].data_ptr() for k in ("count", "id") + _PATCH_F64})
+        st, ps = sw._state(), self._patch_state()
         fb = L.ptr(sw.fields) if fields else None
         addrs = sw._state_addrs()
         with torch.cuda.device(sw.device):
             s = stream if stream is not None else torch.cuda.current_stream()
             with torch.cuda.stream(s):
                 while True:
-                    cnt = np.where(active, reserve + budget, 0).astype(np.int64)
-                    off = np.concatenate([[0], np.cumsum(cnt)[:-1]]).astype(np.int64)
-                    total = int(cnt.sum())
-                    if self._words_host.numel() < total:
-                        self._words_host = torch.zeros(total, dtype=torch.int32).pin_memory()
-                    if self._words.numel() < total:
-                        self._words = torch.zeros(total, dtype=torch.int32, device=sw.device)
+                    end = np.cumsum(cnt)
+                    total = 3 * nb + int(end[-1])
+                    if self._stage_host.numel() < total:
+                        self._stage_host = torch.zeros(total, dtype=torch.int32).pin_memory()
+                    if self._stage.numel() < total:
+                        self._stage = torch.zeros(total, dtype=torch.int32, device=sw.device)
+                    # the pinned buffer is free: every pass ends with a
+                    # synchronising read of _ret on this stream
+                    stage = self._stage_host.numpy()
+                    np.subtract(end, cnt, out=stage[:2 * nb].view(np.int64))
+                    stage[2 * nb:3 * nb] = cnt
                     L.check(self.lib.abm_mt19937_peek32(addrs.ctypes.data_as(C.c_void_p), nb,
                                                         cnt.ctypes.data_as(C.c_void_p),
-                                                        self._words_host.data_ptr()))
-                    self._words[:total].copy_(self._words_host[:total], non_blocking=True)
-                    self._woff.copy_(torch.from_numpy(off))
-                    self._wcnt.copy_(torch.from_numpy(cnt.astype(np.int32)))
+                                                        self._stage_host.data_ptr() + 12 * nb))
+                    self._stage[:total].copy_(self._stage_host[:total], non_blocking=True)
+                    base = self._stage.data_ptr()
                     L.check(self.lib.abm_forage_world_run(
                         self.handle, ph, C.byref(st), L.ptr(self.pool_success), C.byref(ps),
-                        L.ptr(self._words), L.ptr(self._woff), L.ptr(self._wcnt), L.ptr(self._ret[0]),
-                        L.ptr(self._ret[1]), fb, L.stream_ptr(s)))
+                        C.c_void_p(base + 12 * nb), C.c_void_p(base), C.c_void_p(base + 8 * nb),
+                        L.ptr(self._ret[0]), L.ptr(self._ret[1]), fb, L.stream_ptr(s)))
                     used, status = self._ret.cpu().numpy()
                     L.check(self.lib.abm_mt19937_skip32(addrs.ctypes.data_as(C.c_void_p), nb,
                                                         used.astype(np.int64).ctypes.data_as(C.c_void_p)))
+                    if not status.any():   # WORLD_DONE
+                        return
                     if np.any(status[active] == L.WORLD_TIMEOUT):
                         raise Exception(TIMEOUT_MESSAGE)
                     if np.any(status == L.WORLD_BAD_COUNT):
@@ -475,13 +488,13 @@ class ResourceWorld:
                     budget = max(16 * budget, 64)
                     if budget > (1 << 24):
                         raise L.AbmError(L.ABM_ERR_UNSUPPORTED, "patch placement needs more than 2^24 words")
+                    cnt = np.where(need, reserve + budget, 0)
                     ph, active = L.WORLD_RESUME, need
                     self.resumes += 1
 
     def _run_dev(self, phase, fields, stream):
         sw = self.swarm
-        st = L.ForageState(**{k: sw.t[k].data_ptr() for k in _F64 + ("novelty",) + _I32})
-        ps = L.PatchState(**{k: self.p[k].data_ptr() for k in ("count", "id") + _PATCH_F64})
+        st, ps = sw._state(), self._patch_state()
         fb = L.ptr(sw.fields) if fields else None
         with torch.cuda.device(sw.device):
             s = stream if stream is not None else torch.cuda.current_stream()

@@ -41,25 +41,29 @@ def ensemble_stats_arrays(agent_offset, x, y, theta, periodic=False, width=0.0, 
     """Statistics of replicas given as device tensors: ``agent_offset``
     (int32, n_replicas + 1), ``x``, ``y``, ``theta`` (float32 or float64, all
     of one dtype).  Returns a float64 (n_replicas, 4) device tensor."""
-    lib = L.load()
     n = int(agent_offset.shape[0]) - 1
     if n < 0 or agent_offset.dtype != torch.int32:
         raise L.AbmError(L.ABM_ERR_INVALID, "agent_offset must be int32 (n_replicas + 1,)")
+    # the offsets bound every state read: check them on the host
+    return _stats(agent_offset, agent_offset.cpu().numpy(), x, y, theta, periodic, width, height, stream)
+
+
+def _stats(agent_offset, off, x, y, theta, periodic, width, height, stream):
+    """As above, with the offsets' values on the host (``off``)."""
+    n = len(off) - 1
     if not (x.dtype == y.dtype == theta.dtype) or x.dtype not in (torch.float32, torch.float64):
         raise L.AbmError(L.ABM_ERR_INVALID, "x, y, theta must share one float dtype")
     n_agents = int(x.shape[0])
     if y.shape[0] != n_agents or theta.shape[0] != n_agents:
         raise L.AbmError(L.ABM_ERR_INVALID, "x, y, theta must have one length")
-    # the offsets bound every state read: check them on the host
-    off = agent_offset.cpu().numpy()
-    if n >= 0 and (off[0] != 0 or off[-1] != n_agents or np.any(np.diff(off) < 0)):
+    if off[0] != 0 or off[-1] != n_agents or np.any(off[1:] < off[:-1]):
         raise L.AbmError(L.ABM_ERR_INVALID, "agent_offset must rise from 0 to the agent count")
-    out = torch.empty((max(n, 0), 4), dtype=torch.float64, device=x.device)
+    out = torch.empty((n, 4), dtype=torch.float64, device=x.device)
     if n == 0:
         return out
-    L.check(lib.abm_ensemble_stats(n, L.ptr(agent_offset), L.ptr(x), L.ptr(y), L.ptr(theta),
-                                   1 if x.dtype == torch.float32 else 0, 1 if periodic else 0,
-                                   float(width), float(height), L.ptr(out), L.stream_ptr(stream)))
+    L.check(L.load().abm_ensemble_stats(n, L.ptr(agent_offset), L.ptr(x), L.ptr(y), L.ptr(theta),
+                                        1 if x.dtype == torch.float32 else 0, 1 if periodic else 0,
+                                        float(width), float(height), L.ptr(out), L.stream_ptr(stream)))
     return out
 
 
@@ -72,9 +76,12 @@ def ensemble_stats(swarm, periodic=None, stream=None):
         x, y, th, ao = swarm.x, swarm.y, swarm.theta, swarm.batch.agent_offset
     else:                                        # ForageSwarm
         x, y, th, ao = swarm.t["x"], swarm.t["y"], swarm.t["theta"], swarm.agent_offset
+    # the swarm's offsets, on the device from its first call on: their values
+    # are known on the host, so a call on the current stream does not wait
+    off = np.asarray(ao, dtype=np.int32)
     offs = getattr(swarm, "_stats_offsets", None)
     if offs is None:
-        offs = torch.as_tensor(np.asarray(ao, dtype=np.int32), device=x.device)
+        offs = torch.as_tensor(off, device=x.device)
         swarm._stats_offsets = offs
     cfgs = getattr(getattr(swarm, "batch", swarm), "configs", None) or []
     if periodic is None:
@@ -85,7 +92,9 @@ def ensemble_stats(swarm, periodic=None, stream=None):
         if len(sizes) != 1:
             raise L.AbmError(L.ABM_ERR_INVALID, "torus statistics need one arena size per batch")
         W, H = sizes.pop()
-    return ensemble_stats_arrays(offs, x, y, th, periodic, W, H, stream)
+    if stream is not None:   # the state may come from another stream: wait for it, as for any tensors
+        return ensemble_stats_arrays(offs, x, y, th, periodic, W, H, stream)
+    return _stats(offs, off, x, y, th, periodic, W, H, stream)
 
 
 def polarization(swarm):
