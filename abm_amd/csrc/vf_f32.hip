@@ -1534,8 +1534,8 @@ __device__ inline void chain_barrier() {
 // path of dependences times an agent's latency (about 4 thousand cycles), where
 // the id order takes 2.5 thousand cycles for every agent.  Measured, a step, id
 // order and this: 8192 agents, a twelfth of the others in sight, R = 2048, 9.12
-// and 4.26 ms; 2100 agents with walls at R = 2048, a third in sight 2.98 and 2.21,
-// 0.7 3.94 and 3.73, 0.85 4.57 and 4.92 (hence kFlowShare, looked at after a
+// and 3.77 ms (32 segments of 106 us: 5 to load, 11 to list the dependences, 90); 2100 agents with walls at R = 2048, a third in sight 2.98 and 2.11,
+// 0.7 3.94 and 3.64, 0.85 4.48 and 4.92 (hence kFlowShare, looked at after a
 // sample of the agents first, since listing them all costs 2 % of such a step).
 constexpr float kFlowMargin = 16.f;   // + 4 |v|: the displacement allowed for
 constexpr float kFlowShare = 0.7f;    // of a segment's pairs that may depend
@@ -1563,7 +1563,7 @@ vf_step_f32_segment_kernel(const VFRep* __restrict__ rp, const RayTab32* __restr
     __shared__ uint16_t after[kChainWaves][kChainSeg];       // the dependents of a wave's agent
     __shared__ int ctl[4];                                   // next to take, free so far, dependences, out of bounds
     const RepConst C = rep_const(rp);
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const bool want_diag = !PLAIN && (flags & ABM_WANT_DIAG) != 0 && diag != nullptr;
     const bool count = !PLAIN && (flags & (ABM_COUNT_RECHECKS | ABM_VERIFY_FAST_PATH)) != 0 && counters;
     const bool verify = !PLAIN && (flags & ABM_VERIFY_FAST_PATH) != 0 && counters != nullptr;
@@ -1576,26 +1576,45 @@ vf_step_f32_segment_kernel(const VFRep* __restrict__ rp, const RayTab32* __restr
             sdyn[i] = make_float4(st.v[g], st.alp0 ? st.alp0[g] : a0d, st.bet0 ? st.bet0[g] : b0d,
                                   st.v0 ? st.v0[g] : v0d);
         }
-        for (int w = tid; w < n * 64; w += kChainThreads) {
-            const int i = w >> 6, c = w & 63;
-            rows[i][c] = c < C.W ? fields[(size_t)(s0 + i) * C.W + c] : 0u;
+        for (int w0 = tid; w0 < n * 64; w0 += 8 * kChainThreads) {   // eight loads in flight
+            uint32_t q[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int i = (w0 + e * kChainThreads) >> 6;
+                q[e] = i < n && lane < C.W ? fields[(size_t)(s0 + i) * C.W + lane] : 0u;
+            }
+#pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const int i = (w0 + e * kChainThreads) >> 6;
+                if (i < n) rows[i][lane] = q[e];
+            }
         }
     };
-    load();
     if (tid < 2) dirty[tid] = 0;
     const bool may_flow = !count && !verify;
     if (tid < 4) ctl[tid] = 0;
     for (int i = tid; i < kChainSeg; i += kChainThreads) { pend[i] = 0; ready[i] = -1; }
-    // in a summing wave (wave 1, or all) lane l owns rays [l RPL, (l + 1) RPL) and their table entries
+    // in a summing wave (wave 1, or all) lane l owns rays [l RPL, (l + 1) RPL) and
+    // their table entries, which come through the rows' LDS (read from global
+    // memory lane by lane they took 25 thousand cycles for eight waves)
     RayTab32 T[RPL];
-    if (wave == 1 || may_flow) {
+    {
+        static_assert(sizeof(RayTab32) == sizeof(float4) && sizeof(rows) >= 64 * (RPL + 1) * sizeof(float4), "staging");
+        float4* stage = reinterpret_cast<float4*>(&rows[0][0]);   // a lane's entries, and one that shifts the banks
+        const float4* tab = reinterpret_cast<const float4*>(tab32 + rp->table_offset);
+        for (int r = tid; r < C.R; r += kChainThreads) stage[r / RPL * (RPL + 1) + r % RPL] = tab[r];
+        __syncthreads();
+        if (wave == 1 || may_flow) {
 #pragma unroll
-        for (int i = 0; i < RPL; ++i) {
-            const int r = lane * RPL + i;
-            if (r < C.R) T[i] = tab32[rp->table_offset + r];
-            else T[i].wcos = T[i].wsin = T[i].cos = T[i].sin = 0.f;
+            for (int i = 0; i < RPL; ++i) {
+                float4 e = make_float4(0.f, 0.f, 0.f, 0.f);
+                if (lane * RPL + i < C.R) e = stage[lane * (RPL + 1) + i];
+                T[i].wcos = e.x; T[i].wsin = e.y; T[i].cos = e.z; T[i].sin = e.w;
+            }
         }
+        __syncthreads();
     }
+    load();
     // wave 1: the sums of local agent kk's field into red[buf]
     auto sums = [&](int kk, int buf) {
         const float4 d = sdyn[kk];
@@ -1618,29 +1637,53 @@ vf_step_f32_segment_kernel(const VFRep* __restrict__ rp, const RayTab32* __restr
     bool flow = false;
     if (may_flow) {   // uniform
         // ---- the dependences: wave w the agents j = w mod 8, lanes over the later ones
-        float4 f[kChainSeg / 64];
+        float fx[kChainSeg / 64], fy[kChainSeg / 64];   // centres
         int waits[kChainSeg / 64];
 #pragma unroll
         for (int c = 0; c < kChainSeg / 64; ++c) {
-            f[c] = srec[min(64 * c + lane, n - 1)];
+            const int m = 64 * c + lane;
+            fx[c] = m < n ? srec[m].x + srec[m].z : 1e30f;   // out of sight
+            fy[c] = m < n ? srec[m].y + srec[m].z : 1e30f;
             waits[c] = 0;
         }
-        int total = 0;
+        int total = 0;   // wave-uniform
         bool tight = false;   // a torus too small for the nearest image alone to matter
-        auto depend = [&](int j) {
-            const float4 o = srec[j];
-            const float lim = o.z * cull_c + margin(sdyn[j].x) + 1.f;
-            tight = tight || (C.torus && !(fminf(C.hw, C.hh) - C.tguard > lim));
+        static_assert(kChainSeg <= 64 * kChainWaves, "a lane per agent of a wave's share");
+        float jx = 0.f, jy = 0.f, jlim = 0.f;   // lane q: agent wave + 8 q, its reach
+        if (wave + kChainWaves * lane < n) {
+            const float4 o = srec[wave + kChainWaves * lane];
+            jx = o.x + o.z;
+            jy = o.y + o.z;
+            const float lim = o.z * cull_c + margin(sdyn[wave + kChainWaves * lane].x) + 1.f;
+            jlim = lim * lim;
+            tight = C.torus && !(fminf(C.hw, C.hh) - C.tguard > lim);
+        }
+        tight = __ballot(tight) != 0;
+        auto depend = [&](int q) {
+            const int j = wave + kChainWaves * q;
+            const float ox = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(jx), q));
+            const float oy = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(jy), q));
+            const float lim2 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(jlim), q));
+            uint64_t mk[kChainSeg / 64];
 #pragma unroll
             for (int c = 0; c < kChainSeg / 64; ++c) {
-                const int m = 64 * c + lane;
-                float dx = (o.x + o.z) - (f[c].x + f[c].z), dy = (o.y + o.z) - (f[c].y + f[c].z);
-                image(dx, dy);
-                const bool near = m > j && m < n && !(fmaf(dy, dy, dx * dx) > lim * lim);
-                const uint64_t mk = __ballot(near);
+                mk[c] = 0;
+                if (64 * c + 63 <= j) continue;   // (uniform)
+                float dx = fabsf(ox - fx[c]), dy = fabsf(oy - fy[c]);
+                if (C.torus) {   // to the nearest image
+                    dx = fminf(dx, fabsf(C.fW - dx));
+                    dy = fminf(dy, fabsf(C.fH - dy));
+                }
+                const bool near = 64 * c + lane > j && !(fmaf(dy, dy, dx * dx) > lim2);
+                mk[c] = __ballot(near);
                 waits[c] += near ? 1 : 0;
-                total += (int)__popcll(mk);
-                if (lane == 0) dep[j][c] = mk;
+                total += __builtin_amdgcn_readfirstlane((int)__popcll(mk[c]));
+            }
+            if (lane < kChainSeg / 64) {
+                uint64_t mine = mk[0];
+#pragma unroll
+                for (int c = 1; c < kChainSeg / 64; ++c) mine = lane == c ? mk[c] : mine;
+                dep[j][lane] = mine;
             }
         };
         auto tally = [&]() {
@@ -1653,11 +1696,11 @@ vf_step_f32_segment_kernel(const VFRep* __restrict__ rp, const RayTab32* __restr
             return ctl[3] == 0;
         };
         const int n1 = min(n, 2 * kChainWaves);   // a sample first
-        for (int j = wave; j < n1; j += kChainWaves) depend(j);
+        for (int q = 0; wave + kChainWaves * q < n1; ++q) depend(q);
         flow = tally() && ctl[2] <= kFlowShare * n1 * (n - n1 / 2);
         if (flow) {   // uniform
             __syncthreads();
-            for (int j = n1 + wave; j < n; j += kChainWaves) depend(j);
+            for (int q = n1 / kChainWaves; wave + kChainWaves * q < n; ++q) depend(q);
 #pragma unroll
             for (int c = 0; c < kChainSeg / 64; ++c)
                 if (waits[c]) atomicAdd(&pend[64 * c + lane], waits[c]);
