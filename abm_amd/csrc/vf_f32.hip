@@ -1075,15 +1075,18 @@ __device__ __forceinline__ uint32_t span_mask(int a, int b, int rs) {
 // segment kernel, which thereby give the same results bit for bit.  A lane's
 // rays lie in one word (RPL divides 32), its neighbours' rays come from the
 // lanes beside it, so one LDS read starts the sums; `more` holds rays that are
-// not in Fk yet.
-template <int RPL>
+// not in Fk yet.  SPANS = 2: the sums as two waves of half as many rays a lane
+// take them (float32 over a half, the halves' sum the first of the float32 adds).
+template <int RPL, int SPANS = 1>
 __device__ __forceinline__ void one_wave_sums(const uint32_t* Fk, const RayTab32* T, int lane, const RepConst& C,
                                               bool want_diag, float alp0, float bet0, const Pieces& more,
                                               double& Sv, double& Sp, double& Bc, double& Bs, double& Ec,
                                               double& Es) {
+    static_assert(SPANS == 1 || SPANS == 2, "whole lanes or halves");
     const int rs = lane * RPL;
     const int rn = rs >= C.R ? 0 : (C.R - rs < RPL ? C.R - rs : RPL);
     float bc = 0.f, bs = 0.f, ec = 0.f, es = 0.f;
+    float hv = 0.f, hp = 0.f, hbc = 0.f, hbs = 0.f, hec = 0.f, hes = 0.f;   // the first half's
     {
         const uint32_t m = low_mask(rn);
         uint32_t cur = Fk[min(rs >> 5, C.W - 1)] >> (rs & 31);
@@ -1115,15 +1118,31 @@ __device__ __forceinline__ void one_wave_sums(const uint32_t* Fk, const RayTab32
             bs = __builtin_fmaf(vb, T[i].wsin, bs);
             ec = __builtin_fmaf(sb, T[i].cos, ec);
             es = __builtin_fmaf(sb, T[i].sin, es);
+            if (SPANS == 2 && i == RPL / 2 - 1) {
+                if (!want_diag) {
+                    hv = alp0 * (-bc) + (alp0 * C.alp1) * ec;
+                    hp = bet0 * (-bs) + (bet0 * C.bet1) * es;
+                } else {
+                    hbc = bc; hbs = bs; hec = ec; hes = es;
+                }
+                bc = bs = ec = es = 0.f;
+            }
         }
     }
     Bc = Bs = Ec = Es = 0.0;
     if (!want_diag) {
-        Sv = wave_total(alp0 * (-bc) + (alp0 * C.alp1) * ec);
-        Sp = wave_total(bet0 * (-bs) + (bet0 * C.bet1) * es);
+        const float v = alp0 * (-bc) + (alp0 * C.alp1) * ec;
+        const float p = bet0 * (-bs) + (bet0 * C.bet1) * es;
+        Sv = SPANS == 2 ? pair_total(hv + v) : wave_total(v);
+        Sp = SPANS == 2 ? pair_total(hp + p) : wave_total(p);
+    } else if (SPANS == 2) {
+        Bc = pair_total(hbc + bc); Bs = pair_total(hbs + bs);
+        Ec = pair_total(hec + ec); Es = pair_total(hes + es);
     } else {
         Bc = wave_total(bc); Bs = wave_total(bs);
         Ec = wave_total(ec); Es = wave_total(es);
+    }
+    if (want_diag) {
         Sv = (double)alp0 * -Bc + (double)(alp0 * C.alp1) * Ec;
         Sp = (double)bet0 * -Bs + (double)(bet0 * C.bet1) * Es;
     }
@@ -1190,7 +1209,8 @@ __device__ inline void push_culled_check(float4 f, float4 o, const VFRep* rp, bo
 
 // PLAIN: a step with no fields, diagnostics or counters out (the flags and
 // pointers that ask for them are ignored), so their tests leave the kernel.
-template <int RPL, bool PLAIN>
+// HALVES: replicas up to kBigClass agents sum as two waves do (SPANS = 2).
+template <int RPL, bool PLAIN, bool HALVES>
 __global__ void __launch_bounds__(kPushThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 vf_step_f32_push_kernel(const VFRep* __restrict__ reps, const int32_t* __restrict__ order,
                         const RayTab32* __restrict__ tab32, abm_vf_state_f32 st,
@@ -1201,6 +1221,8 @@ vf_step_f32_push_kernel(const VFRep* __restrict__ reps, const int32_t* __restric
     const RepConst C = rep_const(rp);
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
     const int W1 = C.W + 1;
+    const bool halves = HALVES && C.N <= kBigClass;
+    constexpr int kSpans = HALVES ? 2 : 1;
     const bool want_diag = !PLAIN && (flags & ABM_WANT_DIAG) != 0 && diag != nullptr;
     const bool count = !PLAIN && (flags & (ABM_COUNT_RECHECKS | ABM_VERIFY_FAST_PATH)) != 0 && counters;
     const bool verify = !PLAIN && (flags & ABM_VERIFY_FAST_PATH) != 0 && counters != nullptr;
@@ -1301,7 +1323,8 @@ vf_step_f32_push_kernel(const VFRep* __restrict__ reps, const int32_t* __restric
     auto sums_into = [&](int i, const Pieces& more, double* r) {   // wave 1
         const float4 d = dyn[i];
         double Sv, Sp, Bc, Bs, Ec, Es;
-        one_wave_sums<RPL>(F + (size_t)i * W1, T, lane, C, want_diag, d.y, d.z, more, Sv, Sp, Bc, Bs, Ec, Es);
+        if (halves) one_wave_sums<RPL, kSpans>(F + (size_t)i * W1, T, lane, C, want_diag, d.y, d.z, more, Sv, Sp, Bc, Bs, Ec, Es);
+        else one_wave_sums<RPL>(F + (size_t)i * W1, T, lane, C, want_diag, d.y, d.z, more, Sv, Sp, Bc, Bs, Ec, Es);
         if (lane == 0) {
             r[0] = Sv; r[1] = Sp;
             if (want_diag) { r[2] = Bc; r[3] = Bs; r[4] = Ec; r[5] = Es; }
@@ -1340,7 +1363,10 @@ vf_step_f32_push_kernel(const VFRep* __restrict__ reps, const int32_t* __restric
                     for (int w = lane; w < C.W; w += 64) dst[w] = Fk[w];
                 }
             }
-            if (!hit) one_wave_sums<RPL>(Fk, T, lane, C, want_diag, alp0, bet0, more, Sv, Sp, Bc, Bs, Ec, Es);
+            if (!hit) {
+                if (halves) one_wave_sums<RPL, kSpans>(Fk, T, lane, C, want_diag, alp0, bet0, more, Sv, Sp, Bc, Bs, Ec, Es);
+                else one_wave_sums<RPL>(Fk, T, lane, C, want_diag, alp0, bet0, more, Sv, Sp, Bc, Bs, Ec, Es);
+            }
             // ---- agent k's move
             float vel, o, dv, dpsi;
             steer(C, fth, dk.x, v0, (float)Sv, (float)Sp, &o, &vel, &dv, &dpsi);
@@ -1430,9 +1456,11 @@ bool push_fits_in(const abm_vf_batch* b, bool all) {
 
 template <int RPL>
 int launch_push(abm_vf_batch* b, const abm_vf_state_f32* st, uint32_t* bits, float* diag,
-                uint32_t flags, hipStream_t s, const int32_t* order, int n_rep, size_t lds) {
+                uint32_t flags, hipStream_t s, const int32_t* order, int n_rep, size_t lds, bool halves) {
     const bool plain = bits == nullptr && (flags & (ABM_WANT_DIAG | ABM_COUNT_RECHECKS | ABM_VERIFY_FAST_PATH)) == 0;
-    auto kern = plain ? vf_step_f32_push_kernel<RPL, true> : vf_step_f32_push_kernel<RPL, false>;
+    constexpr bool kHalves = RPL > 4;   // (a lane's four rays are not halved)
+    auto kern = halves && kHalves ? (plain ? vf_step_f32_push_kernel<RPL, true, kHalves> : vf_step_f32_push_kernel<RPL, false, kHalves>)
+                                  : (plain ? vf_step_f32_push_kernel<RPL, true, false> : vf_step_f32_push_kernel<RPL, false, false>);
     if (lds > 65536) {
         if (int rc = check_hip(hipFuncSetAttribute((const void*)kern,
                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
@@ -1447,9 +1475,11 @@ int launch_push(abm_vf_batch* b, const abm_vf_state_f32* st, uint32_t* bits, flo
 
 // The push kernel over order[0 .. n_rep): every replica (all) or the large
 // size class.  Rays per lane of wave 0 follow the one-wave per-replica
-// kernel's rule for the largest R of the launch.
+// kernel's rule for the largest R of the launch.  halves: replicas up to
+// kBigClass agents sum as the per-replica kernel's two waves do.
 int launch_push_any(abm_vf_batch* b, const abm_vf_state_f32* st, uint32_t* bits, float* diag,
-                    uint32_t flags, hipStream_t s, const int32_t* order, int n_rep, bool all) {
+                    uint32_t flags, hipStream_t s, const int32_t* order, int n_rep, bool all,
+                    bool halves = false) {
     const size_t lds = all ? b->push_lds_all : b->push_lds_big;
     if (!push_fits_in(b, all))
         return set_error(ABM_ERR_UNSUPPORTED,
@@ -1457,10 +1487,10 @@ int launch_push_any(abm_vf_batch* b, const abm_vf_state_f32* st, uint32_t* bits,
                          "for its fields, device max %d; up to %d agents)", lds, b->dev_max_lds,
                          kWideThreshold);
     const int rpl = push_rpl(all ? b->max_rays : b->big_max_rays);
-    if (rpl == 4) return launch_push<4>(b, st, bits, diag, flags, s, order, n_rep, lds);
-    if (rpl == 8) return launch_push<8>(b, st, bits, diag, flags, s, order, n_rep, lds);
-    if (rpl == 16) return launch_push<16>(b, st, bits, diag, flags, s, order, n_rep, lds);
-    return launch_push<32>(b, st, bits, diag, flags, s, order, n_rep, lds);
+    if (rpl == 4) return launch_push<4>(b, st, bits, diag, flags, s, order, n_rep, lds, halves);
+    if (rpl == 8) return launch_push<8>(b, st, bits, diag, flags, s, order, n_rep, lds, halves);
+    if (rpl == 16) return launch_push<16>(b, st, bits, diag, flags, s, order, n_rep, lds, halves);
+    return launch_push<32>(b, st, bits, diag, flags, s, order, n_rep, lds, halves);
 }
 
 // ---------------------------------------------------------------------------
@@ -2145,6 +2175,8 @@ int selected_group_size(const abm_vf_batch* b) {
     return 1;
 }
 
+constexpr int kFewReplicas = 8;
+
 // Waves per replica of the per-replica kernel: four while the batch gives each
 // CU at most two such workgroups, two while it fits at 16 waves per CU, else
 // one (measured on MI355X: 1024 replicas of 100 agents take 0.223 ms on two
@@ -2226,13 +2258,33 @@ int launch_vf_step_f32(abm_vf_batch* b, const abm_vf_state_f32* st, uint32_t* bi
     if (nw == 16)   // the 16-wave kernel for every replica
         return launch_big_any(b, st, bits, diag, flags, s, b->order_dev, b->n_replicas, b->max_agents,
                               b->max_rays);
-    const int nb = b->n_big_class;
-    const bool push_ok = !sync_order && nb > 0 && push_fits(b, false);
     // The push kernel holds one replica per CU (eight waves of up to 256
-    // VGPRs), so it shortens the step only while the large class's agents,
-    // spread over the CUs, do not outlast the chain of its largest replica;
-    // beyond that (many replicas of similar size) the per-replica kernel's
-    // occupancy wins.
+    // VGPRs), so it shortens the step only while the agents, spread over the
+    // CUs, do not outlast the chain of the largest replica; beyond that (many
+    // replicas of similar size) the per-replica kernel's occupancy wins.  A
+    // replica counts four agents more, its start and end.  Where that holds for
+    // the whole batch, all of it goes there: ms a step on this kernel and
+    // otherwise, one replica of 8 agents 0.0159 and 0.0169, of 33 0.046 and 0.063;
+    // 256 of 8 to 60 0.074 and 0.100 (512 of 60: 0.141 and 0.112, which the rule
+    // leaves); 250 of 60 at R = 2048 0.106 and 0.140; 64 of 8 to 200 0.218 and
+    // 0.311, 1000 of 8 to 512 0.82 and 0.92 (the small ones first, on the other
+    // kernel).  A batch of a few replicas of both classes keeps a kernel for
+    // each, as its callers may rely on.
+    const int nb = b->n_big_class;
+    const bool few = b->n_replicas <= kFewReplicas && nb > 0 && nb < b->n_replicas;
+    if (nw == 0 && !sync_order && !few && push_fits(b, true) &&
+        (int64_t)b->n_agents_total + 4 * (int64_t)b->n_replicas <= ((int64_t)b->max_agents + 4) * b->n_cu) {
+        // the sums as the kernels of the two classes take them, bit for bit (but
+        // for the order of the last float64 adds): the same rays a lane, or half
+        // as many on two waves
+        const int ns = b->n_replicas - nb, rpl = push_rpl(b->max_rays), r = nb > 0 ? b->small_max_rays : b->max_rays;
+        const int waves = ns > 0 ? default_waves(b, nb > 0 ? b->small_max_agents : b->max_agents, ns) : 1;
+        const int small = ns > 0 ? push_rpl((r + waves - 1) / waves) : rpl;
+        if ((nb == 0 || push_rpl(b->big_max_rays) == rpl) && (small == rpl || 2 * small == rpl))
+            return launch_push_any(b, st, bits, diag, flags, s, b->order_dev, b->n_replicas, true, small != rpl);
+    }
+    // else for the class of large replicas alone
+    const bool push_ok = !sync_order && nb > 0 && push_fits(b, false);
     const bool push = push_ok && b->big_sum_agents <= (int64_t)b->big_max_agents * b->n_cu;
     if (nw == 0 && nb > 0 && !sync_order && (push || (!push_ok && nb < b->n_replicas))) {
         // size classes: the small replicas on the per-replica kernel, then

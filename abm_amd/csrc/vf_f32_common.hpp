@@ -53,6 +53,21 @@ __device__ inline double wave_total(float x) {
     return __hiloint2double(hi, lo);
 }
 
+// The same total where a lane's x is already the sum of two neighbouring terms:
+// float32 adds over 16 terms as there (eight lanes), float64 beyond.
+__device__ inline double pair_total(float x) {
+    x += dpp_f32<0xB1>(x);
+    x += dpp_f32<0x4E>(x);
+    x += dpp_f32<0x141>(x);
+    double v = (double)x;
+    v += (double)dpp_f32<0x140>(x);
+    v += dpp_f64_masked<0x142, 0xa>(v);
+    v += dpp_f64_masked<0x143, 0xc>(v);
+    const int lo = __builtin_amdgcn_readlane(__double2loint(v), 63);
+    const int hi = __builtin_amdgcn_readlane(__double2hiint(v), 63);
+    return __hiloint2double(hi, lo);
+}
+
 __device__ inline float lane_f32(float v, int lane) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), lane));
 }
