@@ -167,16 +167,17 @@ class ForageSwarm:
         return slice(int(self.agent_offset[b]), int(self.agent_offset[b + 1]))
 
     def set_path(self, path: str = "auto"):
-        """How replicas are updated: "auto" (one workgroup each for replicas
-        that fit its LDS, a sweep over the whole GPU for larger ones) or
-        "sweep" (that sweep for every replica without visual exclusion; the
-        same results, used to compare the two)."""
+        """How replicas are updated: "auto" (one workgroup each, or launches
+        over the whole GPU for those beyond its LDS and for large ones of
+        batches too small to fill the GPU) or
+        "sweep" (those launches for every replica without visual exclusion;
+        the same results, used to compare the two)."""
         code = {"auto": L.FORAGE_PATH_AUTO, "sweep": L.FORAGE_PATH_SWEEP}[path]
         L.check(self.lib.abm_forage_set_path(self.handle, code))
 
     def sweep_counts(self):
-        """(replica updates made by sweeps over the whole GPU, sweeps they took:
-        one each) since creation."""
+        """(replica updates made over the whole GPU, sweeps of their agents that
+        they took: one each) since creation."""
         u, s = C.c_int64(), C.c_int64()
         L.check(self.lib.abm_forage_sweep_counts(self.handle, C.byref(u), C.byref(s)))
         return u.value, s.value

@@ -221,11 +221,16 @@ def other_workload(args):
         for prec in ("f32", "f64"):
             sw = VFSwarm([cfg], x, y, th, 0.0, radius=5, precision=prec)
             res[prec] = time_steps(sw, args.steps, args.warmup, not args.no_graph)[0]
+
+        class PlainStep:   # every pair in float64: the float64 step that counts its near ties
+            step = staticmethod(lambda: sw.step(count=True))
+        res["plain"] = time_steps(PlainStep, args.steps, args.warmup, not args.no_graph)[0]
         ops = ops_per_agent_step(Ns, Rs) * Ns
         _line(args, f"single VSWRM replica N={Ns}, R={Rs}, 1000x1000 torus, reference order", Ns / (res["f32"] * 1e-3),
               res["f32"], "f32", {"replicas": 1, "agents_per_replica": Ns, "rays": Rs},
-              plain_f64={"agent_steps_per_s": Ns / (res["f64"] * 1e-3), "ms_per_step": res["f64"]},
-              speedup_vs_plain_f64=res["f64"] / res["f32"],
+              plain_f64={"agent_steps_per_s": Ns / (res["plain"] * 1e-3), "ms_per_step": res["plain"]},
+              speedup_vs_plain_f64=res["plain"] / res["f32"],
+              float64={"agent_steps_per_s": Ns / (res["f64"] * 1e-3), "ms_per_step": res["f64"]},
               roofline={"bound": "valu", "achieved": ops / (res["f32"] * 1e-3) / 1e12,
                         "peak": VALU_PEAK_TOPS, "unit": "Tops/s",
                         "frac": ops / (res["f32"] * 1e-3) / 1e12 / VALU_PEAK_TOPS, "traffic": None,
@@ -642,7 +647,7 @@ def c5_overlay_workload(args):
     (the foraging agent's only boundary, agent.py:279), 64 resource patches
     of radius 30 with quality U[0.5, 1] and 200..1000 units, the C1 decision
     values, vision range 2000, generators on the device.  The replica
-    exceeds one workgroup's LDS, so the update runs by sweeps."""
+    exceeds one workgroup's LDS, so the update runs over the whole GPU."""
     import torch
     from abm_amd.forage import ForageConfig, ForageSwarm, ResourceWorld, WorldConfig
     N, R, W, r = 8192, 2048, 4000, 2
@@ -677,19 +682,18 @@ def c5_overlay_workload(args):
     achieved = ops / (ms * 1e-3) / 1e12
     extra = {"roofline": {"bound": "valu", "achieved": achieved, "peak": VALU_PEAK_TOPS,
                           "unit": "Tops/s", "frac": achieved / VALU_PEAK_TOPS, "traffic": None,
-                          "note": "latency-bound: a few sweeps of small launches per step, "
-                                  "host-synchronised once per round; ops counted once per "
-                                  "agent-step with the exploiting cues at the end of the run"}}
+                          "note": "latency-bound: six small launches per step; ops counted once "
+                                  "per agent-step with the exploiting cues at the end of the run"}}
     if cpu is not None:
         extra["cpu_baseline"] = cpu
     _line(args, f"foraging overlay of the large flock: N={N} agents of radius 2, R={R}, 4000x4000 "
                 f"walls, 64 patches (radius 30, quality U[0.5, 1]), resource loop and Agent.update "
-                f"in id order (sweeps) on the device",
+                f"in id order on the device",
           N / (ms * 1e-3), ms, "f64", {"replicas": 1, "agents_per_replica": N, "rays": R,
                                         "patches": 64},
           ms_per_step_median=q50, ms_per_step_iqr=[q25, q75],
           sweeps_per_step=(w1 - w0) / max(1, s1 - s0), exploiting_cues_at_end=expl,
-          note="wall time per step (the sweeps read a few control words per round)", **extra)
+          note="wall time per step", **extra)
 
 
 def main():
@@ -778,8 +782,12 @@ def main():
     sw64 = VFSwarm(cfgs, x, y, th, 0.0, radius=RADIUS, precision="f64")
     ms32_mean, ms32_med, wall32 = time_steps(sw32, args.steps, args.warmup, not args.no_graph)
     iqr32, replays32 = getattr(time_steps, "last_iqr", None), getattr(time_steps, "last_replays", (0, 0))
-    ms64_mean, ms64_med, wall64 = time_steps(sw64, args.steps_f64, min(args.warmup, 3),
+
+    class PlainStep:   # every pair in float64: the float64 step that counts its near ties
+        step = staticmethod(lambda: sw64.step(count=True))
+    ms64_mean, ms64_med, wall64 = time_steps(PlainStep, args.steps_f64, min(args.warmup, 3),
                                              not args.no_graph)
+    ms64g_mean = time_steps(sw64, args.steps_f64, min(args.warmup, 3), not args.no_graph)[0]
     swk = VFSwarm(cfgs, x, y, th, 0.0, radius=RADIUS, precision="f32")
 
     class KahanStep:
@@ -812,10 +820,12 @@ def main():
         "plain_f64": {"agent_steps_per_s": rate64, "ms_per_step": ms64_mean,
                       "steps": args.steps_f64,
                       "roofline_frac": ops / (ms64_mean * 1e-3) / 1e12 / VALU_PEAK_TOPS,
-                      "note": ("the same lane-op count over the float64 kernel's time; its float64 "
-                               "transcendentals and one wave per replica keep VALUBusy near 58 % "
-                               "(rocprofv3), against about 82 % for the fused kernel")},
+                      "note": ("the same lane-op count over the plain float64 kernel's time (near-tie "
+                               "counts on); its float64 transcendentals and one wave per replica keep "
+                               "VALUBusy near 58 % (rocprofv3), against about 82 % for the fused kernel")},
         "speedup_vs_plain_f64": rate32 / rate64,
+        "float64": {"agent_steps_per_s": agents / (ms64g_mean * 1e-3), "ms_per_step": ms64g_mean,
+                    "note": "the default float64 step: decisions in guarded float32, all else in float64"},
         "fixed_error": {
             "one_step_rel_err_vs_f64": float(e_sync.max()),
             "fields_bit_exact_vs_f64": bool(same_sync.all()),

@@ -171,14 +171,16 @@ int abm_vf_f64_near_ties(abm_vf_batch* batch, int64_t* near_ties, void* stream);
  * give one workgroup to each replica: the 16-wave kernel (every pose in LDS,
  * the pairs of each agent decided in its turn) and the push kernel (every
  * agent's field in LDS, the pairs decided off the id-order chain as soon as
- * their object has moved), which by default runs the large size class of a
- * batch (replicas above 64 agents) when their fields fit and the class's
- * agents, spread over the CUs, are no more than its largest replica's chain
- * (one push workgroup per CU), next to the per-replica kernel for the rest;
+ * their object has moved), which by default runs batches whose fields fit and
+ * whose agents, spread over the CUs, are no more than the largest replica's
+ * chain (one push workgroup per CU).  Where that holds only for the large size
+ * class (replicas above 64 agents), or the batch has at most eight replicas of
+ * both classes, it runs that class next to the per-replica kernel for the rest;
  * the 16-wave kernel takes the class when its fields do not fit.
  * Batches of flocks above 2048 agents in the reference order take the chain
  * step: each agent's pairs with later agents at their start poses over the
- * whole GPU, then segments of 256 agents moved in id order by one workgroup,
+ * whole GPU, then segments of 256 agents moved by one workgroup (in id order,
+ * or each agent once the earlier ones it can see have moved: the same moves),
  * each segment's new poses decided in the later agents' fields over the
  * whole GPU (the push kernel's sums and moves, so the same results).
  * abm_vf_set_launch selects the per-replica kernel with waves_per_group waves
