@@ -1051,7 +1051,9 @@ int launch_big_any(abm_vf_batch* b, const abm_vf_state_f32* st, uint32_t* bits, 
 // on the other waves' LDS traffic.  Measured, one replica of 100 agents at
 // R = 1024: 0.160 ms a step with the sums and their LDS round trips on the
 // chain, 0.141 with the pair handed over in registers, 0.123 with wave 1
-// summing ahead; 1000 replicas of 8 to 512 agents, 1.025, 0.989, 0.931.
+// summing ahead, 0.121 with the rays between a span's ends stored rather than
+// ORed and a pushing lane's agent in registers; 1000 replicas of 8 to 512 agents,
+// 1.025, 0.989, 0.931, 0.921 (0.811 with the small ones in the same launch).
 constexpr int kPushThreads = 64 * kPushWaves;
 
 // Rays added to a field in registers: up to two pieces [a, b) (wave-uniform).
@@ -1172,12 +1174,15 @@ __device__ inline bool decide_pair(PairF32& pr, float2 u, float4 f, float4 o, co
     return pr.drawn;
 }
 
+template <bool LDS = true>   // where the field lies
 __device__ inline void push_pair(uint32_t* Fm, float2 u, float4 f, float4 o, const VFRep* rp,
                                  const RepConst& C, bool count, bool verify, unsigned long long& n_pairs,
                                  unsigned long long& n_recheck, unsigned long long& n_disagree) {
     PairF32 pr;
-    if (decide_pair(pr, u, f, o, rp, C, count, verify, n_pairs, n_recheck, n_disagree))
-        raster(Fm, pr.start, pr.end, C.R);
+    if (decide_pair(pr, u, f, o, rp, C, count, verify, n_pairs, n_recheck, n_disagree)) {
+        if (LDS) raster_lds(Fm, pr.start, pr.end, C.R);
+        else raster(Fm, pr.start, pr.end, C.R);
+    }
 }
 
 // Whether a pair lies beyond the visibility cut-off d > size cot(2 pi / R)
@@ -1219,7 +1224,7 @@ vf_step_f32_push_kernel(const VFRep* __restrict__ reps, const int32_t* __restric
     extern __shared__ __align__(16) double smem_d[];
     const VFRep* rp = reps + order[blockIdx.x];
     const RepConst C = rep_const(rp);
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63;
+    const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
     const int W1 = C.W + 1;
     const bool halves = HALVES && C.N <= kBigClass;
     constexpr int kSpans = HALVES ? 2 : 1;
@@ -1337,6 +1342,10 @@ vf_step_f32_push_kernel(const VFRep* __restrict__ reps, const int32_t* __restric
     const int last = C.N - 1;
     float4 f0 = P0[0], f1 = P0[min(1, last)];   // wave 0: start poses of agents k, k + 1
     float2 u1 = U[min(1, last)];
+    // a pushing lane's agents m0, m0 + 384 ..: the first one's start pose stays in registers
+    const int m0 = 2 + (wave - 2) * 64 + lane;
+    const float4 fm = P0[min(max(m0, 0), last)];
+    const float2 um = U[min(max(m0, 0), last)];
     Pieces more{0, 0, 0, 0};   // wave 0: the rays of the pair (k, k - 1)
     bool hit = true;           // wave 0: they are the ones wave 1 summed with
     for (int k = 0; k < C.N; ++k) {
@@ -1393,9 +1402,13 @@ vf_step_f32_push_kernel(const VFRep* __restrict__ reps, const int32_t* __restric
             if (there && !culled &&
                 decide_pair(pr, u, f, moved, rp, C, count && once, verify && once, n_pairs, n_recheck, n_disagree))
                 vf_pieces(pr.start, pr.end, C.R, &q.a0, &q.b0, &q.a1, &q.b1);
-            if (lane == 1) {
-                or_range(F + (size_t)(k + 2) * W1, q.a0, q.b0);
-                or_range(F + (size_t)(k + 2) * W1, q.a1, q.b1);
+            {   // the odd lanes' rays into agent k + 2's field, a word a lane
+                const Pieces z{__builtin_amdgcn_readlane(q.a0, 1), __builtin_amdgcn_readlane(q.b0, 1),
+                               __builtin_amdgcn_readlane(q.a1, 1), __builtin_amdgcn_readlane(q.b1, 1)};
+                uint32_t bits = 0;
+                if (z.b0 > z.a0) bits = span_mask<32>(z.a0, z.b0, 32 * lane);
+                if (z.b1 > z.a1) bits |= span_mask<32>(z.a1, z.b1, 32 * lane);
+                if (bits) atomicOr(&F[(size_t)(k + 2) * W1 + lane], bits);   // (rays < R: words < W)
             }
             more.a0 = __builtin_amdgcn_readfirstlane(q.a0); more.b0 = __builtin_amdgcn_readfirstlane(q.b0);
             more.a1 = __builtin_amdgcn_readfirstlane(q.a1); more.b1 = __builtin_amdgcn_readfirstlane(q.b1);
@@ -1422,12 +1435,18 @@ vf_step_f32_push_kernel(const VFRep* __restrict__ reps, const int32_t* __restric
         } else if (k >= 1) {
             // ---- agent k - 1's new pose into the fields of agents k + 2 ..
             const float4 ob = P1[k - 1];
-            for (int m = k + 2 + (wave - 2) * 64 + lane; m < C.N; m += (kPushWaves - 2) * 64) {
-                const float4 f = P0[m];
+            for (int m = m0; m < C.N; m += (kPushWaves - 2) * 64) {
+                if (m < k + 2) continue;
+                float4 f = fm;
+                float2 u = um;
+                if (m != m0) {
+                    f = P0[m];
+                    u = U[m];
+                }
                 if (push_culled(f, ob, C, cull_c)) {
                     push_culled_check(f, ob, rp, count, verify, n_pairs, n_disagree);
                 } else {
-                    push_pair(F + (size_t)m * W1, U[m], f, ob, rp, C, count, verify, n_pairs, n_recheck, n_disagree);
+                    push_pair(F + (size_t)m * W1, u, f, ob, rp, C, count, verify, n_pairs, n_recheck, n_disagree);
                 }
             }
         }
@@ -1879,7 +1898,7 @@ vf_step_f32_segment_kernel(const VFRep* __restrict__ rp, const RayTab32* __restr
                 } else {
                     PairF32 pr;
                     if (decide_pair(pr, su[m], f, ob, rp, C, count, verify, n_pairs, n_recheck, n_disagree)) {
-                        raster(rows[m], pr.start, pr.end, C.R);
+                        raster_lds(rows[m], pr.start, pr.end, C.R);
                         drew = true;
                     }
                 }
@@ -1990,7 +2009,7 @@ vf_step_f32_chain_push_kernel(const VFRep* __restrict__ rp, abm_vf_state_f32 st,
         if (head + lane < tail) {
             int m;
             const float4 f = focal((int)wq[(head + lane) & (kChainQueue - 1)], m, true);
-            push_pair(fields + (size_t)m * C.W, ustart[m], f, o, rp, C, count, verify, n_pairs, n_recheck,
+            push_pair<false>(fields + (size_t)m * C.W, ustart[m], f, o, rp, C, count, verify, n_pairs, n_recheck,
                       n_disagree);
         }
     };

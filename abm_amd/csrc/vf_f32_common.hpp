@@ -88,6 +88,25 @@ __device__ inline void or_range(uint32_t* F, int a, int b) {
     }
 }
 
+// The same in a field in LDS: its first and last word by atomics, the words
+// between, which all become ones, by plain (relaxed) stores.
+__device__ inline void or_span(uint32_t* F, int a, int b) {
+    if (a >= b) return;
+    int w = a >> 5;
+    const int e = (b - 1) >> 5;
+    const uint32_t first = 0xffffffffu << (a & 31), last = 0xffffffffu >> (31 - ((b - 1) & 31));
+    atomicOr(&F[w], w == e ? first & last : first);
+    if (w != e) atomicOr(&F[e], last);
+    for (++w; w < e; ++w) __hip_atomic_store(&F[w], 0xffffffffu, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+
+__device__ inline void raster_lds(uint32_t* F, int start, int end, int R) {
+    int p0, p1, q0, q1;
+    vf_pieces(start, end, R, &p0, &p1, &q0, &q1);
+    or_span(F, p0, p1);
+    or_span(F, q0, q1);
+}
+
 __device__ inline void raster(uint32_t* F, int start, int end, int R) {
     int p0, p1, q0, q1;
     vf_pieces(start, end, R, &p0, &p1, &q0, &q1);
