@@ -595,26 +595,54 @@ vf_step_f32_wide_kernel(const VFRep* __restrict__ rp, const RayTab32* __restrict
     }
 }
 
+// Inclusive prefix sum over the 64 lanes: inside rows of 16, then rows 0 and 2
+// into 1 and 3, then the lower half into the upper.
+__device__ inline int wave_scan(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);
+    return v;
+}
+
 // One block: the replica's grid (cells no narrower than the largest
 // visibility cut-off r_max * cull_c, plus 0.1 % and 1 px) and its agents
 // sorted by cell (counting sort in LDS).  The order inside a cell is free:
-// the field is an OR of rasters.
+// the field is an OR of rasters.  Bound by latency: the agents' loads, a few
+// barriers, the scatter.  The first 8192 agents stay in registers from one load
+// to the scatter, the radii meet by wave and the counts are summed by wave
+// (before, three passes over global memory, 1024 atomics to one word and twenty
+// barriers: 16.6 us for 8192 agents, 10.5 now, of 87.8 and 81.6 in a synchronous
+// step).
 __global__ void __launch_bounds__(1024)
 wide_grid_kernel(const VFRep* __restrict__ rp, abm_vf_state_f32 st, float cull_c,
                  float4* __restrict__ sorted, int32_t* __restrict__ cell_start,
                  WideGrid* __restrict__ grid) {
     __shared__ int cnt[kWideGridMaxCells + 1];
-    __shared__ int part[1024];
+    __shared__ int part[16];
     __shared__ int rmax;
     __shared__ WideGrid G;
     const RepConst C = rep_const(rp);
-    const int tid = threadIdx.x, nthr = blockDim.x;
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    constexpr int nthr = 1024;
     if (tid == 0) rmax = 0;
-    __syncthreads();
-    // eight agents per thread per pass, their loads issued together
+    // eight agents per thread per pass, their loads issued together; the first
+    // pass's stay
     constexpr int kPer = 8;
+    float px[kPer], py[kPer];
+    int pr[kPer], cell[kPer];
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+        const int i = q * nthr + tid, g = C.a0 + (i < C.N ? i : 0);
+        px[q] = st.x[g]; py[q] = st.y[g]; pr[q] = (int)st.radius[g];
+    }
+    for (int c = tid; c <= kWideGridMaxCells; c += nthr) cnt[c] = 0;
     int rm = 0;
-    for (int base = 0; base < C.N; base += nthr * kPer) {
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) rm = max(rm, q * nthr + tid < C.N ? pr[q] : 0);
+    for (int base = nthr * kPer; base < C.N; base += nthr * kPer) {
         int rv[kPer];
 #pragma unroll
         for (int q = 0; q < kPer; ++q) {
@@ -624,7 +652,9 @@ wide_grid_kernel(const VFRep* __restrict__ rp, abm_vf_state_f32 st, float cull_c
 #pragma unroll
         for (int q = 0; q < kPer; ++q) rm = max(rm, rv[q]);
     }
-    atomicMax(&rmax, rm);
+    for (int o = 32; o > 0; o >>= 1) rm = max(rm, __shfl_xor(rm, o, 64));
+    __syncthreads();
+    if (lane == 0) atomicMax(&rmax, rm);
     __syncthreads();
     if (tid == 0) {
         WideGrid g;
@@ -642,38 +672,37 @@ wide_grid_kernel(const VFRep* __restrict__ rp, abm_vf_state_f32 st, float cull_c
     __syncthreads();
     if (!G.ok) return;
     const int ncell = G.nx * G.ny;
-    for (int c = tid; c <= ncell; c += nthr) cnt[c] = 0;
-    __syncthreads();
-    for (int base = 0; base < C.N; base += nthr * kPer) {
-        float px[kPer], py[kPer], pr[kPer];
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+        const float r = (float)pr[q];
+        cell[q] = grid_cell(G, px[q] + r, py[q] + r);
+        if (q * nthr + tid < C.N) atomicAdd(&cnt[cell[q]], 1);
+    }
+    for (int base = nthr * kPer; base < C.N; base += nthr * kPer) {
+        float x[kPer], y[kPer], r[kPer];
 #pragma unroll
         for (int q = 0; q < kPer; ++q) {
             const int i = base + q * nthr + tid;
             const int g = C.a0 + (i < C.N ? i : 0);
-            px[q] = st.x[g]; py[q] = st.y[g]; pr[q] = (float)st.radius[g];
+            x[q] = st.x[g]; y[q] = st.y[g]; r[q] = (float)st.radius[g];
         }
 #pragma unroll
         for (int q = 0; q < kPer; ++q)
-            if (base + q * nthr + tid < C.N) atomicAdd(&cnt[grid_cell(G, px[q] + pr[q], py[q] + pr[q])], 1);
+            if (base + q * nthr + tid < C.N) atomicAdd(&cnt[grid_cell(G, x[q] + r[q], y[q] + r[q])], 1);
     }
     __syncthreads();
-    // exclusive scan of the counts: per-thread runs of 4 cells, then a
-    // Hillis-Steele scan of the run totals
+    // exclusive scan of the counts: a run of cells per thread, the runs by wave
     const int per = (ncell + nthr - 1) / nthr;
     int run = 0;
     for (int q = 0; q < per; ++q) {
         const int c = tid * per + q;
         if (c < ncell) run += cnt[c];
     }
-    part[tid] = run;
+    const int upto = wave_scan(run);
+    if (lane == 63) part[wave] = upto;
     __syncthreads();
-    for (int o = 1; o < nthr; o <<= 1) {
-        const int v = tid >= o ? part[tid - o] : 0;
-        __syncthreads();
-        part[tid] += v;
-        __syncthreads();
-    }
-    int acc = part[tid] - run;
+    int acc = upto - run;
+    for (int w = 0; w < wave; ++w) acc += part[w];
     for (int q = 0; q < per; ++q) {
         const int c = tid * per + q;
         if (c < ncell) {
@@ -685,21 +714,25 @@ wide_grid_kernel(const VFRep* __restrict__ rp, abm_vf_state_f32 st, float cull_c
     }
     if (tid == 0) cell_start[ncell] = C.N;
     __syncthreads();
-    for (int base = 0; base < C.N; base += nthr * kPer) {
-        float px[kPer], py[kPer], pr[kPer];
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+        const int i = q * nthr + tid;
+        if (i < C.N) sorted[atomicAdd(&cnt[cell[q]], 1)] = make_float4(px[q], py[q], (float)pr[q], __int_as_float(i));
+    }
+    for (int base = nthr * kPer; base < C.N; base += nthr * kPer) {
+        float x[kPer], y[kPer], r[kPer];
 #pragma unroll
         for (int q = 0; q < kPer; ++q) {
             const int i = base + q * nthr + tid;
             const int g = C.a0 + (i < C.N ? i : 0);
-            px[q] = st.x[g]; py[q] = st.y[g]; pr[q] = (float)st.radius[g];
+            x[q] = st.x[g]; y[q] = st.y[g]; r[q] = (float)st.radius[g];
         }
 #pragma unroll
         for (int q = 0; q < kPer; ++q) {
             const int i = base + q * nthr + tid;
-            if (i < C.N) {
-                const int at = atomicAdd(&cnt[grid_cell(G, px[q] + pr[q], py[q] + pr[q])], 1);
-                sorted[at] = make_float4(px[q], py[q], pr[q], __int_as_float(i));
-            }
+            if (i < C.N)
+                sorted[atomicAdd(&cnt[grid_cell(G, x[q] + r[q], y[q] + r[q])], 1)] =
+                    make_float4(x[q], y[q], r[q], __int_as_float(i));
         }
     }
 }
