@@ -133,7 +133,7 @@ vf_step_f32_kernel(const VFRep* __restrict__ reps, const int32_t* __restrict__ o
                     S.rfast[slot] = fast_code(p.start, p.end, p.drawn, C.R);
                     if (!p.ok) continue;
                 }
-                if (p.drawn) raster(S.F, p.start, p.end, C.R);
+                if (p.drawn) raster_lds(S.F, p.start, p.end, C.R);
             }
             __syncthreads();
             // ------------------------------------- pairs re-decided in float64
@@ -149,7 +149,7 @@ vf_step_f32_kernel(const VFRep* __restrict__ reps, const int32_t* __restrict__ o
                     n_disagree += dis;
                     if (e & kEntryForced) {
                         if (count) ++n_recheck;
-                        if (r >= 0) raster(S.F, (r & 0x7fff) - 2 * C.R, ((r >> 15) & 0x7fff) - 2 * C.R, C.R);
+                        if (r >= 0) raster_lds(S.F, (r & 0x7fff) - 2 * C.R, ((r >> 15) & 0x7fff) - 2 * C.R, C.R);
                     }
                 }
                 __syncthreads();
@@ -309,7 +309,7 @@ __device__ __forceinline__ void wide_decide(const float4 o, float u1x, float u1y
         exact_pair(fx, fy, fth, fr, o.x, o.y, o.z, rp, &es, &ee, &ed);
         p.start = es; p.end = ee; p.drawn = ed != 0;
     }
-    if (p.drawn) raster(F, p.start, p.end, C.R);
+    if (p.drawn) raster_lds(F, p.start, p.end, C.R);
 }
 
 // LDS written by some lanes of a wave and read by others: in-order per
@@ -504,7 +504,7 @@ vf_step_f32_wide_kernel(const VFRep* __restrict__ rp, const RayTab32* __restrict
                 }
             }
             if (culled) continue;
-            if (p.drawn) raster(F, p.start, p.end, C.R);
+            if (p.drawn) raster_lds(F, p.start, p.end, C.R);
         }
     }
     if (!use_grid) __syncthreads();
@@ -932,7 +932,7 @@ vf_step_f32_big_kernel(const VFRep* __restrict__ reps, const int32_t* __restrict
                     pr.start = es; pr.end = ee; pr.drawn = ed != 0;
                 }
             }
-            if (pr.drawn) raster(F, pr.start, pr.end, C.R);
+            if (pr.drawn) raster_lds(F, pr.start, pr.end, C.R);
         }
         __syncthreads();
         // ---- sums over this thread's rays
