@@ -365,6 +365,8 @@ int abm_vf_batch_create(const abm_vf_replica* reps, int32_t n, abm_vf_batch** ou
                                 "hipMalloc(chain fields)");
         if (!rc && max_r <= 2048)
             rc = check_hip(hipMalloc(&bt->chain_u, sizeof(float) * 2 * (size_t)max_n), "hipMalloc(chain u)");
+        if (!rc && max_r <= 2048)
+            rc = check_hip(hipMalloc(&bt->chain_dep, kChainDepBytes * (size_t)max_n), "hipMalloc(chain dependences)");
     }
     if (!rc) {
         bt->tab_sin = bt->tab_cos + ray_total;
@@ -412,6 +414,7 @@ int abm_vf_batch_destroy(abm_vf_batch* b) {
     if (b->grid_start) (void)hipFree(b->grid_start);
     if (b->chain_fields) (void)hipFree(b->chain_fields);
     if (b->chain_u) (void)hipFree(b->chain_u);
+    if (b->chain_dep) (void)hipFree(b->chain_dep);
     if (b->grid_param) (void)hipFree(b->grid_param);
     for (GroupPlan& gp : b->gplan) {
         if (gp.groups) (void)hipFree(gp.groups);
@@ -511,6 +514,7 @@ int abm_vf_set_launch(abm_vf_batch* b, int32_t waves) {
         if (!rc && !b->chain_fields)
             rc = check_hip(hipMalloc(&b->chain_fields, sizeof(uint32_t) * n * words), "hipMalloc(chain fields)");
         if (!rc && !b->chain_u) rc = check_hip(hipMalloc(&b->chain_u, sizeof(float) * 2 * n), "hipMalloc(chain u)");
+        if (!rc && !b->chain_dep) rc = check_hip(hipMalloc(&b->chain_dep, kChainDepBytes * n), "hipMalloc(chain dependences)");
         if (rc) return rc;
     }
     b->waves_per_group = waves;

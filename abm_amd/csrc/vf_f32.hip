@@ -1609,19 +1609,70 @@ __device__ inline void chain_barrier() {
 // need not wait for each other: agent m waits only for the agents j < m whose new
 // pose it can see, those within the cut-off plus j's margin of its start pose
 // (a displacement beyond the margin is detected, and the segment taken again in id
-// order).  The kernel lists these dependences first (dep, pend) and, where they are
-// few (kFlowShare), runs them as they come free: each wave takes the next ready
+// order).  A kernel of its own lists these dependences (dep, pend) and, where they are
+// few (kFlowShare), a segment runs them as they come free: each wave takes the next ready
 // agent, sums and moves it, decides its new pose for its dependents and counts
 // them down.  The same fields and moves, in another order.  Bound by the longest
 // path of dependences times an agent's latency (about 4 thousand cycles), where
 // the id order takes 2.5 thousand cycles for every agent.  Measured, a step, id
 // order and this: 8192 agents, a twelfth of the others in sight, R = 2048, 9.12
-// and 3.77 ms (32 segments of 106 us: 5 to load, 11 to list the dependences, 90); 2100 agents with walls at R = 2048, a third in sight 2.98 and 2.11,
-// 0.7 3.94 and 3.64, 0.85 4.48 and 4.92 (hence kFlowShare, looked at after a
-// sample of the agents first, since listing them all costs 2 % of such a step).
+// and 3.47 ms; 2100 agents with walls at R = 2048, a third in sight 2.98 and 2.02,
+// 0.7 3.94 and 3.49, 0.85 4.48 and 4.92 (hence kFlowShare).
 constexpr float kFlowMargin = 16.f;   // + 4 |v|: the displacement allowed for
 constexpr float kFlowShare = 0.7f;    // of a segment's pairs that may depend
 constexpr int kFlowSpins = 1 << 20;   // waits end (the dependences are acyclic); the bound is never met
+
+constexpr int kDepWords = kChainSeg / 64;
+static_assert(kChainDepBytes == 8 * kDepWords + 4, "an agent's dependences");
+
+// The dependences of every agent inside its segment, from the start poses: the
+// later agents that wait for it (dep), and how many earlier ones it waits for
+// (pend; negative, all bits inverted: on a torus too small for the nearest image
+// alone to matter).  One wave per agent over the whole GPU, since no segment's
+// moves change it: 5 us for 8192 agents, where each segment's own workgroup took
+// 11 us for 256 (a step of 3.78 ms then, 3.47 now).
+__global__ void __launch_bounds__(256)
+vf_step_f32_depend_kernel(const VFRep* __restrict__ rp, abm_vf_state_f32 st, float cull_c,
+                          uint64_t* __restrict__ dep, int32_t* __restrict__ pend) {
+    const RepConst C = rep_const(rp);
+    const int lane = threadIdx.x & 63;
+    const int a = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
+    if (a >= C.N) return;   // whole waves, no barrier below
+    const int s0 = a / kChainSeg * kChainSeg, n = min(kChainSeg, C.N - s0), al = a - s0;
+    float x[kDepWords], y[kDepWords], lim[kDepWords];   // centres, reach of a new pose
+    float ax = 0.f, ay = 0.f, alim = 0.f;               // agent a's
+#pragma unroll
+    for (int c = 0; c < kDepWords; ++c) {
+        const int i = 64 * c + lane, g = C.a0 + s0 + min(i, n - 1);
+        const float r = (float)st.radius[g];
+        x[c] = st.x[g] + r;
+        y[c] = st.y[g] + r;
+        lim[c] = r * cull_c + (kFlowMargin + 4.f * fabsf(st.v[g])) + 1.f;
+        if (c == al >> 6) {
+            ax = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(x[c]), al & 63));
+            ay = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(y[c]), al & 63));
+            alim = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(lim[c]), al & 63));
+        }
+    }
+    int waits = 0;
+    uint64_t mine = 0;
+#pragma unroll
+    for (int c = 0; c < kDepWords; ++c) {
+        const int i = 64 * c + lane;
+        float dx = fabsf(ax - x[c]), dy = fabsf(ay - y[c]);
+        if (C.torus) {   // to the nearest image
+            dx = fminf(dx, fabsf(C.fW - dx));
+            dy = fminf(dy, fabsf(C.fH - dy));
+        }
+        const float d2 = fmaf(dy, dy, dx * dx);
+        const uint64_t after = __ballot(i > al && i < n && !(d2 > alim * alim));
+        waits += (int)__popcll(__ballot(i < al && !(d2 > lim[c] * lim[c])));
+        if (lane == c) mine = after;
+    }
+    if (lane < kDepWords) dep[(size_t)a * kDepWords + lane] = mine;
+    const bool tight = C.torus && !(fminf(C.hw, C.hh) - C.tguard > alim);
+    if (lane == 0) pend[a] = tight ? ~waits : waits;
+}
 
 template <int RPL, bool PLAIN>   // PLAIN: as the push kernel's
 __global__ void __launch_bounds__(kChainThreads)
@@ -1629,6 +1680,7 @@ vf_step_f32_segment_kernel(const VFRep* __restrict__ rp, const RayTab32* __restr
                            abm_vf_state_f32 st, const uint32_t* __restrict__ fields,
                            const float2* __restrict__ ustart, uint32_t* __restrict__ bits_out,
                            float* __restrict__ diag, uint32_t flags, unsigned long long* __restrict__ counters,
+                           const uint64_t* __restrict__ dep_all, const int32_t* __restrict__ pend_all,
                            float cull_c, int s0, int n) {
     __shared__ uint32_t rows[kChainSeg][64];
     __shared__ float4 srec[kChainSeg];     // start poses (x, y, radius, theta)
@@ -1639,7 +1691,7 @@ vf_step_f32_segment_kernel(const VFRep* __restrict__ rp, const RayTab32* __restr
     __shared__ int dirty[2];               // the pair (k, k - 1) drew after k's sums were taken
     __shared__ uint16_t cq[2][kChainCullWaves][kChainSeg];   // listed rows, by step parity and cull wave
     __shared__ int cn[2][kChainCullWaves];
-    __shared__ uint64_t dep[kChainSeg][kChainSeg / 64];      // agents that wait for an agent
+    __shared__ uint64_t dep[kChainSeg][kDepWords];           // agents that wait for an agent
     __shared__ int pend[kChainSeg];                          // agents it waits for
     __shared__ int ready[kChainSeg];                         // in the order they come free (-1: not yet)
     __shared__ uint16_t after[kChainWaves][kChainSeg];       // the dependents of a wave's agent
@@ -1675,7 +1727,7 @@ vf_step_f32_segment_kernel(const VFRep* __restrict__ rp, const RayTab32* __restr
     if (tid < 2) dirty[tid] = 0;
     const bool may_flow = !count && !verify;
     if (tid < 4) ctl[tid] = 0;
-    for (int i = tid; i < kChainSeg; i += kChainThreads) { pend[i] = 0; ready[i] = -1; }
+    for (int i = tid; i < kChainSeg; i += kChainThreads) ready[i] = -1;
     // in a summing wave (wave 1, or all) lane l owns rays [l RPL, (l + 1) RPL) and
     // their table entries, which come through the rows' LDS (read from global
     // memory lane by lane they took 25 thousand cycles for eight waves)
@@ -1717,77 +1769,21 @@ vf_step_f32_segment_kernel(const VFRep* __restrict__ rp, const RayTab32* __restr
         }
     };
     bool flow = false;
-    if (may_flow) {   // uniform
-        // ---- the dependences: wave w the agents j = w mod 8, lanes over the later ones
-        float fx[kChainSeg / 64], fy[kChainSeg / 64];   // centres
-        int waits[kChainSeg / 64];
-#pragma unroll
-        for (int c = 0; c < kChainSeg / 64; ++c) {
-            const int m = 64 * c + lane;
-            fx[c] = m < n ? srec[m].x + srec[m].z : 1e30f;   // out of sight
-            fy[c] = m < n ? srec[m].y + srec[m].z : 1e30f;
-            waits[c] = 0;
+    if (may_flow) {   // uniform: the dependences, and whether they are few
+        uint64_t* flat = &dep[0][0];
+        for (int w = tid; w < n * kDepWords; w += kChainThreads) flat[w] = dep_all[(size_t)s0 * kDepWords + w];
+        int waits = 0;
+        for (int m = tid; m < n; m += kChainThreads) {
+            const int q = pend_all[s0 + m];
+            waits = q < 0 ? ~q : q;
+            pend[m] = waits;
+            if (q < 0) ctl[3] = 1;
         }
-        int total = 0;   // wave-uniform
-        bool tight = false;   // a torus too small for the nearest image alone to matter
-        static_assert(kChainSeg <= 64 * kChainWaves, "a lane per agent of a wave's share");
-        float jx = 0.f, jy = 0.f, jlim = 0.f;   // lane q: agent wave + 8 q, its reach
-        if (wave + kChainWaves * lane < n) {
-            const float4 o = srec[wave + kChainWaves * lane];
-            jx = o.x + o.z;
-            jy = o.y + o.z;
-            const float lim = o.z * cull_c + margin(sdyn[wave + kChainWaves * lane].x) + 1.f;
-            jlim = lim * lim;
-            tight = C.torus && !(fminf(C.hw, C.hh) - C.tguard > lim);
-        }
-        tight = __ballot(tight) != 0;
-        auto depend = [&](int q) {
-            const int j = wave + kChainWaves * q;
-            const float ox = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(jx), q));
-            const float oy = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(jy), q));
-            const float lim2 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(jlim), q));
-            uint64_t mk[kChainSeg / 64];
-#pragma unroll
-            for (int c = 0; c < kChainSeg / 64; ++c) {
-                mk[c] = 0;
-                if (64 * c + 63 <= j) continue;   // (uniform)
-                float dx = fabsf(ox - fx[c]), dy = fabsf(oy - fy[c]);
-                if (C.torus) {   // to the nearest image
-                    dx = fminf(dx, fabsf(C.fW - dx));
-                    dy = fminf(dy, fabsf(C.fH - dy));
-                }
-                const bool near = 64 * c + lane > j && !(fmaf(dy, dy, dx * dx) > lim2);
-                mk[c] = __ballot(near);
-                waits[c] += near ? 1 : 0;
-                total += __builtin_amdgcn_readfirstlane((int)__popcll(mk[c]));
-            }
-            if (lane < kChainSeg / 64) {
-                uint64_t mine = mk[0];
-#pragma unroll
-                for (int c = 1; c < kChainSeg / 64; ++c) mine = lane == c ? mk[c] : mine;
-                dep[j][lane] = mine;
-            }
-        };
-        auto tally = [&]() {
-            if (lane == 0) {
-                atomicAdd(&ctl[2], total);
-                if (tight) ctl[3] = 1;
-            }
-            total = 0;
-            __syncthreads();
-            return ctl[3] == 0;
-        };
-        const int n1 = min(n, 2 * kChainWaves);   // a sample first
-        for (int q = 0; wave + kChainWaves * q < n1; ++q) depend(q);
-        flow = tally() && ctl[2] <= kFlowShare * n1 * (n - n1 / 2);
-        if (flow) {   // uniform
-            __syncthreads();
-            for (int q = n1 / kChainWaves; wave + kChainWaves * q < n; ++q) depend(q);
-#pragma unroll
-            for (int c = 0; c < kChainSeg / 64; ++c)
-                if (waits[c]) atomicAdd(&pend[64 * c + lane], waits[c]);
-            flow = tally() && ctl[2] <= kFlowShare * n * n / 2;
-        }
+        static_assert(kChainSeg <= kChainThreads, "an agent a thread");
+        const int total = wave_scan(waits);
+        if (lane == 63 && total > 0) atomicAdd(&ctl[2], total);
+        __syncthreads();
+        flow = ctl[3] == 0 && ctl[2] <= kFlowShare * n * n / 2;
     }
     if (flow) {
         for (int m = tid; m < n; m += kChainThreads)
@@ -1814,7 +1810,7 @@ vf_step_f32_segment_kernel(const VFRep* __restrict__ rp, const RayTab32* __restr
             // its dependents, the first 64 to registers before the sums
             int cnt = 0;   // wave-uniform
 #pragma unroll
-            for (int c = 0; c < kChainSeg / 64; ++c) {
+            for (int c = 0; c < kDepWords; ++c) {
                 const uint64_t mk = dep[m][c];
                 if ((mk >> lane) & 1ull)
                     after[wave][cnt + (int)__popcll(mk & ((1ull << lane) - 1ull))] = (uint16_t)(64 * c + lane);
@@ -2100,7 +2096,7 @@ int launch_chain_start(abm_vf_batch* b, const abm_vf_state_f32* st, uint32_t fla
 // whether it does by default: every replica above kWideThreshold agents (a
 // single large flock).
 bool chain_ready(const abm_vf_batch* b) {
-    return b->chain_fields != nullptr && b->chain_u != nullptr && b->grid_sorted != nullptr &&
+    return b->chain_fields != nullptr && b->chain_u != nullptr && b->chain_dep != nullptr && b->grid_sorted != nullptr &&
            b->grid_start != nullptr && b->grid_param != nullptr && b->n_replicas > 0 && b->max_rays <= 2048;
 }
 bool chain_fits(const abm_vf_batch* b) { return chain_ready(b) && b->min_agents > kWideThreshold; }
@@ -2124,6 +2120,13 @@ int launch_chain(abm_vf_batch* b, const abm_vf_state_f32* st, uint32_t* bits, fl
         else if (need <= 16) rc = launch_chain_start<16>(b, st, flags, s, rep, cull_c, N);
         else rc = launch_chain_start<32>(b, st, flags, s, rep, cull_c, N);
         if (rc) return rc;
+        uint64_t* dep = (uint64_t*)b->chain_dep;
+        int32_t* pend = (int32_t*)(dep + (size_t)b->max_agents * kDepWords);
+        if (!counting) {
+            hipLaunchKernelGGL(vf_step_f32_depend_kernel, dim3((N + 3) / 4), dim3(256), 0, s, b->reps_dev + rep, *st,
+                               cull_c, dep, pend);
+            if (int rc2 = check_hip(hipGetLastError(), "vf_step_f32_depend_kernel launch")) return rc2;
+        }
         for (int s0 = 0; s0 < N; s0 += kChainSeg) {
             const int n = std::min(kChainSeg, N - s0);
             // rays per lane of the summing wave: the push kernel's rule for the batch
@@ -2133,7 +2136,8 @@ int launch_chain(abm_vf_batch* b, const abm_vf_state_f32* st, uint32_t* bits, fl
                                   : vf_step_f32_segment_kernel<RPLV, false>),                               \
                            dim3(1), dim3(kChainThreads), 0, s,                                              \
                            b->reps_dev + rep, b->tab32, *st, (const uint32_t*)b->chain_fields,             \
-                           (const float2*)b->chain_u, bits, diag, flags, b->counters, cull_c, s0, n);
+                           (const float2*)b->chain_u, bits, diag, flags, b->counters, (const uint64_t*)dep,        \
+                           (const int32_t*)pend, cull_c, s0, n);
             ABM_SEGMENT(4) ABM_SEGMENT(8) ABM_SEGMENT(16) ABM_SEGMENT(32)
 #undef ABM_SEGMENT
             if (int rc2 = check_hip(hipGetLastError(), "vf_step_f32_segment_kernel launch")) return rc2;
