@@ -63,8 +63,9 @@ struct GroupPlan {
 // kernel) updates them, the per-replica kernel the rest.
 constexpr int kBigClass = 64;
 
-// Bytes of an agent's dependences in the chain step (its segment's 256 bits and a count).
-constexpr size_t kChainDepBytes = 36;
+// Bytes of an agent's dependences in the chain step (64 indices, its segment's
+// 256 bits and a count).
+constexpr size_t kChainDepBytes = 100;
 
 // The push kernel (one workgroup of 8 waves per replica): rays per lane of
 // its summing wave for a launch whose largest R is r (the one-wave
@@ -127,7 +128,7 @@ struct abm_vf_batch {
     void* grid_param = nullptr;     // wide step: the grid of the current replica (WideGrid)
     uint32_t* chain_fields = nullptr;   // chain step: every agent's field (max_agents x words)
     void* chain_u = nullptr;        // chain step: start heading vectors (float2 per agent)
-    void* chain_dep = nullptr;      // chain step: dependences (four 64-bit words and an int32 per agent)
+    void* chain_dep = nullptr;      // chain step: dependences (64 bytes, four 64-bit words, an int32 per agent)
     int32_t min_agents = 0;         // of the smallest replica
     abm::GroupPlan gplan[3];        // G = 1, 2, 4
     // host copies

@@ -1613,27 +1613,28 @@ __device__ inline void chain_barrier() {
 // few (kFlowShare), a segment runs them as they come free: each wave takes the next ready
 // agent, sums and moves it, decides its new pose for its dependents and counts
 // them down.  The same fields and moves, in another order.  Bound by the longest
-// path of dependences times an agent's latency (about 4 thousand cycles), where
+// path of dependences times an agent's latency (about 5 thousand cycles), where
 // the id order takes 2.5 thousand cycles for every agent.  Measured, a step, id
 // order and this: 8192 agents, a twelfth of the others in sight, R = 2048, 9.12
-// and 3.47 ms; 2100 agents with walls at R = 2048, a third in sight 2.98 and 2.02,
-// 0.7 3.94 and 3.49, 0.85 4.48 and 4.92 (hence kFlowShare).
+// and 3.29 ms; 2100 agents with walls at R = 2048, a third in sight 2.98 and 1.93,
+// 0.7 3.94 and 3.47, 0.85 4.48 and 4.92 (hence kFlowShare).
 constexpr float kFlowMargin = 16.f;   // + 4 |v|: the displacement allowed for
 constexpr float kFlowShare = 0.7f;    // of a segment's pairs that may depend
 constexpr int kFlowSpins = 1 << 20;   // waits end (the dependences are acyclic); the bound is never met
 
 constexpr int kDepWords = kChainSeg / 64;
-static_assert(kChainDepBytes == 8 * kDepWords + 4, "an agent's dependences");
+static_assert(kChainDepBytes == 64 + 8 * kDepWords + 4, "an agent's dependences");
 
 // The dependences of every agent inside its segment, from the start poses: the
-// later agents that wait for it (dep), and how many earlier ones it waits for
-// (pend; negative, all bits inverted: on a torus too small for the nearest image
+// later agents that wait for it (dep, and the first 64 of them by index: first), and
+// how many earlier ones it waits for (pend; negative, all bits inverted: on a torus too small for the nearest image
 // alone to matter).  One wave per agent over the whole GPU, since no segment's
-// moves change it: 5 us for 8192 agents, where each segment's own workgroup took
-// 11 us for 256 (a step of 3.78 ms then, 3.47 now).
+// moves change it: 6 us for 8192 agents, where each segment's own workgroup took
+// 11 us for 256 (a step of 3.78 ms then, 3.47 after; 3.29 with the indices, whose
+// agents then load in one go, where a wave made its list from the bits).
 __global__ void __launch_bounds__(256)
 vf_step_f32_depend_kernel(const VFRep* __restrict__ rp, abm_vf_state_f32 st, float cull_c,
-                          uint64_t* __restrict__ dep, int32_t* __restrict__ pend) {
+                          uint8_t* __restrict__ first, uint64_t* __restrict__ dep, int32_t* __restrict__ pend) {
     const RepConst C = rep_const(rp);
     const int lane = threadIdx.x & 63;
     const int a = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
@@ -1654,7 +1655,7 @@ vf_step_f32_depend_kernel(const VFRep* __restrict__ rp, abm_vf_state_f32 st, flo
             alim = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(lim[c]), al & 63));
         }
     }
-    int waits = 0;
+    int waits = 0, cnt = 0;
     uint64_t mine = 0;
 #pragma unroll
     for (int c = 0; c < kDepWords; ++c) {
@@ -1668,7 +1669,11 @@ vf_step_f32_depend_kernel(const VFRep* __restrict__ rp, abm_vf_state_f32 st, flo
         const uint64_t after = __ballot(i > al && i < n && !(d2 > alim * alim));
         waits += (int)__popcll(__ballot(i < al && !(d2 > lim[c] * lim[c])));
         if (lane == c) mine = after;
+        const int at = cnt + (int)__popcll(after & ((1ull << lane) - 1ull));
+        if (((after >> lane) & 1ull) && at < 64) first[(size_t)a * 64 + at] = (uint8_t)i;
+        cnt += (int)__popcll(after);
     }
+    if (lane >= cnt) first[(size_t)a * 64 + lane] = 0;   // (not used)
     if (lane < kDepWords) dep[(size_t)a * kDepWords + lane] = mine;
     const bool tight = C.torus && !(fminf(C.hw, C.hh) - C.tguard > alim);
     if (lane == 0) pend[a] = tight ? ~waits : waits;
@@ -1680,7 +1685,7 @@ vf_step_f32_segment_kernel(const VFRep* __restrict__ rp, const RayTab32* __restr
                            abm_vf_state_f32 st, const uint32_t* __restrict__ fields,
                            const float2* __restrict__ ustart, uint32_t* __restrict__ bits_out,
                            float* __restrict__ diag, uint32_t flags, unsigned long long* __restrict__ counters,
-                           const uint64_t* __restrict__ dep_all, const int32_t* __restrict__ pend_all,
+                           const uint8_t* __restrict__ first_all, const uint64_t* __restrict__ dep_all, const int32_t* __restrict__ pend_all,
                            float cull_c, int s0, int n) {
     __shared__ uint32_t rows[kChainSeg][64];
     __shared__ float4 srec[kChainSeg];     // start poses (x, y, radius, theta)
@@ -1692,9 +1697,10 @@ vf_step_f32_segment_kernel(const VFRep* __restrict__ rp, const RayTab32* __restr
     __shared__ uint16_t cq[2][kChainCullWaves][kChainSeg];   // listed rows, by step parity and cull wave
     __shared__ int cn[2][kChainCullWaves];
     __shared__ uint64_t dep[kChainSeg][kDepWords];           // agents that wait for an agent
+    __shared__ uint32_t first[kChainSeg][16];                // the first 64 of them, a byte each
     __shared__ int pend[kChainSeg];                          // agents it waits for
     __shared__ int ready[kChainSeg];                         // in the order they come free (-1: not yet)
-    __shared__ uint16_t after[kChainWaves][kChainSeg];       // the dependents of a wave's agent
+    __shared__ uint16_t after[kChainWaves][kChainSeg];       // all dependents of a wave's agent (beyond 64)
     __shared__ int ctl[4];                                   // next to take, free so far, dependences, out of bounds
     const RepConst C = rep_const(rp);
     const int tid = threadIdx.x, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
@@ -1772,6 +1778,8 @@ vf_step_f32_segment_kernel(const VFRep* __restrict__ rp, const RayTab32* __restr
     if (may_flow) {   // uniform: the dependences, and whether they are few
         uint64_t* flat = &dep[0][0];
         for (int w = tid; w < n * kDepWords; w += kChainThreads) flat[w] = dep_all[(size_t)s0 * kDepWords + w];
+        const uint32_t* lists = reinterpret_cast<const uint32_t*>(first_all) + (size_t)s0 * 16;
+        for (int w = tid; w < n * 16; w += kChainThreads) (&first[0][0])[w] = lists[w];
         int waits = 0;
         for (int m = tid; m < n; m += kChainThreads) {
             const int q = pend_all[s0 + m];
@@ -1808,16 +1816,11 @@ vf_step_f32_segment_kernel(const VFRep* __restrict__ rp, const RayTab32* __restr
             const int gk = C.a0 + s0 + m;
             const float4 pk = srec[m], dk = sdyn[m];
             // its dependents, the first 64 to registers before the sums
+            int mm = reinterpret_cast<const uint8_t*>(first[m])[lane];
             int cnt = 0;   // wave-uniform
 #pragma unroll
-            for (int c = 0; c < kDepWords; ++c) {
-                const uint64_t mk = dep[m][c];
-                if ((mk >> lane) & 1ull)
-                    after[wave][cnt + (int)__popcll(mk & ((1ull << lane) - 1ull))] = (uint16_t)(64 * c + lane);
-                cnt += (int)__popcll(mk);
-            }
-            wave_lds_sync();
-            int mm = lane < cnt ? after[wave][lane] : m;
+            for (int c = 0; c < kDepWords; ++c) cnt += (int)__popcll(dep[m][c]);
+            if (lane >= cnt) mm = m;
             float4 fm = srec[mm];
             float2 um = su[mm];
             double Sv, Sp, Bc, Bs, Ec, Es;
@@ -1845,6 +1848,18 @@ vf_step_f32_segment_kernel(const VFRep* __restrict__ rp, const RayTab32* __restr
                     dd[4] = C.phi_ok ? (float)((double)dk.z * -Bs) : 0.f;
                     dd[5] = C.phi_ok ? (float)((double)(dk.z * C.bet1) * Es) : 0.f;
                 }
+            }
+            cnt = __builtin_amdgcn_readfirstlane(cnt);
+            if (cnt > 64) {
+                int at = 0;
+#pragma unroll
+                for (int c = 0; c < kDepWords; ++c) {
+                    const uint64_t mk = dep[m][c];
+                    if ((mk >> lane) & 1ull)
+                        after[wave][at + (int)__popcll(mk & ((1ull << lane) - 1ull))] = (uint16_t)(64 * c + lane);
+                    at += (int)__popcll(mk);
+                }
+                wave_lds_sync();
             }
             for (int e = lane; e < cnt; e += 64) {
                 if (e >= 64) {
@@ -2120,11 +2135,12 @@ int launch_chain(abm_vf_batch* b, const abm_vf_state_f32* st, uint32_t* bits, fl
         else if (need <= 16) rc = launch_chain_start<16>(b, st, flags, s, rep, cull_c, N);
         else rc = launch_chain_start<32>(b, st, flags, s, rep, cull_c, N);
         if (rc) return rc;
-        uint64_t* dep = (uint64_t*)b->chain_dep;
+        uint8_t* first = (uint8_t*)b->chain_dep;
+        uint64_t* dep = (uint64_t*)(first + (size_t)b->max_agents * 64);
         int32_t* pend = (int32_t*)(dep + (size_t)b->max_agents * kDepWords);
         if (!counting) {
             hipLaunchKernelGGL(vf_step_f32_depend_kernel, dim3((N + 3) / 4), dim3(256), 0, s, b->reps_dev + rep, *st,
-                               cull_c, dep, pend);
+                               cull_c, first, dep, pend);
             if (int rc2 = check_hip(hipGetLastError(), "vf_step_f32_depend_kernel launch")) return rc2;
         }
         for (int s0 = 0; s0 < N; s0 += kChainSeg) {
@@ -2136,7 +2152,8 @@ int launch_chain(abm_vf_batch* b, const abm_vf_state_f32* st, uint32_t* bits, fl
                                   : vf_step_f32_segment_kernel<RPLV, false>),                               \
                            dim3(1), dim3(kChainThreads), 0, s,                                              \
                            b->reps_dev + rep, b->tab32, *st, (const uint32_t*)b->chain_fields,             \
-                           (const float2*)b->chain_u, bits, diag, flags, b->counters, (const uint64_t*)dep,        \
+                           (const float2*)b->chain_u, bits, diag, flags, b->counters, (const uint8_t*)first,       \
+                           (const uint64_t*)dep,                                                            \
                            (const int32_t*)pend, cull_c, s0, n);
             ABM_SEGMENT(4) ABM_SEGMENT(8) ABM_SEGMENT(16) ABM_SEGMENT(32)
 #undef ABM_SEGMENT
