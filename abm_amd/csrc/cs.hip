@@ -209,8 +209,9 @@ __device__ inline CSFocal cs_focal(const CSArgs& A, int f) {
     F.cy = F.py + F.radius;
     double sn, cs;
     if (!f32::sincos_f64_small(F.theta, &sn, &cs)) sincos(F.theta, &sn, &cs);
-    F.ux = (float)cs;
-    F.uy = -(float)sn;
+    const bool kept = heading_kept(F.px, F.py, F.radius);   // else NaN, which no guard lets through
+    F.ux = kept ? (float)cs : NAN;
+    F.uy = kept ? -(float)sn : NAN;
     return F;
 }
 

@@ -116,6 +116,15 @@ ABM_HD Focal make_focal(double px, double py, double theta, double radius) {
     return f;
 }
 
+// Whether unit(v1) is the heading (cos th, -sin th) to within 1e-6 rad.  The
+// reference forms v1 from the agent's position (make_focal), so it loses the
+// heading in the position's rounding, an angle of about 2e-16 |position| /
+// radius: below 6e-7 up to 3e9 radii, but bins apart from the heading at 1e11.
+// At radius 0 it has none, and at a negative one the opposite.
+ABM_HD bool heading_kept(double px, double py, double radius) {
+    return radius > 0.0 && fabs(px) <= 1e9 * radius && fabs(py) <= 1e9 * radius;
+}
+
 // Raster decision of one object for the VSWRM field (vf_supcalc.py:55-119).
 struct PairVF {
     int skipped;       // coincident positions (:57)

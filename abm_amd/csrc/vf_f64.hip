@@ -197,7 +197,8 @@ vf_step_f64_kernel(const VFRep* __restrict__ reps, const double* __restrict__ tc
 // the float32 angle is within 1e-6 rad of the exact one and the guard bands of
 // the fused kernels (4e-6 rad around a bin tie and the +-pi wrap, 4e-6 relative
 // + 1e-6 around an integer half-width) cover it and the reference's own error
-// (vf_f32_common.hpp).  About 1 pair in 1000 takes the replica.
+// (vf_f32_common.hpp).  About 1 pair in 1000 takes the replica, and every pair of
+// a focal agent whose heading the reference loses (heading_kept).
 //
 // One workgroup of NW waves per replica, largest first.  Lanes over objects
 // decide and OR each interval into a bit-packed field in LDS; every lane owns
@@ -335,7 +336,8 @@ vf_step_f64_guard_kernel(const VFRep* __restrict__ reps, const int32_t* __restri
         S.b0[i] = st.bet0 ? st.bet0[g] : rp->bet0;
         S.v0[i] = st.v0 ? st.v0[g] : rp->v0;
         const double2 sc = sincos_f64(th);
-        S.u[i] = make_float2((float)sc.y, -(float)sc.x);   // unit(v1) = (cos th, -sin th)
+        // unit(v1) = (cos th, -sin th), or NaN, which no guard lets through
+        S.u[i] = heading_kept(S.x[i], S.y[i], (double)S.rad[i]) ? make_float2((float)sc.y, -(float)sc.x) : make_float2(NAN, NAN);
         if (sync_order) { S.ox[i] = S.x[i]; S.oy[i] = S.y[i]; }
     }
     const bool torus = rp->boundary == ABM_BOUNDARY_INFINITE;
