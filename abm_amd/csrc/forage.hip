@@ -24,6 +24,7 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <utility>
 #include <vector>
 
 #include "../../include/abm_amd.h"
@@ -3280,9 +3281,9 @@ int wide_updates(const abm_forage_batch* bt, int64_t* total) {
     return ABM_OK;
 }
 
-// The wide replicas' chunks and scratch, laid out once per plan.
+// The wide replicas' chunks and scratch, laid out once per plan.  bt->wide_mem is
+// a new allocation; the one before it stays its caller's.
 int plan_wide(abm_forage_batch* bt) {
-    if (bt->wide_mem) (void)hipFree(bt->wide_mem);
     bt->wide_mem = nullptr;
     bt->wide_chunks = 0;
     bt->wide_keys = 0;
@@ -3346,7 +3347,12 @@ size_t wide_world_carve(void* base, const abm_forage_world* w, WideWorld* m) {
 // 0.093, 100 of 8 to 512 0.064 and 0.113; 300 of 100 0.085 and 0.074, 1000 of 8
 // to 512 0.226 and 0.148).  A kernel's blocks take their replicas
 // largest first (the cost grows with the agents; rays add to each agent's).
-int plan_paths(abm_forage_batch* bt, int path) {
+int plan_paths(abm_forage_batch* batch, int path) {
+    // updates counted so far, and no launch left on the scratch that goes
+    int64_t made = 0;
+    if (int rc = wide_updates(batch, &made)) return rc;
+    // the plan is made beside the one in use and takes its place when it is whole
+    abm_forage_batch plan = *batch, *bt = &plan;
     const int n = bt->n_replicas;
     std::vector<int32_t> plain, occl, crowd, big;
     int64_t agents = 0;
@@ -3383,15 +3389,19 @@ int plan_paths(abm_forage_batch* bt, int path) {
     extent(plain, bt->n_plain, bt->plain_max_agents, bt->plain_max_rays);
     extent(occl, bt->n_occl, bt->occl_max_agents, bt->occl_max_rays);
     extent(crowd, bt->n_crowd, bt->crowd_max_agents, bt->crowd_max_rays);
-    // updates counted so far, and no launch left on the scratch that goes
-    int64_t made = 0;
-    if (int rc = wide_updates(bt, &made)) return rc;
     bt->wide_steps += made;
     bt->wide = big;
     bt->path = path;
-    if (int rc = plan_wide(bt)) return rc;
-    return check_hip(hipMemcpy(bt->order_dev, bt->order_host.data(), sizeof(int32_t) * n,
-                               hipMemcpyHostToDevice), "upload forage order");
+    int rc = plan_wide(bt);
+    if (!rc) rc = check_hip(hipMemcpy(bt->order_dev, bt->order_host.data(), sizeof(int32_t) * n,
+                                      hipMemcpyHostToDevice), "upload forage order");
+    if (rc) {
+        if (bt->wide_mem) (void)hipFree(bt->wide_mem);
+        return rc;
+    }
+    if (batch->wide_mem) (void)hipFree(batch->wide_mem);
+    *batch = std::move(plan);
+    return ABM_OK;
 }
 
 // Waves of the update kernel's workgroups: sixteen, so that a large replica's
@@ -3421,6 +3431,7 @@ int check_state(const abm_forage_state* st, const char* who) {
 int launch_wide(abm_forage_batch* b, const abm_forage_state* st, const double* uniforms,
                 const uint32_t* words, const int64_t* offset, const int32_t* count, int32_t* used,
                 int32_t* status, uint32_t* field_bits, hipStream_t s, abm_mt19937_state* mt) {
+    if (!b->wide_mem) return set_error(ABM_ERR_HIP, "forage update over the whole GPU: no scratch");
     WideMem m;
     const int n = (int)b->wide.size(), chunks = b->wide_chunks, W = (b->wide_max_rays + 31) / 32;
     wide_carve(b->wide_mem, n, chunks, (size_t)b->wide_keys, &m);
