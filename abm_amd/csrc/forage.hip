@@ -3238,7 +3238,7 @@ namespace {
 
 constexpr int kForageMaxAgents = 65536;
 constexpr int kWideMaxRays = 8192;   // of the update over the whole GPU
-constexpr int kWideMinAgents = 64, kWideMaxPerCu = 96;   // where it is the better one (plan_paths)
+constexpr int kWideMinAgents = 64, kWideMaxPerCu = 96;   // where it is the better one (plan_classes)
 
 // Generator keys a step may twist to while making 2M words.
 int wide_key_slots(int M) { return (2 * M + kMtN) / kMtN + 1; }
@@ -3265,51 +3265,57 @@ size_t wide_carve(void* base, size_t reps, size_t chunks, size_t key_words, Wide
     return at;
 }
 
-// Updates the wide replicas' move kernels have made since the plan.
+WideMem wide_mem(const WidePlan& w) {
+    WideMem m;
+    wide_carve(w.mem, w.reps.size(), (size_t)w.chunks, (size_t)w.keys, &m);
+    return m;
+}
+
+// Updates the wide replicas' move kernels have made.
 int wide_updates(const abm_forage_batch* bt, int64_t* total) {
     *total = 0;
-    if (!bt->wide_mem) return ABM_OK;
-    WideMem m;
-    const size_t n = bt->wide.size();
-    wide_carve(bt->wide_mem, n, (size_t)bt->wide_chunks, (size_t)bt->wide_keys, &m);
-    std::vector<int32_t> ctl(kWdWords * n);
-    if (int rc = check_hip(hipDeviceSynchronize(), "hipDeviceSynchronize")) return rc;
-    if (int rc = check_hip(hipMemcpy(ctl.data(), m.ctl, sizeof(int32_t) * ctl.size(), hipMemcpyDeviceToHost),
-                           "read wide control"))
-        return rc;
-    for (size_t i = 0; i < n; ++i) *total += ctl[kWdWords * i + kWdUpdates];
+    for (const WidePlan& w : bt->wide) {
+        if (!w.mem) continue;
+        std::vector<int32_t> ctl(kWdWords * w.reps.size());
+        if (int rc = check_hip(hipDeviceSynchronize(), "hipDeviceSynchronize")) return rc;
+        if (int rc = check_hip(hipMemcpy(ctl.data(), wide_mem(w).ctl, sizeof(int32_t) * ctl.size(),
+                                         hipMemcpyDeviceToHost), "read wide control"))
+            return rc;
+        for (size_t i = 0; i < w.reps.size(); ++i) *total += ctl[kWdWords * i + kWdUpdates];
+    }
     return ABM_OK;
 }
 
-// The wide replicas' chunks and scratch, laid out once per plan.  bt->wide_mem is
-// a new allocation; the one before it stays its caller's.
-int plan_wide(abm_forage_batch* bt) {
-    bt->wide_mem = nullptr;
-    bt->wide_chunks = 0;
-    bt->wide_keys = 0;
-    bt->wide_max_rays = 0;
-    if (bt->wide.empty()) return ABM_OK;
+// The scratch of a plan, made whole before the plan has it.
+int make_wide(const abm_forage_batch* bt, WidePlan& w) {
+    if (w.mem || w.reps.empty()) return ABM_OK;
     std::vector<WideRep> rep;
     std::vector<int32_t> of;
-    for (int b : bt->wide) {
-        rep.push_back(WideRep{b, (int32_t)of.size(), bt->wide_keys});
+    int64_t keys = 0;
+    for (int b : w.reps) {
+        rep.push_back(WideRep{b, (int32_t)of.size(), keys});
         of.insert(of.end(), (bt->rep_n[b] + 63) / 64, (int32_t)rep.size() - 1);
-        bt->wide_keys += (int64_t)kMtN * wide_key_slots(bt->rep_n[b]);
-        bt->wide_max_rays = std::max(bt->wide_max_rays, bt->rep_r[b]);
+        keys += (int64_t)kMtN * wide_key_slots(bt->rep_n[b]);
     }
-    bt->wide_chunks = (int32_t)of.size();
+    WidePlan made = w;
+    made.chunks = (int32_t)of.size();
+    made.keys = keys;
     WideMem m;
-    const size_t bytes = wide_carve(nullptr, rep.size(), of.size(), (size_t)bt->wide_keys, &m);
-    int rc = check_hip(hipMalloc(&bt->wide_mem, bytes), "hipMalloc(wide update)");
-    if (rc) return rc;
-    wide_carve(bt->wide_mem, rep.size(), of.size(), (size_t)bt->wide_keys, &m);
-    rc = check_hip(hipMemcpy(const_cast<WideRep*>(m.rep), rep.data(), sizeof(WideRep) * rep.size(),
-                             hipMemcpyHostToDevice), "upload wide replicas");
+    const size_t bytes = wide_carve(nullptr, rep.size(), of.size(), (size_t)keys, &m);
+    if (int rc = check_hip(hipMalloc(&made.mem, bytes), "hipMalloc(wide update)")) return rc;
+    m = wide_mem(made);
+    int rc = check_hip(hipMemcpy(const_cast<WideRep*>(m.rep), rep.data(), sizeof(WideRep) * rep.size(),
+                                 hipMemcpyHostToDevice), "upload wide replicas");
     if (!rc) rc = check_hip(hipMemcpy(const_cast<int32_t*>(m.of), of.data(), sizeof(int32_t) * of.size(),
                                       hipMemcpyHostToDevice), "upload wide chunks");
     if (!rc) rc = check_hip(hipMemset(m.ctl, 0, sizeof(int32_t) * kWdWords * rep.size()), "clear wide control");
     if (!rc) rc = check_hip(hipDeviceSynchronize(), "plan wide update");
-    return rc;
+    if (rc) {
+        (void)hipFree(made.mem);
+        return rc;
+    }
+    w = std::move(made);
+    return ABM_OK;
 }
 
 // Device memory of the resource loop over the whole GPU; with base null only
@@ -3347,60 +3353,57 @@ size_t wide_world_carve(void* base, const abm_forage_world* w, WideWorld* m) {
 // 0.093, 100 of 8 to 512 0.064 and 0.113; 300 of 100 0.085 and 0.074, 1000 of 8
 // to 512 0.226 and 0.148).  A kernel's blocks take their replicas
 // largest first (the cost grows with the agents; rays add to each agent's).
-int plan_paths(abm_forage_batch* batch, int path) {
-    // updates counted so far, and no launch left on the scratch that goes
-    int64_t made = 0;
-    if (int rc = wide_updates(batch, &made)) return rc;
-    // the plan is made beside the one in use and takes its place when it is whole
-    abm_forage_batch plan = *batch, *bt = &plan;
+// The lists are made once: a captured step keeps order_dev's address, and its
+// replays take the same replicas whatever path is chosen later.
+int plan_classes(abm_forage_batch* bt) {
     const int n = bt->n_replicas;
-    std::vector<int32_t> plain, occl, crowd, big;
+    std::vector<int32_t> plain, narrow, occl, crowd, big, spread;
     int64_t agents = 0;
     int largest = 0;
-    for (int b = 0; b < n; ++b)
-        if (!bt->exclusion[b] && bt->rep_r[b] <= kWideMaxRays) {
+    for (int b = 0; b < n; ++b) {
+        const bool wideable = !bt->exclusion[b] && bt->rep_r[b] <= kWideMaxRays;
+        if (wideable) {
             agents += bt->rep_n[b];
             largest = std::max(largest, bt->rep_n[b]);
         }
-    const bool spread = path == ABM_FORAGE_PATH_SWEEP ||
-                        (largest >= kWideMinAgents && agents <= (int64_t)kWideMaxPerCu * bt->cus);
-    for (int b = 0; b < n; ++b) {
-        const bool wideable = !bt->exclusion[b] && bt->rep_r[b] <= kWideMaxRays;
-        if (bt->too_big[b] || (spread && wideable)) big.push_back(b);
-        else (!bt->exclusion[b] ? plain : bt->rep_n[b] <= kOcclMaxAgents ? occl : crowd).push_back(b);
+        if (bt->too_big[b]) big.push_back(b);
+        else if (bt->exclusion[b]) (bt->rep_n[b] <= kOcclMaxAgents ? occl : crowd).push_back(b);
+        else plain.push_back(b);
+        if (!bt->too_big[b] && !bt->exclusion[b] && !wideable) narrow.push_back(b);
+        if (bt->too_big[b] || wideable) spread.push_back(b);
     }
+    bt->spread_auto = largest >= kWideMinAgents && agents <= (int64_t)kWideMaxPerCu * bt->cus;
     auto cost = [&](int b) { return (double)bt->rep_n[b] * (64.0 + bt->rep_r[b] / 32.0); };
-    auto larger = [&](int a, int c) { return cost(a) > cost(c); };
-    std::stable_sort(plain.begin(), plain.end(), larger);
-    std::stable_sort(occl.begin(), occl.end(), larger);
-    std::stable_sort(crowd.begin(), crowd.end(), larger);
-    bt->order_host = plain;
-    bt->order_host.insert(bt->order_host.end(), occl.begin(), occl.end());
-    bt->order_host.insert(bt->order_host.end(), crowd.begin(), crowd.end());
-    bt->order_host.insert(bt->order_host.end(), big.begin(), big.end());
-    auto extent = [&](const std::vector<int32_t>& v, int32_t& count, int32_t& agents, int32_t& rays) {
-        count = (int32_t)v.size();
-        agents = rays = 0;
+    std::vector<int32_t> order;
+    auto add = [&](std::vector<int32_t>& v, ForageClass& c) {
+        std::stable_sort(v.begin(), v.end(), [&](int a, int d) { return cost(a) > cost(d); });
+        c.first = (int32_t)order.size();
+        c.count = (int32_t)v.size();
         for (int b : v) {
-            agents = std::max(agents, bt->rep_n[b]);
-            rays = std::max(rays, bt->rep_r[b]);
+            c.max_agents = std::max(c.max_agents, bt->rep_n[b]);
+            c.max_rays = std::max(c.max_rays, bt->rep_r[b]);
         }
+        order.insert(order.end(), v.begin(), v.end());
     };
-    extent(plain, bt->n_plain, bt->plain_max_agents, bt->plain_max_rays);
-    extent(occl, bt->n_occl, bt->occl_max_agents, bt->occl_max_rays);
-    extent(crowd, bt->n_crowd, bt->crowd_max_agents, bt->crowd_max_rays);
-    bt->wide_steps += made;
-    bt->wide = big;
+    add(plain, bt->plain);
+    add(narrow, bt->narrow);
+    add(occl, bt->occl);
+    add(crowd, bt->crowd);
+    bt->wide[0].reps = big;
+    bt->wide[1].reps = spread;
+    for (WidePlan& w : bt->wide)
+        for (int b : w.reps) w.max_rays = std::max(w.max_rays, bt->rep_r[b]);
+    const size_t bytes = sizeof(int32_t) * order.size();
+    if (int rc = check_hip(hipMalloc(&bt->order_dev, std::max(bytes, sizeof(int32_t))), "hipMalloc(forage order)")) return rc;
+    return check_hip(hipMemcpy(bt->order_dev, order.data(), bytes, hipMemcpyHostToDevice), "upload forage order");
+}
+
+// Takes a path, with the scratch it needs; a failure leaves the one in use.
+int take_path(abm_forage_batch* bt, int path) {
+    const bool spread = path == ABM_FORAGE_PATH_SWEEP || bt->spread_auto;
+    if (int rc = make_wide(bt, bt->wide[spread])) return rc;
     bt->path = path;
-    int rc = plan_wide(bt);
-    if (!rc) rc = check_hip(hipMemcpy(bt->order_dev, bt->order_host.data(), sizeof(int32_t) * n,
-                                      hipMemcpyHostToDevice), "upload forage order");
-    if (rc) {
-        if (bt->wide_mem) (void)hipFree(bt->wide_mem);
-        return rc;
-    }
-    if (batch->wide_mem) (void)hipFree(batch->wide_mem);
-    *batch = std::move(plan);
+    bt->spread = spread;
     return ABM_OK;
 }
 
@@ -3411,9 +3414,9 @@ int plan_paths(abm_forage_batch* batch, int path) {
 // replica has work for more (1000 replicas of 10 agents: 0.048 ms with four,
 // 0.070 with sixteen; of 50: 0.068, 0.090; of 128: 0.121, 0.137).  Fewer too
 // where the waves' fields would not fit in LDS.
-int upd_waves(const abm_forage_batch* b) {
-    int waves = b->n_plain > 2 * b->cus && b->plain_max_agents <= 128 ? 4 : 16;
-    while (waves > 4 && upd_lds_bytes(b->plain_max_agents, b->plain_max_rays, waves) > (size_t)163840 - sizeof(FGRep))
+int upd_waves(const ForageClass& c, int cus) {
+    int waves = c.count > 2 * cus && c.max_agents <= 128 ? 4 : 16;
+    while (waves > 4 && upd_lds_bytes(c.max_agents, c.max_rays, waves) > (size_t)163840 - sizeof(FGRep))
         waves /= 2;
     return waves;
 }
@@ -3431,10 +3434,10 @@ int check_state(const abm_forage_state* st, const char* who) {
 int launch_wide(abm_forage_batch* b, const abm_forage_state* st, const double* uniforms,
                 const uint32_t* words, const int64_t* offset, const int32_t* count, int32_t* used,
                 int32_t* status, uint32_t* field_bits, hipStream_t s, abm_mt19937_state* mt) {
-    if (!b->wide_mem) return set_error(ABM_ERR_HIP, "forage update over the whole GPU: no scratch");
-    WideMem m;
-    const int n = (int)b->wide.size(), chunks = b->wide_chunks, W = (b->wide_max_rays + 31) / 32;
-    wide_carve(b->wide_mem, n, chunks, (size_t)b->wide_keys, &m);
+    const WidePlan& plan = b->wide[b->spread];
+    if (!plan.mem) return set_error(ABM_ERR_HIP, "forage update over the whole GPU: no scratch");
+    const WideMem m = wide_mem(plan);
+    const int n = (int)plan.reps.size(), chunks = plan.chunks, W = (plan.max_rays + 31) / 32;
     const FGRep* reps = (const FGRep*)b->reps_dev;
     const int blocks = (chunks + 3) / 4;
     hipLaunchKernelGGL(wide_drive_kernel, dim3(blocks), dim3(256), 0, s, reps, chunks, *st, status, used,
@@ -3455,9 +3458,10 @@ int launch_forage_step(abm_forage_batch* b, const abm_forage_state* st, const do
                        const uint32_t* words, const int64_t* offset, const int32_t* count,
                        int32_t* used, int32_t* status, uint32_t* field_bits, void* stream,
                        abm_mt19937_state* mt = nullptr) {
-    if (b->n_plain > 0) {
-        const int waves = upd_waves(b);
-        const size_t lds = upd_lds_bytes(b->plain_max_agents, b->plain_max_rays, waves);
+    const int32_t* const order = (const int32_t*)b->order_dev;
+    if (const ForageClass& c = b->spread ? b->narrow : b->plain; c.count > 0) {
+        const int waves = upd_waves(c, b->cus);
+        const size_t lds = upd_lds_bytes(c.max_agents, c.max_rays, waves);
         auto kern = field_bits ? forage_update_kernel<true> : forage_update_kernel<false>;
         if (lds > 65536) {
             if (int rc = check_hip(hipFuncSetAttribute((const void*)kern,
@@ -3465,14 +3469,14 @@ int launch_forage_step(abm_forage_batch* b, const abm_forage_state* st, const do
                                    "hipFuncSetAttribute"))
                 return rc;
         }
-        hipLaunchKernelGGL(kern, dim3(b->n_plain), dim3(64 * waves), lds, (hipStream_t)stream,
+        hipLaunchKernelGGL(kern, dim3(c.count), dim3(64 * waves), lds, (hipStream_t)stream,
                            (const FGRep*)b->reps_dev, *st, uniforms, words, offset, count, used, status,
-                           field_bits, (const int32_t*)b->order_dev, mt, b->plain_max_agents);
+                           field_bits, order + c.first, mt, c.max_agents);
         if (int rc = check_hip(hipGetLastError(), "forage_update_kernel launch")) return rc;
     }
-    if (b->n_occl > 0) {
-        const int K = b->occl_max_agents <= 64 ? 1 : (b->occl_max_agents <= 128 ? 2 : 4);
-        const size_t lds = occl_lds_bytes(b->occl_max_agents, b->occl_max_rays, K);
+    if (const ForageClass& c = b->occl; c.count > 0) {
+        const int K = c.max_agents <= 64 ? 1 : (c.max_agents <= 128 ? 2 : 4);
+        const size_t lds = occl_lds_bytes(c.max_agents, c.max_rays, K);
         auto kern = field_bits ? (K == 1 ? forage_occlude_kernel<1, true>
                                          : (K == 2 ? forage_occlude_kernel<2, true> : forage_occlude_kernel<4, true>))
                                : (K == 1 ? forage_occlude_kernel<1, false>
@@ -3483,13 +3487,13 @@ int launch_forage_step(abm_forage_batch* b, const abm_forage_state* st, const do
                                    "hipFuncSetAttribute"))
                 return rc;
         }
-        hipLaunchKernelGGL(kern, dim3(b->n_occl), dim3(64 * kOcclWaves), lds, (hipStream_t)stream,
+        hipLaunchKernelGGL(kern, dim3(c.count), dim3(64 * kOcclWaves), lds, (hipStream_t)stream,
                            (const FGRep*)b->reps_dev, *st, uniforms, words, offset, count, used, status,
-                           field_bits, (const int32_t*)b->order_dev + b->n_plain, mt, b->occl_max_agents);
+                           field_bits, order + c.first, mt, c.max_agents);
         if (int rc = check_hip(hipGetLastError(), "forage_occlude_kernel launch")) return rc;
     }
-    if (b->n_crowd > 0) {   // the replicas with visual exclusion beyond its registers
-        const size_t lds = fg_lds_bytes(b->crowd_max_agents, b->crowd_max_rays);
+    if (const ForageClass& c = b->crowd; c.count > 0) {   // visual exclusion beyond its registers
+        const size_t lds = fg_lds_bytes(c.max_agents, c.max_rays);
         auto kern = field_bits ? forage_step_kernel<true> : forage_step_kernel<false>;
         if (lds > 65536) {
             if (int rc = check_hip(hipFuncSetAttribute((const void*)kern,
@@ -3497,13 +3501,12 @@ int launch_forage_step(abm_forage_batch* b, const abm_forage_state* st, const do
                                    "hipFuncSetAttribute"))
                 return rc;
         }
-        hipLaunchKernelGGL(kern, dim3(b->n_crowd), dim3(512), lds, (hipStream_t)stream,
+        hipLaunchKernelGGL(kern, dim3(c.count), dim3(512), lds, (hipStream_t)stream,
                            (const FGRep*)b->reps_dev, *st, uniforms, words, offset, count, used, status,
-                           field_bits, (const int32_t*)b->order_dev + b->n_plain + b->n_occl, mt,
-                           b->crowd_max_agents, b->crowd_max_rays);
+                           field_bits, order + c.first, mt, c.max_agents, c.max_rays);
         if (int rc = check_hip(hipGetLastError(), "forage_step_kernel launch")) return rc;
     }
-    if (!b->wide.empty())
+    if (!b->wide[b->spread].reps.empty())
         return launch_wide(b, st, uniforms, words, offset, count, used, status, field_bits, (hipStream_t)stream, mt);
     return ABM_OK;
 }
@@ -3583,15 +3586,14 @@ int abm_forage_batch_create(const abm_forage_replica* reps, int32_t n, abm_forag
                            "supports neither visual exclusion nor more than %d rays", b, host[b].n_agents,
                            host[b].n_rays, need, dev_max, kWideMaxRays);
     }
-    bt->order_host.resize(n);
     bt->rep_n.resize(n);
     bt->rep_r.resize(n);
     for (int b = 0; b < n; ++b) { bt->rep_n[b] = host[b].n_agents; bt->rep_r[b] = host[b].n_rays; }
     if (!rc) rc = check_hip(hipMalloc(&bt->reps_dev, sizeof(FGRep) * n), "hipMalloc(forage replicas)");
     if (!rc) rc = check_hip(hipMemcpy(bt->reps_dev, host.data(), sizeof(FGRep) * n, hipMemcpyHostToDevice),
                            "upload forage replicas");
-    if (!rc) rc = check_hip(hipMalloc(&bt->order_dev, sizeof(int32_t) * n), "hipMalloc(forage order)");
-    if (!rc) rc = plan_paths(bt, ABM_FORAGE_PATH_AUTO);
+    if (!rc) rc = plan_classes(bt);
+    if (!rc) rc = take_path(bt, ABM_FORAGE_PATH_AUTO);
     if (rc) { abm_forage_batch_destroy(bt); return rc; }
     bt->agent_offset_host = new int32_t[n + 1];
     bt->field_offset_host = new int64_t[n + 1];
@@ -3609,7 +3611,8 @@ int abm_forage_batch_destroy(abm_forage_batch* b) {
     if (!b) return ABM_OK;
     if (b->reps_dev) (void)hipFree(b->reps_dev);
     if (b->order_dev) (void)hipFree(b->order_dev);
-    if (b->wide_mem) (void)hipFree(b->wide_mem);
+    for (const WidePlan& w : b->wide)
+        if (w.mem) (void)hipFree(w.mem);
     delete[] b->agent_offset_host;
     delete[] b->field_offset_host;
     delete b;
@@ -3635,7 +3638,7 @@ int abm_forage_sweep_counts(const abm_forage_batch* b, int64_t* updates, int64_t
     if (!b || !updates || !sweeps) return set_error(ABM_ERR_INVALID, "abm_forage_sweep_counts: NULL argument");
     int64_t made = 0;
     if (int rc = wide_updates(b, &made)) return rc;
-    *updates = *sweeps = b->wide_steps + made;
+    *updates = *sweeps = made;
     return ABM_OK;
 }
 
@@ -3643,7 +3646,7 @@ int abm_forage_set_path(abm_forage_batch* b, int32_t path) {
     if (!b) return set_error(ABM_ERR_INVALID, "abm_forage_set_path: NULL batch");
     if (path != ABM_FORAGE_PATH_AUTO && path != ABM_FORAGE_PATH_SWEEP)
         return set_error(ABM_ERR_INVALID, "abm_forage_set_path: unknown path %d", path);
-    return plan_paths(b, path);
+    return take_path(b, path);
 }
 
 int abm_forage_step_f64(abm_forage_batch* b, const abm_forage_state* st, const double* uniforms,

@@ -8,6 +8,22 @@
 
 #include "../../include/abm_amd.h"
 
+// Replicas updated over the whole GPU, their 64-agent chunks, largest field and
+// words of twisted generator keys, and the scratch of their launches: allocated
+// when a path first needs it and then kept while the batch lives, since a
+// captured step keeps its address.
+struct WidePlan {
+    std::vector<int32_t> reps;
+    int32_t chunks = 0, max_rays = 0;
+    int64_t keys = 0;
+    void* mem = nullptr;
+};
+
+// Replicas that one kernel takes, a workgroup each: order_dev[first, first + count).
+struct ForageClass {
+    int32_t first = 0, count = 0, max_agents = 0, max_rays = 0;
+};
+
 struct abm_forage_batch {
     int32_t n_replicas = 0;
     int32_t n_agents_total = 0;
@@ -17,26 +33,21 @@ struct abm_forage_batch {
     int device = 0;
     int cus = 0;                       // compute units of the device
     void* reps_dev = nullptr;
-    void* order_dev = nullptr;        // replicas by descending cost: the blocks' update order
+    void* order_dev = nullptr;         // the classes' replicas by descending cost, fixed at creation
     int32_t* agent_offset_host = nullptr;
     int64_t* field_offset_host = nullptr;
-    // Replicas the update kernel takes (the first n_plain of order_dev), those
-    // with visual exclusion, which the occlude kernel takes (the next n_occl) or
-    // the step kernel (the next n_crowd), and the ones beyond one workgroup's
-    // LDS, updated over the whole GPU.
-    int32_t n_plain = 0, n_occl = 0, n_crowd = 0;
-    int32_t plain_max_agents = 0, plain_max_rays = 0, occl_max_agents = 0, occl_max_rays = 0;
-    int32_t crowd_max_agents = 0, crowd_max_rays = 0;
+    // Replicas that fit one workgroup's LDS: those without visual exclusion,
+    // which the update kernel takes, the ones of them that the launches over
+    // the whole GPU cannot take (rays), and those with it, which the occlude
+    // kernel or the step kernel takes.
+    ForageClass plain, narrow, occl, crowd;
+    WidePlan wide[2];                  // replicas beyond that LDS; those and the plain ones but the narrow
     int32_t path = 0;                  // ABM_FORAGE_PATH_*
+    bool spread = false;               // the path in use takes wide[1] (and narrow in the place of plain)
+    bool spread_auto = false;          // what ABM_FORAGE_PATH_AUTO takes
     std::vector<int32_t> rep_n, rep_r; // agents and rays of every replica
-    std::vector<int32_t> order_host;   // every replica: update kernel's, occlude kernel's, step kernel's, wide
     std::vector<uint8_t> too_big;      // [b]: beyond one workgroup's LDS
     std::vector<uint8_t> exclusion;    // [b]: visual exclusion
-    std::vector<int32_t> wide;         // replicas updated over the whole GPU
-    int32_t wide_chunks = 0, wide_max_rays = 0;   // their 64-agent chunks, their largest field
-    int64_t wide_keys = 0;             // words of their generators' twisted keys
-    void* wide_mem = nullptr;          // their map, cues, drives, counts, words, control
-    int64_t wide_steps = 0;            // replica updates made that way under earlier plans
 };
 
 // The resource patches' per-replica constants and pending-placement scratch
