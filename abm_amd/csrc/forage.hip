@@ -24,6 +24,8 @@
 #include <algorithm>
 #include <cmath>
 #include <cstring>
+#include <mutex>
+#include <new>
 #include <utility>
 #include <vector>
 
@@ -2024,8 +2026,16 @@ struct WideMem {
     uint32_t* keys;              // its key after each twist
     uint8_t* walk;               // 1: the agent draws a walk turn
     int32_t* ctl;                // [replica][kWdWords]
+    int32_t* updates;            // [replica]: made so far
 };
-constexpr int kWdCues = 0, kWdSkip = 1, kWdUsed0 = 2, kWdUpdates = 3, kWdWords = 4;
+constexpr int kWdCues = 0, kWdSkip = 1, kWdUsed0 = 2, kWdWords = 4;
+
+// Control words of new scratch.
+__global__ void __launch_bounds__(256)
+wide_clear_kernel(int32_t* __restrict__ ctl, int n) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) ctl[i] = 0;
+}
 
 // One thread per agent: the drive, the focal geometry, the cues.
 __global__ void __launch_bounds__(256)
@@ -2243,7 +2253,7 @@ wide_move_kernel(const FGRep* __restrict__ reps, int n_chunks, abm_forage_state 
     }
     if (lane == 0) {
         ctl[kWdCues] = 0;   // for the next step's drive kernel
-        ctl[kWdUpdates] += 1;
+        atomicAdd(&M.updates[q], 1);
         if (u_used) u_used[rb] = used0 + (words || mt ? 2 : 1) * total;
         if (status) status[rb] = ABM_WORLD_DONE;
     }
@@ -3262,6 +3272,7 @@ size_t wide_carve(void* base, size_t reps, size_t chunks, size_t key_words, Wide
     m->keys = reinterpret_cast<uint32_t*>(take(sizeof(uint32_t) * key_words));
     m->walk = reinterpret_cast<uint8_t*>(take(n));
     m->ctl = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * kWdWords * reps));
+    m->updates = reinterpret_cast<int32_t*>(take(sizeof(int32_t) * reps));
     return at;
 }
 
@@ -3276,19 +3287,21 @@ int wide_updates(const abm_forage_batch* bt, int64_t* total) {
     *total = 0;
     for (const WidePlan& w : bt->wide) {
         if (!w.mem) continue;
-        std::vector<int32_t> ctl(kWdWords * w.reps.size());
+        std::vector<int32_t> made(w.reps.size());
         if (int rc = check_hip(hipDeviceSynchronize(), "hipDeviceSynchronize")) return rc;
-        if (int rc = check_hip(hipMemcpy(ctl.data(), wide_mem(w).ctl, sizeof(int32_t) * ctl.size(),
-                                         hipMemcpyDeviceToHost), "read wide control"))
+        if (int rc = check_hip(hipMemcpy(made.data(), wide_mem(w).updates, sizeof(int32_t) * made.size(),
+                                         hipMemcpyDeviceToHost), "read update counts"))
             return rc;
-        for (size_t i = 0; i < w.reps.size(); ++i) *total += ctl[kWdWords * i + kWdUpdates];
+        for (int32_t n : made) *total += n;
     }
     return ABM_OK;
 }
 
 // The scratch of a plan, made whole before the plan has it.
-int make_wide(const abm_forage_batch* bt, WidePlan& w) {
+int make_wide(abm_forage_batch* bt, WidePlan& w) {
     if (w.mem || w.reps.empty()) return ABM_OK;
+    if (!bt->wide_done)
+        if (int rc = check_hip(hipEventCreateWithFlags(&bt->wide_done, hipEventDisableTiming), "hipEventCreate")) return rc;
     std::vector<WideRep> rep;
     std::vector<int32_t> of;
     int64_t keys = 0;
@@ -3309,6 +3322,7 @@ int make_wide(const abm_forage_batch* bt, WidePlan& w) {
     if (!rc) rc = check_hip(hipMemcpy(const_cast<int32_t*>(m.of), of.data(), sizeof(int32_t) * of.size(),
                                       hipMemcpyHostToDevice), "upload wide chunks");
     if (!rc) rc = check_hip(hipMemset(m.ctl, 0, sizeof(int32_t) * kWdWords * rep.size()), "clear wide control");
+    if (!rc) rc = check_hip(hipMemset(m.updates, 0, sizeof(int32_t) * rep.size()), "clear update counts");
     if (!rc) rc = check_hip(hipDeviceSynchronize(), "plan wide update");
     if (rc) {
         (void)hipFree(made.mem);
@@ -3400,6 +3414,7 @@ int plan_classes(abm_forage_batch* bt) {
 
 // Takes a path, with the scratch it needs; a failure leaves the one in use.
 int take_path(abm_forage_batch* bt, int path) {
+    std::lock_guard<std::mutex> guard(bt->wide_lock);
     const bool spread = path == ABM_FORAGE_PATH_SWEEP || bt->spread_auto;
     if (int rc = make_wide(bt, bt->wide[spread])) return rc;
     bt->path = path;
@@ -3430,13 +3445,10 @@ int check_state(const abm_forage_state* st, const char* who) {
     return ABM_OK;
 }
 
-// Agent.update of the wide replicas (see wide_drive_kernel).
-int launch_wide(abm_forage_batch* b, const abm_forage_state* st, const double* uniforms,
-                const uint32_t* words, const int64_t* offset, const int32_t* count, int32_t* used,
-                int32_t* status, uint32_t* field_bits, hipStream_t s, abm_mt19937_state* mt) {
-    const WidePlan& plan = b->wide[b->spread];
-    if (!plan.mem) return set_error(ABM_ERR_HIP, "forage update over the whole GPU: no scratch");
-    const WideMem m = wide_mem(plan);
+// Agent.update of a plan's replicas (see wide_drive_kernel) on scratch m.
+int wide_launches(const abm_forage_batch* b, const WidePlan& plan, const WideMem& m, const abm_forage_state* st,
+                  const double* uniforms, const uint32_t* words, const int64_t* offset, const int32_t* count,
+                  int32_t* used, int32_t* status, uint32_t* field_bits, hipStream_t s, abm_mt19937_state* mt) {
     const int n = (int)plan.reps.size(), chunks = plan.chunks, W = (plan.max_rays + 31) / 32;
     const FGRep* reps = (const FGRep*)b->reps_dev;
     const int blocks = (chunks + 3) / 4;
@@ -3453,13 +3465,90 @@ int launch_wide(abm_forage_batch* b, const abm_forage_state* st, const double* u
     return ABM_OK;
 }
 
+int wide_clear(const WidePlan& plan, const WideMem& m, hipStream_t s) {
+    const int n = kWdWords * (int)plan.reps.size();
+    hipLaunchKernelGGL(wide_clear_kernel, dim3((n + 255) / 256), dim3(256), 0, s, m.ctl, n);
+    return check_hip(hipGetLastError(), "wide_clear_kernel launch");
+}
+
+// A scratch other than the null stream's, allocated (also while a stream is
+// captured: in relaxed mode) by the first step that needs it and freed with the
+// batch.
+constexpr int kMaxCaptures = 1024;
+int other_scratch(abm_forage_batch* b, int plan, unsigned long long capture, hipStream_t s, WideMem* m,
+                  WideScratch** out) {
+    const WidePlan& w = b->wide[plan];
+    const WideMem base = wide_mem(w);
+    WideScratch* c = b->scratch;
+    while (c && !(c->plan == plan && c->capture == capture && c->stream == s)) c = c->next;
+    if (!c) {
+        if (capture && b->n_captures >= kMaxCaptures)
+            return set_error(ABM_ERR_UNSUPPORTED, "forage update over the whole GPU: %d captures of this batch hold "
+                             "scratch until it is destroyed", kMaxCaptures);
+        c = new (std::nothrow) WideScratch;
+        if (!c) return set_error(ABM_ERR_HIP, "forage update over the whole GPU: out of host memory");
+        hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+        int rc = check_hip(hipThreadExchangeStreamCaptureMode(&mode), "capture mode");
+        if (!rc) {
+            rc = check_hip(hipMalloc(&c->mem, wide_carve(nullptr, w.reps.size(), (size_t)w.chunks, (size_t)w.keys, m)),
+                           "hipMalloc(wide update)");
+            (void)hipThreadExchangeStreamCaptureMode(&mode);
+        }
+        if (rc) {
+            delete c;
+            return rc;
+        }
+        c->plan = plan; c->capture = capture; c->stream = s;
+        c->next = b->scratch;
+        b->scratch = c;
+        b->n_captures += capture != 0;
+    }
+    wide_carve(c->mem, w.reps.size(), (size_t)w.chunks, (size_t)w.keys, m);
+    m->rep = base.rep; m->of = base.of; m->updates = base.updates;
+    *out = c;
+    return ABM_OK;
+}
+
+// Agent.update of the wide replicas.  Calls on one batch may come from several
+// streams and threads, each with its own state, and may not share scratch while
+// they run.  The null stream has its own: its calls are in order, it cannot be
+// destroyed, and an event after each call would cost 3 us (8192 agents 63.4 ->
+// 66.4 us a step).  The other streams share one, each call behind an event of the
+// one before.  A captured step cannot wait for calls outside its graph, nor they
+// for its replays: its capture has scratch of its own.
+int launch_wide(abm_forage_batch* b, int plan, const abm_forage_state* st, const double* uniforms,
+                const uint32_t* words, const int64_t* offset, const int32_t* count, int32_t* used,
+                int32_t* status, uint32_t* field_bits, hipStream_t s, abm_mt19937_state* mt) {
+    std::lock_guard<std::mutex> guard(b->wide_lock);
+    const WidePlan& w = b->wide[plan];
+    if (!w.mem) return set_error(ABM_ERR_HIP, "forage update over the whole GPU: no scratch");
+    WideMem m = wide_mem(w);
+    if (!s) return wide_launches(b, w, m, st, uniforms, words, offset, count, used, status, field_bits, s, mt);
+    hipStreamCaptureStatus state = hipStreamCaptureStatusNone;
+    unsigned long long capture = 0;
+    if (int rc = check_hip(hipStreamGetCaptureInfo(s, &state, &capture), "hipStreamGetCaptureInfo")) return rc;
+    const bool captured = state != hipStreamCaptureStatusNone;
+    WideScratch* c = nullptr;
+    if (int rc = other_scratch(b, plan, captured ? capture : 0, captured ? s : nullptr, &m, &c)) return rc;
+    if (!captured)
+        if (int rc = check_hip(hipStreamWaitEvent(s, b->wide_done, 0), "hipStreamWaitEvent")) return rc;
+    int rc = captured || !c->cleared ? wide_clear(w, m, s) : ABM_OK;
+    c->cleared = rc == ABM_OK;
+    if (!rc) rc = wide_launches(b, w, m, st, uniforms, words, offset, count, used, status, field_bits, s, mt);
+    if (captured) return rc;
+    const int done = check_hip(hipEventRecord(b->wide_done, s), "hipEventRecord");
+    if (done) (void)hipDeviceSynchronize();   // no event to wait for: nothing may be left
+    return rc ? rc : done;
+}
+
 // Agent.update for every replica (all, or those a status array marks ready).
 int launch_forage_step(abm_forage_batch* b, const abm_forage_state* st, const double* uniforms,
                        const uint32_t* words, const int64_t* offset, const int32_t* count,
                        int32_t* used, int32_t* status, uint32_t* field_bits, void* stream,
                        abm_mt19937_state* mt = nullptr) {
     const int32_t* const order = (const int32_t*)b->order_dev;
-    if (const ForageClass& c = b->spread ? b->narrow : b->plain; c.count > 0) {
+    const bool spread = b->spread;
+    if (const ForageClass& c = spread ? b->narrow : b->plain; c.count > 0) {
         const int waves = upd_waves(c, b->cus);
         const size_t lds = upd_lds_bytes(c.max_agents, c.max_rays, waves);
         auto kern = field_bits ? forage_update_kernel<true> : forage_update_kernel<false>;
@@ -3506,8 +3595,8 @@ int launch_forage_step(abm_forage_batch* b, const abm_forage_state* st, const do
                            field_bits, order + c.first, mt, c.max_agents, c.max_rays);
         if (int rc = check_hip(hipGetLastError(), "forage_step_kernel launch")) return rc;
     }
-    if (!b->wide[b->spread].reps.empty())
-        return launch_wide(b, st, uniforms, words, offset, count, used, status, field_bits, (hipStream_t)stream, mt);
+    if (!b->wide[spread].reps.empty())
+        return launch_wide(b, spread, st, uniforms, words, offset, count, used, status, field_bits, (hipStream_t)stream, mt);
     return ABM_OK;
 }
 
@@ -3613,6 +3702,12 @@ int abm_forage_batch_destroy(abm_forage_batch* b) {
     if (b->order_dev) (void)hipFree(b->order_dev);
     for (const WidePlan& w : b->wide)
         if (w.mem) (void)hipFree(w.mem);
+    if (b->wide_done) (void)hipEventDestroy(b->wide_done);
+    while (WideScratch* c = b->scratch) {
+        b->scratch = c->next;
+        (void)hipFree(c->mem);
+        delete c;
+    }
     delete[] b->agent_offset_host;
     delete[] b->field_offset_host;
     delete b;
@@ -3637,6 +3732,7 @@ int abm_forage_batch_get_offsets(const abm_forage_batch* b, int32_t* agent_offse
 int abm_forage_sweep_counts(const abm_forage_batch* b, int64_t* updates, int64_t* sweeps) {
     if (!b || !updates || !sweeps) return set_error(ABM_ERR_INVALID, "abm_forage_sweep_counts: NULL argument");
     int64_t made = 0;
+    std::lock_guard<std::mutex> guard(b->wide_lock);
     if (int rc = wide_updates(b, &made)) return rc;
     *updates = *sweeps = made;
     return ABM_OK;

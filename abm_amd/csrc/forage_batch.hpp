@@ -4,19 +4,34 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <atomic>
+#include <mutex>
 #include <vector>
 
 #include "../../include/abm_amd.h"
 
 // Replicas updated over the whole GPU, their 64-agent chunks, largest field and
-// words of twisted generator keys, and the scratch of their launches: allocated
-// when a path first needs it and then kept while the batch lives, since a
-// captured step keeps its address.
+// words of twisted generator keys, and the scratch of their launches on the null
+// stream (and the lists that every scratch shares): allocated when a path first
+// needs it and then kept while the batch lives, since a captured step keeps its
+// address.
 struct WidePlan {
     std::vector<int32_t> reps;
     int32_t chunks = 0, max_rays = 0;
     int64_t keys = 0;
     void* mem = nullptr;
+};
+
+// Scratch of a plan's steps elsewhere than on the null stream: one for all other
+// streams (capture 0), and one for the steps that a capture of a stream records,
+// whose graph may run beside any other call.
+struct WideScratch {
+    int plan = 0;
+    unsigned long long capture = 0;
+    hipStream_t stream = nullptr;
+    bool cleared = false;              // its control words
+    void* mem = nullptr;
+    WideScratch* next = nullptr;
 };
 
 // Replicas that one kernel takes, a workgroup each: order_dev[first, first + count).
@@ -43,8 +58,15 @@ struct abm_forage_batch {
     ForageClass plain, narrow, occl, crowd;
     WidePlan wide[2];                  // replicas beyond that LDS; those and the plain ones but the narrow
     int32_t path = 0;                  // ABM_FORAGE_PATH_*
-    bool spread = false;               // the path in use takes wide[1] (and narrow in the place of plain)
+    std::atomic<bool> spread{false};   // the path in use takes wide[1] (and narrow in the place of plain)
     bool spread_auto = false;          // what ABM_FORAGE_PATH_AUTO takes
+    // Calls may come from several threads and streams, each with its own state.
+    // One at a time issues its launches; the null stream has wide[].mem to itself,
+    // the other streams wait for each other's launches.
+    mutable std::mutex wide_lock;
+    hipEvent_t wide_done = nullptr;    // after the launches of the last call on another stream
+    WideScratch* scratch = nullptr;
+    int32_t n_captures = 0;
     std::vector<int32_t> rep_n, rep_r; // agents and rays of every replica
     std::vector<uint8_t> too_big;      // [b]: beyond one workgroup's LDS
     std::vector<uint8_t> exclusion;    // [b]: visual exclusion

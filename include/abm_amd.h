@@ -411,9 +411,15 @@ int abm_forage_step_f64(abm_forage_batch* batch, const abm_forage_state* state,
  * exclusion off, at most 8192 rays) by launches over its agents on the whole
  * GPU, in one sweep: what an agent's update makes of it as a social cue does
  * not depend on its own field, so every field can be built at once, in the
- * reference's id-order views.  ABM_FORAGE_PATH_SWEEP takes every replica
- * without visual exclusion that way (same results).  No path synchronises
- * the stream. */
+ * reference's id-order views.  Replicas that fit are taken that way too where
+ * one of them has at least 64 agents and those without visual exclusion at most
+ * 96 a compute unit in all.  ABM_FORAGE_PATH_SWEEP takes every replica without
+ * visual exclusion that way (same results).  No path synchronises the stream.
+ * The launches share scratch: calls on one batch from several threads and
+ * streams, each with its own state, are ordered behind each other where they
+ * would share it, and each capture of a stream has its own until the batch is
+ * destroyed (at most 1024; then ABM_ERR_UNSUPPORTED).  A captured step stays
+ * valid when the path changes. */
 #define ABM_FORAGE_PATH_AUTO  0
 #define ABM_FORAGE_PATH_SWEEP 1
 int abm_forage_set_path(abm_forage_batch* batch, int32_t path);

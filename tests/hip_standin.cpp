@@ -80,6 +80,25 @@ hipError_t hipGetLastError() {
 }
 const char* hipGetErrorString(hipError_t) { return "stand-in error"; }
 
+// ---- events and captures
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) { *e = reinterpret_cast<hipEvent_t>(malloc(1)); return hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t e) { free(e); return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t, hipStream_t s) { note("record on " + hex(s)); return fails("hipEventRecord") ? hipErrorInvalidHandle : hipSuccess; }
+hipError_t hipStreamWaitEvent(hipStream_t s, hipEvent_t, unsigned) { note("wait on " + hex(s)); return hipSuccess; }
+static hipStream_t captured;
+static unsigned long long capture_id;
+void standin_capture(hipStream_t s, unsigned long long id) { captured = s; capture_id = id; }
+hipError_t hipStreamGetCaptureInfo(hipStream_t s, hipStreamCaptureStatus* st, unsigned long long* id) {
+    *st = captured && s == captured ? hipStreamCaptureStatusActive : hipStreamCaptureStatusNone;
+    *id = capture_id;
+    return hipSuccess;
+}
+hipError_t hipThreadExchangeStreamCaptureMode(hipStreamCaptureMode* m) {
+    static hipStreamCaptureMode now = hipStreamCaptureModeGlobal;
+    std::swap(*m, now);
+    return hipSuccess;
+}
+
 // ---- kernels
 void** __hipRegisterFatBinary(const void*) { static void* h; return &h; }
 void __hipUnregisterFatBinary(void**) {}
@@ -95,7 +114,7 @@ hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* lds, hipStream_t*
 }
 hipError_t hipLaunchKernel(const void* f, dim3 g, dim3, void**, size_t, hipStream_t s) {
     if (fails("hipLaunchKernel")) {
-        note("launch failed");
+        note("failed launch");
         return pending = hipErrorLaunchFailure;
     }
     int bad = 0;

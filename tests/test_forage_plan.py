@@ -69,3 +69,57 @@ def test_each_replica_has_one_kernel(standin):
         assert grids(h) == dict(forage_update_kernel=2, forage_occlude_kernel=1, forage_step_kernel=1,
                                 wide_drive_kernel=106, wide_field_kernel=16 * 423, wide_move_kernel=106)
         """)
+
+
+def test_calls_on_several_streams(standin):
+    # the null stream has scratch of its own; the others share one, each call
+    # behind the launches of the one before it, also of one that failed
+    hip_standin.run(standin, """
+        h = forage_batch(replica(200), replica(12, visual_exclusion=1))
+        log()
+        bytes0 = held()[0]
+        for s in (None, 64, None, 128, 128):
+            assert forage_step(h, s) == 0
+            on = "on " + ("(nil)" if s is None else hex(s))
+            calls = [ln for ln in log() if "occlude" not in ln]
+            if held()[0] > bytes0:   # (first on another stream)
+                assert s == 64 and calls.pop(0) == "hipMalloc" and "wide_clear_kernel" in calls.pop(1)
+                bytes0 = held()[0]
+            steps = ["launch"] * 3 if s is None else ["wait", "launch", "launch", "launch", "record"]
+            assert [ln.split()[0] for ln in calls] == steps and all(ln.endswith(on) for ln in calls)
+        for which, launched in ((2, 0), (3, 1), (4, 2)):   # (the first is the other replica's)
+            fail("hipLaunchKernel", which)
+            assert forage_step(h, 64) == L.ABM_ERR_HIP
+            calls = log()
+            assert len(kernels(calls)) == 1 + launched and calls[-1] == "record on 0x40"
+        fail("hipEventRecord")
+        assert forage_step(h, 64) == L.ABM_ERR_HIP
+        assert log()[-1] == "hipDeviceSynchronize"
+        """)
+
+
+def test_captured_steps_have_scratch_of_their_own(standin):
+    hip_standin.run(standin, """
+        h = forage_batch(replica(200), replica(100, 1200))
+        assert forage_step(h, 256) == 0
+        log()
+        one = ["wide_clear_kernel", "wide_drive_kernel", "wide_field_kernel", "wide_move_kernel"]
+        for s, id, steps in ((64, 1, 3), (128, 1, 1), (64, 2, 2)):   # a stream's capture; a branch of it; the next one
+            sim.standin_capture(C.c_void_p(s), C.c_ulonglong(id))
+            before = held()[0]
+            for _ in range(steps):
+                assert forage_step(h, s) == 0
+            calls = log()
+            assert kernels(calls) == steps * one
+            assert calls.count("hipMalloc") == 1 and held()[0] > before
+            assert not [ln for ln in calls if ln.split()[0] in ("wait", "record")]
+            assert forage_step(h, 256) == 0   # not the stream that is captured
+            assert [ln.split()[0] for ln in log()] == ["wait", "launch", "launch", "launch", "record"]
+        fail("hipMalloc")
+        sim.standin_capture(C.c_void_p(64), C.c_ulonglong(3))
+        assert forage_step(h, 64) == L.ABM_ERR_HIP
+        log()
+        assert forage_step(h, 64) == 0 and kernels(log()) == one
+        lib.abm_forage_batch_destroy(h)
+        assert held()[0] == 0
+        """)
