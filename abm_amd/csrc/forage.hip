@@ -3328,6 +3328,7 @@ int make_wide(abm_forage_batch* bt, WidePlan& w) {
         (void)hipFree(made.mem);
         return rc;
     }
+    made.clean = true;
     w = std::move(made);
     return ABM_OK;
 }
@@ -3520,22 +3521,29 @@ int launch_wide(abm_forage_batch* b, int plan, const abm_forage_state* st, const
                 const uint32_t* words, const int64_t* offset, const int32_t* count, int32_t* used,
                 int32_t* status, uint32_t* field_bits, hipStream_t s, abm_mt19937_state* mt) {
     std::lock_guard<std::mutex> guard(b->wide_lock);
-    const WidePlan& w = b->wide[plan];
+    WidePlan& w = b->wide[plan];
     if (!w.mem) return set_error(ABM_ERR_HIP, "forage update over the whole GPU: no scratch");
     WideMem m = wide_mem(w);
-    if (!s) return wide_launches(b, w, m, st, uniforms, words, offset, count, used, status, field_bits, s, mt);
+    bool* clean = &w.clean;
     hipStreamCaptureStatus state = hipStreamCaptureStatusNone;
     unsigned long long capture = 0;
-    if (int rc = check_hip(hipStreamGetCaptureInfo(s, &state, &capture), "hipStreamGetCaptureInfo")) return rc;
+    if (s)
+        if (int rc = check_hip(hipStreamGetCaptureInfo(s, &state, &capture), "hipStreamGetCaptureInfo")) return rc;
     const bool captured = state != hipStreamCaptureStatusNone;
-    WideScratch* c = nullptr;
-    if (int rc = other_scratch(b, plan, captured ? capture : 0, captured ? s : nullptr, &m, &c)) return rc;
-    if (!captured)
-        if (int rc = check_hip(hipStreamWaitEvent(s, b->wide_done, 0), "hipStreamWaitEvent")) return rc;
-    int rc = captured || !c->cleared ? wide_clear(w, m, s) : ABM_OK;
-    c->cleared = rc == ABM_OK;
+    if (s) {
+        WideScratch* c = nullptr;
+        if (int rc = other_scratch(b, plan, captured ? capture : 0, captured ? s : nullptr, &m, &c)) return rc;
+        clean = &c->clean;
+        if (!captured)
+            if (int rc = check_hip(hipStreamWaitEvent(s, b->wide_done, 0), "hipStreamWaitEvent")) return rc;
+    }
+    // The last launch of a step leaves the cue counts 0.  After a call that failed
+    // before it, and on new scratch (a graph's first replay), they are cleared first.
+    int rc = captured || !*clean ? wide_clear(w, m, s) : ABM_OK;
+    *clean = false;
     if (!rc) rc = wide_launches(b, w, m, st, uniforms, words, offset, count, used, status, field_bits, s, mt);
-    if (captured) return rc;
+    *clean = rc == ABM_OK && !captured;
+    if (!s || captured) return rc;
     const int done = check_hip(hipEventRecord(b->wide_done, s), "hipEventRecord");
     if (done) (void)hipDeviceSynchronize();   // no event to wait for: nothing may be left
     return rc ? rc : done;

@@ -20,6 +20,7 @@ struct WidePlan {
     int32_t chunks = 0, max_rays = 0;
     int64_t keys = 0;
     void* mem = nullptr;
+    bool clean = false;                // its cue counts are 0 (each step leaves them so)
 };
 
 // Scratch of a plan's steps elsewhere than on the null stream: one for all other
@@ -29,8 +30,8 @@ struct WideScratch {
     int plan = 0;
     unsigned long long capture = 0;
     hipStream_t stream = nullptr;
-    bool cleared = false;              // its control words
     void* mem = nullptr;
+    bool clean = false;                // as WidePlan's
     WideScratch* next = nullptr;
 };
 

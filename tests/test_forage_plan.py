@@ -123,3 +123,25 @@ def test_captured_steps_have_scratch_of_their_own(standin):
         lib.abm_forage_batch_destroy(h)
         assert held()[0] == 0
         """)
+
+
+@pytest.mark.parametrize("stream", [None, 64])
+def test_a_step_cut_short_leaves_no_cues(standin, stream):
+    # the cues are counted by the first launch and cleared by the last: after a
+    # call that failed between them the next one clears them first
+    hip_standin.run(standin, f"""
+        s = {stream}
+        h = forage_batch(replica(200))
+        assert forage_step(h, s) == 0
+        one = ["wide_drive_kernel", "wide_field_kernel", "wide_move_kernel"]
+        for which in (1, 2, 3):
+            fail("hipLaunchKernel", which)
+            assert forage_step(h, s) == L.ABM_ERR_HIP
+            fail("hipLaunchKernel", 1)
+            assert forage_step(h, s) == L.ABM_ERR_HIP   # the clearing itself
+            log()
+            assert forage_step(h, s) == 0
+            assert kernels(log()) == ["wide_clear_kernel"] + one
+            assert forage_step(h, s) == 0
+            assert kernels(log()) == one
+        """)
