@@ -206,7 +206,7 @@ vf_step_f64_kernel(const VFRep* __restrict__ reps, const double* __restrict__ tc
 // sums meet by DPP.  Bound by VALU
 // issue (batches) or the id-order chain's latency (few replicas).  Against the
 // plain kernel (exact decisions, a byte per ray, tables from memory): 4096
-// replicas of 50 agents at R = 512 0.773 -> 0.169 ms a step (1332 -> 461 VALU
+// replicas of 50 agents at R = 512 0.773 -> 0.168 ms a step (1332 -> 461 VALU
 // instructions per agent-step, an eighth of them the motion's sincos; 0.91 of
 // the VALU issue slots filled), 512 of 37 at R = 300 in a walled arena 0.265 ->
 // 0.088 ms.
@@ -272,17 +272,47 @@ __device__ inline double dpp_f64(double v) {
     return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true),
                             __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true));
 }
-// Wave sum, to every lane: quads, half rows, rows (every lane its row's), then
-// rows carried up to lane 63.
-__device__ inline double wave_total_f64(double x) {
-    x += dpp_f64<0xB1>(x);
+__device__ inline double lane_f64(double x, int l) {
+    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), l),
+                            __builtin_amdgcn_readlane(__double2loint(x), l));
+}
+// The wave sums of four values, to every lane, in one pass over lanes 32, 16, 8,
+// 4, 2 and 1 apart (the plain kernel's order).  A swap of halves leaves the first
+// value's pairs in the lower lanes and the second's in the upper ones, a swap of
+// rows one value a row: 29 instructions, where two sums by themselves are 40.
+__device__ inline void wave_totals_f64(double (&c)[4]) {
+    double h[2];
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {   // c[2q] | c[2q + 1]
+        const auto lo = __builtin_amdgcn_permlane32_swap((uint32_t)__double2loint(c[2 * q]), (uint32_t)__double2loint(c[2 * q + 1]), false, false);
+        const auto hi = __builtin_amdgcn_permlane32_swap((uint32_t)__double2hiint(c[2 * q]), (uint32_t)__double2hiint(c[2 * q + 1]), false, false);
+        h[q] = __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);
+    }
+    const auto lo = __builtin_amdgcn_permlane16_swap((uint32_t)__double2loint(h[0]), (uint32_t)__double2loint(h[1]), false, false);
+    const auto hi = __builtin_amdgcn_permlane16_swap((uint32_t)__double2hiint(h[0]), (uint32_t)__double2hiint(h[1]), false, false);
+    double x = __hiloint2double((int)hi[0], (int)lo[0]) + __hiloint2double((int)hi[1], (int)lo[1]);   // by row: c[0], c[2], c[1], c[3]
+    x += dpp_f64<0x128>(x);
+    x += dpp_f64<0x124>(x);
     x += dpp_f64<0x4E>(x);
-    x += dpp_f64<0x141>(x);
-    x += dpp_f64<0x140>(x);
-    x += f32::dpp_f64_masked<0x142, 0xa>(x);
-    x += f32::dpp_f64_masked<0x143, 0xc>(x);
-    return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(x), 63),
-                            __builtin_amdgcn_readlane(__double2loint(x), 63));
+    x += dpp_f64<0xB1>(x);
+    c[0] = lane_f64(x, 0); c[2] = lane_f64(x, 16); c[1] = lane_f64(x, 32); c[3] = lane_f64(x, 48);
+}
+
+// The sums over the workgroup's NW waves, by way of red (4 NW doubles).
+template <int NW>
+__device__ inline void block_totals_f64(double (&c)[4], double* red) {
+    wave_totals_f64(c);
+    if (NW == 1) return;
+    if ((threadIdx.x & 63) == 0)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) red[4 * (threadIdx.x >> 6) + q] = c[q];
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        c[q] = 0.0;
+#pragma unroll
+        for (int w = 0; w < NW; ++w) c[q] += red[4 * w + q];
+    }
 }
 
 // OR the rays [a, b) into the field: one or two words nearly always.
@@ -424,32 +454,20 @@ vf_step_f64_guard_kernel(const VFRep* __restrict__ reps, const int32_t* __restri
         }
         const double alp0 = S.a0[k], bet0 = S.b0[k], vel = S.v[k];
         const double ae0 = alp0 * rp->alp1, be0 = bet0 * rp->bet1;
-        // blob terms: trapz(cos(PHI) * (-V)) = -sum(w cos V)
-        double Sv, Sp, ab = 0.0, ae = 0.0, bb = 0.0, be = 0.0;
-        if (!want_diag) {
-            Sv = wave_total_f64(__builtin_fma(ae0, ec, -(alp0 * bc)));
-            Sp = wave_total_f64(__builtin_fma(be0, es, -(bet0 * bs)));
-            if (NW > 1) {
-                if (lane == 0) { S.red[2 * (tid >> 6)] = Sv; S.red[2 * (tid >> 6) + 1] = Sp; }
-                __syncthreads();
-                Sv = Sp = 0.0;
-#pragma unroll
-                for (int w = 0; w < NW; ++w) { Sv += S.red[2 * w]; Sp += S.red[2 * w + 1]; }
-            }
-        } else {
-            double c[4] = {wave_total_f64(bc), wave_total_f64(bs), wave_total_f64(ec), wave_total_f64(es)};
-            if (NW > 1) {
-                if (lane == 0)
-                    for (int q = 0; q < 4; ++q) S.red[4 * (tid >> 6) + q] = c[q];
-                __syncthreads();
-                for (int q = 0; q < 4; ++q) {
-                    c[q] = 0.0;
-                    for (int w = 0; w < NW; ++w) c[q] += S.red[4 * w + q];
-                }
-            }
-            ab = alp0 * -c[0]; bb = bet0 * -c[1]; ae = ae0 * c[2]; be = be0 * c[3];
-            Sv = ab + ae;
-            Sp = bb + be;
+        // blob terms: trapz(cos(PHI) * (-V)) = -sum(w cos V).  The speed's two sums
+        // are weighted and added by lane, which rounds least; the heading's stay
+        // apart, as the plain kernel has them: in a field that mirrors itself each
+        // cancels, and a residue could take a heading of 0 to 2 pi.
+        double c[4] = {__builtin_fma(ae0, ec, -(alp0 * bc)), bs, es, 0.0};
+        block_totals_f64<NW>(c, S.red);
+        const double Sv = c[0];
+        double bb = bet0 * -c[1], be = be0 * c[2], ab = 0.0, ae = 0.0;
+        const double Sp = __builtin_fma(be0, c[2], bb);
+        if (want_diag) {
+            double d[4] = {bc, ec, 0.0, 0.0};
+            if (NW > 1) __syncthreads();   // red is read
+            block_totals_f64<NW>(d, S.red);
+            ab = alp0 * -d[0]; ae = ae0 * d[1];
         }
         if (bits_out) {
             uint32_t* dst = bits_out + rp->field_offset + (int64_t)k * W;
