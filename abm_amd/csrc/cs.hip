@@ -209,9 +209,8 @@ __device__ inline CSFocal cs_focal(const CSArgs& A, int f) {
     F.cy = F.py + F.radius;
     double sn, cs;
     if (!f32::sincos_f64_small(F.theta, &sn, &cs)) sincos(F.theta, &sn, &cs);
-    const bool kept = heading_kept(F.px, F.py, F.radius);   // else NaN, which no guard lets through
-    F.ux = kept ? (float)cs : NAN;
-    F.uy = kept ? -(float)sn : NAN;
+    F.ux = heading_kept(F.px, F.py, F.radius) ? (float)cs : NAN;   // NaN: no guard lets it through
+    F.uy = -(float)sn;
     return F;
 }
 

@@ -122,7 +122,7 @@ ABM_HD Focal make_focal(double px, double py, double theta, double radius) {
 // radius: below 6e-7 up to 3e9 radii, but bins apart from the heading at 1e11.
 // At radius 0 it has none, and at a negative one the opposite.
 ABM_HD bool heading_kept(double px, double py, double radius) {
-    return radius > 0.0 && fabs(px) <= 1e9 * radius && fabs(py) <= 1e9 * radius;
+    return fmax(fabs(px), fabs(py)) < 1e9 * radius;
 }
 
 // Raster decision of one object for the VSWRM field (vf_supcalc.py:55-119).

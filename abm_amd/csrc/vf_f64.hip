@@ -367,7 +367,7 @@ vf_step_f64_guard_kernel(const VFRep* __restrict__ reps, const int32_t* __restri
         S.v0[i] = st.v0 ? st.v0[g] : rp->v0;
         const double2 sc = sincos_f64(th);
         // unit(v1) = (cos th, -sin th), or NaN, which no guard lets through
-        S.u[i] = heading_kept(S.x[i], S.y[i], (double)S.rad[i]) ? make_float2((float)sc.y, -(float)sc.x) : make_float2(NAN, NAN);
+        S.u[i] = make_float2(heading_kept(S.x[i], S.y[i], (double)S.rad[i]) ? (float)sc.y : NAN, -(float)sc.x);
         if (sync_order) { S.ox[i] = S.x[i]; S.oy[i] = S.y[i]; }
     }
     const bool torus = rp->boundary == ABM_BOUNDARY_INFINITE;
