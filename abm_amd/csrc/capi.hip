@@ -366,7 +366,7 @@ int abm_vf_batch_create(const abm_vf_replica* reps, int32_t n, abm_vf_batch** ou
         if (!rc && max_r <= 2048)
             rc = check_hip(hipMalloc(&bt->chain_u, sizeof(float) * 2 * (size_t)max_n), "hipMalloc(chain u)");
         if (!rc && max_r <= 2048)
-            rc = check_hip(hipMalloc(&bt->chain_dep, kChainDepBytes * (size_t)max_n), "hipMalloc(chain dependences)");
+            rc = check_hip(hipMalloc(&bt->chain_dep, chain_dep_bytes(max_n)), "hipMalloc(chain dependences)");
     }
     if (!rc) {
         bt->tab_sin = bt->tab_cos + ray_total;
@@ -514,7 +514,7 @@ int abm_vf_set_launch(abm_vf_batch* b, int32_t waves) {
         if (!rc && !b->chain_fields)
             rc = check_hip(hipMalloc(&b->chain_fields, sizeof(uint32_t) * n * words), "hipMalloc(chain fields)");
         if (!rc && !b->chain_u) rc = check_hip(hipMalloc(&b->chain_u, sizeof(float) * 2 * n), "hipMalloc(chain u)");
-        if (!rc && !b->chain_dep) rc = check_hip(hipMalloc(&b->chain_dep, kChainDepBytes * n), "hipMalloc(chain dependences)");
+        if (!rc && !b->chain_dep) rc = check_hip(hipMalloc(&b->chain_dep, chain_dep_bytes(n)), "hipMalloc(chain dependences)");
         if (rc) return rc;
     }
     b->waves_per_group = waves;

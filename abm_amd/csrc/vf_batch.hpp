@@ -66,6 +66,8 @@ constexpr int kBigClass = 64;
 // Bytes of an agent's dependences in the chain step (64 indices, its segment's
 // 256 bits and a count).
 constexpr size_t kChainDepBytes = 100;
+// Those of n agents, and a count of the step's segments.
+constexpr size_t chain_dep_bytes(size_t n) { return kChainDepBytes * n + sizeof(int32_t); }
 
 // The push kernel (one workgroup of 8 waves per replica): rays per lane of
 // its summing wave for a launch whose largest R is r (the one-wave

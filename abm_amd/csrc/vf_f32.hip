@@ -1618,8 +1618,13 @@ __device__ inline void chain_barrier() {
 // order and this: 8192 agents, a twelfth of the others in sight, R = 2048, 9.12
 // and 3.29 ms; 2100 agents with walls at R = 2048, a third in sight 2.98 and 1.93,
 // 0.7 3.94 and 3.47, 0.85 4.48 and 4.92 (hence kFlowShare).
+// A segment with a jump stops at once, and a step in which most segments had one
+// starts the others in id order (kFlowMisses): of the 8192 agents, all jumping
+// 11.41 ms to the end of every segment and 8.96 so, 148 in 30 of 32 segments 10.96
+// and 8.98, 11 in ten 5.87 and 5.36 (id order alone 9.0 here, each time).
 constexpr float kFlowMargin = 16.f;   // + 4 |v|: the displacement allowed for
 constexpr float kFlowShare = 0.7f;    // of a segment's pairs that may depend
+constexpr int kFlowMisses = 2;        // segments taken again, beyond twice the others, that a step tries
 constexpr int kFlowSpins = 1 << 20;   // waits end (the dependences are acyclic); the bound is never met
 
 constexpr int kDepWords = kChainSeg / 64;
@@ -1634,7 +1639,9 @@ static_assert(kChainDepBytes == 64 + 8 * kDepWords + 4, "an agent's dependences"
 // agents then load in one go, where a wave made its list from the bits).
 __global__ void __launch_bounds__(256)
 vf_step_f32_depend_kernel(const VFRep* __restrict__ rp, abm_vf_state_f32 st, float cull_c,
-                          uint8_t* __restrict__ first, uint64_t* __restrict__ dep, int32_t* __restrict__ pend) {
+                          uint8_t* __restrict__ first, uint64_t* __restrict__ dep, int32_t* __restrict__ pend,
+                          int32_t* __restrict__ missed) {
+    if (blockIdx.x == 0 && threadIdx.x == 0) *missed = 0;   // segments of this step not done by dependence
     const RepConst C = rep_const(rp);
     const int lane = threadIdx.x & 63;
     const int a = __builtin_amdgcn_readfirstlane(blockIdx.x * 4 + (threadIdx.x >> 6));
@@ -1685,8 +1692,8 @@ vf_step_f32_segment_kernel(const VFRep* __restrict__ rp, const RayTab32* __restr
                            abm_vf_state_f32 st, const uint32_t* __restrict__ fields,
                            const float2* __restrict__ ustart, uint32_t* __restrict__ bits_out,
                            float* __restrict__ diag, uint32_t flags, unsigned long long* __restrict__ counters,
-                           const uint8_t* __restrict__ first_all, const uint64_t* __restrict__ dep_all, const int32_t* __restrict__ pend_all,
-                           float cull_c, int s0, int n) {
+                           const uint8_t* __restrict__ first_all, const uint64_t* __restrict__ dep_all, int32_t* pend_all,
+                           int32_t* missed, float cull_c, int s0, int n) {
     __shared__ uint32_t rows[kChainSeg][64];
     __shared__ float4 srec[kChainSeg];     // start poses (x, y, radius, theta)
     __shared__ float2 su[kChainSeg];       // start heading vectors
@@ -1774,6 +1781,13 @@ vf_step_f32_segment_kernel(const VFRep* __restrict__ rp, const RayTab32* __restr
             if (fabsf(dy) > C.hh) dy = dy > 0.f ? dy - C.fH : dy + C.fH;
         }
     };
+    // A segment not done by dependence: where that is the rule, the next one's
+    // first agent is marked as on a torus too small.
+    auto miss = [&]() {
+        if (tid != 0 || s0 + n >= C.N) return;
+        const int times = atomicAdd(missed, 1) + 1, q = pend_all[s0 + n];
+        if (times > 2 * (s0 / kChainSeg + 1 - times) + kFlowMisses && q >= 0) pend_all[s0 + n] = ~q;
+    };
     bool flow = false;
     if (may_flow) {   // uniform: the dependences, and whether they are few
         uint64_t* flat = &dep[0][0];
@@ -1792,6 +1806,7 @@ vf_step_f32_segment_kernel(const VFRep* __restrict__ rp, const RayTab32* __restr
         if (lane == 63 && total > 0) atomicAdd(&ctl[2], total);
         __syncthreads();
         flow = ctl[3] == 0 && ctl[2] <= kFlowShare * n * n / 2;
+        if (ctl[3] != 0) miss();
     }
     if (flow) {
         for (int m = tid; m < n; m += kChainThreads)
@@ -1812,6 +1827,7 @@ vf_step_f32_segment_kernel(const VFRep* __restrict__ rp, const RayTab32* __restr
                 if (lane == 0) ctl[3] = 1;
                 break;
             }
+            if (m >= n) break;   // stopped
             asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
             const int gk = C.a0 + s0 + m;
             const float4 pk = srec[m], dk = sdyn[m];
@@ -1834,10 +1850,6 @@ vf_step_f32_segment_kernel(const VFRep* __restrict__ rp, const RayTab32* __restr
             const float4 moved = make_float4(nx, ny, pk.z, o);
             if (!PLAIN && bits_out && lane < C.W) bits_out[C.field_offset + (int64_t)(s0 + m) * C.W + lane] = rows[m][lane];
             if (lane == 0) {
-                float dx = nx - pk.x, dy = ny - pk.y;
-                image(dx, dy);
-                const float mg = margin(dk.x);
-                if (!(fmaf(dy, dy, dx * dx) <= mg * mg)) ctl[3] = 1;
                 srec[m] = moved;   // its start pose is read no more
                 sdyn[m].x = vel;
                 if (want_diag) {
@@ -1872,6 +1884,18 @@ vf_step_f32_segment_kernel(const VFRep* __restrict__ rp, const RayTab32* __restr
                 asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the field first, then the count
                 if (atomicSub(&pend[mm], 1) == 1) *(volatile int*)&ready[atomicAdd(&ctl[1], 1)] = mm;
             }
+            // (its dependents do not wait for this)
+            float jx = nx - pk.x, jy = ny - pk.y;
+            image(jx, jy);
+            const float mg = margin(dk.x);
+            if (!(fmaf(jy, jy, jx * jx) <= mg * mg)) {   // stop: no wave takes or awaits another agent
+                if (lane == 0) {
+                    ctl[3] = 1;
+                    atomicAdd(&ctl[0], n);
+                }
+                for (int i = lane; i < n; i += 64)
+                    if (ready[i] < 0) *(volatile int*)&ready[i] = n;
+            }
             wave_lds_sync();   // after[] is read before the next agent's
         }
         __syncthreads();
@@ -1886,6 +1910,7 @@ vf_step_f32_segment_kernel(const VFRep* __restrict__ rp, const RayTab32* __restr
             }
             return;
         }
+        miss();
         load();   // again, in id order
         __syncthreads();
     }
@@ -2138,9 +2163,10 @@ int launch_chain(abm_vf_batch* b, const abm_vf_state_f32* st, uint32_t* bits, fl
         uint8_t* first = (uint8_t*)b->chain_dep;
         uint64_t* dep = (uint64_t*)(first + (size_t)b->max_agents * 64);
         int32_t* pend = (int32_t*)(dep + (size_t)b->max_agents * kDepWords);
+        int32_t* missed = pend + b->max_agents;
         if (!counting) {
             hipLaunchKernelGGL(vf_step_f32_depend_kernel, dim3((N + 3) / 4), dim3(256), 0, s, b->reps_dev + rep, *st,
-                               cull_c, first, dep, pend);
+                               cull_c, first, dep, pend, missed);
             if (int rc2 = check_hip(hipGetLastError(), "vf_step_f32_depend_kernel launch")) return rc2;
         }
         for (int s0 = 0; s0 < N; s0 += kChainSeg) {
@@ -2154,7 +2180,7 @@ int launch_chain(abm_vf_batch* b, const abm_vf_state_f32* st, uint32_t* bits, fl
                            b->reps_dev + rep, b->tab32, *st, (const uint32_t*)b->chain_fields,             \
                            (const float2*)b->chain_u, bits, diag, flags, b->counters, (const uint8_t*)first,       \
                            (const uint64_t*)dep,                                                            \
-                           (const int32_t*)pend, cull_c, s0, n);
+                           pend, missed, cull_c, s0, n);
             ABM_SEGMENT(4) ABM_SEGMENT(8) ABM_SEGMENT(16) ABM_SEGMENT(32)
 #undef ABM_SEGMENT
             if (int rc2 = check_hip(hipGetLastError(), "vf_step_f32_segment_kernel launch")) return rc2;
