@@ -2090,12 +2090,12 @@ wide_drive_kernel(const FGRep* __restrict__ reps, int n_chunks, abm_forage_state
     }
 }
 
-// One wave per agent, sixteen blocks per chunk: its field from the cues, the
-// counts and whether it walks.  With device generators the first n_reps blocks
-// make each replica's next 2N words meanwhile.
+// One wave per agent, sixteen blocks per chunk from first_chunk on: its field
+// from the cues, the counts and whether it walks.  With device generators the
+// first n_reps blocks make each replica's next 2N words meanwhile.
 template <bool FIELDS>
 __global__ void __launch_bounds__(256)
-wide_field_kernel(const FGRep* __restrict__ reps, int n_reps, abm_forage_state st, WideMem M,
+wide_field_kernel(const FGRep* __restrict__ reps, int n_reps, int first_chunk, abm_forage_state st, WideMem M,
                   const abm_mt19937_state* __restrict__ mt, uint32_t* __restrict__ bits_out) {
 #pragma clang fp contract(off)
     extern __shared__ uint32_t lds_u[];
@@ -2127,7 +2127,7 @@ wide_field_kernel(const FGRep* __restrict__ reps, int n_reps, abm_forage_state s
         }
         block -= n_reps;
     }
-    const int chunk = block >> 4, q = M.of[chunk], chunk0 = M.rep[q].chunk0;
+    const int chunk = first_chunk + (block >> 4), q = M.of[chunk], chunk0 = M.rep[q].chunk0;
     const int32_t* const ctl = M.ctl + kWdWords * q;
     if (ctl[kWdSkip]) return;
     const FGRep& P = reps[M.rep[q].rb];
@@ -3429,10 +3429,11 @@ int take_path(abm_forage_batch* bt, int path) {
 // 0.126, 0.126, 0.179); four where more workgroups than two per CU queue and no
 // replica has work for more (1000 replicas of 10 agents: 0.048 ms with four,
 // 0.070 with sixteen; of 50: 0.068, 0.090; of 128: 0.121, 0.137).  Fewer too
-// where the waves' fields would not fit in LDS.
+// where the waves' fields would not fit in LDS, or a launch would have 2^32 threads.
 int upd_waves(const ForageClass& c, int cus) {
     int waves = c.count > 2 * cus && c.max_agents <= 128 ? 4 : 16;
-    while (waves > 4 && upd_lds_bytes(c.max_agents, c.max_rays, waves) > (size_t)163840 - sizeof(FGRep))
+    while (waves > 4 && (upd_lds_bytes(c.max_agents, c.max_rays, waves) > (size_t)163840 - sizeof(FGRep) ||
+                         ((int64_t)c.count * 64 * waves) >> 32 != 0))
         waves /= 2;
     return waves;
 }
@@ -3446,6 +3447,10 @@ int check_state(const abm_forage_state* st, const char* who) {
     return ABM_OK;
 }
 
+// A launch has fewer than 2^32 threads: 64-agent chunks per field launch (2^30
+// threads, beside one workgroup per replica).
+constexpr int kFieldChunks = 1 << 18;
+
 // Agent.update of a plan's replicas (see wide_drive_kernel) on scratch m.
 int wide_launches(const abm_forage_batch* b, const WidePlan& plan, const WideMem& m, const abm_forage_state* st,
                   const double* uniforms, const uint32_t* words, const int64_t* offset, const int32_t* count,
@@ -3457,9 +3462,13 @@ int wide_launches(const abm_forage_batch* b, const WidePlan& plan, const WideMem
                        (words || mt) ? 1 : 0, m);
     if (int rc = check_hip(hipGetLastError(), "wide_drive_kernel launch")) return rc;
     const size_t lds = sizeof(uint32_t) * (size_t)std::max(kMtN, 4 * W);
-    hipLaunchKernelGGL(field_bits ? wide_field_kernel<true> : wide_field_kernel<false>,
-                       dim3(16 * chunks + (mt ? n : 0)), dim3(256), lds, s, reps, n, *st, m, mt, field_bits);
-    if (int rc = check_hip(hipGetLastError(), "wide_field_kernel launch")) return rc;
+    for (int c = 0; c < chunks; c += kFieldChunks) {
+        const abm_mt19937_state* gen = c == 0 ? mt : nullptr;
+        hipLaunchKernelGGL(field_bits ? wide_field_kernel<true> : wide_field_kernel<false>,
+                           dim3(16 * std::min(kFieldChunks, chunks - c) + (gen ? n : 0)), dim3(256), lds, s, reps, n, c,
+                           *st, m, gen, field_bits);
+        if (int rc = check_hip(hipGetLastError(), "wide_field_kernel launch")) return rc;
+    }
     hipLaunchKernelGGL(wide_move_kernel, dim3(blocks), dim3(256), 0, s, reps, chunks, *st, uniforms, words, offset,
                        count, used, status, mt, m);
     if (int rc = check_hip(hipGetLastError(), "wide_move_kernel launch")) return rc;

@@ -112,8 +112,8 @@ hipError_t __hipPopCallConfiguration(dim3* g, dim3* b, size_t* lds, hipStream_t*
     *g = config.grid; *b = config.block; *lds = config.lds; *s = config.stream;
     return hipSuccess;
 }
-hipError_t hipLaunchKernel(const void* f, dim3 g, dim3, void**, size_t, hipStream_t s) {
-    if (fails("hipLaunchKernel")) {
+hipError_t hipLaunchKernel(const void* f, dim3 g, dim3 b, void**, size_t, hipStream_t s) {
+    if (fails("hipLaunchKernel") || (uint64_t)g.x * b.x >> 32 != 0) {   // (a launch takes fewer than 2^32 threads)
         note("failed launch");
         return pending = hipErrorLaunchFailure;
     }

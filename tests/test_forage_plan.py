@@ -145,3 +145,18 @@ def test_a_step_cut_short_leaves_no_cues(standin, stream):
             assert forage_step(h, s) == 0
             assert kernels(log()) == one
         """)
+
+
+def test_many_agents_take_several_launches(standin):
+    # 67 million agents, beyond the 2^32 threads of one launch at a wave each
+    hip_standin.run(standin, """
+        h = forage_batch(*[replica(65536)] * 1025)
+        log()
+        assert forage_step(h) == 0
+        grids = [int(ln.split()[2]) for ln in log() if "wide_field_kernel" in ln]
+        assert sum(grids) == 16 * 1025 * 1024 and len(grids) > 1 and max(grids) * 256 < 1 << 32
+        h = forage_batch(replica(200), *[replica(1)] * 4200000)   # 16 waves each would be beyond it
+        log()
+        assert forage_step(h) == 0
+        assert kernels(log()) == ["forage_update_kernel"]
+        """)
