@@ -547,8 +547,10 @@ int abm_vf_autotune(abm_vf_batch* b, const abm_vf_state_f32* st, int32_t trial_s
     // candidates: waves per replica of the per-replica kernel (> 0), or minus the
     // replicas per wave of the grouped kernel
     // (16: the 16-wave kernel for every replica; 32: the push kernel for
-    // every replica; 0: the size classes, the per-replica kernel up to
-    // kBigClass agents and the push or 16-wave kernel above)
+    // every replica; 0: the automatic choice for batches with both size
+    // classes or large replicas, the push kernel for all where the CUs hold them
+    // at once, else the per-replica kernel up to kBigClass agents and the push or
+    // 16-wave kernel above)
     std::vector<int> cand{1, 2, 4};
     if (b->max_agents <= 2048) cand.push_back(16);
     if (push_fits(b, true)) cand.push_back(32);

@@ -3679,7 +3679,10 @@ int abm_forage_batch_create(const abm_forage_replica* reps, int32_t n, abm_forag
     if (!rc) rc = check_hip(hipDeviceGetAttribute(&dev_max, hipDeviceAttributeMaxSharedMemoryPerBlock,
                                                   bt->device), "hipDeviceGetAttribute");
     // a replica beyond one workgroup's LDS is updated over the whole GPU,
-    // without visual exclusion and with at most 8192 rays
+    // without visual exclusion and with at most 8192 rays.  One measure for all:
+    // the step kernel's layout, the largest (172 bytes an agent and a byte a ray,
+    // where the update kernel needs 152 and its waves' fields), so what a batch
+    // accepts does not depend on the kernel that takes a replica
     bt->too_big.assign(n, 0);
     bt->exclusion.assign(n, 0);
     for (int b = 0; !rc && b < n; ++b) {
@@ -3930,6 +3933,8 @@ int world_run(abm_forage_world* w, int32_t phase, const abm_forage_state* st, in
         return set_error(ABM_ERR_INVALID, "%s: every patch array is required", who);
     if (!ps->count) return set_error(ABM_ERR_INVALID, "%s: patch count array is required", who);
     abm_forage_batch* b = w->batch;
+    // (the masks of replicas above kWorldBlockAgents lie in global memory, which
+    // does not need this limit; worlds beyond it are untested and refused)
     if (w->member_lds > 65536)
         return set_error(ABM_ERR_UNSUPPORTED, "%s: %zu B of membership masks", who, w->member_lds);
     if (phase == ABM_WORLD_STEP && w->collide_lds > 0) {

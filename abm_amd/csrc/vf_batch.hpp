@@ -130,7 +130,7 @@ struct abm_vf_batch {
     void* grid_param = nullptr;     // wide step: the grid of the current replica (WideGrid)
     uint32_t* chain_fields = nullptr;   // chain step: every agent's field (max_agents x words)
     void* chain_u = nullptr;        // chain step: start heading vectors (float2 per agent)
-    void* chain_dep = nullptr;      // chain step: dependences (64 bytes, four 64-bit words, an int32 per agent)
+    void* chain_dep = nullptr;      // chain step: dependences (64 bytes, four 64-bit words, an int32 per agent), a count
     int32_t min_agents = 0;         // of the smallest replica
     abm::GroupPlan gplan[3];        // G = 1, 2, 4
     // host copies

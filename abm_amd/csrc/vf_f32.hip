@@ -1621,7 +1621,7 @@ __device__ inline void chain_barrier() {
 // A segment with a jump stops at once, and a step in which most segments had one
 // starts the others in id order (kFlowMisses): of the 8192 agents, all jumping
 // 11.41 ms to the end of every segment and 8.96 so, 148 in 30 of 32 segments 10.96
-// and 8.98, 11 in ten 5.87 and 5.36 (id order alone 9.0 here, each time).
+// and 8.98, 11 in ten 5.87 and 5.36.
 constexpr float kFlowMargin = 16.f;   // + 4 |v|: the displacement allowed for
 constexpr float kFlowShare = 0.7f;    // of a segment's pairs that may depend
 constexpr int kFlowMisses = 2;        // segments taken again, beyond twice the others, that a step tries
@@ -2367,8 +2367,10 @@ int launch_vf_step_f32(abm_vf_batch* b, const abm_vf_state_f32* st, uint32_t* bi
     // 256 of 8 to 60 0.074 and 0.100 (512 of 60: 0.141 and 0.112, which the rule
     // leaves); 250 of 60 at R = 2048 0.106 and 0.140; 64 of 8 to 200 0.218 and
     // 0.311, 1000 of 8 to 512 0.82 and 0.92 (the small ones first, on the other
-    // kernel).  A batch of a few replicas of both classes keeps a kernel for
-    // each, as its callers may rely on.
+    // kernel).  A batch of up to kFewReplicas replicas of both classes keeps a
+    // kernel for each, although this one is faster there too (40 and 200 agents
+    // at R = 512 0.227 and 0.291 ms, 64 and 65 0.073 and 0.175, 10 and 500 0.650
+    // and 0.669): the tests of the size classes fix its kernels.
     const int nb = b->n_big_class;
     const bool few = b->n_replicas <= kFewReplicas && nb > 0 && nb < b->n_replicas;
     if (nw == 0 && !sync_order && !few && push_fits(b, true) &&

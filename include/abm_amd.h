@@ -57,7 +57,11 @@ extern "C" {
 #define ABM_ORDER_SEQUENTIAL  0u  /* reference order: agent k sees agents <k moved      */
 #define ABM_ORDER_SYNCHRONOUS 1u  /* every field from the pre-step poses (not reference) */
 #define ABM_WANT_DIAG         2u  /* write per-agent (dv, dpsi, a_blob, a_edge, b_blob, b_edge) */
-#define ABM_COUNT_RECHECKS    4u  /* fused step: count pairs and float64 re-checks       */
+#define ABM_COUNT_RECHECKS    4u  /* fused step: count pairs and float64 re-checks;
+                                     float64 step: count near ties, which decides every
+                                     pair in float64 in a kernel of its own (the same
+                                     decisions and fields; the sums, and so the poses,
+                                     differ in the last bits)                            */
 #define ABM_VERIFY_FAST_PATH  8u  /* fused step: also decide every pair in float64 and
                                      count float32 decisions that differ (testing)     */
 #define ABM_KAHAN_SUMS       16u  /* fused step, grouped kernel: Kahan-compensated ray
@@ -386,11 +390,12 @@ int abm_forage_batch_get_offsets(const abm_forage_batch* batch, int32_t* agent_o
                                  int64_t* field_offset);
 
 /* One Agent.update for every agent, reference order, float64.  One
- * workgroup per replica holds the replica in LDS: about 172 bytes per agent
- * plus one byte per ray, so up to about 920 agents per replica at R = 1200 on
- * gfx950 (160 KB).  Larger replicas (up to 65536 agents) are updated over the
- * whole GPU (see abm_forage_set_path); with visual exclusion they get
- * ABM_ERR_UNSUPPORTED from abm_forage_batch_create. */
+ * workgroup per replica holds the replica in LDS, counted as 172 bytes per agent
+ * plus one byte per ray (the largest layout of the kernels), so up to about 920
+ * agents per replica at R = 1200 on gfx950 (160 KB).  Larger replicas (up to 65536
+ * agents) are updated over the whole GPU, and so are, by default, large ones of
+ * small batches (see abm_forage_set_path); with visual exclusion a larger replica
+ * gets ABM_ERR_UNSUPPORTED from abm_forage_batch_create. */
 /* Arguments:
  * uniforms: per replica, a device array of the next numpy legacy-MT19937
  *   doubles (random_sample) of the global stream, uniform_offset[b] its start
@@ -490,6 +495,12 @@ typedef struct abm_patch_state {
     double* quality;              /* unit_per_timestep */
 } abm_patch_state;
 
+/* A world keeps its replicas' pending placements and the scratch of their loops
+ * from one call to the next, so its calls belong to one state and one set of
+ * patches and are to be in order (one stream, or events between them).  Several
+ * worlds may share a batch and run on streams and threads of their own.  A call
+ * gets ABM_ERR_UNSUPPORTED where n_patches x ceil(n_agents / 64) words of
+ * membership masks of some replica exceed 64 KB (64 patches: 8192 agents). */
 typedef struct abm_forage_world abm_forage_world;   /* opaque */
 
 int abm_forage_world_create(abm_forage_batch* batch, const abm_forage_world_params* params_host,
