@@ -1272,7 +1272,10 @@ vf_step_f32_push_kernel(const VFRep* __restrict__ reps, const int32_t* __restric
     float2* U = reinterpret_cast<float2*>(p); p += sizeof(float2) * (size_t)C.N;     // (cos, -sin) of start headings
     uint32_t* queue = reinterpret_cast<uint32_t*>(p); p += sizeof(uint32_t) * kPushQueue * kPushWaves;
     uint32_t* F = reinterpret_cast<uint32_t*>(p);                                     // [N][W + 1] fields
-    __shared__ double red[2][6];   // Sv, Sp, Bc, Bs, Ec, Es of agents k and k + 1
+    // Sv, Sp, Bc, Bs, Ec, Es of agents k and k + 1: in the queues' place, which are
+    // done with before the chain (a replica may fill the LDS to the last byte); 1000
+    // replicas of 8 to 512 agents 0.815 ms at the queues' start, 0.807 in their middle
+    double (*red)[6] = reinterpret_cast<double (*)[6]>(queue + kPushQueue * kPushWaves / 2);
     const float cull_c = (float)rp->cull_c;
     uint32_t* wq = queue + wave * kPushQueue;   // this wave's ring of queued pairs
     const float a0d = (float)rp->alp0, b0d = (float)rp->bet0, v0d = (float)rp->v0;
