@@ -23,6 +23,7 @@
 //   motion  -- float32 VSWRM update, Euler step, boundary (vf_agent.py:188-204,
 //              263-326; agent.py:347-395, 605-610).
 #include <cmath>
+#include <type_traits>
 
 #include "vf_f32_common.hpp"
 
@@ -1061,7 +1062,8 @@ int launch_big_any(abm_vf_batch* b, const abm_vf_state_f32* st, uint32_t* bits, 
 // of 512 threads per replica, every agent's field in LDS).  Agent m's field
 // is the OR of its pairs with every other agent j, seen at j's new pose for
 // j < m and at its start pose for j > m, and m itself at its start pose.
-// Step k of the chain (one barrier each):
+// Step k of the chain (one barrier each), where the sums are taken ahead
+// (push_ahead):
 //   * wave 0 moves agent k by the sums of its field and decides the pairs
 //     (k + 1, k) and (k + 2, k) at k's new pose;
 //   * wave 1 sums agent k + 1's field, complete but for the pair (k + 1, k),
@@ -1070,6 +1072,8 @@ int launch_big_any(abm_vf_batch* b, const abm_vf_state_f32* st, uint32_t* bits, 
 //     with the decided ones, so a wrong guess costs time and no result;
 //   * waves 2..7 decide the pairs (m, k - 1) for m > k + 1 with agent k - 1's
 //     new pose.
+// Otherwise wave 0 sums agent k's field, moves it and decides the pair (k + 1, k),
+// and waves 1..7 decide agent k - 1's other pairs.
 // The start-pose pairs (m, j > m) are decided before the chain by every
 // wave.  Pairs beyond the visibility cut-off are dropped by a cheap float32
 // test (as in the 16-wave kernel) and the rest queued, so that the exact
@@ -1248,7 +1252,8 @@ __device__ inline void push_culled_check(float4 f, float4 o, const VFRep* rp, bo
 // PLAIN: a step with no fields, diagnostics or counters out (the flags and
 // pointers that ask for them are ignored), so their tests leave the kernel.
 // HALVES: replicas up to kBigClass agents sum as two waves do (SPANS = 2).
-template <int RPL, bool PLAIN, bool HALVES>
+// AHEAD: wave 1 sums agent k + 1's field while agent k moves (push_ahead).
+template <int RPL, bool PLAIN, bool HALVES, bool AHEAD>
 __global__ void __launch_bounds__(kPushThreads) __attribute__((amdgpu_waves_per_eu(2, 2)))
 vf_step_f32_push_kernel(const VFRep* __restrict__ reps, const int32_t* __restrict__ order,
                         const RayTab32* __restrict__ tab32, abm_vf_state_f32 st,
@@ -1289,9 +1294,10 @@ vf_step_f32_push_kernel(const VFRep* __restrict__ reps, const int32_t* __restric
         sincos_f32(q.w, &sth, &cth);
         U[i] = make_float2(cth, -sth);
     }
-    // in waves 0 and 1 lane l owns rays [l RPL, (l + 1) RPL) and their table entries
+    // in the summing waves (0 and 1, or 0) lane l owns rays [l RPL, (l + 1) RPL) and
+    // their table entries
     RayTab32 T[RPL];
-    if (wave <= 1) {
+    if (wave <= (AHEAD ? 1 : 0)) {
 #pragma unroll
         for (int i = 0; i < RPL; ++i) {
             const int r = lane * RPL + i;
@@ -1341,6 +1347,7 @@ vf_step_f32_push_kernel(const VFRep* __restrict__ reps, const int32_t* __restric
                       n_disagree);
         }
     }
+    if constexpr (AHEAD) {
     // ---- where agent i will be if it keeps its heading and speed, and the
     // rays its pair (i + 1, i) then sets: a prediction, left in P1[i + 1] until
     // agent i + 1's new pose goes there
@@ -1396,18 +1403,7 @@ vf_step_f32_push_kernel(const VFRep* __restrict__ reps, const int32_t* __restric
             const Pieces guess = predicted(min(k + 1, last));
             const float fx = f0.x, fy = f0.y, fr = f0.z, fth = f0.w;
             const float alp0 = dk.y, bet0 = dk.z, v0 = dk.w;
-            if (!PLAIN) {
-                if (want_diag) { Bc = r[2]; Bs = r[3]; Ec = r[4]; Es = r[5]; }
-                if (bits_out) {   // the one pair that is not in the row
-                    if (lane == 0) {
-                        or_range(F + (size_t)k * W1, more.a0, more.b0);
-                        or_range(F + (size_t)k * W1, more.a1, more.b1);
-                    }
-                    wave_lds_sync();
-                    uint32_t* dst = bits_out + C.field_offset + (int64_t)k * C.W;
-                    for (int w = lane; w < C.W; w += 64) dst[w] = Fk[w];
-                }
-            }
+            if (!PLAIN && want_diag) { Bc = r[2]; Bs = r[3]; Ec = r[4]; Es = r[5]; }
             if (!hit) {
                 if (halves) one_wave_sums<RPL, kSpans>(Fk, T, lane, C, want_diag, alp0, bet0, more, Sv, Sp, Bc, Bs, Ec, Es);
                 else one_wave_sums<RPL>(Fk, T, lane, C, want_diag, alp0, bet0, more, Sv, Sp, Bc, Bs, Ec, Es);
@@ -1448,6 +1444,13 @@ vf_step_f32_push_kernel(const VFRep* __restrict__ reps, const int32_t* __restric
             }
             more.a0 = __builtin_amdgcn_readfirstlane(q.a0); more.b0 = __builtin_amdgcn_readfirstlane(q.b0);
             more.a1 = __builtin_amdgcn_readfirstlane(q.a1); more.b1 = __builtin_amdgcn_readfirstlane(q.b1);
+            if (!PLAIN && bits_out) {   // into agent k + 1's field, which wave 1 writes out
+                // (and may be summing with the guessed rays: the same ones, or the sums are taken again)
+                uint32_t bits = 0;
+                if (more.b0 > more.a0) bits = span_mask<32>(more.a0, more.b0, 32 * lane);
+                if (more.b1 > more.a1) bits |= span_mask<32>(more.a1, more.b1, 32 * lane);
+                if (bits) atomicOr(&F[(size_t)(k + 1) * W1 + lane], bits);
+            }
             hit = more.a0 == __builtin_amdgcn_readfirstlane(guess.a0) && more.b0 == __builtin_amdgcn_readfirstlane(guess.b0) &&
                   more.a1 == __builtin_amdgcn_readfirstlane(guess.a1) && more.b1 == __builtin_amdgcn_readfirstlane(guess.b1);
             f0 = f1; f1 = f2; u1 = u2;
@@ -1468,6 +1471,10 @@ vf_step_f32_push_kernel(const VFRep* __restrict__ reps, const int32_t* __restric
             // ---- agent k + 1's sums: its row lacks only the pair (k + 1, k),
             // whose rays are the predicted ones
             if (k + 1 < C.N) sums_into(k + 1, predicted(k + 1), red[(k + 1) & 1]);
+            if (!PLAIN && bits_out) {   // agent k's field, complete since the step before
+                uint32_t* dst = bits_out + C.field_offset + (int64_t)k * C.W;
+                for (int w = lane; w < C.W; w += 64) dst[w] = F[(size_t)k * W1 + w];
+            }
         } else if (k >= 1) {
             // ---- agent k - 1's new pose into the fields of agents k + 2 ..
             const float4 ob = P1[k - 1];
@@ -1487,6 +1494,112 @@ vf_step_f32_push_kernel(const VFRep* __restrict__ reps, const int32_t* __restric
             }
         }
         __syncthreads();
+    }
+    } else {
+    __syncthreads();
+    if (wave == 0) __builtin_amdgcn_s_setprio(3);   // the chain's wave issues first
+    float4 f1 = P0[0], d1 = dyn[0];   // wave 0: the next agent's
+    Pieces more{0, 0, 0, 0};          // wave 0: the pair (k, k - 1)'s rays, not in F
+    for (int k = 0; k < C.N; ++k) {
+        if (wave == 0) {
+            // ---- agent k's sums, as the one-wave per-replica kernel; the next
+            // agent's start pose, heading and parameters (constant over the
+            // step) load meanwhile
+            const uint32_t* Fk = F + (size_t)k * W1;
+            const float4 fp = f1, dk = d1;
+            const int k1 = min(k + 1, C.N - 1);
+            f1 = P0[k1];
+            d1 = dyn[k1];
+            const float2 u1 = U[k1];
+            const float fx = fp.x, fy = fp.y, fr = fp.z, fth = fp.w;
+            const float alp0 = dk.y, bet0 = dk.z, v0 = dk.w;
+            double Sv, Sp, Bc, Bs, Ec, Es;
+            if (halves) one_wave_sums<RPL, kSpans>(Fk, T, lane, C, want_diag, alp0, bet0, more, Sv, Sp, Bc, Bs, Ec, Es);
+            else one_wave_sums<RPL>(Fk, T, lane, C, want_diag, alp0, bet0, more, Sv, Sp, Bc, Bs, Ec, Es);
+            if (!PLAIN && bits_out) {
+                uint32_t* dst = bits_out + C.field_offset + (int64_t)k * C.W;
+                for (int w = lane; w < C.W; w += 64) dst[w] = Fk[w];
+            }
+            // ---- agent k's move, then the pair (k + 1, k) at its new pose
+            float vel, o, dv, dpsi;
+            steer(C, fth, dk.x, v0, (float)Sv, (float)Sp, &o, &vel, &dv, &dpsi);
+            float so, co;
+            sincos_f32(o, &so, &co);
+            float nx, ny;
+            euler_boundary(C, fx, fy, fr, vel, so, co, &o, &nx, &ny);
+            const float4 moved = make_float4(nx, ny, fr, o);
+            if (lane == 0) {
+                const int gk = C.a0 + k;
+                P1[k] = moved;
+                st.v[gk] = vel;
+                if (want_diag) {
+                    float* dd = diag + 6 * (int64_t)gk;
+                    dd[0] = dv; dd[1] = dpsi;
+                    dd[2] = C.phi_ok ? (float)((double)alp0 * -Bc) : 0.f;
+                    dd[3] = C.phi_ok ? (float)((double)(alp0 * C.alp1) * Ec) : 0.f;
+                    dd[4] = C.phi_ok ? (float)((double)bet0 * -Bs) : 0.f;
+                    dd[5] = C.phi_ok ? (float)((double)(bet0 * C.bet1) * Es) : 0.f;
+                }
+                if (!PLAIN && k + 1 < C.N) {
+                    if (push_culled(f1, moved, C, cull_c))
+                        push_culled_check(f1, moved, rp, count, verify, n_pairs, n_disagree);
+                    else
+                        push_pair(F + (size_t)(k + 1) * W1, u1, f1, moved, rp, C, count, verify,
+                                  n_pairs, n_recheck, n_disagree);
+                }
+            }
+            if (PLAIN) {
+                // on every lane alike: its rays go into agent k + 1's sums
+                // from registers (a pair beyond the cut-off decides to none; with
+                // few rays most are beyond it and it is tested first: 64 rays, 1000
+                // agents 1063 us against 1248, 250 rays 1474 against 1417)
+                PairF32 pr;
+                more = Pieces{0, 0, 0, 0};
+                if (!(RPL == 4 && push_culled(f1, moved, C, cull_c)) &&
+                    decide_pair(pr, u1, f1, moved, rp, C, false, false, n_pairs, n_recheck, n_disagree)) {
+                    Pieces q;
+                    vf_pieces(pr.start, pr.end, C.R, &q.a0, &q.b0, &q.a1, &q.b1);
+                    more.a0 = __builtin_amdgcn_readfirstlane(q.a0); more.b0 = __builtin_amdgcn_readfirstlane(q.b0);
+                    more.a1 = __builtin_amdgcn_readfirstlane(q.a1); more.b1 = __builtin_amdgcn_readfirstlane(q.b1);
+                }
+            }
+        } else if (k >= 1) {
+            // ---- agent k - 1's new pose into the fields of agents k + 1 ..:
+            // each wave tests its focal agents against the cut-off 64 at a
+            // time and queues the rest in a ring of 128 in LDS, deciding 64
+            // at a time
+            const float4 ob = P1[k - 1];
+            int head = 0, tail = 0;   // wave-uniform ring positions
+            for (int mb = k + 1 + (wave - 1) * 64; mb < C.N; mb += kPushThreads - 64) {
+                const int m = mb + lane;
+                bool keep = false;
+                if (m < C.N) {
+                    const float4 f = P0[m];
+                    if (!(ob.x == f.x && ob.y == f.y)) {   // coincident pairs are skipped (vf_supcalc.py:57)
+                        keep = !push_culled(f, ob, C, cull_c);
+                        if (!keep) push_culled_check(f, ob, rp, count, verify, n_pairs, n_disagree);
+                    }
+                }
+                const uint64_t mk = __ballot(keep);
+                if (keep) wq[(tail + (int)__popcll(mk & ((1ull << lane) - 1ull))) & (kPushQueue - 1)] = (uint32_t)m;
+                tail += (int)__popcll(mk);
+                wave_lds_sync();
+                if (tail - head >= 64) {
+                    const int mm = (int)wq[(head + lane) & (kPushQueue - 1)];
+                    push_pair(F + (size_t)mm * W1, U[mm], P0[mm], ob, rp, C, count, verify, n_pairs, n_recheck,
+                              n_disagree);
+                    head += 64;
+                    wave_lds_sync();
+                }
+            }
+            if (lane < tail - head) {
+                const int mm = (int)wq[(head + lane) & (kPushQueue - 1)];
+                push_pair(F + (size_t)mm * W1, U[mm], P0[mm], ob, rp, C, count, verify, n_pairs, n_recheck,
+                          n_disagree);
+            }
+        }
+        __syncthreads();
+    }
     }
     for (int i = tid; i < C.N; i += kPushThreads) {
         const int g = C.a0 + i;
@@ -1509,13 +1622,36 @@ bool push_fits_in(const abm_vf_batch* b, bool all) {
            (all ? b->max_agents : b->big_max_agents) <= kWideThreshold;
 }
 
+// Whether wave 1 sums ahead, or wave 0 sums in its turn and wave 1 pushes too.
+// Ahead shortens the chain's link, but leaves six waves to push, each lane with its
+// own agents, where seven test 64 agents at a time and decide the rest together: in
+// large replicas the pushing outlasts the link, and where few rays leave most pairs
+// beyond the cut-off there is little to decide.  us a step, ahead and in turn, one
+// replica at 1e-4 agents per unit^2: R = 512, 100 agents 118 and 122, 300 338 and 366,
+// 512 647 and 648, 600 875 and 786, 1000 1875 and 1493; R = 250, 60 agents 64 and 69,
+// 450 493 and 539; R = 128 60 and 63, 466 and 485, but 458 and 413 at a fifth of that
+// density; R = 64 61 and 55, 456 and 401.  The step with outputs holds more values per
+// pushed pair: at R = 512 300 agents 402 and 407, 450 649 and 626, at R = 250 with few
+// in sight 300 359 and 339, at R = 2000 33 agents 65 and 70, 200 424 and 421, counting,
+// 200 at R = 512 285 and 274.
+bool push_ahead(int rpl, int max_n, int max_r, bool plain, bool counts) {
+    if (plain) return max_n <= (max_r <= 128 ? 64 : 512);
+    return !counts && max_n <= (rpl == 4 ? 0 : (rpl == 32 ? 64 : 384));
+}
+
 template <int RPL>
 int launch_push(abm_vf_batch* b, const abm_vf_state_f32* st, uint32_t* bits, float* diag,
-                uint32_t flags, hipStream_t s, const int32_t* order, int n_rep, size_t lds, bool halves) {
+                uint32_t flags, hipStream_t s, const int32_t* order, int n_rep, int max_n, int max_r,
+                size_t lds, bool halves) {
     const bool plain = bits == nullptr && (flags & (ABM_WANT_DIAG | ABM_COUNT_RECHECKS | ABM_VERIFY_FAST_PATH)) == 0;
     constexpr bool kHalves = RPL > 4;   // (a lane's four rays are not halved)
-    auto kern = halves && kHalves ? (plain ? vf_step_f32_push_kernel<RPL, true, kHalves> : vf_step_f32_push_kernel<RPL, false, kHalves>)
-                                  : (plain ? vf_step_f32_push_kernel<RPL, true, false> : vf_step_f32_push_kernel<RPL, false, false>);
+    auto pick = [&](auto ahead) {
+        constexpr bool A = decltype(ahead)::value;
+        return halves && kHalves ? (plain ? vf_step_f32_push_kernel<RPL, true, kHalves, A> : vf_step_f32_push_kernel<RPL, false, kHalves, A>)
+                                 : (plain ? vf_step_f32_push_kernel<RPL, true, false, A> : vf_step_f32_push_kernel<RPL, false, false, A>);
+    };
+    const bool counts = (flags & (ABM_COUNT_RECHECKS | ABM_VERIFY_FAST_PATH)) != 0;
+    auto kern = push_ahead(RPL, max_n, max_r, plain, counts) ? pick(std::true_type{}) : pick(std::false_type{});
     if (lds > 65536) {
         if (int rc = check_hip(hipFuncSetAttribute((const void*)kern,
                                                    hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds),
@@ -1541,11 +1677,12 @@ int launch_push_any(abm_vf_batch* b, const abm_vf_state_f32* st, uint32_t* bits,
                          "abm_vf_step_f32: the push kernel holds no replica of this batch (%zu B of LDS "
                          "for its fields, device max %d; up to %d agents)", lds, b->dev_max_lds,
                          kWideThreshold);
-    const int rpl = push_rpl(all ? b->max_rays : b->big_max_rays);
-    if (rpl == 4) return launch_push<4>(b, st, bits, diag, flags, s, order, n_rep, lds, halves);
-    if (rpl == 8) return launch_push<8>(b, st, bits, diag, flags, s, order, n_rep, lds, halves);
-    if (rpl == 16) return launch_push<16>(b, st, bits, diag, flags, s, order, n_rep, lds, halves);
-    return launch_push<32>(b, st, bits, diag, flags, s, order, n_rep, lds, halves);
+    const int max_n = all ? b->max_agents : b->big_max_agents, max_r = all ? b->max_rays : b->big_max_rays;
+    const int rpl = push_rpl(max_r);
+    if (rpl == 4) return launch_push<4>(b, st, bits, diag, flags, s, order, n_rep, max_n, max_r, lds, halves);
+    if (rpl == 8) return launch_push<8>(b, st, bits, diag, flags, s, order, n_rep, max_n, max_r, lds, halves);
+    if (rpl == 16) return launch_push<16>(b, st, bits, diag, flags, s, order, n_rep, max_n, max_r, lds, halves);
+    return launch_push<32>(b, st, bits, diag, flags, s, order, n_rep, max_n, max_r, lds, halves);
 }
 
 // ---------------------------------------------------------------------------
