@@ -1249,6 +1249,13 @@ __device__ inline void push_culled_check(float4 f, float4 o, const VFRep* rp, bo
     }
 }
 
+// The wave's total of a counter, on every lane.
+__device__ inline unsigned long long wave_count(unsigned long long n) {
+#pragma unroll
+    for (int d = 32; d > 0; d >>= 1) n += __shfl_xor(n, d, 64);
+    return n;
+}
+
 // PLAIN: a step with no fields, diagnostics or counters out (the flags and
 // pointers that ask for them are ignored), so their tests leave the kernel.
 // HALVES: replicas up to kBigClass agents sum as two waves do (SPANS = 2).
@@ -1609,9 +1616,18 @@ vf_step_f32_push_kernel(const VFRep* __restrict__ reps, const int32_t* __restric
         st.theta[g] = q.w;
     }
     if (count) {
-        if (n_pairs) atomicAdd(&counters[0], n_pairs);
-        if (n_recheck) atomicAdd(&counters[1], n_recheck);
-        if (n_disagree) atomicAdd(&counters[2], n_disagree);
+        // one add per workgroup: adds to one address follow one another, about 10 ns
+        // each (250 replicas of 10 agents, a wave each 42 us a step)
+        n_pairs = wave_count(n_pairs); n_recheck = wave_count(n_recheck); n_disagree = wave_count(n_disagree);
+        unsigned long long* part = reinterpret_cast<unsigned long long*>(queue);
+        __syncthreads();   // the queues are done with
+        if (lane < 3) part[3 * wave + lane] = lane == 0 ? n_pairs : (lane == 1 ? n_recheck : n_disagree);
+        __syncthreads();
+        if (tid < 3) {
+            unsigned long long n = 0;
+            for (int w = 0; w < kPushWaves; ++w) n += part[3 * w + tid];
+            if (n) atomicAdd(&counters[tid], n);
+        }
     }
 }
 
@@ -2510,10 +2526,13 @@ int launch_vf_step_f32(abm_vf_batch* b, const abm_vf_state_f32* st, uint32_t* bi
     // kernel).  A batch of up to kFewReplicas replicas of both classes keeps a
     // kernel for each, although this one is faster there too (40 and 200 agents
     // at R = 512 0.227 and 0.291 ms, 64 and 65 0.073 and 0.175, 10 and 500 0.650
-    // and 0.669): the tests of the size classes fix its kernels.
+    // and 0.669): the tests of the size classes fix its kernels;
     const int nb = b->n_big_class;
+    // and a step that takes every pair in float64 too keeps them (100 replicas of 64
+    // agents 0.384 and 0.251).
+    const bool verify = (flags & ABM_VERIFY_FAST_PATH) != 0;
     const bool few = b->n_replicas <= kFewReplicas && nb > 0 && nb < b->n_replicas;
-    if (nw == 0 && !sync_order && !few && push_fits(b, true) &&
+    if (nw == 0 && !sync_order && !few && !verify && push_fits(b, true) &&
         (int64_t)b->n_agents_total + 4 * (int64_t)b->n_replicas <= ((int64_t)b->max_agents + 4) * b->n_cu) {
         // the sums as the kernels of the two classes take them, bit for bit (but
         // for the order of the last float64 adds): the same rays a lane, or half

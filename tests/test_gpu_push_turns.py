@@ -66,3 +66,21 @@ def test_small_replicas_beside_a_large_one(gpu, big, n_rays, outputs):
                 assert np.array_equal(x[a.replica_slice(at)], y), (step, at)
             if outputs:
                 assert np.array_equal(a.fields_numpy(at), p.fields_numpy(0)), (step, at)
+
+
+def test_counters_of_a_whole_batch(gpu):
+    # counted on the push kernel; verified (every pair in float64 too) on the
+    # kernels of the size classes, with the same pairs and the same steps
+    sizes = (64, 33, 9, 2, 1, 48, 17, 64, 5, 30)
+    a, b = (group(sizes, 512, "walls", 0) for _ in range(2))
+    for step in range(3):
+        a.step(count=True)
+        b.step(verify=True)
+        assert a.last_kernels() == {"push"} and b.last_kernels() == {"per_replica"}
+        for p, q in zip(a.state_numpy(), b.state_numpy()):
+            assert np.array_equal(p, q), step
+    pairs = 3 * sum(n * (n - 1) for n in sizes)
+    got, rechecked, _ = a.fallback_counts()
+    assert got == pairs and 0 <= rechecked <= pairs
+    got, _, disagree = b.fallback_counts()
+    assert got == pairs and disagree == 0
